@@ -14,29 +14,29 @@ def rnd(shape, seed, scale=1.0):
     return torch.randn(shape, generator=torch.Generator().manual_seed(seed)) * scale
 
 
-@pytest.mark.parametrize("per_channel", [False, True])
-@pytest.mark.parametrize("H,G,D,V,lens,slots", [
-    (2, 1, 128, 128, [65, 1, 64, 200], [3, 0, 1, 4]), (4, 2, 64, 48, [129, 0, 63], [2, 3, 0]), (3, 3, 128, 16, [70], [1]),
-    (2, 2, 64, 192, [5, 66], [-1, 2]), (1, 1, 128, 112, [400], [0])])
-@pytest.mark.parametrize("pace", [-4.0, 0.0, 6.0])
-def test_chunks_against_float64(per_channel, H, G, D, V, lens, slots, pace, monkeypatch):
-    """``pace`` moves the decays: near one, about a half a token, and down to e^-60 a token.  A token's outputs are float32
-    sums of at most D + 64 terms behind two triangular products, and decays whose logarithms carry the rounding of their
-    sum over a block of 16 tokens (2^-24 of at most 1,000 at the strongest decays, where all but the last few tokens are
-    forgotten)."""
-    ops = gpu_ops()
-    monkeypatch.setattr(ops, "_delta_chunks_pay", lambda *sizes: True)
-    T, wide = sum(lens), H * D if per_channel else H
-    qkv, gates = rnd((T, 2 * G * D + H * V), 1), rnd((T, 2 * H + 1), 2)
-    decay, a_log, dt_bias = rnd((T, wide + 3), 3) + pace, 2 * torch.rand((H,), generator=torch.Generator().manual_seed(4)), rnd((wide,), 5, 0.3)
-    before = rnd((5, 7 + H * D * V), 6, 0.3)
+def tables(lens, slots):
     cu = [0]
     for n in lens:
         cu.append(cu[-1] + n)
-    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
-    state, out = before.to(DEV), torch.empty((T, H, V), device=DEV)
-    ops.delta_rule(qkv.to(DEV), gates.to(DEV), 2, H, a_log.to(DEV), dt_bias.to(DEV), state, 7, i32(cu), i32(slots), out, H, G, D, V,
+    return cu, *(torch.tensor(v, dtype=torch.int32, device=DEV) for v in (cu, slots))
+
+
+def chunked(ops, monkeypatch, per_channel, H, G, D, V, lens, slots, qkv, gates, decay, a_log, dt_bias, before):
+    """Outputs and state of the chunk kernels, which are made to take every request and seen to run."""
+    monkeypatch.setattr(ops, "_delta_chunks_pay", lambda *sizes: True)
+    assert ops.lib.atom_delta_chunks_supports(D, V)
+    ran, kernel = [], ops.lib.atom_delta_chunks
+    monkeypatch.setattr(ops.lib, "atom_delta_chunks", lambda *a: ran.append(1) or kernel(*a))
+    _, cu, slot = tables(lens, slots)
+    state, out = before.to(DEV), torch.empty((sum(lens), H, V), device=DEV)
+    ops.delta_rule(qkv.to(DEV), gates.to(DEV), 2, H, a_log.to(DEV), dt_bias.to(DEV), state, 7, cu, slot, out, H, G, D, V,
                    decay=decay.to(DEV), per_channel=per_channel)
+    assert ran == [1]
+    return out, state
+
+
+def check(out, state, H, G, D, V, lens, slots, qkv, gates, decay, a_log, dt_bias, before, bound):
+    cu, wide = tables(lens, slots)[0], dt_bias.numel()
     unit = lambda z: z / torch.sqrt((z * z).sum(-1, keepdim=True) + 1e-6)  # noqa: E731
     for s, (n, slot) in enumerate(zip(lens, slots)):
         rows = slice(cu[s], cu[s + 1])
@@ -54,6 +54,38 @@ def test_chunks_against_float64(per_channel, H, G, D, V, lens, slots, pace, monk
                                 before[slot, 7:].double().view(H, D, V))
         for got, exact in ((out[rows], want), (state[slot, 7:].view(H, D, V), S)):
             off = float((got.double().cpu() - exact).norm() / exact.norm())
-            assert off <= (1e-6 if pace < 1 else 2e-5), off
+            assert off <= bound, off
     idle = [s for s in range(5) if s not in slots]
     assert torch.equal(state.cpu()[idle], before[idle])
+
+
+@pytest.mark.parametrize("per_channel", [False, True])
+@pytest.mark.parametrize("H,G,D,V,lens,slots", [
+    (2, 1, 128, 128, [65, 1, 64, 200], [3, 0, 1, 4]), (4, 2, 64, 48, [129, 0, 63], [2, 3, 0]), (3, 3, 128, 16, [70], [1]),
+    (2, 2, 64, 192, [5, 66], [-1, 2]), (1, 1, 128, 112, [400], [0])])
+@pytest.mark.parametrize("pace", [-4.0, 0.0, 6.0])
+def test_chunks_against_float64(per_channel, H, G, D, V, lens, slots, pace, monkeypatch):
+    """``pace`` moves the decays: near one, about a half a token, and down to e^-60 a token.  A token's outputs are float32
+    sums of at most D + 64 terms behind two triangular products."""
+    T, wide = sum(lens), H * D if per_channel else H
+    qkv, gates = rnd((T, 2 * G * D + H * V), 1), rnd((T, 2 * H + 1), 2)
+    decay, a_log, dt_bias = rnd((T, wide + 3), 3) + pace, 2 * torch.rand((H,), generator=torch.Generator().manual_seed(4)), rnd((wide,), 5, 0.3)
+    given = qkv, gates, decay, a_log, dt_bias, rnd((5, 7 + H * D * V), 6, 0.3)
+    sizes = H, G, D, V, lens, slots
+    check(*chunked(gpu_ops(), monkeypatch, per_channel, *sizes, *given), *sizes, *given, 1e-6)
+
+
+@pytest.mark.parametrize("per_channel", [False, True])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("forgets", [lambda t: t % 16 < 1, lambda t: t % 16 < 14, lambda t: t % 2 == 0, lambda t: t % 10 == 3])
+def test_chunks_forget_then_hold(per_channel, D, forgets, monkeypatch):
+    """Tokens that forget by e^-100 among tokens that keep nearly everything: the weights between those that keep are as
+    exact as where nobody forgets, however large the sum of logarithms before them."""
+    H, G, V, lens, slots = 2, 1, 32, [150, 90], [2, 0]
+    T, wide = sum(lens), H * D if per_channel else H
+    strong = torch.tensor([forgets(t) for n in lens for t in range(n)])
+    decay = torch.where(strong[:, None], 12.5, -7.0) + rnd((T, wide + 3), 3, 0.3)
+    a_log, dt_bias = torch.full((H,), 8.0).log(), rnd((wide,), 5, 0.1)
+    given = rnd((T, 2 * G * D + H * V), 1), rnd((T, 2 * H + 1), 2), decay, a_log, dt_bias, rnd((5, 7 + H * D * V), 6, 0.3)
+    sizes = H, G, D, V, lens, slots
+    check(*chunked(gpu_ops(), monkeypatch, per_channel, *sizes, *given), *sizes, *given, 1e-6)
