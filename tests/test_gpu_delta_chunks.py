@@ -89,3 +89,32 @@ def test_chunks_forget_then_hold(per_channel, D, forgets, monkeypatch):
     given = rnd((T, 2 * G * D + H * V), 1), rnd((T, 2 * H + 1), 2), decay, a_log, dt_bias, rnd((5, 7 + H * D * V), 6, 0.3)
     sizes = H, G, D, V, lens, slots
     check(*chunked(gpu_ops(), monkeypatch, per_channel, *sizes, *given), *sizes, *given, 1e-6)
+
+
+@pytest.mark.parametrize("per_channel", [False, True])
+@pytest.mark.parametrize("D,V", [(64, 48), (128, 32)])
+@pytest.mark.parametrize("what", ["q", "k", "v", "beta", "decay", "state"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+@pytest.mark.parametrize("where", [5, 64 + 21, 79])
+def test_what_is_not_finite_stays_behind_its_token(per_channel, D, V, what, value, where, monkeypatch):
+    """A NaN or an infinity in a token's input reaches that token and those behind it and nothing else: the same outputs and
+    entries of the state are finite as in the walk token by token, and those are close to it."""
+    ops = gpu_ops()
+    H, G, lens, slots = 2, 1, [150, 90], [2, 0]
+    T, wide = sum(lens), H * D if per_channel else H
+    qkv, gates, decay = rnd((T, 2 * G * D + H * V), 1), rnd((T, 2 * H + 1), 2), rnd((T, wide + 3), 3)
+    before = rnd((5, 7 + H * D * V), 6, 0.3)
+    {"q": qkv, "k": qkv, "v": qkv, "beta": gates, "decay": decay, "state": before}[what][
+        2 if what == "state" else where, {"q": 3, "k": D + 9, "v": 2 * D + V + 17, "beta": H + 1, "decay": 2 + wide // 2, "state": 7 + 5}[what]] = value
+    sizes, given = (H, G, D, V, lens, slots), (qkv, gates, decay, rnd((H,), 4, 0.3), rnd((wide,), 5, 0.3), before)
+    got = chunked(ops, monkeypatch, per_channel, *sizes, *given)
+    monkeypatch.setattr(ops, "use_delta_chunks", False)
+    _, cu, slot = tables(lens, slots)
+    state, out = before.to(DEV), torch.empty((T, H, V), device=DEV)
+    ops.delta_rule(qkv.to(DEV), gates.to(DEV), 2, H, given[3].to(DEV), given[4].to(DEV), state, 7, cu, slot, out, H, G, D, V,
+                   decay=decay.to(DEV), per_channel=per_channel)
+    assert what == "state" or bool(out[:where].isfinite().all())
+    for mine, walk in zip(got, (out, state)):
+        held = walk.isfinite()
+        assert torch.equal(mine.isfinite(), held)
+        assert float((mine[held] - walk[held]).norm()) <= 1e-6 * float(walk[held].norm())
