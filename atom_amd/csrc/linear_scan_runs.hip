@@ -11,7 +11,9 @@
 // before.
 //
 // Everything is float32; the logarithms are summed in float64 and kept as two floats, so that a difference of two of them
-// is as exact as the decays' own products are.
+// is as exact as the decays' own products are.  An infinity or a NaN of a token reaches that token and those behind it only,
+// as in the walk token by token: a wave whose 16 tokens' values hold any takes their triangle term by term, because a zero
+// above the diagonal times such a value is not zero.
 //
 // Against a walk of the runs token by token (which it replaces for these sizes): 5,569 tokens of 64 heads of 128 x 64,
 // 106 + 85 + 214 us for the three launches, 289 + 87 + 528 so.  At the smallest, 65 tokens of 32 heads, 30 us and 76.
@@ -45,7 +47,8 @@ __device__ __forceinline__ double run_times(const ScanArgs& a, RunTimes& times, 
   if (lane < n) {
     const float z = raw + a.w_bias[h];
     step = z > 20.f ? z : log1pf(expf(z));
-    c = -(double)(expf(a.a_log[h]) * step);
+    const float l = expf(a.a_log[h]) * step;
+    c = l > 110.f ? -110.0 : -(double)l;   // e^-110 is zero in float32; larger ones would take the digits of those behind
   }
 #pragma unroll
   for (int off = 1; off < kWave; off <<= 1) {
@@ -279,7 +282,16 @@ __global__ void __launch_bounds__(kReadThreads) scan_read_kernel(ScanArgs a, int
       acc[1][i] *= grown;
     }
     const float hi = times.hi[row], lo = times.lo[row];
-    for (int u = 0; u <= mt; ++u) {
+    // the diagonal tile's values hold no infinity or NaN: their products with zero are zeros
+    float zeros = 0.f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const float* v = v_rows + (16 * mt + 4 * quarter + t) * kVRow + 16 * j0 + side;
+      zeros += fmaf(v[0], 0.f, v[16] * 0.f);
+    }
+    const bool whole = __builtin_expect(__all(zeros == 0.f), 1);
+    const int tiles = whole ? mt + 1 : mt;
+    for (int u = 0; u < tiles; ++u) {
       const f32x4 g = *reinterpret_cast<const f32x4*>(scores + row * kGRow + 16 * u + 4 * quarter);
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
@@ -288,6 +300,19 @@ __global__ void __launch_bounds__(kReadThreads) scan_read_kernel(ScanArgs a, int
         const float* v = v_rows + i * kVRow + 16 * j0 + side;
         acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, v[0], acc[0], 0, 0, 0);
         acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, v[16], acc[1], 0, 0, 0);
+      }
+    }
+    if (!whole) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int t = 16 * mt + 4 * quarter + r;
+#pragma unroll 1
+        for (int i = 16 * mt; i <= t; ++i) {
+          const float x = scores[t * kGRow + i] * times.step[i] * expf((times.hi[t] - times.hi[i]) + (times.lo[t] - times.lo[i]));
+          const float* v = v_rows + i * kVRow + 16 * j0 + side;
+          acc[0][r] += x * v[0];
+          acc[1][r] += x * v[16];
+        }
       }
     }
     const float skip = a.skip != nullptr ? a.skip[h] : 0.f;

@@ -45,6 +45,7 @@ def test_runs_against_float64_and_the_walk(H, G, K, V, lens, slots, pace):
     a_log, skip = torch.log(1 + 7 * torch.rand((H,), generator=torch.Generator().manual_seed(4))), rnd((H,), 5)
     got, state = scan(ops, H, G, K, V, lens, slots, raw, bias, a_log, skip, x, odd=False)
     walked, walked_state = scan(ops, H, G, K, V, lens, slots, raw, bias, a_log, skip, x, odd=True)
+    assert not torch.equal(got, walked)      # two kernels, two orders of sums
     before = rnd((5, 7 + H * K * V), 9, 0.5).double()
     at = 0
     for n, slot in zip(lens, slots):
@@ -63,3 +64,28 @@ def test_runs_against_float64_and_the_walk(H, G, K, V, lens, slots, pace):
             assert off <= 3e-6 and off <= 2 * walk_off + 2e-7, (off, walk_off)
     idle = [s for s in range(5) if s not in slots]
     assert torch.equal(state[idle], before.float().double()[idle])
+
+
+@pytest.mark.parametrize("H,G,K,V", [(4, 2, 64, 48), (2, 1, 128, 64)])
+@pytest.mark.parametrize("what", ["v", "k", "r", "step"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), 1e30])
+@pytest.mark.parametrize("where", [5, 64 + 21, 79])
+def test_what_is_not_finite_stays_behind_its_token(H, G, K, V, what, value, where):
+    """A NaN, an infinity or a huge number in a token's input reaches that token and those behind it and nothing else: the
+    same outputs and entries of the state are finite as in the walk token by token, and each token's are close to it."""
+    ops = gpu_ops()
+    lens, slots = [150, 90], [2, 0]
+    T = sum(lens)
+    x, raw, bias = rnd((T, H * V + 2 * G * K), 1), rnd((T, H + 3), 2), rnd((H,), 3, 0.3) - 2
+    (raw if what == "step" else x)[where, {"v": V + 17, "k": H * V + 3, "r": H * V + G * K + 9, "step": 3}[what]] = value
+    a_log, skip = torch.log(1 + 7 * torch.rand((H,), generator=torch.Generator().manual_seed(4))), rnd((H,), 5)
+    mine, walk = (scan(ops, H, G, K, V, lens, slots, raw, bias, a_log, skip, x, odd=odd) for odd in (False, True))
+    assert bool(walk[0][:where].isfinite().all())
+    for got, want in zip(mine, walk):
+        held = want.isfinite()
+        assert torch.equal(got.isfinite(), held)
+        got, want = (torch.where(held, z, 0.0) for z in (got, want))
+        # a token's row (a slot's of the state): float32 sums of K + 64 terms of the size of its largest outputs; behind a huge
+        # number a row is one product r . k scaled, whose own terms cancel by up to two digits
+        bound = 1e-3 if value == 1e30 else 1e-5
+        assert bool(((got - want).norm(dim=1) <= bound * want.norm(dim=1)).all())
