@@ -17,6 +17,8 @@
 //                     to 16 adjacent lanes, so the columns never meet; q, k and the gates of a run of tokens are
 //                     staged in LDS
 //   delta_out         o / rms(o) * w * silu(gate) (or sigmoid(gate)), rounded to the serving type
+#include <climits>
+
 #include "common.h"
 
 #include <type_traits>
@@ -185,8 +187,16 @@ __device__ __forceinline__ float group_sum(float v) {
 __global__ void __launch_bounds__(256)
 delta_prepare_kernel(float* __restrict__ qkv, int channels, float* __restrict__ dec, int ld_dec, int a_off,
                      const float* __restrict__ a_log, const float* __restrict__ dt_bias, int heads, int kv_heads, int dim,
-                     int per_head, int row_parts) {
+                     int per_head, int row_parts, const int* __restrict__ cu_seqlens, int num_seqs, int below) {
   const size_t t = blockIdx.x;
+  if (below != INT_MAX) {   // a token of a request that goes in chunks is left as it is
+    int lo = 0, hi = num_seqs - 1;
+    while (lo < hi) {       // the last request that begins at t or before
+      const int mid = (lo + hi + 1) >> 1;
+      if (cu_seqlens[mid] <= (int)t) lo = mid; else hi = mid - 1;
+    }
+    if (cu_seqlens[lo + 1] - cu_seqlens[lo] >= below) return;
+  }
   if ((int)blockIdx.y < row_parts) {
     const int row = blockIdx.y * (256 / kWave) + threadIdx.x / kWave, lane = threadIdx.x % kWave;
     if (row >= 2 * kv_heads) return;
@@ -226,7 +236,7 @@ delta_rule_kernel(const float* __restrict__ qkv, int channels, const float* __re
                   int b_off,
                   float* __restrict__ state, long slot_stride, long state_off, const int* __restrict__ cu_seqlens,
                   const int* __restrict__ slot_of_seq, float* __restrict__ out, int heads, int kv_heads, int dim,
-                  int vdim) {
+                  int vdim, int below) {
   constexpr int DMAX = DPL * LPC;
   __shared__ __attribute__((aligned(16))) float qs[kRun][DMAX];
   __shared__ __attribute__((aligned(16))) float ks[kRun][DMAX];
@@ -239,6 +249,7 @@ delta_rule_kernel(const float* __restrict__ qkv, int channels, const float* __re
   const int kvh = head / (heads / kv_heads);
   const int begin = cu_seqlens[seq], end = cu_seqlens[seq + 1];
   const int slot = slot_of_seq[seq];
+  if (end - begin >= below) return;                       // atom_delta_chunks takes this request
   const bool live = col < vdim;
   if (slot < 0) {
     for (int t = begin; t < end; ++t)
@@ -375,13 +386,14 @@ delta_rule_kernel(const float* __restrict__ qkv, int channels, const float* __re
   }
 }
 
-// qkv and the decay inputs are changed in place (see delta_prepare_kernel); tokens is the number of their rows.
+// qkv and the decay inputs are changed in place (see delta_prepare_kernel); tokens is the number of their rows.  Requests of
+// `below` tokens or more are left alone, inputs, outputs and state (INT_MAX: every request is walked).
 ATOM_EXPORT int atom_delta_rule(float* qkv, int tokens, int channels, const float* ab, int ld_ab, float* dec, int ld_dec,
                                 int a_off, int b_off, int per_channel,
                                 const float* a_log, const float* dt_bias, float* state, long slot_stride,
                                 long state_off, const int* cu_seqlens, const int* slot_of_seq, int num_seqs, float* out,
-                                int heads, int kv_heads, int dim, int vdim, hipStream_t stream) {
-  if (heads <= 0 || kv_heads <= 0 || heads % kv_heads || dim <= 0 || vdim <= 0 || num_seqs < 0) return ATOM_BAD_SHAPE;
+                                int heads, int kv_heads, int dim, int vdim, int below, hipStream_t stream) {
+  if (heads <= 0 || kv_heads <= 0 || heads % kv_heads || dim <= 0 || vdim <= 0 || num_seqs < 0 || below < 1) return ATOM_BAD_SHAPE;
   if (channels != 2 * kv_heads * dim + heads * vdim) return ATOM_BAD_SHAPE;
   if (a_off < 0 || b_off < 0 || b_off + heads > ld_ab) return ATOM_BAD_SHAPE;
   if (a_off + heads * (per_channel ? dim : 1) > ld_dec) return ATOM_BAD_SHAPE;
@@ -392,7 +404,8 @@ ATOM_EXPORT int atom_delta_rule(float* qkv, int tokens, int channels, const floa
   if (num_seqs > 65535 || heads > 65535) return ATOM_TOO_LARGE;
   const int row_parts = (2 * kv_heads + 3) / 4, decays = heads * (per_channel ? dim : 1);
   hipLaunchKernelGGL(delta_prepare_kernel, dim3(tokens, row_parts + (decays + 255) / 256), dim3(256), 0, stream, qkv, channels,
-                     dec, ld_dec, a_off, a_log, dt_bias, heads, kv_heads, dim, per_channel ? dim : 1, row_parts);
+                     dec, ld_dec, a_off, a_log, dt_bias, heads, kv_heads, dim, per_channel ? dim : 1, row_parts, cu_seqlens,
+                     num_seqs, below);
   int lpc = 1;
   while (lpc * kDPL < dim) lpc *= 2;
   const bool narrow = dim > 64 && dim <= 128;   // 16 lanes of 8 entries instead of 8 lanes of 16
@@ -402,7 +415,8 @@ ATOM_EXPORT int atom_delta_rule(float* qkv, int tokens, int channels, const floa
   if (grid.z > 65535) return ATOM_TOO_LARGE;
 #define LAUNCH_AS(L, C)                                                                                          \
   hipLaunchKernelGGL((delta_rule_kernel<L, C>), grid, block, 0, stream, qkv, channels, ab, ld_ab, dec, ld_dec, a_off, \
-                     b_off, state, slot_stride, state_off, cu_seqlens, slot_of_seq, out, heads, kv_heads, dim, vdim)
+                     b_off, state, slot_stride, state_off, cu_seqlens, slot_of_seq, out, heads, kv_heads, dim, vdim, \
+                     below)
 #define LAUNCH(L)                  \
   do {                             \
     if (per_channel) {             \
@@ -415,11 +429,11 @@ ATOM_EXPORT int atom_delta_rule(float* qkv, int tokens, int channels, const floa
     if (per_channel)
       hipLaunchKernelGGL((delta_rule_kernel<16, true, 8>), grid, block, 0, stream, qkv, channels, ab, ld_ab, dec, ld_dec,
                          a_off, b_off, state, slot_stride, state_off, cu_seqlens, slot_of_seq, out, heads, kv_heads, dim,
-                         vdim);
+                         vdim, below);
     else
       hipLaunchKernelGGL((delta_rule_kernel<16, false, 8>), grid, block, 0, stream, qkv, channels, ab, ld_ab, dec, ld_dec,
                          a_off, b_off, state, slot_stride, state_off, cu_seqlens, slot_of_seq, out, heads, kv_heads, dim,
-                         vdim);
+                         vdim, below);
     return launch_status();
   }
   switch (lpc) {

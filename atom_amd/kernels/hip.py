@@ -1303,21 +1303,18 @@ class HipKernels:
             0 if activation == "silu" else 1, self._stream()))
         return out
 
-    def _delta_chunks_pay(self, tokens: int, seqs: int, heads: int, vdim: int, per_channel: bool) -> bool:
-        """Whether the delta rule takes a step in chunks.  The walk token by token costs 0.28 us a token of the longest
-        request (which has at least the mean of them), more once its blocks outnumber the chip's places; chunks cost 0.06
-        us a token and, ahead of that, a round of forming them over the CUs: 27 us with one decay per head, 52 with one per
-        key channel.  Measured with 16 heads of 128 x 128, chunks and walk: 128 tokens 36 and 43 us (channels 63 and 46),
-        300 tokens 51 and 93 (79 and 98), 2,048 tokens 185 and 577 (242 and 601), four requests of 5,571 tokens together
-        430 and 647 (596 and 741); 70 tokens 35 and 28."""
-        places = tokens // 64 + seqs
-        rounds = -(-places * heads // self.num_cus)
-        crowd = max(1.0, heads * seqs * vdim / 16 / (2 * self.num_cus))
-        return 0.25 * tokens / max(seqs, 1) * crowd > 15 + rounds * (52 if per_channel else 27)
+    # Tokens of a request's portion from which on the delta rule takes it in chunks, with one decay per head and with one per
+    # key channel.  Nothing but the request's own portion enters, so that its result does not depend on what else is in the
+    # step.  Walk and chunks, us, with 16 heads of 128 x 128: one request of 96 / 128 / 192 tokens 34 / 43 / 62 and 34 / 35 / 39,
+    # four of them 43 / 54 / 74 and 52 / 53 / 61, sixteen 143 / 185 / 266 and 137 / 140 / 214; with decays per channel one of
+    # 192 / 256 / 320 65 / 84 / 102 and 68 / 73 / 80, four 86 / 110 / 132 and 91 / 100 / 157, sixteen 304 / 396 / 488 and
+    # 340 / 389 / 533.  Heads of 64 channels gain more alone (16 heads, 256 tokens: 84 and 30) and lose where many portions fill
+    # the chip with walks (sixteen: 102 and 123).
+    DELTA_CHUNKS_FROM = {False: 128, True: 256}
 
     def delta_rule(self, qkv, gates, a_off: int, b_off: int, a_log, dt_bias, state, state_off: int, cu_seqlens_q,
                    slot_of_seq, out, heads: int, kv_heads: int, dim: int, vdim: int, decay=None,
-                   per_channel: bool = False):
+                   per_channel: bool = False, max_q_len: int | None = None, min_q_len: int = 1):
         """The gated delta recurrence over each request's tokens.  ``qkv`` float32 [tokens, 2 kv_heads dim + heads
         vdim] (q | k | v after convolution and SiLU); ``gates`` float32 [tokens, *] with the raw beta inputs at
         ``b_off`` and, unless ``decay`` (float32 [tokens, *]) holds them, the raw decay inputs at ``a_off``: one
@@ -1326,8 +1323,9 @@ class HipKernels:
         vdim].  ``qkv`` and the decay inputs are used up: q and k are made unit vectors and the raw decay inputs
         become the decays, in place, for all tokens side by side before the recurrence walks them.
 
-        Steps with prompts take chunks of 64 tokens as matrix products (heads of 64 or 128 key channels) where
-        ``_delta_chunks_pay``; the inputs are then left as they are."""
+        Requests that bring ``DELTA_CHUNKS_FROM`` tokens or more take chunks of 64 tokens as matrix products (heads of 64 or
+        128 key channels); their inputs are left as they are.  ``max_q_len`` and ``min_q_len``: the most and the fewest tokens
+        a request brings, or bounds of them (default: all tokens, and one), which say what need not be launched."""
         tokens, channels = qkv.shape
         seqs = slot_of_seq.numel()
         decay = gates if decay is None else decay
@@ -1343,8 +1341,10 @@ class HipKernels:
         self._check("cu_seqlens_q", cu_seqlens_q, torch.int32, (seqs + 1,))
         self._check("slot_of_seq", slot_of_seq, torch.int32, (seqs,))
         self._check("delta out", out, torch.float32, (tokens, heads, vdim))
-        if (self.use_delta_chunks and tokens > seqs and self.lib.atom_delta_chunks_supports(dim, vdim)
-                and self._delta_chunks_pay(tokens, seqs, heads, vdim, per_channel)):
+        least, longest = self.DELTA_CHUNKS_FROM[bool(per_channel)], tokens if max_q_len is None else min(tokens, max_q_len)
+        if not (self.use_delta_chunks and longest >= least and self.lib.atom_delta_chunks_supports(dim, vdim)):
+            least = 2 ** 31 - 1                     # no request goes in chunks
+        else:
             places = tokens // 64 + seqs
             scratch = torch.empty((places, self.lib.atom_delta_chunks_floats(heads, dim, vdim)), dtype=torch.float32,
                                   device=qkv.device)
@@ -1352,13 +1352,14 @@ class HipKernels:
                 _ptr(qkv), tokens, channels, _ptr(gates), gates.shape[1], _ptr(decay), decay.shape[1], a_off, b_off,
                 int(bool(per_channel)), _ptr(a_log), _ptr(dt_bias), _ptr(state),
                 ctypes.c_long(state.shape[1]), ctypes.c_long(state_off), _ptr(cu_seqlens_q), _ptr(slot_of_seq), seqs,
-                _ptr(out), heads, kv_heads, dim, vdim, _ptr(scratch), places, self._stream()))
-            return out
+                _ptr(out), heads, kv_heads, dim, vdim, least, _ptr(scratch), places, self._stream()))
+            if min_q_len >= least:
+                return out
         self._done("delta_rule", self.lib.atom_delta_rule(
             _ptr(qkv), tokens, channels, _ptr(gates), gates.shape[1], _ptr(decay), decay.shape[1], a_off, b_off,
             int(bool(per_channel)), _ptr(a_log), _ptr(dt_bias), _ptr(state),
             ctypes.c_long(state.shape[1]), ctypes.c_long(state_off), _ptr(cu_seqlens_q), _ptr(slot_of_seq), seqs,
-            _ptr(out), heads, kv_heads, dim, vdim, self._stream()))
+            _ptr(out), heads, kv_heads, dim, vdim, least, self._stream()))
         return out
 
     def delta_out(self, o, gates, gate_off: int, weight, eps: float, out, activation: str = "silu"):

@@ -373,7 +373,7 @@ class PlainKernels:
         return out
 
     def delta_rule(self, qkv, gates, a_off, b_off, a_log, dt_bias, state, state_off, cu_seqlens_q, slot_of_seq, out,
-                   heads, kv_heads, dim, vdim, decay=None, per_channel=False):
+                   heads, kv_heads, dim, vdim, decay=None, per_channel=False, max_q_len=None, min_q_len=1):
         if per_channel:
             return self._delta_rule_channels(qkv, gates, a_off, b_off, a_log, dt_bias, state, state_off, cu_seqlens_q,
                                              slot_of_seq, out, heads, kv_heads, dim, vdim,

@@ -23,7 +23,7 @@ def tables(lens, slots):
 
 def chunked(ops, monkeypatch, per_channel, H, G, D, V, lens, slots, qkv, gates, decay, a_log, dt_bias, before):
     """Outputs and state of the chunk kernels, which are made to take every request and seen to run."""
-    monkeypatch.setattr(ops, "_delta_chunks_pay", lambda *sizes: True)
+    monkeypatch.setattr(ops, "DELTA_CHUNKS_FROM", {False: 1, True: 1})
     assert ops.lib.atom_delta_chunks_supports(D, V)
     ran, kernel = [], ops.lib.atom_delta_chunks
     monkeypatch.setattr(ops.lib, "atom_delta_chunks", lambda *a: ran.append(1) or kernel(*a))
@@ -118,3 +118,53 @@ def test_what_is_not_finite_stays_behind_its_token(per_channel, D, V, what, valu
         held = walk.isfinite()
         assert torch.equal(mine.isfinite(), held)
         assert float((mine[held] - walk[held]).norm()) <= 1e-6 * float(walk[held].norm())
+
+
+@pytest.mark.parametrize("per_channel", [False, True])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("step", [0, -1, 1, 200])
+@pytest.mark.parametrize("others", [[1] * 24, [500], [1, 127, 128, 255, 256, 3]])
+def test_a_request_is_worked_alike_alone_and_beside_others(per_channel, D, step, others):
+    """Walk or chunks is a matter of a request's own tokens: around the number where one gives way to the other, outputs
+    and state have the same bits alone and in steps with single tokens, shorter and longer portions."""
+    ops = gpu_ops()
+    n = ops.DELTA_CHUNKS_FROM[per_channel] + step
+    H, G, V = 2, 1, 32
+    for lens in ([n] + others, others + [n]):
+        at, place, T = sum(lens[:lens.index(n)]), lens.index(n), sum(lens)
+        wide = H * D if per_channel else H
+        qkv, gates, decay = rnd((T, 2 * G * D + H * V), 1), rnd((T, 2 * H + 1), 2), rnd((T, wide + 3), 3)
+        a_log, dt_bias = rnd((H,), 4, 0.3).to(DEV), rnd((wide,), 5, 0.3).to(DEV)
+        got = []
+        for rows, some in ((slice(0, T), lens), (slice(at, at + n), [n])):
+            _, cu, slots = tables(some, list(range(len(some))) if len(some) > 1 else [place])
+            state = rnd((len(lens), 7 + H * D * V), 6, 0.3).to(DEV)
+            out = torch.empty((sum(some), H, V), device=DEV)
+            ops.delta_rule(qkv[rows].contiguous().to(DEV), gates[rows].contiguous().to(DEV), 2, H, a_log, dt_bias, state, 7, cu,
+                           slots, out, H, G, D, V, decay=decay[rows].contiguous().to(DEV), per_channel=per_channel,
+                           max_q_len=max(some), min_q_len=min(some))
+            got.append((out if len(some) == 1 else out[at:at + n], state[place]))
+        for whole, alone in zip(*got):
+            assert torch.equal(whole, alone)
+
+
+@pytest.mark.parametrize("per_channel", [False, True])
+def test_chunks_begin_where_they_are_said_to(per_channel, monkeypatch):
+    """Which kernels a step launches: by the longest and the shortest request, whatever the number of either."""
+    ops = gpu_ops()
+    least = ops.DELTA_CHUNKS_FROM[per_channel]
+    H, G, D, V = 2, 1, 64, 16
+    ran = []
+    for name in ("atom_delta_chunks", "atom_delta_rule"):
+        monkeypatch.setattr(ops.lib, name, lambda *a, name=name, kernel=getattr(ops.lib, name): ran.append(name) or kernel(*a))
+    for lens, want in (([least], ["atom_delta_chunks"]), ([least - 1] * 3, ["atom_delta_rule"]), ([1] * 40, ["atom_delta_rule"]),
+                       ([least, 2 * least], ["atom_delta_chunks"]), ([1] * 40 + [least], ["atom_delta_chunks", "atom_delta_rule"])):
+        T, wide = sum(lens), H * D if per_channel else H
+        _, cu, slots = tables(lens, list(range(len(lens))))
+        state, out = torch.zeros((len(lens), H * D * V), device=DEV), torch.empty((T, H, V), device=DEV)
+        ran.clear()
+        ops.delta_rule(rnd((T, 2 * G * D + H * V), 1).to(DEV), rnd((T, H), 2).to(DEV), 0, 0, rnd((H,), 4).to(DEV),
+                       rnd((wide,), 5).to(DEV), state, 0, cu, slots, out, H, G, D, V, decay=rnd((T, wide), 3).to(DEV),
+                       per_channel=per_channel, max_q_len=max(lens), min_q_len=min(lens))
+        assert ran == want
+        assert bool(out.isfinite().all())
