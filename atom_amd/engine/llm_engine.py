@@ -121,7 +121,7 @@ class LLMEngine:
 
     def _cache_budget(self) -> int:
         """Bytes for the cache: the share of device memory ``gpu_memory_utilization`` allows minus what is
-        in use, minus what the decode graphs will take and a 2 % margin
+        in use, minus what the decode graphs and the largest scratch memory of a part will take and a 2 % margin
         (atom/model_engine/model_runner.py:1591-1611, 1737-1749)."""
         dev = torch.device(self.config.device)
         if dev.type != "cuda":
@@ -129,11 +129,14 @@ class LLMEngine:
         free, total = torch.cuda.mem_get_info(dev)
         used = total - free
         graphs = 0 if self.config.enforce_eager else self._graph_estimate()
+        scratch = max((part.scratch_bytes(self.ops, self.config.max_num_batched_tokens, self.config.max_num_seqs)
+                       for block in self.model.blocks for part in block.walk()), default=0)
         safety = int(total * 0.02)
-        budget = max(0, min(int(total * self.config.gpu_memory_utilization) - used - graphs - safety, free))
+        budget = max(0, min(int(total * self.config.gpu_memory_utilization) - used - graphs - scratch - safety, free))
         logger.info("Memory budget: total_gpu=%.2fGB, free=%.2fGB, utilization=%s, in_use=%.2fGB, "
-                    "cudagraph_est=%.2fGB, safety=%.2fGB, available_for_kv=%.2fGB", total / 2**30, free / 2**30,
-                    self.config.gpu_memory_utilization, used / 2**30, graphs / 2**30, safety / 2**30, budget / 2**30)
+                    "cudagraph_est=%.2fGB, scratch=%.2fGB, safety=%.2fGB, available_for_kv=%.2fGB", total / 2**30, free / 2**30,
+                    self.config.gpu_memory_utilization, used / 2**30, graphs / 2**30, scratch / 2**30, safety / 2**30,
+                    budget / 2**30)
         return budget
 
     def _graph_estimate(self) -> int:

@@ -1311,6 +1311,18 @@ class HipKernels:
     # 340 / 389 / 533.  Heads of 64 channels gain more alone (16 heads, 256 tokens: 84 and 30) and lose where many portions fill
     # the chip with walks (sixteen: 102 and 123).
     DELTA_CHUNKS_FROM = {False: 128, True: 256}
+    # The most scratch memory the chunks of a step take; what is beyond it is worked afterwards in the same memory (14,000
+    # tokens of 32 heads of 128 x 128 fit).
+    DELTA_SCRATCH_BYTES = 1 << 30
+
+    def delta_scratch(self, tokens: int, seqs: int, heads: int, dim: int, vdim: int, per_channel: bool) -> tuple[int, int]:
+        """Places (64 tokens of a request, or what is left of it) and floats a place of the scratch memory that a step of
+        ``tokens`` tokens takes the delta rule's chunks through; (0, 0) where none of its requests can go in chunks."""
+        if not (self.use_delta_chunks and tokens >= self.DELTA_CHUNKS_FROM[per_channel]
+                and self.lib.atom_delta_chunks_supports(dim, vdim)):
+            return 0, 0
+        floats = self.lib.atom_delta_chunks_floats(heads, dim, vdim)
+        return min(tokens // 64 + seqs, max(1, self.DELTA_SCRATCH_BYTES // (4 * floats))), floats
 
     def delta_rule(self, qkv, gates, a_off: int, b_off: int, a_log, dt_bias, state, state_off: int, cu_seqlens_q,
                    slot_of_seq, out, heads: int, kv_heads: int, dim: int, vdim: int, decay=None,
@@ -1341,18 +1353,17 @@ class HipKernels:
         self._check("cu_seqlens_q", cu_seqlens_q, torch.int32, (seqs + 1,))
         self._check("slot_of_seq", slot_of_seq, torch.int32, (seqs,))
         self._check("delta out", out, torch.float32, (tokens, heads, vdim))
-        least, longest = self.DELTA_CHUNKS_FROM[bool(per_channel)], tokens if max_q_len is None else min(tokens, max_q_len)
-        if not (self.use_delta_chunks and longest >= least and self.lib.atom_delta_chunks_supports(dim, vdim)):
-            least = 2 ** 31 - 1                     # no request goes in chunks
-        else:
-            places = tokens // 64 + seqs
-            scratch = torch.empty((places, self.lib.atom_delta_chunks_floats(heads, dim, vdim)), dtype=torch.float32,
-                                  device=qkv.device)
+        least, room = 2 ** 31 - 1, 0                # no request goes in chunks
+        if max_q_len is None or max_q_len >= self.DELTA_CHUNKS_FROM[bool(per_channel)]:
+            room, floats = self.delta_scratch(tokens, seqs, heads, dim, vdim, bool(per_channel))
+        if room:
+            least = self.DELTA_CHUNKS_FROM[bool(per_channel)]
+            scratch = torch.empty((room, floats), dtype=torch.float32, device=qkv.device)
             self._done("delta_chunks", self.lib.atom_delta_chunks(
                 _ptr(qkv), tokens, channels, _ptr(gates), gates.shape[1], _ptr(decay), decay.shape[1], a_off, b_off,
                 int(bool(per_channel)), _ptr(a_log), _ptr(dt_bias), _ptr(state),
                 ctypes.c_long(state.shape[1]), ctypes.c_long(state_off), _ptr(cu_seqlens_q), _ptr(slot_of_seq), seqs,
-                _ptr(out), heads, kv_heads, dim, vdim, least, _ptr(scratch), places, self._stream()))
+                _ptr(out), heads, kv_heads, dim, vdim, least, _ptr(scratch), room, self._stream()))
             if min_q_len >= least:
                 return out
         self._done("delta_rule", self.lib.atom_delta_rule(

@@ -90,6 +90,10 @@ class Part:
         for child in self.children():
             yield from child.walk()
 
+    def scratch_bytes(self, ops, tokens: int, seqs: int) -> int:
+        """Device memory that a step of ``tokens`` tokens of ``seqs`` requests takes in this part beside the activations."""
+        return 0
+
     def full_name(self, local: str) -> str:
         """The checkpoint name of ``local`` under this part's prefix; an empty ``local`` names the prefix itself
         (a checkpoint that calls a norm's weight ``l0.norm1`` and its bias ``l0.norm1.b``)."""

@@ -64,6 +64,12 @@ class GatedDeltaRule(Mixer):
     def cache_need(self):
         return StateNeed((self.conv_floats + self.num_heads * self.head_dim * self.value_dim,), torch.float32)
 
+    def scratch_bytes(self, ops, tokens, seqs):
+        if not hasattr(ops, "delta_scratch"):
+            return 0
+        places, floats = ops.delta_scratch(tokens, seqs, self.num_heads, self.head_dim, self.value_dim, self.decay == "channel")
+        return 4 * places * floats
+
     @property
     def decay_width(self) -> int:
         return self.num_heads * (self.head_dim if self.decay == "channel" else 1)

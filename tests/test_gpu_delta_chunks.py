@@ -168,3 +168,25 @@ def test_chunks_begin_where_they_are_said_to(per_channel, monkeypatch):
                        per_channel=per_channel, max_q_len=max(lens), min_q_len=min(lens))
         assert ran == want
         assert bool(out.isfinite().all())
+
+
+@pytest.mark.parametrize("per_channel", [False, True])
+@pytest.mark.parametrize("room", [1, 2, 5, 9, 1000])
+def test_bounded_scratch_memory(per_channel, room, monkeypatch):
+    """Places beyond the scratch memory's bound are worked afterwards in the same memory, with the same bits, wherever the
+    bound cuts a request."""
+    ops = gpu_ops()
+    H, G, D, V, lens, slots = 2, 1, 64, 48, [300, 0, 64, 65, 511, 1], [0, 4, 2, -1, 3, 1]
+    T, wide = sum(lens), H * D if per_channel else H
+    given = (rnd((T, 2 * G * D + H * V), 1), rnd((T, 2 * H + 1), 2), rnd((T, wide + 3), 3), rnd((H,), 4, 0.3), rnd((wide,), 5, 0.3),
+             rnd((5, 7 + H * D * V), 6, 0.3))
+    whole = chunked(ops, monkeypatch, per_channel, H, G, D, V, lens, slots, *given)
+    monkeypatch.undo()
+    place = 4 * ops.lib.atom_delta_chunks_floats(H, D, V)
+    monkeypatch.setattr(ops, "DELTA_SCRATCH_BYTES", room * place + 4, raising=False)
+    taken, empty = [], torch.empty
+    monkeypatch.setattr(torch, "empty", lambda *a, **k: taken.append(empty(*a, **k)) or taken[-1])
+    cut = chunked(ops, monkeypatch, per_channel, H, G, D, V, lens, slots, *given)
+    assert max(t.numel() * 4 for t in taken if t.shape[-1] * 4 == place) <= room * place
+    for a, b in zip(whole, cut):
+        assert torch.equal(a, b)
