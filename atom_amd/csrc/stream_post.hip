@@ -194,9 +194,11 @@ ATOM_EXPORT int atom_rmsnorm_rows(const float* x, const float* weight, float eps
 
 // stream[r] = (init ? 0 : stream[r]) + x[r] for float32 rows, and out[r] = norm(stream[r]) * weight in out's type: a
 // float32 summand (an embedding's output) starts the stream or joins it, and the stream is normed for the sublayer
-// that reads it next.  A block a row, the row's sum kept in LDS between the two walks.
+// that reads it next.  A block a row, the row's sum kept in LDS between the two walks.  256 threads whatever the number of
+// rows, so that a row's sum of squares has one order; the eight entries a thread asks for together are what a launch of few
+// rows is spent on.
 template <typename TO>
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__(256)
 stream_norm_kernel(float* __restrict__ stream, const float* __restrict__ x, const float* __restrict__ weight, float eps,
                    TO* __restrict__ out, int width, int init) {
   extern __shared__ float smem[];
@@ -206,8 +208,8 @@ stream_norm_kernel(float* __restrict__ stream, const float* __restrict__ x, cons
   float* sr = stream + r * width;
   const float* xr = x + r * width;
   float ss = 0.f;
-#pragma unroll 4
-  for (int i = threadIdx.x; i < width; i += blockDim.x) {
+#pragma unroll 8
+  for (int i = threadIdx.x; i < width; i += 256) {
     const float v = init ? xr[i] : sr[i] + xr[i];
     sr[i] = v;
     vals[i] = v;
@@ -215,8 +217,8 @@ stream_norm_kernel(float* __restrict__ stream, const float* __restrict__ x, cons
   }
   ss = block_sum(ss, scratch);
   const float inv = 1.f / sqrtf(ss / (float)width + eps);
-#pragma unroll 4
-  for (int i = threadIdx.x; i < width; i += blockDim.x) out[r * width + i] = from_f32<TO>(vals[i] * inv * weight[i]);
+#pragma unroll 8
+  for (int i = threadIdx.x; i < width; i += 256) out[r * width + i] = from_f32<TO>(vals[i] * inv * weight[i]);
 }
 
 ATOM_EXPORT int atom_stream_norm(float* stream_rows, const float* x, const float* weight, float eps, void* out, int out_dtype,
@@ -225,8 +227,7 @@ ATOM_EXPORT int atom_stream_norm(float* stream_rows, const float* x, const float
   if (width > 32768) return ATOM_TOO_LARGE;
   if (num_rows == 0) return ATOM_OK;
   const size_t smem = (size_t)(width + 16) * sizeof(float);
-  const int threads = num_rows < device_cus() && width >= 1024 ? 1024 : 256;   // few rows: shorter walks
-  ATOM_DISPATCH_DTYPE(out_dtype, hipLaunchKernelGGL((stream_norm_kernel<T>), dim3(num_rows), dim3(threads), smem, stream,
+  ATOM_DISPATCH_DTYPE(out_dtype, hipLaunchKernelGGL((stream_norm_kernel<T>), dim3(num_rows), dim3(256), smem, stream,
                                                      stream_rows, x, weight, eps, (T*)out, width, init));
   return launch_status();
 }

@@ -116,3 +116,19 @@ def test_float32_gate_in_the_product(m, inter, k, biased, wdtype):
     ops.silu_mul(ops.linear(x, w, b), want)
     assert act.shape == (m, inter) and act.dtype == torch.float32
     assert torch.equal(act, want)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width", [53, 1024, 2050, 4096])
+@pytest.mark.parametrize("init", [True, False])
+def test_stream_norm_rows_do_not_depend_on_batch(dtype, width, init):
+    """A row alone, among a few and among more than there are compute units: the same bits."""
+    ops = gpu_ops()
+    stream, x, w = rnd((600, width), 1).to(DEV), rnd((600, width), 2).to(DEV), (1 + rnd((width,), 3, 0.2)).to(DEV)
+    got = []
+    for rows in (slice(0, 600), slice(7, 12), slice(9, 10)):
+        s, out = stream[rows].clone(), torch.empty((len(stream[rows]), width), dtype=dtype, device=DEV)
+        ops.stream_norm(s, x[rows].contiguous(), w, 2e-5, out, init=init)
+        got.append((s, out))
+    for mine, few, alone in zip(*got):
+        assert torch.equal(mine[7:12], few) and torch.equal(mine[9:10], alone)
