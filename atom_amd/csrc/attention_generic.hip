@@ -50,7 +50,7 @@ paged_attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ k_
                                const int* __restrict__ block_tables, int max_blocks, int hq, int hkv,
                                int d, int page_size, float scale, int window, int chunk, float softcap,
                                const float* __restrict__ sink, const float* __restrict__ slopes,
-                               const float* __restrict__ gate, long gate_ld, int od) {
+                               const float* __restrict__ gate, long gate_ld, int od, int key_fours, int value_fours) {
   extern __shared__ __align__(16) float smem[];
   float* qs = smem;                  // d
   float* probs = qs + (d + 3) / 4 * 4;   // kAttnChunk
@@ -100,7 +100,7 @@ paged_attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ k_
       const int off = key % page_size;
       const T* kr = k_cache + (((size_t)page * hkv + kvh) * page_size + off) * (size_t)d;
       float s = 0.f;
-      if (d % 4 == 0) {   // rows of four-element pieces: a piece a load
+      if (key_fours) {   // rows of four-element pieces: a piece a load
 #pragma unroll 8
         for (int i = 0; i < d; i += 4) {
           const Four<T> four = *reinterpret_cast<const Four<T>*>(kr + i);
@@ -146,7 +146,7 @@ paged_attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ k_
           const T* vr = v_cache + (((size_t)table[key / page_size] * hkv + kvh) * d + entry) * (size_t)page_size + off;
           const float* pr = probs + (key - lo);
           int j = 0;
-          if (page_size % 4 == 0 && off % 4 == 0) {
+          if (value_fours && off % 4 == 0) {
             for (; j + 4 <= here; j += 4) {
               const Four<T> four = *reinterpret_cast<const Four<T>*>(vr + j);
 #pragma unroll
@@ -187,11 +187,16 @@ ATOM_EXPORT int atom_paged_attention_generic(const void* q, const void* k_cache,
   if (tokens == 0) return ATOM_OK;
   const size_t smem = (size_t)((d + 3) / 4 * 4 + kAttnChunk + 16 + kAttnItems) * sizeof(float);
   const dim3 grid(tokens, hq);
+  // four keys' entries, or an entry of four keys, a load where they begin at multiples of their size in memory
+  const size_t four = dtype == ATOM_F32 ? 16 : 8;
+  const int key_fours = d % 4 == 0 && (uintptr_t)k_cache % four == 0;
+  const int value_fours = page_size % 4 == 0 && (uintptr_t)v_cache % four == 0;
 #define LAUNCH(PER)                                                                                                  \
   ATOM_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((paged_attention_generic_kernel<T, PER>), grid, dim3(kAttnItems / PER), smem, \
                                                  stream, (const T*)q, (const T*)k_cache, (const T*)v_cache, (T*)out,  \
                                                  token_seq, positions, block_tables, max_blocks, hq, hkv, d, page_size, \
-                                                 scale, window, chunk, softcap, sink, slopes, gate, gate_ld, od))
+                                                 scale, window, chunk, softcap, sink, slopes, gate, gate_ld, od, key_fours, \
+                                                 value_fours))
   if ((long)tokens * hq <= kAttnFew) LAUNCH(1);
   else LAUNCH(4);
 #undef LAUNCH

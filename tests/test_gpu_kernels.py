@@ -316,6 +316,26 @@ def test_general_attention_with_few_and_many_blocks(hq, d, page, window):
     close(outs[0], want, torch.float32)
 
 
+@pytest.mark.parametrize("dtype,d,page", [(torch.float32, 128, 16), (torch.float32, 20, 4), (torch.bfloat16, 100, 12)])
+@pytest.mark.parametrize("shift_k,shift_v", [(1, 0), (0, 1), (2, 3), (4, 4)])
+def test_general_attention_over_pages_that_begin_anywhere(dtype, d, page, shift_k, shift_v):
+    """A cache that is a view into the middle of a buffer: loads of four elements only where they are aligned, and the same
+    bits either way, because the order of the sums does not change."""
+    q, kc, vc, meta = _attention_case(dtype, 9, 3, d, page, None, [3, 1], [200, 77], seed=d)
+
+    def at(t, shift):
+        buffer = torch.zeros(t.numel() + shift, dtype=dtype, device=DEV)
+        buffer[shift:] = t.to(DEV).view(-1)
+        return buffer[shift:].view(t.shape)
+
+    outs = []
+    for k, v in ((kc.to(DEV), vc.to(DEV)), (at(kc, shift_k), at(vc, shift_v))):
+        out = torch.empty_like(q, device=DEV)
+        gpu_ops().paged_attention(q.to(DEV), k, v, out, meta(DEV), d ** -0.5, None)
+        outs.append(out)
+    assert torch.equal(*outs)
+
+
 TILED_SHAPES = [  # hq, hkv, d, page: groups of 4, 2, 1, 3 and 8; pages of 8, 16, 32 and 64 keys
     (8, 2, 64, 16), (32, 8, 128, 16), (6, 3, 128, 8), (5, 5, 64, 32), (3, 1, 256, 8), (16, 2, 192, 64),
 ]
