@@ -177,7 +177,7 @@ template <typename T, int ACC, int TH>
 __global__ void __launch_bounds__(TH)
 attention_together_kernel(const T* __restrict__ q, const T* __restrict__ k_cache, const T* __restrict__ v_cache,
                           T* __restrict__ out, TogetherArgs a) {
-  extern __shared__ float lds[];
+  extern __shared__ __align__(16) float lds[];
   const int t = blockIdx.x;
   const int HB = a.talk != nullptr ? a.H : a.H / a.G;   // heads of this block
   const int h0 = a.talk != nullptr ? 0 : blockIdx.y * HB;
@@ -278,7 +278,7 @@ template <typename T, int PASS, int ACC, int TH>
 __global__ void __launch_bounds__(TH)
 attention_together_part_kernel(const T* __restrict__ q, const T* __restrict__ k_cache, const T* __restrict__ v_cache,
                                TogetherArgs a) {
-  extern __shared__ float lds[];
+  extern __shared__ __align__(16) float lds[];
   const int t = blockIdx.x, part = blockIdx.z;
   const int HB = a.talk != nullptr ? a.H : a.H / a.G;
   const int h0 = a.talk != nullptr ? 0 : blockIdx.y * HB;
