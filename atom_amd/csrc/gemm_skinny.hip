@@ -566,7 +566,10 @@ static SkinnyPlan skinny_plan(int m, int tiles, int k) {
 // A round more costs as much as 16 rows x 2,048 of K: with a quarter of that, slices were cut finer than their starts are worth
 // (64 and 16 rows of x: 10,240 x 5,120 33 and 23 us in five slices and two rounds, 29 and 22 in two slices and one;
 // 20,992 x 4,096 50 and 36 in four, 38 and 31 whole; 39,936 x 8,192 162 and 140, 128 and 103; with half of it 33,792 x 3,072 66
-// and 45 in three, 55 and 40 whole; 12,288 x 2,560 25.5 and 17.4 in three, 22.6 and 17.0 in two).
+// and 45 in three, 55 and 40 whole; 12,288 x 2,560 25.5 and 17.4 in three, 22.6 and 17.0 in two).  With 65 rows or more, where
+// the plan says whether this kernel takes the product at all, a round costs that quarter: plans that the larger figure turns into
+// one round of four waves are slower than the BLAS library (14,592 x 5,120 at 65 and 128 rows 62 and 67 us, 36 and 43 there;
+// 15,360 x 9,216 102 and 112, 66 and 71).
 struct MidPlan {
   int waves, tiles, splits, kslice;
 };
@@ -582,6 +585,7 @@ static MidPlan mid_plan(int m, int groups, int k, int gate) {
     plan.kslice = units * kMidSlice;
     return plan;
   }
+  const double round_cost = m > 64 ? 0.5 : 2.0;
   double best = 1e30;
   for (int s = 1; s <= min(units, 32); ++s) {
     const int per = (units + s - 1) / s;
@@ -590,7 +594,7 @@ static MidPlan mid_plan(int m, int groups, int k, int gate) {
     for (int w = 8; w >= 4; --w) {
       const long tiles = (groups + w - 1) / w;
       const long rounds = (tiles * splits + cus - 1) / cus;
-      const double cost = (double)rounds * w * per * (1. + 1. / w) + 2.0 * rounds + 0.15 * splits * groups / (double)cus;
+      const double cost = (double)rounds * w * per * (1. + 1. / w) + round_cost * rounds + 0.15 * splits * groups / (double)cus;
       if (cost < best - 1e-9) {
         best = cost;
         plan.waves = w;

@@ -700,6 +700,18 @@ def test_skinny_gemm_very_wide(n, k, all_rows):
         assert torch.equal(y, full[:m])
 
 
+def test_which_products_of_65_to_128_rows_are_streamed():
+    """Products whose blocks of four waves fill one round only because a second one is dear go to the library, as they are
+    faster there; those that are streamed have the slices they have at 64 rows."""
+    ops = gpu_ops()
+    for n, k in ((14592, 4608), (14592, 5120), (14848, 9216), (15360, 8704), (16128, 9216)):
+        assert not any(ops.lib.atom_gemm_skinny_supports(m, n, k) for m in (65, 100, 128)), (n, k)
+    streamed = [(n, k) for n in range(512, 24577, 512) for k in range(512, 16385, 512) if ops.lib.atom_gemm_skinny_supports(100, n, k)]
+    assert len(streamed) > 100
+    for n, k in streamed:
+        assert ops.lib.atom_gemm_skinny_splits(100, n, k, 0) == ops.lib.atom_gemm_skinny_splits(64, n, k, 0), (n, k)
+
+
 @pytest.mark.parametrize("m,n,k", [(65, 4096, 4096), (96, 2560, 9728), (128, 6144, 2560), (200, 130, 12288),
                                    (256, 5120, 5120), (129, 517, 1024), (255, 4096, 12288), (70, 7, 64),
                                    (100, 1031, 192), (256, 8192, 576)])
