@@ -555,10 +555,12 @@ static SkinnyPlan skinny_plan(int m, int tiles, int k) {
 
 // More than 16 rows.  `groups` is the number of 16-row groups of w (8 columns each for SiLU-gate).
 // Blocks of 5 to 8 waves run one a CU, blocks of 4 waves two.  Very wide products (three rounds of
-// blocks or more whatever the choice) take K whole, and four waves up to 16 rows of x: with two blocks a CU one block's
-// start and end overlap another's work.  From 17 rows on, where reading x for every block weighs more than that, plain ones
-// take eight: the head of 151,936 columns with four and with eight, us: K 4,096 at 64 / 32 / 16 rows 280 / 219 / 200 and
-// 257 / 220 / 197, K 5,120 359 / 302 / 257 and 319 / 288 / 257, K 2,560 188 / 154 / 130 and 178 / 154 / 140.
+// blocks or more whatever the choice) take K whole and four waves: with two blocks a CU one block's start and end overlap
+// another's work.  Reading x for every block weighs more than that only with many rows, a long K and, below 49 rows, many
+// columns; there plain ones take eight.  Four and eight waves, us, at 17 / 33 / 48 / 64 rows: 66,000 x 1,024 27 / 30 / 33 / 36 and
+// 37 / 40 / 42 / 45, 151,936 x 2,048 101 / 114 / 125 / 139 and 109 / 120 / 128 / 133, 100,000 x 3,072 102 / 117 / 126 / 140 and
+// 117 / 127 / 133 / 141, 100,000 x 4,096 130 / 144 / 155 / 173 and 145 / 157 / 163 / 171, 151,936 x 4,096 189 / 207 / 223 / 252 and
+// 189 / 206 / 218 / 229, 262,144 x 8,192 671 / 698 / 741 / 780 and 665 / 700 / 700 / 695.
 // For the others the number of waves and of K slices (multiples
 // of 1024) is the one with the least work on the busiest CU: rounds of a block a CU x rows x k a block,
 // a little more for fewer waves (x is read once per block), for every round (a block's start and end)
@@ -566,7 +568,9 @@ static SkinnyPlan skinny_plan(int m, int tiles, int k) {
 // A round more costs as much as 16 rows x 2,048 of K: with a quarter of that, slices were cut finer than their starts are worth
 // (64 and 16 rows of x: 10,240 x 5,120 33 and 23 us in five slices and two rounds, 29 and 22 in two slices and one;
 // 20,992 x 4,096 50 and 36 in four, 38 and 31 whole; 39,936 x 8,192 162 and 140, 128 and 103; with half of it 33,792 x 3,072 66
-// and 45 in three, 55 and 40 whole; 12,288 x 2,560 25.5 and 17.4 in three, 22.6 and 17.0 in two).  With 65 rows or more, where
+// and 45 in three, 55 and 40 whole; 12,288 x 2,560 25.5 and 17.4 in three, 22.6 and 17.0 in two).  Of 70 shapes taken at
+// random whose plan it changed, 69 gained 2 to 35 %; a band about 34,400 x 12,288 and 17,200 x 14,336, whose five rounds become
+// three or four, loses 1 to 8 % (144 -> 154 us at 9 rows).  With 65 rows or more, where
 // the plan says whether this kernel takes the product at all, a round costs that quarter: plans that the larger figure turns into
 // one round of four waves are slower than the BLAS library (14,592 x 5,120 at 65 and 128 rows 62 and 67 us, 36 and 43 there;
 // 15,360 x 9,216 102 and 112, 66 and 71).
@@ -579,7 +583,8 @@ static MidPlan mid_plan(int m, int groups, int k, int gate) {
   const int units = (k + kMidSlice - 1) / kMidSlice;
   const int cus = device_cus();
   if ((groups + 7) / 8 > 2 * cus) {
-    plan.waves = m > 16 && !gate ? 8 : 4;
+    const bool wide = !gate && (m > 48 ? k >= 3072 : m > 32 && k >= 4096 && groups > 28 * cus);
+    plan.waves = wide ? 8 : 4;
     plan.tiles = (groups + plan.waves - 1) / plan.waves;
     plan.splits = 1;
     plan.kslice = units * kMidSlice;

@@ -700,6 +700,22 @@ def test_skinny_gemm_very_wide(n, k, all_rows):
         assert torch.equal(y, full[:m])
 
 
+@pytest.mark.parametrize("n,k", [(65584, 3080), (65552, 4096), (114720, 4104), (114704, 3072)])
+def test_skinny_gemm_very_wide_and_deep(n, k, all_rows):
+    """Where blocks of four waves give way to blocks of eight by rows, K and columns: close to the float64 product, and each
+    row the same bits on both sides of every line."""
+    ops = all_rows
+    g = torch.Generator(device=DEV).manual_seed(n + k)
+    w = torch.randn((n, k), generator=g, device=DEV).mul_(0.05).to(torch.bfloat16)
+    x = torch.randn((64, k), generator=g, device=DEV).to(torch.bfloat16)
+    y = ops.linear(x, w, out_dtype=torch.float32)
+    for lo in range(0, n, 16384):
+        want = x.double() @ w[lo:lo + 16384].double().T
+        assert float((y[:, lo:lo + 16384].double() - want).abs().max()) <= 1e-4 * float(want.abs().max())
+    for m in (49, 48, 33, 32, 17, 16, 9):
+        assert torch.equal(ops.linear(x[:m].contiguous(), w, out_dtype=torch.float32), y[:m]), m
+
+
 def test_which_products_of_65_to_128_rows_are_streamed():
     """Products whose blocks of four waves fill one round only because a second one is dear go to the library, as they are
     faster there; those that are streamed have the slices they have at 64 rows."""
