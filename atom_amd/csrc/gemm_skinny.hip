@@ -235,10 +235,11 @@ __global__ void __launch_bounds__(256) gemm_skinny_kernel(SkinnyParams p) {
 // block comes twice, side by side in the grid, each with half of the rows of x.  The pair reads its
 // rows of w at about the same time, so memory delivers them once.
 constexpr int kMidSlice = 1024;   // K is cut in multiples of this
+constexpr int kMidNarrow = 65536; // columns up to which walks of eight chunks start by eighths
 constexpr int kMidAhead = 4;      // chunks in flight a wave (3 and 5 measure the same)
 
-// EXACT: the block's range of K is whole chunks, so no load needs a guard.  TURN: K is not cut, and every
-// tile starts its walk through K at another eighth.
+// EXACT: the block's range of K is whole chunks, so no load needs a guard.  TURN: K is not cut, and the walks
+// through K start at different places.
 template <int MT, bool GATE, bool EXACT, bool TURN>
 __global__ void __launch_bounds__(512) gemm_mid_kernel(SkinnyParams p) {
   extern __shared__ __attribute__((aligned(16))) char lds[];   // two chunks of 16 W + 16 MT rows
@@ -261,14 +262,18 @@ __global__ void __launch_bounds__(512) gemm_mid_kernel(SkinnyParams p) {
   const int chunk_bytes = (16 * waves + 16 * MT) * kARow;
   // Blocks that start together would all read the same stretch of their rows, a row's length apart in memory,
   // and so the same few memory channels at any moment: where K is not cut (slices start apart anyway, and
-  // measure worse with this) the walks through K start at different places.  SiLU-gate: every tile at another eighth,
-  // the same one for the tiles of an XCD (one round of blocks, which share the rows of x in their L2).  Plain products
-  // (many rounds): seven chunks further for every 512 columns, so that the blocks that run in one XCD at a time start at
-  // different ones; the place is a function of the columns, so a sum's order does not depend on the number of waves.
+  // measure worse with this) the walks through K start at different places.  SiLU-gate, and plain products of eight
+  // chunks and few columns: every tile at another eighth, the same one for the tiles of an XCD (which share the rows of x in
+  // their L2).  Other plain products: seven chunks further for every 512 columns, so that the blocks that run in one XCD at a
+  // time start at different ones.  The place comes from a tile's first column, so blocks of four and of eight waves, which
+  // take turns by the number of rows in very wide products of a longer K, sum in one order (blocks of five to seven reach
+  // into the next 512 columns, but their number is the same for all rows).
   // A head of 151,936 x 4,096, whose rows lie 8 KB apart, by eighths and so: 306 and 280 us at 64 rows, 237 and 219 at 32,
-  // 217 and 200 at 16; with rows of 5 and 10 KB both are equal.  The gate of 12,288 x 4,096: 35.5 and 36.8 at 24 rows.
+  // 217 and 200 at 16; with rows of 5 and 10 KB both are equal.  The gate of 12,288 x 4,096: 35.5 and 36.8 at 24 rows.  K 1,024 at
+  // 32 rows: 47,584 columns 23.4 and 24.5, 66,000 30.0 and 28.7.
+  const bool eighths = GATE || (total == 8 && p.n <= kMidNarrow);
   const int first = !(TURN && total >= 8) ? 0
-                    : GATE ? (tile & 7) * (total >> 3) : (int)(((unsigned)(tile * waves) >> 5) * 7u % (unsigned)total);
+                    : eighths ? (tile & 7) * (total >> 3) : (int)(((unsigned)(tile * waves) >> 5) * 7u % (unsigned)total);
   auto k_of = [&](int ci) {
     if (!TURN) return k_begin + 128 * ci;
     const int c = ci + first;
