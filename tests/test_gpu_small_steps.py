@@ -132,3 +132,26 @@ def test_stream_norm_rows_do_not_depend_on_batch(dtype, width, init):
         got.append((s, out))
     for mine, few, alone in zip(*got):
         assert torch.equal(mine[7:12], few) and torch.equal(mine[9:10], alone)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width", [512, 1300])
+@pytest.mark.parametrize("lens", [[1, 2, 1], [1020, 1, 2], [1021, 1, 2], [700, 800]])
+def test_shifted_rows_in_pieces_and_whole(dtype, width, lens):
+    """Rows cut over several blocks, and from four tokens a compute unit on whole: each mixed with the one before it, the
+    first of a request with what its slot holds, which then holds the last."""
+    ops = gpu_ops()
+    T, S = sum(lens), len(lens)
+    x, mu, kept = rnd((T, width), 1).to(dtype), torch.rand((width,), generator=torch.Generator().manual_seed(2)), rnd((S, 3 + width), 3)
+    cu = [sum(lens[:i]) for i in range(S + 1)]
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    state, out = kept.to(DEV), torch.empty((T, width), dtype=dtype, device=DEV)
+    ops.shift_rows(x.to(DEV), mu.to(DEV), out, state, 3, i32(cu), i32(list(range(S))), i32([s for s in range(S) for _ in range(lens[s])]))
+    cur = x.double()
+    prev = torch.cat((cur[:1], cur[:-1]))
+    for s in range(S):
+        prev[cu[s]] = kept[s, 3:].double()
+    want = cur + (prev - cur) * mu.double()
+    tol = {torch.float32: 1e-6, torch.bfloat16: 2.0 ** -8}[dtype]
+    assert bool(((out.double().cpu() - want).abs() <= tol * (want.abs() + 1)).all())
+    assert torch.equal(state.cpu()[:, 3:], x.float()[[c - 1 for c in cu[1:]]]) and torch.equal(state.cpu()[:, :3], kept[:, :3])
