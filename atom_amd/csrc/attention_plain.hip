@@ -15,7 +15,9 @@
 #include "common.h"
 
 // A wave a (token, head), value heads among them: a decode step's launch is one head's chain of waits and not that of all
-// the heads a wave of a token's block had in turn (4 tokens of 16 + 2 x 4 heads: 3.7 us, 8.1 so).
+// the heads a wave of a token's block had in turn (4 tokens of 16 + 2 x 4 heads: 3.7 us, 8.1 so).  From four tokens a CU on a
+// token has one block, whose waves take its heads in turn: so many short blocks cost more than the chains (4,096 tokens of
+// 16 + 2 x 4 heads, float32: 41 us with a wave a head, 35 so).
 template <typename T>
 __global__ void __launch_bounds__(256)
 qkv_plain_write_kernel(const float* __restrict__ proj, long ld, T* __restrict__ q_out, T* __restrict__ k_cache,
@@ -23,35 +25,35 @@ qkv_plain_write_kernel(const float* __restrict__ proj, long ld, T* __restrict__ 
                        int G, int D, int DV, int DP, int page_size, int unit_norm, float eps, float coef, int every) {
   const size_t t = blockIdx.x;
   const int lane = threadIdx.x & (kWave - 1);
-  const int head = blockIdx.y * (256 / kWave) + threadIdx.x / kWave;
-  if (head >= H + 2 * G) return;
   const int slot = slots != nullptr ? slots[t] : -1;
   const int page = slot >= 0 ? slot / page_size : 0, off = slot >= 0 ? slot % page_size : 0;
-  if (head >= H + G) {
-    if (slot < 0) return;
-    const int g = head - H - G;
-    const float* src = proj + t * ld + (size_t)(H + G) * D + (size_t)g * DV;
-    T* dst = v_cache + (((size_t)page * G + g) * DP) * (size_t)page_size + off;
-    for (int i = lane; i < DV; i += kWave) dst[(size_t)i * page_size] = from_f32<T>(src[i]);
-    return;
-  }
-  const bool is_k = head >= H;
-  const float* src = proj + t * ld + (size_t)head * D;
-  float factor = 1.f;
-  if (unit_norm) {
-    float ss = 0.f;
+  float temp = 1.f;
+  if (coef != 0.f) temp = 1.f + coef * logf((float)((positions[t] + 1) / every) + 1.f);
+  for (int head = blockIdx.y * (256 / kWave) + threadIdx.x / kWave; head < H + 2 * G; head += gridDim.y * (256 / kWave)) {
+    if (head >= H + G) {
+      if (slot < 0) return;
+      const int g = head - H - G;
+      const float* src = proj + t * ld + (size_t)(H + G) * D + (size_t)g * DV;
+      T* dst = v_cache + (((size_t)page * G + g) * DP) * (size_t)page_size + off;
+      for (int i = lane; i < DV; i += kWave) dst[(size_t)i * page_size] = from_f32<T>(src[i]);
+      continue;
+    }
+    const bool is_k = head >= H;
+    const float* src = proj + t * ld + (size_t)head * D;
+    float factor = 1.f;
+    if (unit_norm) {
+      float ss = 0.f;
 #pragma unroll 2
-    for (int i = lane; i < D; i += kWave) ss += src[i] * src[i];
-    factor = 1.f / sqrtf(wave_sum(ss) / (float)D + eps);
-  }
-  if (!is_k) {
-    float temp = 1.f;
-    if (coef != 0.f) temp = 1.f + coef * logf((float)((positions[t] + 1) / every) + 1.f);
-    T* dst = q_out + (t * H + head) * (size_t)DP;
-    for (int i = lane; i < DP; i += kWave) dst[i] = from_f32<T>(i < D ? src[i] * factor * temp : 0.f);
-  } else if (slot >= 0) {
-    T* dst = k_cache + (((size_t)page * G + (head - H)) * page_size + off) * (size_t)DP;
-    for (int i = lane; i < D; i += kWave) dst[i] = from_f32<T>(src[i] * factor);
+      for (int i = lane; i < D; i += kWave) ss += src[i] * src[i];
+      factor = 1.f / sqrtf(wave_sum(ss) / (float)D + eps);
+    }
+    if (!is_k) {
+      T* dst = q_out + (t * H + head) * (size_t)DP;
+      for (int i = lane; i < DP; i += kWave) dst[i] = from_f32<T>(i < D ? src[i] * factor * temp : 0.f);
+    } else if (slot >= 0) {
+      T* dst = k_cache + (((size_t)page * G + (head - H)) * page_size + off) * (size_t)DP;
+      for (int i = lane; i < D; i += kWave) dst[i] = from_f32<T>(src[i] * factor);
+    }
   }
 }
 
@@ -65,8 +67,7 @@ ATOM_EXPORT int atom_qkv_plain_write(const float* proj, long ld, void* q_out, vo
   if (slots != nullptr && (k_cache == nullptr || v_cache == nullptr)) return ATOM_BAD_SHAPE;
   if (coef != 0.f && (positions == nullptr || every <= 0)) return ATOM_BAD_SHAPE;
   if (tokens == 0) return ATOM_OK;
-  if (H + 2 * G > 65535) return ATOM_TOO_LARGE;
-  const dim3 grid(tokens, (H + 2 * G + 3) / 4);
+  const dim3 grid(tokens, tokens < 4 * device_cus() ? min((H + 2 * G + 3) / 4, 65535) : 1);
   ATOM_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((qkv_plain_write_kernel<T>), grid, dim3(256), 0, stream, proj, ld,
                                                  (T*)q_out, (T*)k_cache, (T*)v_cache, positions, slots, H, G, D, DV, DP,
                                                  page_size, unit_norm, eps, coef, every));

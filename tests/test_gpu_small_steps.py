@@ -155,3 +155,33 @@ def test_shifted_rows_in_pieces_and_whole(dtype, width, lens):
     tol = {torch.float32: 1e-6, torch.bfloat16: 2.0 ** -8}[dtype]
     assert bool(((out.double().cpu() - want).abs() <= tol * (want.abs() + 1)).all())
     assert torch.equal(state.cpu()[:, 3:], x.float()[[c - 1 for c in cu[1:]]]) and torch.equal(state.cpu()[:, :3], kept[:, :3])
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,G,D,DV", [(5, 2, 72, 40), (1, 1, 16, 20), (16, 4, 128, 128)])
+def test_plain_heads_of_few_and_many_tokens(dtype, H, G, D, DV):
+    """A wave a head up to four tokens a compute unit, a block a token from there on: the same bits, and every head there."""
+    ops = gpu_ops()
+    T, page, DP = 1100, 16, max(D, DV)
+    proj = rnd((T, (H + G) * D + G * DV), 1).to(DEV)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    slots = torch.randperm(T, generator=torch.Generator().manual_seed(2)).tolist()
+    slots[7] = -1
+    got = []
+    for n in (T, 1023, 9):
+        q = torch.full((n, H, DP), float("nan"), dtype=dtype, device=DEV)
+        k_cache = torch.zeros((T // page + 1, G, page, DP), dtype=dtype, device=DEV)
+        v_cache = torch.zeros((T // page + 1, G, DP, page), dtype=dtype, device=DEV)
+        ops.qkv_plain_write(proj[:n].contiguous(), q, k_cache, v_cache, i32(list(range(n))), i32(slots[:n]), H, G, D, DV, page,
+                            True, 1e-5, (0.1, 64))
+        at = [slots[t] for t in range(9) if slots[t] >= 0]
+        pg, off = torch.tensor(at, device=DEV) // page, torch.tensor(at, device=DEV) % page
+        got.append((q[:9], k_cache[pg, :, off], v_cache[pg, :, :, off]))
+    for few in got[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(got[0], few))
+    x = proj[:9].double()
+    k = x[:, H * D:(H + G) * D].view(9, G, D)
+    k = k / torch.sqrt((k * k).mean(-1, keepdim=True) + 1e-5)
+    keep = [t for t in range(9) if slots[t] >= 0]
+    for mine, want in ((got[0][1][:, :, :D], k[keep]), (got[0][2][:, :, :DV], x[keep, (H + G) * D:].view(-1, G, DV))):
+        assert bool(((mine.double() - want).abs() <= (2.0 ** -8 if dtype == torch.bfloat16 else 1e-5) * want.abs().max()).all())
