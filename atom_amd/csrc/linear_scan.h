@@ -19,6 +19,7 @@ struct ScanArgs {
   float* state; long slot_stride; long state_off;
   const int* cu_seqlens; const int* slot_of_seq;
   int num_seqs, H, K, V, lpc, waves;
+  int most;                                  // the walk leaves out requests of more tokens (0: none)
   int run_len;                               // R, a multiple of kScanStage; 0: a request is one run whatever its length
   float* run_state;                          // [places, H, K, V]: B of a run after pass 1, the state before it after pass 2
   float* run_decay;                          // [places, H, K]: the product of a run's decays
@@ -42,7 +43,7 @@ __device__ __forceinline__ bool scan_place(const ScanArgs& a, int b, int& seq, i
   return run >= 0 && run < runs;
 }
 
-// Whether the runs of this scan are worked as matrix products (linear_scan_runs.hip), and their launches; `need` is the
-// number of scratch places.
+// Whether the runs of this scan are worked as matrix products (linear_scan_runs.hip), and their launches, which leave out
+// requests of one run; `need` is the number of scratch places.
 bool scan_runs_takes(const ScanArgs& a);
-int scan_runs_launch(const ScanArgs& a, long need, hipStream_t stream);
+int scan_runs_launch(const ScanArgs& a, long need, int tokens, hipStream_t stream);

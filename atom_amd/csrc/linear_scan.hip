@@ -24,7 +24,8 @@
 //      the slot.
 // Run j of request s (tokens from t0) has the scratch place t0 / R + s + j, which no other run has.  A token's
 // result depends on its own request only; cutting a request differently changes the order of roundings, no more.
-// Runs with one decay per head go to the matrix cores where the sizes allow (linear_scan_runs.hip).
+// Runs with one decay per head go to the matrix cores where the sizes allow (linear_scan_runs.hip); requests of one run are
+// walked beside them, so that these too have the same bits alone and beside longer ones.
 //
 // Around it: token_shift (a token's input mixed with the previous token's, the previous token kept per request),
 // step_decay (softplus step sizes and the decays exp(-exp(A_log) dt) of a state-space layer), group_norm_gate (RMS
@@ -79,6 +80,7 @@ linear_scan_kernel(ScanArgs a) {
   if (!scan_place(a, blockIdx.x, seq, run, runs)) return;
   if (PASS == 1 && run == runs - 1) return;  // nothing follows a request's last run
   const int s0 = a.cu_seqlens[seq], s1 = a.cu_seqlens[seq + 1];
+  if (PASS == 0 && a.most > 0 && s1 - s0 > a.most) return;
   const int t0 = a.run_len == 0 ? s0 : s0 + run * a.run_len;
   const int t1 = a.run_len == 0 ? s1 : min(s1, t0 + a.run_len);
   const int slot = a.slot_of_seq[seq];
@@ -313,12 +315,13 @@ __global__ void __launch_bounds__(256) linear_scan_fold_kernel(ScanArgs a) {
   }
 }
 
+// shortest: a lower bound of the tokens a request brings, which says what need not be launched.
 ATOM_EXPORT int atom_linear_scan(const float* r, long ldr, int r_div, const float* k, long ldk, int k_div, const float* v,
                                  long ldv, const float* w, long ldw, int w_per_channel, const float* w_bias, int w_mode,
                                  const float* a_log, const float* v_scale, long ldvs, const float* bonus, const float* skip, float* out,
                                  long ldo, float* state, long slot_stride, long state_off, const int* cu_seqlens,
                                  const int* slot_of_seq, int num_seqs, int H, int K, int V, int tokens, int run_len,
-                                 float* run_state, float* run_decay, long places, hipStream_t stream) {
+                                 float* run_state, float* run_decay, long places, int shortest, hipStream_t stream) {
   if (H <= 0 || K <= 0 || V <= 0 || num_seqs < 0 || r_div <= 0 || k_div <= 0 || tokens < 0) return ATOM_BAD_SHAPE;
   if (r == nullptr || k == nullptr || v == nullptr || w == nullptr || out == nullptr || state == nullptr) return ATOM_BAD_SHAPE;
   if (cu_seqlens == nullptr || slot_of_seq == nullptr) return ATOM_BAD_SHAPE;
@@ -338,15 +341,21 @@ ATOM_EXPORT int atom_linear_scan(const float* r, long ldr, int r_div, const floa
   // long requests in runs: four columns a lane, so that a staged row serves four columns, where that still leaves
   // waves enough to fill the chip; otherwise one column a lane, which gives the most waves
   const bool wide = run_len > 0 && V >= 4 * cols && need * H * ((V + 4 * cols - 1) / (4 * cols)) >= 2048;
-  const int cpl = wide ? 4 : 1;
-  const int waves = min(kScanWaves, (V + cols * cpl - 1) / (cols * cpl));
-  const int vw = waves * cols * cpl;
-  const long blocks_x = run_len > 0 ? need : num_seqs;
+  int cpl = wide ? 4 : 1;
+  int waves = min(kScanWaves, (V + cols * cpl - 1) / (cols * cpl));
+  int vw = waves * cols * cpl;
+  long blocks_x = run_len > 0 ? need : num_seqs;
   if (blocks_x > 0x7fffffff || H > 65535 || (V + vw - 1) / vw > 65535 || ((long)K * V + 255) / 256 > 65535) return ATOM_TOO_LARGE;
   ScanArgs a{r, ldr, r_div, k, ldk, k_div, v, ldv, w, ldw, w_per_channel, w_bias, w_mode, a_log, v_scale, ldvs, bonus, skip,
-             out, ldo, state, slot_stride, state_off, cu_seqlens, slot_of_seq, num_seqs, H, K, V, lpc, waves, run_len,
+             out, ldo, state, slot_stride, state_off, cu_seqlens, slot_of_seq, num_seqs, H, K, V, lpc, waves, 0, run_len,
              run_len > 0 ? run_state : nullptr, run_len > 0 ? run_decay : nullptr};
-  if (scan_runs_takes(a)) return scan_runs_launch(a, need, stream);
+  const int narrow = min(kScanWaves, (V + cols - 1) / cols);
+  if (scan_runs_takes(a) && (V - 1) / (narrow * cols) < 65535) {
+    const int status = scan_runs_launch(a, need, tokens, stream);
+    if (status != ATOM_OK || shortest > run_len) return status;
+    cpl = 1, waves = a.waves = narrow, vw = waves * cols, blocks_x = num_seqs;   // the requests of one run, as without longer ones
+    a.most = run_len, a.run_len = 0, a.run_state = nullptr, a.run_decay = nullptr;
+  }
   const bool perhead = !w_per_channel && bonus == nullptr;   // one staged decay a token instead of one a row
   const size_t smem = (size_t)(cpl > 1 ? kScanStage / 2 : kScanStage) *
                       ((perhead ? 2 : 3) * lpc * kScanRows + ((vw + 5) & ~3)) * sizeof(float);
@@ -366,7 +375,7 @@ ATOM_EXPORT int atom_linear_scan(const float* r, long ldr, int r_div, const floa
     case 8: ATOM_SCAN_LAUNCH(PASS, 8, CPL); break;        \
     default: ATOM_SCAN_LAUNCH(PASS, 16, CPL); break;      \
   }
-  if (run_len > 0) {
+  if (a.run_len > 0) {
     if (cpl == 4) { ATOM_SCAN_BY_LPC(1, 4) } else { ATOM_SCAN_BY_LPC(1, 1) }
     hipLaunchKernelGGL(linear_scan_fold_kernel, dim3(num_seqs, H, (unsigned)(((long)K * V + 255) / 256)), dim3(256), 0, stream, a);
   }

@@ -15,10 +15,15 @@
 // as in the walk token by token: a wave whose 16 tokens' values hold any takes their triangle term by term, because a zero
 // above the diagonal times such a value is not zero.
 //
+// Requests of one run (64 tokens or fewer) are left to the walk token by token, which follows for them alone: they take it
+// without longer ones beside them too, so a token's result does not depend on those, and a single token does not pay for a
+// run (64 heads of 128 x 64, 512 tokens beside 24 single ones: 175 us with runs for all, 115 so; beside three of 40 tokens 73
+// and 95).
+//
 // Against a walk of the runs token by token (which it replaces for these sizes): 5,569 tokens of 64 heads of 128 x 64,
-// 106 + 85 + 214 us for the three launches, 289 + 87 + 528 so.  At the smallest, 65 tokens of 32 heads, 30 us and 76.
-// Bound by the float32 rate of the matrix cores and, in the middle launch, by the bytes of the states (1.6 MB a run of 64
-// heads).
+// 99 + 81 + 203 us for the three launches, 263 + 80 + 486 so.  At the smallest, 65 tokens of 32 heads, 30 us and 77.
+// The first and the last are bound by their blocks' waits between the stages of a head (they run at 0.37 and 0.26 of the float32
+// rate of the matrix cores), the middle one by the bytes of the states (2.1 MB a run of 64 heads, read and written).
 #include "linear_scan.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -83,7 +88,7 @@ __global__ void __launch_bounds__(kFormThreads) scan_form_kernel(ScanArgs a, int
   float* k_rows = lds;                  // [64][ks]
   float* v_rows = lds + kRun * ks;      // [64][kVRow]
   int seq, run, runs;
-  if (!scan_place(a, blockIdx.x, seq, run, runs)) return;
+  if (!scan_place(a, blockIdx.x, seq, run, runs) || runs < 2) return;
   if (a.slot_of_seq[seq] < 0) return;
   const int t0 = a.cu_seqlens[seq] + run * kRun, n = min(kRun, a.cu_seqlens[seq + 1] - t0);
   const size_t place = (size_t)(a.cu_seqlens[seq] / kRun + seq + run);
@@ -153,7 +158,7 @@ __global__ void __launch_bounds__(256) scan_join_kernel(ScanArgs a) {
   if (e >= a.K * a.V) return;
   const int slot = a.slot_of_seq[seq];
   const int t0 = a.cu_seqlens[seq], len = a.cu_seqlens[seq + 1] - t0;
-  if (slot < 0 || len <= 0) return;
+  if (slot < 0 || len <= kRun) return;
   const int runs = (len + kRun - 1) / kRun;
   const size_t first = ((size_t)(t0 / kRun + seq) * a.H + h), state = (size_t)a.K * a.V;
   float* B = a.run_state + first * state + e;
@@ -198,7 +203,7 @@ __global__ void __launch_bounds__(kReadThreads) scan_read_kernel(ScanArgs a, int
   float* v_rows = scores + kRun * kGRow;      // [64][kVRow]
   float* s_rows = v_rows + kRun * kVRow;      // [K][kVRow]; the keys [64][ks] until the scores are formed
   int seq, run, runs;
-  if (!scan_place(a, blockIdx.x, seq, run, runs)) return;
+  if (!scan_place(a, blockIdx.x, seq, run, runs) || runs < 2) return;
   const int t0 = a.cu_seqlens[seq] + run * kRun, n = min(kRun, a.cu_seqlens[seq + 1] - t0);
   const size_t place = (size_t)(a.cu_seqlens[seq] / kRun + seq + run);
   const int h0 = blockIdx.y * heads, col0 = blockIdx.z * kCols;
@@ -338,11 +343,13 @@ bool scan_runs_takes(const ScanArgs& a) {
          ends % 16 == 0;
 }
 
-int scan_runs_launch(const ScanArgs& a, long need, hipStream_t stream) {
+int scan_runs_launch(const ScanArgs& a, long need, int tokens, hipStream_t stream) {
   const int blocks_v = (a.V + kCols - 1) / kCols;
-  // heads a block: as many as share r and k, up to eight, while every CU keeps two blocks
+  // heads a block: as many as share r and k, up to eight, while every CU keeps two blocks (a request of several runs leaves
+  // at most every second one part empty)
+  const long busy = min(need, 2L * tokens / kRun);
   int heads = 8;
-  while (heads > 1 && (a.r_div % heads || need * (a.H / heads) * blocks_v < 2L * device_cus())) heads /= 2;
+  while (heads > 1 && (a.r_div % heads || busy * (a.H / heads) * blocks_v < 2L * device_cus())) heads /= 2;
   const dim3 grid((unsigned)need, a.H / heads, blocks_v);
   if (need > 0x7fffffL || a.H > 65535 || blocks_v > 65535) return ATOM_TOO_LARGE;
   const size_t form = (size_t)kRun * (a.K + 4 + kVRow) * sizeof(float);

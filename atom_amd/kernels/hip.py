@@ -1399,7 +1399,7 @@ class HipKernels:
     def linear_scan(self, r, r_off: int, r_heads: int, k, k_off: int, k_heads: int, v, v_off: int, w, w_off: int,
                     state, state_off: int, cu_seqlens_q, slot_of_seq, out, heads: int, dim: int, vdim: int,
                     per_channel: bool = True, w_bias=None, v_scale=None, bonus=None, skip=None,
-                    max_q_len: int | None = None, step_bias=None, a_log=None):
+                    max_q_len: int | None = None, step_bias=None, a_log=None, min_q_len: int = 1):
         """A linear recurrence with a state of ``dim`` x ``vdim`` per head over each request's tokens:
         ``S <- diag(w) S + k v^T`` with the read-out ``o = (S_before + diag(bonus) k v^T)^T r`` where ``bonus``
         [heads, dim] is given, else ``o = S_after^T r``.  All inputs float32 [tokens, *], read from a column offset:
@@ -1412,7 +1412,8 @@ class HipKernels:
         given) to the read-out.  The heads' matrices [heads, dim, vdim] start at ``state_off`` of a slot's row of
         ``state``; requests with slot -1 are padding.  ``out`` float32 [tokens, heads * vdim].  ``max_q_len``: the most tokens a
         request brings (an upper bound; default: all tokens); beyond ``SCAN_RUN`` tokens requests are cut into runs of
-        that length that are worked side by side, through scratch memory of a state per run."""
+        that length that are worked side by side, through scratch memory of a state per run.  ``min_q_len``: the fewest (a
+        lower bound), which says whether shorter requests have to be looked for beside them."""
         tokens = out.shape[0]
         seqs = slot_of_seq.numel()
         if heads % r_heads or heads % k_heads:
@@ -1454,7 +1455,8 @@ class HipKernels:
             self._at(v, v_off), L(v.shape[1]), self._at(w, w_off), L(w.shape[1]), int(bool(per_channel)), _ptr(bias),
             mode, _ptr(a_log), _ptr(v_scale), L(heads), _ptr(bonus), _ptr(skip), _ptr(out),
             L(heads * vdim), _ptr(state), L(state.shape[1]), L(state_off), _ptr(cu_seqlens_q), _ptr(slot_of_seq), seqs,
-            heads, dim, vdim, tokens, run_len, _ptr(run_state), _ptr(run_decay), L(places), self._stream()))
+            heads, dim, vdim, tokens, run_len, _ptr(run_state), _ptr(run_decay), L(places),
+            int(min_q_len), self._stream()))
         return out
 
     def token_shift(self, x, mu, mixes, state, state_off: int, cu_seqlens_q, slot_of_seq, token_seq):

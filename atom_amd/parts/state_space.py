@@ -80,7 +80,8 @@ class StateSpaceMixer(Mixer):
         # the raw step sizes are the product's last columns: the scan forms softplus(dt + dt_bias) and the decays
         ops.linear_scan(xbc, inner + G * N, G, xbc, inner, G, xbc, 0, proj, inner + C, cache.state, self.conv_floats,
                         ctx.cu_seqlens_q, ctx.slot_of_seq, y, H, N, V, per_channel=False, skip=self.params["D"],
-                        max_q_len=ctx.max_q_len, step_bias=self.params["dt_bias"], a_log=self.params["A_log"])
+                        max_q_len=ctx.max_q_len, step_bias=self.params["dt_bias"], a_log=self.params["A_log"],
+                        min_q_len=min(ctx.seq_lens) if ctx.max_q_len > 1 and ctx.seq_lens else 1)
         out = torch.empty((T, inner), dtype=x.dtype, device=x.device)
         ops.group_norm_gate(y, self.norm_groups, self.params["norm.weight"], self.norm_eps, out, gate=proj, gate_off=0,
                             gate_first=True)

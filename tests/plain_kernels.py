@@ -478,7 +478,7 @@ class PlainKernels:
 
     def linear_scan(self, r, r_off, r_heads, k, k_off, k_heads, v, v_off, w, w_off, state, state_off, cu_seqlens_q,
                     slot_of_seq, out, heads, dim, vdim, per_channel=True, w_bias=None, v_scale=None, bonus=None,
-                    skip=None, max_q_len=None, step_bias=None, a_log=None):
+                    skip=None, max_q_len=None, step_bias=None, a_log=None, min_q_len=1):
         if a_log is not None:      # raw step sizes in w's place: the steps multiply v, the decays follow from them
             steps = pl.softplus(w[:, w_off:w_off + heads].to(WIDE) + step_bias.to(WIDE))
             w, w_off, v_scale = torch.exp(-torch.exp(a_log.to(WIDE)) * steps), 0, steps

@@ -89,3 +89,31 @@ def test_what_is_not_finite_stays_behind_its_token(H, G, K, V, what, value, wher
         # number a row is one product r . k scaled, whose own terms cancel by up to two digits
         bound = 1e-3 if value == 1e30 else 1e-5
         assert bool(((got - want).norm(dim=1) <= bound * want.norm(dim=1)).all())
+
+
+@pytest.mark.parametrize("H,G,K,V", [(4, 2, 64, 48), (16, 1, 128, 64)])
+@pytest.mark.parametrize("n", [1, 17, 64, 65, 200])
+@pytest.mark.parametrize("others", [[1] * 24, [500], [3, 64, 65, 128]])
+def test_a_request_is_worked_alike_alone_and_beside_others(H, G, K, V, n, others):
+    """Walk or runs is a matter of a request's own tokens: outputs and state have the same bits alone and in steps with single
+    tokens, shorter and longer portions, before it and behind it, a padded request among them."""
+    ops = gpu_ops()
+    for lens in ([n, 2] + others, others + [2, n]):
+        place, pad, T = (0, 1, sum(lens)) if lens[0] == n else (len(lens) - 1, len(lens) - 2, sum(lens))
+        at = sum(lens[:place])
+        x, raw = rnd((T, H * V + 2 * G * K + 4), 1).to(DEV), rnd((T, H), 2).to(DEV)
+        bias, a_log, skip = rnd((H,), 3, 0.3).to(DEV), rnd((H,), 4, 0.3).to(DEV), rnd((H,), 5).to(DEV)
+        slots = [-1 if s == pad else s for s in range(len(lens))]
+        got = []
+        for rows, some, slot in ((slice(0, T), lens, slots), (slice(at, at + n), [n], [place])):
+            i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+            state = rnd((len(lens), 7 + H * K * V), 6, 0.3).to(DEV)
+            out = torch.full((sum(some), H * V), float("nan"), device=DEV)
+            part = x[rows].contiguous()
+            cu = [sum(some[:i]) for i in range(len(some) + 1)]
+            ops.linear_scan(part, H * V + G * K, G, part, H * V, G, part, 0, raw[rows].contiguous(), 0, state, 7, i32(cu), i32(slot),
+                            out, H, K, V, per_channel=False, skip=skip, max_q_len=max(some), step_bias=bias, a_log=a_log)
+            assert bool(out.isfinite().all())
+            got.append((out[at:at + n] if len(some) > 1 else out, state[place]))
+        for beside, alone in zip(*got):
+            assert torch.equal(beside, alone)
