@@ -43,27 +43,43 @@ __device__ __forceinline__ int row_of_w(const GemmF32Params& p, int at) {
 
 __device__ __forceinline__ float silu_times(float gate, float up) { return gate / (1.f + expf(-gate)) * up; }
 
-// Four consecutive terms of a row from k0 on.  WHOLE: K is a multiple of 16 and rows begin at multiples of four
-// elements in memory; else term by term, zeros behind the row's end.
-template <typename T, bool WHOLE>
+// How a row's terms are read, four at a time.  kWhole: K is a multiple of 16 and rows begin at multiples of four elements in
+// memory.  kAny: any K from 4 on and any rows, with loads that need no more than their elements' alignment; the four that would
+// reach behind the row's end are its last four, which last_terms moves into place before they are used.  kTerms: term by
+// term, for the K below 4.  (4,096 columns at 2,048 rows, K 4,095, bfloat16 x: 1,867 us term by
+// term, 795 with loads of four; one row 36 and 17.)
+enum Loads : int { kTerms, kAny, kWhole };
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef bf16_t bf16x4_any __attribute__((ext_vector_type(4), aligned(2)));
+
+template <typename T, int LOADS>
 __device__ __forceinline__ f32x4 four_terms(const T* __restrict__ row, int k0, int k) {
   f32x4 v;
-  if constexpr (WHOLE) {
-    if constexpr (sizeof(T) == 4) {
-      v = *reinterpret_cast<const f32x4*>(row + k0);
-    } else {
-      const bf16x4 h = *reinterpret_cast<const bf16x4*>(row + k0);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = to_f32(h[i]);
-    }
-  } else {
+  if constexpr (LOADS == kTerms) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] = k0 + i < k ? to_f32(row[k0 + i]) : 0.f;
+  } else if constexpr (sizeof(T) == 4) {
+    if constexpr (LOADS == kWhole) v = *reinterpret_cast<const f32x4*>(row + k0);
+    else v = *reinterpret_cast<const f32x4_any*>(row + min(k0, k - 4));
+  } else {
+    bf16x4 h;
+    if constexpr (LOADS == kWhole) h = *reinterpret_cast<const bf16x4*>(row + k0);
+    else h = *reinterpret_cast<const bf16x4_any*>(row + min(k0, k - 4));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = to_f32(h[i]);
   }
   return v;
 }
 
-template <typename TX, typename TW, int MT, int NT, int DEPTH, bool WHOLE>
+// The terms from k0 on of what four_terms<kAny> read: `late` (1 to 3, or more for none) of the four were read too early, and
+// zeros stand behind the row's end.
+__device__ __forceinline__ void last_terms(f32x4& v, int late) {
+  if (late & 1) v = f32x4{v[1], v[2], v[3], 0.f};
+  if (late & 2) v = f32x4{v[2], v[3], 0.f, 0.f};
+  if (late > 3) v = f32x4{0.f, 0.f, 0.f, 0.f};
+}
+
+template <typename TX, typename TW, int MT, int NT, int DEPTH, int LOADS>
 __global__ void __launch_bounds__(kSlices* kWave)
 gemm_f32_kernel(GemmF32Params p) {
   __shared__ float met[kSlices][MT * kSide * kSide];
@@ -91,6 +107,8 @@ gemm_f32_kernel(GemmF32Params p) {
   const int begin = min(wave * share, steps);
   const int count = __builtin_amdgcn_readfirstlane(min(begin + share, steps) - begin);
 
+  const int ends = __builtin_amdgcn_readfirstlane(p.k / kStep - begin);   // kAny: the step that the row ends in
+
   f32x4 acc[MT][NT];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
@@ -105,9 +123,9 @@ gemm_f32_kernel(GemmF32Params p) {
   const auto fetch = [&](int d, int step) {
     const int at = min(begin + min(step, max(count - 1, 0)), steps - 1) * kStep + quarter * 4;
 #pragma unroll
-    for (int j = 0; j < NT; ++j) b[d][j] = four_terms<TW, WHOLE>(wr[j], at, p.k);
+    for (int j = 0; j < NT; ++j) b[d][j] = four_terms<TW, LOADS>(wr[j], at, p.k);
 #pragma unroll
-    for (int i = 0; i < MT; ++i) a[d][i] = four_terms<TX, WHOLE>(xr[i], at, p.k);
+    for (int i = 0; i < MT; ++i) a[d][i] = four_terms<TX, LOADS>(xr[i], at, p.k);
   };
 #pragma unroll
   for (int d = 0; d < DEPTH; ++d) {
@@ -118,6 +136,15 @@ gemm_f32_kernel(GemmF32Params p) {
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) {
       if (base + d < count) {
+        if constexpr (LOADS == kAny) {
+          if (base + d == ends) {
+            const int late = max(p.k / kStep * kStep + quarter * 4 - (p.k - 4), 0);
+#pragma unroll
+            for (int i = 0; i < MT; ++i) last_terms(a[d][i], late);
+#pragma unroll
+            for (int j = 0; j < NT; ++j) last_terms(b[d][j], late);
+          }
+        }
         // term by term over all tiles: an instruction's sum is needed only MT NT instructions later
         f32x4 part[MT][NT];
 #pragma unroll
@@ -353,9 +380,11 @@ static int launch_gemm_f32(GemmF32Params p, hipStream_t stream) {
   const dim3 grid((unsigned)(tiles + kXcds - 1) / kXcds * kXcds), block(kSlices * kWave);
   const bool whole = p.k % kStep == 0 && (uintptr_t)p.x % (4 * sizeof(TX)) == 0 && (uintptr_t)p.w % (4 * sizeof(TW)) == 0;
   if (whole)
-    hipLaunchKernelGGL((gemm_f32_kernel<TX, TW, MT, NT, DEPTH, true>), grid, block, 0, stream, p);
-  else
-    hipLaunchKernelGGL((gemm_f32_kernel<TX, TW, MT, NT, (DEPTH > 2 ? 2 : DEPTH), false>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((gemm_f32_kernel<TX, TW, MT, NT, DEPTH, kWhole>), grid, block, 0, stream, p);
+  else if (MT * NT < 16 || p.k >= 4)
+    hipLaunchKernelGGL((gemm_f32_kernel<TX, TW, MT, NT, DEPTH, kAny>), grid, block, 0, stream, p);
+  else if constexpr (MT * NT == 16)
+    hipLaunchKernelGGL((gemm_f32_kernel<TX, TW, MT, NT, DEPTH, kTerms>), grid, block, 0, stream, p);
   return launch_status();
 }
 
@@ -364,6 +393,7 @@ static int choose_gemm_f32(const GemmF32Params& p, hipStream_t stream) {
   // Tiles two wide read x half as often, which pays from where there is one for most CUs on.  24,576 x 4,096, narrow and
   // wide: 16 rows 111 and 93 us, 32 rows 155 and 116; 4,096 x 12,288 (128
   // wide tiles): 32 rows 89 and 116 us.
+  if (p.k < 4) return launch_gemm_f32<TX, TW, 4, 4, 2>(p, stream);
   const long cus = device_cus();
   const bool wide_fills = p.n / 32 >= cus * 3 / 4;
   if (p.m <= 16) {

@@ -130,6 +130,29 @@ def test_gemm_f32_tiles(xd, wd, m, n, k):
         assert torch.equal(ops.linear(x[lo:hi].contiguous(), w, out_dtype=torch.float32), y[lo:hi])
 
 
+@pytest.mark.parametrize("xd,wd", [(torch.float32, torch.float32), (torch.bfloat16, torch.float32), (torch.float32, torch.bfloat16)])
+@pytest.mark.parametrize("m,n", [(1, 40), (9, 6160), (18, 70), (20, 6160), (40, 70), (64, 8200), (300, 8200)])
+@pytest.mark.parametrize("k", [1, 3, 4, 5, 6, 7, 15, 17, 18, 30, 32, 131])
+@pytest.mark.parametrize("start", [0, 1])
+def test_gemm_f32_of_any_length(xd, wd, m, n, k, start):
+    """A K that is no multiple of 16, and rows that begin anywhere in memory, give the same bits as rows filled up with zeros:
+    nothing before or behind a row's own terms enters."""
+    ops = gpu_ops()
+
+    def placed(t):   # `start` elements into a buffer of NaN
+        buffer = torch.full((t.numel() + 8,), float("nan"), dtype=t.dtype, device=DEV)
+        view = buffer[start:start + t.numel()].view(t.shape)
+        view.copy_(t)
+        return view
+
+    x, w = rnd((m, k), xd, 8), rnd((n, k), wd, 9)
+    w[n // 2, 0] = float("inf")
+    filled = [torch.nn.functional.pad(t, (0, -k % 16)).to(DEV) for t in (x, w)]
+    got = ops.linear(placed(x), placed(w), out_dtype=torch.float32)
+    assert bool(got.isfinite().all(0)[:n // 2].all())
+    assert torch.equal(got, ops.linear(*filled, out_dtype=torch.float32))
+
+
 def test_linear_bf16_library_path():
     ops = gpu_ops()
     x, w, b = rnd((33, 136), torch.bfloat16, 13), rnd((517, 136), torch.bfloat16, 14), rnd((517,), torch.float32, 15)
