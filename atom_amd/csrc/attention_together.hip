@@ -20,7 +20,8 @@
 #include "common.h"
 
 constexpr int kTogetherThreads = 1024;   // a decode step's launch is a chain of waits: the more waves share a chunk, the shorter
-constexpr int kTogetherFew = 256;        // threads where a thread of many would own more than two pairs: registers for 32
+constexpr int kTogetherFew = 256;        // threads where they own no more than one pair each, or where a thread of many would own more
+                                         // than two: registers for 32
 constexpr int kTogetherChunk = 64;     // keys a pass; a wave's width, so a head's chunk is reduced by one wave
 constexpr int kTogetherAcc = 32;       // (head, value entry) pairs a thread may own, of the few
 
@@ -476,8 +477,14 @@ ATOM_EXPORT int atom_attention_together(const void* q, const void* k_cache, cons
     hipLaunchKernelGGL((together_sum_parts_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, stream, ws_o, (T*)out,      \
                        parts, H * DV, total);                                                                            \
   } while (0)
+  // A block with no more pairs, nor scores of a chunk, than the few threads are leaves three quarters of the many idle at every
+  // barrier (16 heads in 4 sets of 64 entries, bfloat16: 300 tokens behind 200 keys 164 us with many, 80 with few; 8 behind
+  // 4,000 72 and 45; one behind 100 keys 22 and 23).  Many from there on, also where the blocks fill the chip (8 mixed heads of 128,
+  // 300 tokens behind 200 keys: 148, 139 with 256 threads and 32 copies of the loop; 64 behind 1,000 87 and 125).
+  const bool few = HB * max(DV, kTogetherChunk) <= kTogetherFew;
   ATOM_DISPATCH_DTYPE(dtype, {
-    if (pairs <= 1) ATOM_TOGETHER(T, 1, kTogetherThreads);
+    if (few) ATOM_TOGETHER(T, 1, kTogetherFew);
+    else if (pairs <= 1) ATOM_TOGETHER(T, 1, kTogetherThreads);
     else if (pairs <= 2) ATOM_TOGETHER(T, 2, kTogetherThreads);
     else ATOM_TOGETHER(T, kTogetherAcc, kTogetherFew);
   });

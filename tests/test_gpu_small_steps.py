@@ -101,6 +101,15 @@ def test_heads_together_by_pairs_a_thread(dtype, how, H, G, D, DV, page, talk):
     attention_against_plain(dtype, how, H, G, D, DV, page, 150, True, talk, True)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("how", ["blocks", "parts"])
+@pytest.mark.parametrize("H,G,D,DV,page,talk", [(8, 2, 32, 64, 16, False), (4, 2, 32, 64, 6, True), (8, 2, 32, 66, 8, False),
+                                                (10, 2, 16, 48, 16, False)])
+def test_heads_together_by_threads_a_block(dtype, how, H, G, D, DV, page, talk):
+    """Blocks of few threads up to 256 pairs and scores, of many from there on."""
+    attention_against_plain(dtype, how, H, G, D, DV, page, 150, True, talk, True)
+
+
 @pytest.mark.parametrize("wdtype", DTYPES)
 @pytest.mark.parametrize("m,inter,k,biased", [(1, 13, 96, True), (5, 3080, 96, False), (5, 3081, 64, True), (17, 1, 20, True),
                                               (33, 160, 96, False), (65, 1003, 144, True), (130, 4100, 64, False),
