@@ -11,7 +11,7 @@ from dataclasses import dataclass, field
 import torch
 
 from ..cache.kinds import kind_of
-from ..parts.base import BLOCKS, EMBEDDINGS, HEADS, JOINS, NORMS, Part, PartChoice
+from ..parts.base import BLOCKS, EMBEDDINGS, HEADS, JOINS, NORMS, Part, PartChoice, PendingPost
 
 
 @dataclass(frozen=True)
@@ -149,11 +149,16 @@ class CausalLM(Part):
             hidden = first = self.embedding.forward(ctx, token_ids)
         residual = None
         for run, cache in zip(self.order, caches):
+            block = self.blocks[run.layer]
+            if isinstance(hidden, PendingPost) and (run.enters or not block.accepts_pending_post):
+                hidden = hidden.resolve(ctx)
             if run.enters:
                 hidden, residual = self.join.forward(ctx, hidden, residual, first)
-            hidden, residual = self.blocks[run.layer].forward(ctx, hidden, residual, cache)
+            hidden, residual = block.forward(ctx, hidden, residual, cache)
         if want_rows is None or want_rows.numel() == 0:
             return None
+        if isinstance(hidden, PendingPost):
+            hidden = hidden.resolve(ctx)
         if not self.final_norm.accepts_deferred:
             hidden = ctx.ops.materialize(hidden)
         normed = self.final_norm.forward_rows(ctx, hidden, residual, want_rows)

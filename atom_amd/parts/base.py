@@ -167,6 +167,18 @@ class ScaledSum:
     dtype = torch.float32
 
 
+class PendingPost:
+    """A sublayer's result whose own norm has not been applied yet: ``norm(x)`` is to join the residual stream.  A block
+    that ``accepts_pending_post`` forms it, adds it and norms the stream for its first sublayer in one kernel; anything
+    else is handed ``resolve(ctx)``, the summand itself in float32."""
+
+    def __init__(self, x, norm):
+        self.x, self.norm = x, norm
+
+    def resolve(self, ctx):
+        return self.norm.forward(ctx, self.x, out_dtype=torch.float32)
+
+
 class StreamUpdate:
     """A sublayer's result that has not joined a residual of several streams yet: with ``y = layer_scale * sum_i
     scales[i] * terms[i]`` (``layer_scale`` None: ones) the streams x_1 .. x_S become ``x_t <- sum_s mix[s, t] x_s +
@@ -281,6 +293,9 @@ class FeedForward(Part):
 
 
 class Block(Part):
+    #: True when ``forward`` takes a ``PendingPost`` for ``hidden``
+    accepts_pending_post = False
+
     def forward(self, ctx, hidden: torch.Tensor, residual: torch.Tensor | None, cache):
         """Returns (hidden, residual) for the next block."""
         raise NotImplementedError
