@@ -222,7 +222,7 @@ class HipKernels:
                    "atom_attention_together", "atom_attention_together_tiles", "atom_attention_together_tiles_supports",
                    "atom_together_sum_parts", "atom_streams_step", "atom_embedding_sinusoid", "atom_softcap_rows",
                    "atom_selective_scan", "atom_step_sizes", "atom_experts_few", "atom_experts_few_supports", "atom_keys_as_values_heads_write",
-                   "atom_delta_chunks", "atom_delta_chunks_supports"):
+                   "atom_delta_chunks", "atom_delta_chunks_supports", "atom_delta_step", "atom_delta_step_supports"):
             getattr(self.lib, fn).restype = ctypes.c_int
         self.lib.atom_delta_chunks_floats.restype = ctypes.c_long
         self.allow_library_gemm = True
@@ -248,6 +248,7 @@ class HipKernels:
         self.prefill_low_blocks = None   # True / False forces 16 / 32 tokens a wave in the blocks of eight waves
         self.use_fused_decode = True    # decode-only steps of few rows: norm, rotation and cache write inside attention
         self.use_delta_chunks = True   # the delta rule of prompts in chunks of 64 tokens
+        self.use_delta_step = True     # ... and of single tokens in one launch with what is before and behind it
         self.use_together_tiles = True  # attention with the heads together on the matrix cores, for prompt portions
         self.use_mfma_latent = True     # attention over latent pages on the matrix cores (bfloat16, sizes it is built for)
         self.use_latent_tiles = True    # ... its form for a latent of 128, 256 or 512 entries and 64 rotated ones
@@ -1386,6 +1387,45 @@ class HipKernels:
         self._done("delta_out", self.lib.atom_delta_out(
             _ptr(o), _ptr(gates), gates.shape[1], gate_off, _ptr(weight), ctypes.c_float(eps), _ptr(out),
             self._code(out), tokens, heads, vdim, 0 if activation == "silu" else 1, self._stream()))
+        return out
+
+    def delta_step(self, proj, taps_weight, state, state_off: int, cu_seqlens_q, slot_of_seq, b_off: int, a_off: int,
+                   decay2, gate_off: int, gate2, a_log, dt_bias, weight, eps: float, out, heads: int, kv_heads: int, dim: int,
+                   vdim: int, per_channel: bool, activation: str):
+        """For steps whose requests bring one token each: ``conv_silu_state``, ``delta_rule`` and ``delta_out`` in one launch,
+        from the projection ``proj`` (float32 [tokens, *]; q | k | v first, the rest at its offsets) to ``out`` [tokens, heads
+        vdim].  ``decay2`` [decays, rank] / ``gate2`` [heads vdim, rank]: the columns at ``a_off`` / ``gate_off`` are the inner
+        vectors of low-rank products with these (None: the raw decays and gates themselves).  Returns ``out``, or None where
+        the kernel does not take these sizes: heads of 64 or 128 channels, one or two a q/k head, four taps, ranks of 16 to 64
+        in steps of 16."""
+        ranks = tuple(0 if w is None else w.shape[1] for w in (decay2, gate2))
+        if (not self.use_delta_step or taps_weight.dtype != out.dtype or state.shape[1] % 4 or state_off % 4
+                or not self.lib.atom_delta_step_supports(heads, kv_heads, dim, vdim, taps_weight.shape[1], *ranks)):
+            return None
+        tokens, seqs = proj.shape[0], slot_of_seq.numel()
+        channels, decays = (2 * kv_heads + heads) * dim, heads * (dim if per_channel else 1)
+        if activation not in ("silu", "sigmoid"):
+            raise KernelError(f"delta_step: unknown activation {activation!r}")
+        dt = out.dtype
+        self._check("delta projection", proj, torch.float32)
+        self._check("taps", taps_weight, dt, (channels, 4))
+        self._check("state", state, torch.float32, (None, None))
+        self._check("cu_seqlens_q", cu_seqlens_q, torch.int32, (seqs + 1,))
+        self._check("slot_of_seq", slot_of_seq, torch.int32, (seqs,))
+        self._check("A_log", a_log, torch.float32, (heads,))
+        self._check("dt_bias", dt_bias, torch.float32, (decays,))
+        self._check("read-out norm weight", weight, torch.float32, (vdim,))
+        self._check("gated read-out", out, (torch.float32, torch.bfloat16), (tokens, heads * vdim))
+        if decay2 is not None:
+            self._check("decay weight", decay2, dt, (decays, ranks[0]))
+        if gate2 is not None:
+            self._check("gate weight", gate2, dt, (heads * vdim, ranks[1]))
+        self._done("delta_step", self.lib.atom_delta_step(
+            _ptr(proj), ctypes.c_long(proj.shape[1]), _ptr(taps_weight), self._code(out), _ptr(state),
+            ctypes.c_long(state.shape[1]), ctypes.c_long(state_off), _ptr(cu_seqlens_q), _ptr(slot_of_seq), seqs, b_off, a_off,
+            ranks[0], _ptr(decay2), gate_off, ranks[1], _ptr(gate2), int(bool(per_channel)), _ptr(a_log), _ptr(dt_bias),
+            _ptr(weight), ctypes.c_float(eps), _ptr(out), heads, kv_heads, dim, 0 if activation == "silu" else 1,
+            self._stream()))
         return out
 
     # ------------------------------------------------------------------ linear recurrences with a matrix state

@@ -132,11 +132,19 @@ class GatedDeltaRule(Mixer):
         T = x.shape[0]
         H, dv, C = self.num_heads, self.value_dim, self.channels
         proj = ops.linear(x, self.params["proj.weight"], None, out_dtype=torch.float32)
+        at = self._layout()[1]
+        step = getattr(ops, "delta_step", None) if ctx.max_q_len == 1 else None
+        if step is not None:
+            out = torch.empty((T, H * dv), dtype=x.dtype, device=x.device)
+            if step(proj, self.params["conv.weight"], cache.state, self.conv_floats, ctx.cu_seqlens_q, ctx.slot_of_seq,
+                    at["beta"], at["decay"], self.p("decay2.weight"), at["gate"], self.p("gate2.weight"), self.params["A_log"],
+                    self.params["dt_bias"], self.params["norm.weight"], self.norm_eps, out, H, self.num_kv_heads,
+                    self.head_dim, dv, self.decay == "channel", self.gate_activation) is not None:
+                return ops.linear(out, self.params["o.weight"], None, defer=True)
         qkv = torch.empty((T, C), dtype=torch.float32, device=x.device)
         ops.conv_silu_state(proj, C, self.params["conv.weight"], cache.state, ctx.cu_seqlens_q, ctx.slot_of_seq, qkv,
                             max_q_len=ctx.max_q_len)
         read = torch.empty((T, H, dv), dtype=torch.float32, device=x.device)
-        at = self._layout()[1]
         decay, decay_off = proj, at["decay"]
         if self.decay_low_rank:
             decay, decay_off = self._second(ops, proj, at["decay"], self.params["decay2.weight"]), 0

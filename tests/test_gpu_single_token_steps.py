@@ -1,0 +1,69 @@
+"""Kernels that take a decode step's single tokens through several operations in one launch, against the operations one by
+one in float64."""
+
+import pytest
+import torch
+
+from helpers import gpu_ops
+from plain_kernels import PlainKernels
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+PLAIN = PlainKernels()
+
+
+def rnd(shape, seed, scale=1.0):
+    return torch.randn(shape, generator=torch.Generator().manual_seed(seed)) * scale
+
+
+def i32(values):
+    return torch.tensor(values, dtype=torch.int32)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("per_channel,a_rank,g_rank,act", [(False, 0, 0, "silu"), (True, 64, 64, "sigmoid"), (True, 0, 16, "silu"),
+                                                           (False, 48, 0, "sigmoid"), (True, 16, 0, "silu")])
+@pytest.mark.parametrize("heads,kv_heads,dim", [(2, 2, 64), (6, 3, 64), (3, 3, 128), (4, 2, 128)])
+def test_delta_step(heads, kv_heads, dim, per_channel, a_rank, g_rank, act, dtype):
+    """Requests with and without a token, one that is padding; states beside theirs stay as they are."""
+    ops = gpu_ops()
+    lens, slots = [1, 1, 0, 1, 1], [4, 0, 2, -1, 1]
+    T, C, decays = sum(lens), (2 * kv_heads + heads) * dim, heads * (dim if per_channel else 1)
+    widths = [C, heads, a_rank or decays, g_rank or heads * dim]
+    b_off, a_off, g_off = C, C + heads, C + heads + widths[2]
+    proj = rnd((T, sum(widths) + 3), 1)
+    taps = rnd((C, 4), 2, 0.5).to(dtype)
+    decay2 = rnd((decays, a_rank), 3, 0.2).to(dtype) if a_rank else None
+    gate2 = rnd((heads * dim, g_rank), 4, 0.2).to(dtype) if g_rank else None
+    a_log, dt_bias, norm = rnd((heads,), 5, 0.5), rnd((decays,), 6) - 1, 1 + rnd((dim,), 7, 0.2)
+    off = 3 * C + 4
+    state = rnd((5, off + heads * dim * dim), 8, 0.3)
+    cu = i32([0, 1, 2, 2, 3, 4])
+
+    want_state, some, places = state.double(), i32([0, 1, 2, 3, 4]), i32([s for n, s in zip(lens, slots) if n])
+    qkv = torch.empty((T, C), dtype=torch.float64)
+    PLAIN.conv_silu_state(proj, C, taps, want_state, some, places, qkv)
+    decay, d_off = (proj, a_off) if decay2 is None else (proj[:, a_off:a_off + a_rank].double() @ decay2.double().T, 0)
+    gate, gate_off = (proj, g_off) if gate2 is None else (proj[:, g_off:g_off + g_rank].double() @ gate2.double().T, 0)
+    read = torch.empty((T, heads, dim), dtype=torch.float64)
+    PLAIN.delta_rule(qkv, proj, d_off, b_off, a_log, dt_bias, want_state, off, some, places, read, heads, kv_heads, dim, dim,
+                     decay=decay, per_channel=per_channel)
+    want = torch.empty((T, heads * dim), dtype=torch.float64)
+    PLAIN.delta_out(read, gate, gate_off, norm, 1e-5, want, activation=act)
+
+    dev = lambda t: None if t is None else t.to(DEV)  # noqa: E731
+    got, out = dev(state), torch.full((T, heads * dim), 7.0, dtype=dtype, device=DEV)
+    assert ops.delta_step(dev(proj), dev(taps), got, off, dev(cu), dev(i32(slots)), b_off, a_off, dev(decay2), g_off, dev(gate2),
+                          dev(a_log), dev(dt_bias), dev(norm), 1e-5, out, heads, kv_heads, dim, dim, per_channel, act) is out
+    # sums of up to 128 float32 terms; the output is rounded to its type
+    assert float((got.cpu().double() - want_state).norm() / want_state.norm()) <= 2e-6
+    assert float((out.cpu().double() - want).norm() / want.norm()) <= (4e-3 if dtype == torch.bfloat16 else 4e-6)
+    assert float(out[2].abs().max()) == 0
+    assert torch.equal(got[2:4].cpu(), state[2:4]), "slots 2 (no token) and 3 (no request) are not touched"
+
+
+def test_delta_step_leaves_other_sizes_alone():
+    ops = gpu_ops()
+    for sizes in ((4, 2, 32, 32, 4, 0, 0), (4, 2, 64, 128, 4, 0, 0), (6, 2, 64, 64, 4, 0, 0), (4, 2, 64, 64, 3, 0, 0),
+                  (4, 2, 64, 64, 4, 24, 0), (4, 2, 64, 64, 4, 0, 80)):
+        assert not ops.lib.atom_delta_step_supports(*sizes)
