@@ -264,7 +264,7 @@ class DecodeGraphs:
 
     # ------------------------------------------------------------------ capture and replay
 
-    def _capture(self, shape: tuple[int, int, int]) -> _Captured:
+    def _capture(self, shape: tuple[int, int, int], collect: bool = True) -> _Captured:
         core = self.core
         cap = _Captured(shape)
         total = self._layout(cap)
@@ -286,7 +286,8 @@ class DecodeGraphs:
         # No garbage collection while the stream is capturing: a collected tensor, event or older graph
         # frees device objects, which is not allowed during capture and aborts the process (the reference
         # pauses it for the same reason, atom/model_engine/model_runner.py:4046-4055).
-        gc.collect()
+        if collect:
+            gc.collect()
         gc_was_enabled = gc.isenabled()
         gc.disable()
         try:
@@ -305,20 +306,18 @@ class DecodeGraphs:
     def capture_all(self) -> int:
         """Captures every decode bucket now, largest first (atom/model_engine/model_runner.py:3973), so that no
         decode step of a running engine pays for a capture.  Returns how many graphs there are."""
-        if self.usable:
-            for size in sorted(self.sizes, reverse=True):
-                if (0, 0, size) not in self.captured:
-                    self._capture((0, 0, size))
-            for p in sorted(self.prefill_sizes, reverse=True):
-                for size in sorted(self.mixed_sizes, reverse=True):
-                    if (p, self.prefill_slots, size) not in self.captured:
-                        self._capture((p, self.prefill_slots, size))
+        shapes = [(0, 0, size) for size in sorted(self.sizes, reverse=True)]
+        shapes += [(p, self.prefill_slots, size) for p in sorted(self.prefill_sizes, reverse=True)
+                   for size in sorted(self.mixed_sizes, reverse=True)]
+        missing = [shape for shape in shapes if shape not in self.captured] if self.usable else []
+        for i, shape in enumerate(missing):
+            self._capture(shape, collect=i == 0)   # one collection (some 20 ms) before all of them
         return len(self.captured)
 
     def run(self, entries, cached: list[int]) -> torch.Tensor | None:
         """Float32 logits at the entries' wanted places (a portion's last row, a single token), in the
-        order of the entries; None if nothing is wanted.  The tensor is the graph's own output or a
-        selection of it, valid until the graph's next replay."""
+        order of the entries; None if nothing is wanted.  For a step of single tokens the tensor may be the graph's own
+        output, valid until the graph's next replay."""
         shape = self.shape_for(entries)
         cap = self.captured.get(shape) or self._capture(shape)
         logits_row = self._fill(cap, entries, cached)
@@ -332,7 +331,14 @@ class DecodeGraphs:
         picked = [row for row, e in zip(logits_row, entries) if e.want]
         if not picked:
             return None
-        if picked == list(range(len(picked))):
-            return cap.logits[:len(picked)]
-        index = torch.tensor(picked, dtype=torch.long, device=self.core.device)
-        return cap.logits.index_select(0, index)
+        # neighbouring rows as slices: an index array would be a copy from host memory that waits for the replay
+        runs = []
+        for row in picked:
+            if runs and runs[-1][1] == row:
+                runs[-1][1] = row + 1
+            else:
+                runs.append([row, row + 1])
+        parts = [cap.logits[lo:hi] for lo, hi in runs]
+        if len(parts) > 1:
+            return torch.cat(parts)
+        return parts[0].clone() if shape[0] else parts[0]

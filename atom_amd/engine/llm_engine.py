@@ -101,7 +101,7 @@ class LLMEngine:
             max_num_seqs=cfg.max_num_seqs, max_model_len=cfg.max_model_len,
             max_num_batched_tokens=cfg.max_num_batched_tokens,
             graph_sizes=None if cfg.enforce_eager else cfg.cudagraph_capture_sizes,
-            graph_prefill_sizes=cfg.cudagraph_prefill_sizes, graph_prefill_slots=cfg.cudagraph_prefill_slots,
+            graph_prefill_sizes=self._prefill_graph_sizes(), graph_prefill_slots=cfg.cudagraph_prefill_slots,
             prefix_caching=cfg.enable_prefix_caching)
         self._log_capacity()
         if self.core.graphs is not None:   # as the reference's engine does before it serves (engine_core.py:131-138)
@@ -139,6 +139,26 @@ class LLMEngine:
                     budget / 2**30)
         return budget
 
+    # Where no sizes are configured, steps with prompt portions are replayed if the token budget is at most this ...
+    SMALL_BUDGET_TOKENS = 128
+    # ... and a layer's weights are below this.  Launching a layer takes the host some 110 us (nine launches of 12 us, the
+    # step's arrays apart), working it some 36 us beside its bytes at 5 TB/s, and rows up to 128 are padded for next to
+    # nothing because the weights' bytes bound the products.  Three layers of 96 in float32, 16 tokens a step beside up to
+    # three decoding requests: 390 us launched, 95 replayed.
+    SMALL_LAYER_BYTES = 256 << 20
+
+    def _prefill_graph_sizes(self) -> list[int]:
+        """Portion sizes (tokens of a step's prompt portions together) that graphs are captured for."""
+        cfg = self.config
+        if cfg.cudagraph_prefill_sizes:
+            return list(cfg.cudagraph_prefill_sizes)
+        budget = min(cfg.max_num_batched_tokens, cfg.max_model_len or cfg.max_num_batched_tokens)
+        heaviest = max((sum(p.numel() * p.element_size() for part in block.walk() for p in part.params.values())
+                        for block in self.model.blocks), default=0)
+        if budget > self.SMALL_BUDGET_TOKENS or heaviest > self.SMALL_LAYER_BYTES:
+            return []
+        return sorted({n for n in (budget // 4, budget) if n >= 2})
+
     def _graph_estimate(self) -> int:
         """Bytes the decode graphs' shared pool will hold: every bucket keeps its float32 logits, and the
         buckets share the memory of one step's activations (what a layer frees during capture the next
@@ -150,12 +170,13 @@ class LLMEngine:
         widest = max((int(p.shape[0]) for block in self.model.blocks for part in block.walk()
                       for p in part.params.values() if p.dim() == 2), default=spec.hidden_size)
         rows, logits_rows = max(sizes), sum(sizes)
-        if cfg.cudagraph_prefill_sizes:
+        prefill_sizes = self._prefill_graph_sizes()
+        if prefill_sizes:
             # a graph per (portion tokens P, single tokens N >= 8): logits at the portion slots and the single
             # tokens, activations for P + N rows
             mixed = [s for s in sizes if s >= 8] or sizes[-1:]
-            logits_rows += len(cfg.cudagraph_prefill_sizes) * sum(cfg.cudagraph_prefill_slots + n for n in mixed)
-            rows = max(rows, max(cfg.cudagraph_prefill_sizes) + max(mixed))
+            logits_rows += len(prefill_sizes) * sum(cfg.cudagraph_prefill_slots + n for n in mixed)
+            rows = max(rows, max(prefill_sizes) + max(mixed))
         live = rows * (4 * spec.hidden_size + 8 * widest) * 4
         return logits_rows * spec.vocab_size * 4 + 2 * live + (128 << 20)
 
