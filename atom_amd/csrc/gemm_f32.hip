@@ -1,27 +1,38 @@
-// y[M, N] = x[M, K] * w[N, K]^T (+ bias[N]) in true float32: the matrix cores' float32 instructions, every product
-// and every sum in 32 bits.  X and W may be float32 or bfloat16 independently (read, widened, multiplied in float32).
+// y[M, N] = x[M, K] * w[N, K]^T (+ bias[N]) with float32 operands and float32 sums (X and W may be float32 or bfloat16
+// independently), on the matrix cores' bfloat16 instructions, whose rate is sixteen times that of the float32 ones.
 //
-// K is walked 16 terms at a time.  The 16 are summed apart and join the sum of their slice; K is cut into 8 slices, whose
-// sums are added four and four in order, then the two.  That order is the same whatever M is and whichever tile and kernel
-// a launch uses, so a row's result does not depend on its batch.
+// A float32 value is the sum of three bfloat16 pieces, hi + mid + lo, each the rounded rest of what the pieces before it
+// leave: 3 x 8 bits hold its 24.  A product of two values is the six products of pieces that reach its last bits (hi lo, lo
+// hi, mid mid, hi mid, mid hi, hi hi; the three left out are below 2^-24 of it, a rounding of float32, at most, and a
+// sixth of the sums' own roundings on average), each exact in float32 and added there.  An operand that is bfloat16 is one
+// piece.  Two kinds of results are summed again, term by term in float32: those that are not finite (a piece behind an
+// infinity is a NaN), and those below 1e-18 and not 0, whose operands may have pieces below bfloat16's range.
+//
+// K is walked 32 terms at a time.  The 32 are summed apart, smallest pieces first, and join the sum of their slice; K is cut
+// into 8 slices, whose sums are added four and four in order, then the two.  That order is the same whatever M is and
+// whichever tile and kernel a launch uses, so a row's result does not depend on its batch.  Against float64 (random normal
+// operands, 2-norm of the difference over that of the result): 9.9e-8 at K 4,096
+// and 1.43e-7 at 12,288, where the float32 instructions' sums of 16 terms are 1.38e-7 and 2.00e-7 off.
 //
 // A block is 8 waves, one a slice, all on the same output tile of 16 MT rows and 16 NT columns; a wave reads its
 // operands straight from memory into the registers that the matrix instructions take, DEPTH steps ahead of their use
-// (no LDS before the slices meet: at 64 x 64 a step's 8 KB feed 64 instructions of 32 cycles, so the caches keep up).
-// Few rows are bound by the weights' bytes: one row by 24,576 x 4,096 takes 71 us, 5.6 TB/s.  Many are bound by what the
-// loads cost (16 rows of 64 bytes an instruction) and take the kernel with LDS below where its tiles fill the chip, bound by
-// the float32 rate of the matrix cores.  (The multiply-add kernel of 64 x 64 tiles that these replaced: the products of two
-// 8B layers at 465 rows, once, and at 2 rows, four times, with the heads, took 44 ms, 7.0 now.)
+// (no LDS before the slices meet).  Few rows are bound by the weights' bytes: one row by 24,576 x 4,096 takes 69 us, 5.8 TB/s
+// (72 with the float32 instructions), 8 rows 74 (88), 32 rows 112 (120).  Many rows take the kernel
+// with LDS below where its tiles fill the chip.
 #include "common.h"
 #include "lds_loads.h"
 
+#include <type_traits>
+
 constexpr int kSlices = 8;      // slices of K, and waves of a block
-constexpr int kStep = 16;       // terms summed apart
+constexpr int kStep = 32;       // terms summed apart
+constexpr int kLane = 8;        // of them, those a lane brings
 constexpr int kXcds = 8;        // dies of the chip, each with an L2 of its own
 constexpr int kSide = 16;       // rows and columns of a matrix instruction
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef bf16_t bf16x4 __attribute__((ext_vector_type(4)));
+typedef bf16_t bf16x8 __attribute__((ext_vector_type(8)));
 
 struct GemmF32Params {
   const void* x;
@@ -31,6 +42,7 @@ struct GemmF32Params {
   int m, n, k;
   int row_tiles, tiles;
   int y_bf16;
+  const bf16_t* pieces;   // the wide kernel: x as three planes [m, k] of pieces
   int inter;   // SiLU-gate: w holds `inter` gate rows, then as many up rows (n = 2 inter); 0: a plain product
 };
 
@@ -43,51 +55,149 @@ __device__ __forceinline__ int row_of_w(const GemmF32Params& p, int at) {
 
 __device__ __forceinline__ float silu_times(float gate, float up) { return gate / (1.f + expf(-gate)) * up; }
 
-// How a row's terms are read, four at a time.  kWhole: K is a multiple of 16 and rows begin at multiples of four elements in
+// The pieces of a value; an operand that is bfloat16 has one.
+template <typename T>
+constexpr int kPieces = sizeof(T) == 4 ? 3 : 1;
+
+// (Two values at a time: the instruction that rounds takes two, and their widened pieces are its result's halves.)
+__device__ __forceinline__ void pieces_of(const float (&v)[kLane], bf16x8 (&p)[3]) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef bf16_t bf16x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int e = 0; e < kLane; e += 2) {
+    float a = v[e], b = v[e + 1];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const bf16x2 both = __builtin_convertvector(f32x2{a, b}, bf16x2);
+      p[i][e] = both[0];
+      p[i][e + 1] = both[1];
+      const unsigned bits = __builtin_bit_cast(unsigned, both);
+      a -= __uint_as_float(bits << 16);
+      b -= __uint_as_float(bits & 0xffff0000u);
+    }
+  }
+}
+
+// The products of pieces that are formed, smallest first: (piece of x, piece of w).
+template <int PX, int PW>
+struct Products;
+template <>
+struct Products<3, 3> {
+  static constexpr int count = 6, x[6] = {0, 2, 1, 0, 1, 0}, w[6] = {2, 0, 1, 1, 0, 0};
+};
+template <>
+struct Products<3, 1> {
+  static constexpr int count = 3, x[3] = {2, 1, 0}, w[3] = {0, 0, 0};
+};
+template <>
+struct Products<1, 3> {
+  static constexpr int count = 3, x[3] = {0, 0, 0}, w[3] = {2, 1, 0};
+};
+template <>
+struct Products<1, 1> {
+  static constexpr int count = 1, x[1] = {0}, w[1] = {0};
+};
+
+// The matrix instruction cuts its 32 products off below the largest one's last bits, downwards whatever their sign: a mean
+// error of its own, the same in all rows, which an average over rows (of values, by attention) does not take down with it.
+// Every other step of K is therefore formed from x's negatives and subtracted (without that 1.21e-7 and 1.87e-7 in the figures
+// above, but 9.1e-7 for 4.6e-7 in attention's averages over 300 rows).
+__device__ __forceinline__ unsigned flip_of(int step) { return step & 1 ? 0x80000000u : 0u; }
+__device__ __forceinline__ float sign_of(int step) { return step & 1 ? -1.f : 1.f; }
+
+// Whether a result is one of those that pieces may have spoilt, and the result summed in float32, in the kernels' order.
+__device__ __forceinline__ bool spoilt(float v) {
+  const float a = fabsf(v);
+  return !(a < INFINITY) || (a < 1e-18f && a > 0.f);
+}
+
+template <typename TX, typename TW>
+__device__ __noinline__ float summed_again(const TX* x, const TW* w, int k) {
+  const int steps = (k + kStep - 1) / kStep, share = (steps + kSlices - 1) / kSlices;
+  float total = 0.f, half = 0.f;
+  for (int slice = 0; slice < kSlices; ++slice) {
+    float sum = 0.f;
+    for (int step = slice * share; step < min((slice + 1) * share, steps); ++step) {
+      float part = 0.f;
+      for (int i = step * kStep; i < min((step + 1) * kStep, k); ++i) part = fmaf(to_f32(x[i]), to_f32(w[i]), part);
+      sum += part;
+    }
+    half = slice % (kSlices / 2) ? half + sum : sum;
+    if (slice % (kSlices / 2) == kSlices / 2 - 1) total = slice < kSlices / 2 ? half : total + half;
+  }
+  return total;
+}
+
+// How a row's terms are read, four at a time.  kWhole: K is a multiple of 32 and rows begin at multiples of 16 bytes in
 // memory.  kAny: any K from 4 on and any rows, with loads that need no more than their elements' alignment; the four that would
 // reach behind the row's end are its last four, which last_terms moves into place before they are used.  kTerms: term by
-// term, for the K below 4.  (4,096 columns at 2,048 rows, K 4,095, bfloat16 x: 1,867 us term by
-// term, 795 with loads of four; one row 36 and 17.)
+// term, for the K below 4.
 enum Loads : int { kTerms, kAny, kWhole };
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 typedef bf16_t bf16x4_any __attribute__((ext_vector_type(4), aligned(2)));
 
-template <typename T, int LOADS>
-__device__ __forceinline__ f32x4 four_terms(const T* __restrict__ row, int k0, int k) {
-  f32x4 v;
-  if constexpr (LOADS == kTerms) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = k0 + i < k ? to_f32(row[k0 + i]) : 0.f;
-  } else if constexpr (sizeof(T) == 4) {
-    if constexpr (LOADS == kWhole) v = *reinterpret_cast<const f32x4*>(row + k0);
-    else v = *reinterpret_cast<const f32x4_any*>(row + min(k0, k - 4));
-  } else {
-    bf16x4 h;
-    if constexpr (LOADS == kWhole) h = *reinterpret_cast<const bf16x4*>(row + k0);
-    else h = *reinterpret_cast<const bf16x4_any*>(row + min(k0, k - 4));
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = to_f32(h[i]);
-  }
-  return v;
-}
+// A lane's eight terms as they lie in memory: of a step's 32 terms from `k0` on lane quarter q brings four from 4 q on and four
+// from 16 + 4 q on, so that the quarters' reads lie side by side.  Operands agree on that order, which is all it takes.
+__device__ __forceinline__ int quad_at(int quarter, int h) { return 16 * h + 4 * quarter; }
 
-// The terms from k0 on of what four_terms<kAny> read: `late` (1 to 3, or more for none) of the four were read too early, and
-// zeros stand behind the row's end.
-__device__ __forceinline__ void last_terms(f32x4& v, int late) {
-  if (late & 1) v = f32x4{v[1], v[2], v[3], 0.f};
-  if (late & 2) v = f32x4{v[2], v[3], 0.f, 0.f};
-  if (late > 3) v = f32x4{0.f, 0.f, 0.f, 0.f};
-}
+template <typename T>
+struct Terms {
+  typedef typename std::conditional<sizeof(T) == 4, f32x4, bf16x4>::type Quad;
+  typedef typename std::conditional<sizeof(T) == 4, f32x4_any, bf16x4_any>::type QuadAny;
+  Quad q[2];
+
+  template <int LOADS>
+  __device__ __forceinline__ void read(const T* __restrict__ row, int k0, int quarter, int k) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int at = k0 + quad_at(quarter, h);
+      if constexpr (LOADS == kWhole) {
+        q[h] = *reinterpret_cast<const Quad*>(row + at);
+      } else if constexpr (LOADS == kAny) {
+        q[h] = *reinterpret_cast<const QuadAny*>(row + min(at, k - 4));
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) q[h][i] = at + i < k ? row[at + i] : from_f32<T>(0.f);
+      }
+    }
+  }
+  // After read<kAny> of the step from k0 on: four that were read too early (up to 3 places, or more for those that lie
+  // behind the row's end altogether) move into place, with zeros behind them.
+  __device__ __forceinline__ void last_terms(int k0, int quarter, int k) {
+    const T zero = from_f32<T>(0.f);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int late = max(k0 + quad_at(quarter, h) - (k - 4), 0);
+      if (late & 1) q[h] = Quad{q[h][1], q[h][2], q[h][3], zero};
+      if (late & 2) q[h] = Quad{q[h][2], q[h][3], zero, zero};
+      if (late > 3) q[h] = Quad{zero, zero, zero, zero};
+    }
+  }
+  // `flip`: the sign bit, or 0; with it the pieces are those of the terms' negatives.
+  __device__ __forceinline__ void pieces(bf16x8 (&p)[kPieces<T>], unsigned flip = 0) const {
+    if constexpr (sizeof(T) == 4) {
+      float v[kLane];
+#pragma unroll
+      for (int e = 0; e < kLane; ++e) v[e] = __uint_as_float(__float_as_uint(q[e / 4][e % 4]) ^ flip);
+      pieces_of(v, p);
+    } else {
+      typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+      const bf16x8 all = __builtin_shufflevector(q[0], q[1], 0, 1, 2, 3, 4, 5, 6, 7);
+      p[0] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, all) ^ (flip | flip >> 16));
+    }
+  }
+};
 
 template <typename TX, typename TW, int MT, int NT, int DEPTH, int LOADS>
 __global__ void __launch_bounds__(kSlices* kWave)
 gemm_f32_kernel(GemmF32Params p) {
+  using Order = Products<kPieces<TX>, kPieces<TW>>;
   __shared__ float met[kSlices][MT * kSide * kSide];
   const int tid = threadIdx.x;
   const int wave = tid / kWave;
   const int lane = tid % kWave;
   const int side = lane % kSide;       // the row of x and the row of w whose terms this lane brings
-  const int quarter = lane / kSide;    // which 4 of a step's 16 terms
+  const int quarter = lane / kSide;    // which 8 of a step's 32 terms
   // blocks go to the chip's XCDs in turn: each XCD gets a range of columns, with all their rows one after the other, so
   // that weights are read into one L2 only
   const int tile = blockIdx.x % kXcds * (gridDim.x / kXcds) + blockIdx.x / kXcds;
@@ -104,9 +214,8 @@ gemm_f32_kernel(GemmF32Params p) {
 
   const int steps = (p.k + kStep - 1) / kStep;
   const int share = (steps + kSlices - 1) / kSlices;
-  const int begin = min(wave * share, steps);
+  const int begin = __builtin_amdgcn_readfirstlane(min(wave * share, steps));
   const int count = __builtin_amdgcn_readfirstlane(min(begin + share, steps) - begin);
-
   const int ends = __builtin_amdgcn_readfirstlane(p.k / kStep - begin);   // kAny: the step that the row ends in
 
   f32x4 acc[MT][NT];
@@ -115,21 +224,18 @@ gemm_f32_kernel(GemmF32Params p) {
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // The largest tile asks for a later step's operands in every step, the last ones for the last step's again: with loads
-  // in all paths alike the compiler knows how many are in flight and waits for the oldest only (1,024 x 4,096 x 4,096:
-  // 388 us without, 336 with).  The small tiles are bound by what the loads cost and ask for nothing twice.
-  constexpr bool kSteady = MT * NT >= 16;
-  f32x4 a[DEPTH][MT], b[DEPTH][NT];
+  Terms<TX> a[DEPTH][MT];
+  Terms<TW> b[DEPTH][NT];
   const auto fetch = [&](int d, int step) {
-    const int at = min(begin + min(step, max(count - 1, 0)), steps - 1) * kStep + quarter * 4;
+    const int at = (begin + step) * kStep;
 #pragma unroll
-    for (int j = 0; j < NT; ++j) b[d][j] = four_terms<TW, LOADS>(wr[j], at, p.k);
+    for (int j = 0; j < NT; ++j) b[d][j].template read<LOADS>(wr[j], at, quarter, p.k);
 #pragma unroll
-    for (int i = 0; i < MT; ++i) a[d][i] = four_terms<TX, LOADS>(xr[i], at, p.k);
+    for (int i = 0; i < MT; ++i) a[d][i].template read<LOADS>(xr[i], at, quarter, p.k);
   };
 #pragma unroll
   for (int d = 0; d < DEPTH; ++d) {
-    if (kSteady || d < count) fetch(d, d);
+    if (d < count) fetch(d, d);
     __builtin_amdgcn_sched_barrier(0);
   }
   for (int base = 0; base < count; base += DEPTH) {
@@ -138,32 +244,36 @@ gemm_f32_kernel(GemmF32Params p) {
       if (base + d < count) {
         if constexpr (LOADS == kAny) {
           if (base + d == ends) {
-            const int late = max(p.k / kStep * kStep + quarter * 4 - (p.k - 4), 0);
+            const int at = p.k / kStep * kStep;
 #pragma unroll
-            for (int i = 0; i < MT; ++i) last_terms(a[d][i], late);
+            for (int i = 0; i < MT; ++i) a[d][i].last_terms(at, quarter, p.k);
 #pragma unroll
-            for (int j = 0; j < NT; ++j) last_terms(b[d][j], late);
+            for (int j = 0; j < NT; ++j) b[d][j].last_terms(at, quarter, p.k);
           }
         }
-        // term by term over all tiles: an instruction's sum is needed only MT NT instructions later
-        f32x4 part[MT][NT];
+        const float sign = sign_of(begin + base + d);
+        bf16x8 ap[MT][kPieces<TX>];
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
+        for (int i = 0; i < MT; ++i) a[d][i].pieces(ap[i], flip_of(begin + base + d));
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          bf16x8 bp[kPieces<TW>];
+          b[d][j].pieces(bp);
+          f32x4 part[MT];
+#pragma unroll
+          for (int t = 0; t < Order::count; ++t)
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+              part[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ap[i][Order::x[t]], bp[Order::w[t]],
+                                                                t ? part[i] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
           for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int j = 0; j < NT; ++j)
-              part[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                  a[d][i][t], b[d][j][t], t ? part[i][j] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-          for (int j = 0; j < NT; ++j)
-#pragma unroll
-            for (int t = 0; t < 4; ++t) acc[i][j][t] += part[i][j][t];
+            for (int t = 0; t < 4; ++t) acc[i][j][t] = fmaf(part[i][t], sign, acc[i][j][t]);
+        }
       }
       __builtin_amdgcn_sched_barrier(0);
-      if (kSteady || base + d + DEPTH < count) fetch(d, base + d + DEPTH);
+      if (base + d + DEPTH < count) fetch(d, base + d + DEPTH);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
@@ -177,7 +287,7 @@ gemm_f32_kernel(GemmF32Params p) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) met[wave][(i * kSide + quarter * 4 + t) * kSide + side] = acc[i][j][t];
     __syncthreads();
-    const auto sum_of = [&](int e) {
+    const auto sum_of = [&](int e) {   // entry e % 16 of row e / 16, of rows and columns that are there
       float sum = 0.f;
 #pragma unroll
       for (int half = 0; half < kSlices; half += kSlices / 2) {
@@ -185,6 +295,11 @@ gemm_f32_kernel(GemmF32Params p) {
 #pragma unroll
         for (int s = 1; s < kSlices / 2; ++s) part += met[half + s][e];
         sum = half ? sum + part : part;
+      }
+      if constexpr (kPieces<TX> * kPieces<TW> > 1) {
+        if (spoilt(sum))
+          sum = summed_again((const TX*)p.x + (size_t)(row0 + e / kSide) * p.k,
+                             (const TW*)p.w + (size_t)row_of_w(p, col0 + j * kSide + e % kSide) * p.k, p.k);
       }
       return sum;
     };
@@ -211,136 +326,190 @@ gemm_f32_kernel(GemmF32Params p) {
   }
 }
 
-// Many rows, float32 operands, K a multiple of 16: tiles of 64 rows and 128 columns whose operands go through LDS, in whole
-// cache lines straight from memory.  A block is two groups of four waves, each with four of the slices, a wave with 32 x 64
-// of the tile.  A stage is 32 terms of the tile's 192 rows, double buffered; the eight 16-byte pieces of a row change
-// places by its row number, so that the 16 rows a wave reads at once lie in different banks.  465 rows by 24,576 x 4,096
-// take 932 us, 100 TFLOP/s (1,039 in tiles of 64 x 64 without LDS), by 4,096 x 4,096 157 (177); 1,024 rows 110 TFLOP/s
-// (102).
-constexpr int kWideRows = 64, kWideCols = 128, kWideStage = 32;
-constexpr int kStageFloats = (kWideRows + kWideCols) * kWideStage;
+// Many rows, float32 operands, K a multiple of 32: tiles of 64 rows and 128 columns whose operands go through LDS, in whole
+// cache lines straight from memory.  x comes as planes of pieces, made once by a kernel of its own; pieces of w are formed by
+// the one wave that multiplies them.  A block is two groups of four waves, each with four of the slices, a wave with 64 x 32
+// of the tile, so that a step's splitting (two of w's 16-row parts) takes a third of the cycles of its 48 matrix
+// instructions; in 32 x 64 it would take more than they do.  A stage is 32 terms of the tile's 192 rows, double buffered; the
+// 16-byte pieces of a row change places by its row number, so that the rows a wave reads at once lie in different banks.
+// While a stage is multiplied, the next one's operands are read from LDS and the stage behind that comes from memory: 56 KB a
+// stage and CU, at the 35 to 40 KB a microsecond that a CU draws, are what bounds it.  465 rows by 24,576 x 4,096 take 645 us,
+// 145 TFLOP/s (945 with the float32 instructions, whose rate is 157 at most), by 4,096 x 4,096 109 (161), by 4,096 x 12,288
+// 305 (475).  Five stages in LDS with all eight waves on each (32 x 32 of the tile a wave) took 705, 120 and 340.
+constexpr int kWideRows = 64, kWideCols = 128;
+constexpr int kPlaneBytes = kWideRows * kStep * 2;                     // a stage of one plane of x
+constexpr int kStageBytes = 3 * kPlaneBytes + kWideCols * kStep * 4;
+
+__global__ void __launch_bounds__(256) split_f32_kernel(const float* __restrict__ x, bf16_t* __restrict__ pieces, size_t eights,
+                                                                  int steps) {
+  const size_t at = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (at >= eights) return;
+  Terms<float> v;   // four eights a step, in the order of the lanes' quarters
+  v.read<kWhole>(x + at / 4 * kStep, 0, at % 4, kStep);
+  bf16x8 p[3];
+  v.pieces(p, flip_of(at / 4 % steps));
+#pragma unroll
+  for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(pieces + (i * eights + at) * kLane) = p[i];
+}
 
 __global__ void __launch_bounds__(kSlices* kWave) gemm_f32_wide_kernel(GemmF32Params p) {
-  extern __shared__ __align__(16) float wide[];   // [group][buffer][kStageFloats]
+  extern __shared__ __align__(16) char wide[];   // [group][buffer][kStageBytes]: x's planes, then w
   const int tile = blockIdx.x % kXcds * (gridDim.x / kXcds) + blockIdx.x / kXcds;
   if (tile >= p.tiles) return;
   const int row0 = tile % p.row_tiles * kWideRows;
   const int col0 = tile / p.row_tiles * kWideCols;
   const int tid = threadIdx.x, lane = tid % kWave, side = lane % kSide, quarter = lane / kSide;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), group = wave / 4, w4 = wave % 4;
-  const int r0 = w4 % 2 * 32, c0 = kWideRows + w4 / 2 * 64;   // the wave's first row and column among the staged rows
 
   const int steps = p.k / kStep;
   const int share = (steps + kSlices - 1) / kSlices;
   const int low = min(steps, 4 * share);
   const int count = group ? steps - low : low;      // this group's steps
-  const int stages = (low + 1) / 2;
   const int k0 = group ? low * kStep : 0;
 
-  // piece `lane % 8` of row 8 (6 w4 + j) + lane / 8 in LDS holds the row's piece of that number turned by the row
-  constexpr int LOADS = (kWideRows + kWideCols) / 8 / 4;
-  const float* from[LOADS];
-  int at[LOADS];
+  // Loads of a stage: 16 rows of a plane of x each (piece `lane % 4` of a row in LDS is the row's piece of that number turned
+  // by the row), then 8 rows of w each (piece `lane % 8`).
+  constexpr int X_LOADS = 3 * kWideRows / 16, LOADS = (X_LOADS + kWideCols / 8) / 4;
+  const char* from[LOADS];
+  int size[LOADS];                                  // bytes of a term
 #pragma unroll
   for (int j = 0; j < LOADS; ++j) {
-    const int r = 8 * (LOADS * w4 + j) + lane / 8;
-    from[j] = r < kWideRows ? (const float*)p.x + (size_t)min(row0 + r, p.m - 1) * p.k
-                            : (const float*)p.w + (size_t)row_of_w(p, col0 + r - kWideRows) * p.k;
-    at[j] = k0 + (lane % 8 ^ (r >> 1 & 7)) * 4;
+    const int load = LOADS * w4 + j;
+    if (load < X_LOADS) {
+      const int r = load % 4 * 16 + lane / 4;
+      from[j] = (const char*)(p.pieces + ((size_t)(load / 4) * p.m + min(row0 + r, p.m - 1)) * p.k + k0 +
+                              (lane % 4 ^ (r >> 2 & 3)) * 8);
+      size[j] = 2;
+    } else {
+      const int r = (load - X_LOADS) * 8 + lane / 8;
+      from[j] = (const char*)((const float*)p.w + (size_t)row_of_w(p, col0 + r) * p.k + k0 + (lane % 8 ^ (r >> 1 & 7)) * 4);
+      size[j] = 4;
+    }
   }
-  float* mine = wide + group * 2 * kStageFloats;
-  const auto fetch = [&](int buffer, int stage) {
+  char* mine = wide + group * 2 * kStageBytes;
+  const auto fetch = [&](int buffer, int stage) {   // a group without steps of its own left reads its last stage again
+    const int term = min(stage, max(count - 1, 0)) * kStep;
 #pragma unroll
-    for (int j = 0; j < LOADS; ++j)   // pieces behind the row's end: its last again, never used
-      load_to_lds(from[j] + min(at[j] + stage * kWideStage, p.k - 4),
-                  lds_address(mine + buffer * kStageFloats + (LOADS * w4 + j) * 8 * kWideStage));
+    for (int j = 0; j < LOADS; ++j)
+      load_to_lds(from[j] + term * size[j], lds_address(mine + buffer * kStageBytes + (LOADS * w4 + j) * 1024));
   };
-  const auto piece = [&](const float* buffer, int r, int half) {
-    return *reinterpret_cast<const f32x4*>(buffer + r * kWideStage + ((4 * half + quarter) ^ (r >> 1 & 7)) * 4);
-  };
-  f32x4 acc[2][4], total[2][4];
+  f32x4 acc[4][2], total[4][2];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < 2; ++j) acc[i][j] = total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  fetch(0, 0);
+  using Order = Products<3, 3>;
+  struct Operands {
+    bf16x8 a[4][3];
+    Terms<float> b[2];
+  };
+  const auto read = [&](Operands& o, int stage) {
+    const char* xs = mine + (stage & 1) * kStageBytes;
+    const char* ws = xs + 3 * kPlaneBytes;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int r = 32 * w4 + 16 * j + side;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        o.b[j].q[h] = *reinterpret_cast<const f32x4*>(ws + r * kStep * 4 + ((quad_at(quarter, h) / 4) ^ (r >> 1 & 7)) * 16);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = 16 * i + side;
+#pragma unroll
+      for (int t = 0; t < 3; ++t)
+        o.a[i][t] = *reinterpret_cast<const bf16x8*>(xs + t * kPlaneBytes + r * kStep * 2 + (quarter ^ (r >> 2 & 3)) * 16);
+    }
+  };
   int until = share;                                // steps until the slice ends
-  for (int stage = 0; stage < stages; ++stage) {
-    arrived();
-    lds_barrier();                                  // the stage is there, the one before has been read
-    if (stage + 1 < stages) fetch(stage + 1 & 1, stage + 1);
-    const float* buffer = mine + (stage & 1) * kStageFloats;
-    f32x4 a2[2][2], b2[2][4];                       // both halves' operands at once: one wait for LDS a stage
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-#pragma unroll
-      for (int i = 0; i < 2; ++i) a2[half][i] = piece(buffer, r0 + 16 * i + side, half);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) b2[half][j] = piece(buffer, c0 + 16 * j + side, half);
-    }
+  const auto multiply = [&](const Operands& o, float sign, bool last) {
+    bf16x8 bp[2][3];
+    f32x4 part[2][4];
+    o.b[0].pieces(bp[0]);
     __builtin_amdgcn_sched_barrier(0);
+    o.b[1].pieces(bp[1]);
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      if (2 * stage + half < count) {
-        const f32x4(&a)[2] = a2[half];
-        const f32x4(&b)[4] = b2[half];
-        f32x4 part[2][4];
+    for (int j = 0; j < 2; ++j) {
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < Order::count; ++t)
 #pragma unroll
-          for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < 4; ++i)
+          part[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.a[i][Order::x[t]], bp[j][Order::w[t]],
+                                                               t ? part[j][i] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-              part[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][t], b[j][t], t ? part[i][j] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int t = 0; t < 4; ++t) acc[i][j][t] += part[i][j][t];
-        if (--until == 0 || 2 * stage + half + 1 == count) {
-          until = share;
-#pragma unroll
-          for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-#pragma unroll
-              for (int t = 0; t < 4; ++t) total[i][j][t] += acc[i][j][t];
-              acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-            }
-        }
-      }
+        for (int t = 0; t < 4; ++t) acc[i][j][t] = fmaf(part[j][i][t], sign, acc[i][j][t]);
     }
+    // matrix instructions with the second half's splitting, then the first half's adding up, between them
+#pragma unroll
+    for (int t = 0; t < 48; ++t) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+    }
+    if (--until == 0 || last) {
+      until = share;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+#pragma unroll
+          for (int t = 0; t < 4; ++t) total[i][j][t] += acc[i][j][t];
+          acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+  };
+  // A stage's operands are read from LDS while the stage before is multiplied; its buffer then takes the stage after next.
+  Operands even, odd;
+  if (count > 0) fetch(0, 0);
+  arrived();
+  lds_barrier();
+  if (count > 0) read(even, 0);
+  if (count > 1) fetch(1, 1);
+  const auto pass = [&](const Operands& now, Operands& next, int stage) {
+    arrived();
+    lds_barrier();                                  // the next stage is there, and all have read this one
+    __builtin_amdgcn_s_waitcnt(0xc07f);             // (the barrier's wait for LDS once more, for the compiler's count)
+    if (stage + 2 < count) fetch(stage & 1, stage + 2);
+    if (stage + 1 < count) read(next, stage + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    if (stage < count) multiply(now, sign_of(k0 / kStep + stage), stage + 1 == count);
+  };
+  for (int stage = 0; stage < low; stage += 2) {
+    pass(even, odd, stage);
+    if (stage + 1 < low) pass(odd, even, stage + 1);
   }
 
   // the second group's half of the sum joins the first's
   __syncthreads();
-  float* met = wide + w4 * 32 * 64;                 // the wave's 32 x 64
+  float* met = (float*)wide + w4 * 64 * 32;         // the wave's 64 x 32
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        float* there = met + (16 * i + 4 * quarter + t) * 64 + 16 * j + side;
+        float* there = met + (16 * i + 4 * quarter + t) * 32 + 16 * j + side;
         if (group) *there = total[i][j][t];
       }
   __syncthreads();
   if (group) return;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int at = col0 + c0 - kWideRows + 16 * j + side;
+    for (int j = 0; j < 2; ++j) {
+      const int at = col0 + 32 * w4 + 16 * j + side;
       const int c = p.inter == 0 ? at : at / kSide * 8 + side % 8;     // the column of y
       if (c >= (p.inter == 0 ? p.n : p.inter)) continue;               // (gate and up lanes of a column go together)
       const float bias = p.bias != nullptr ? p.bias[c + (p.inter != 0 && side >= 8 ? p.inter : 0)] : 0.f;
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        const int r = row0 + r0 + 16 * i + 4 * quarter + t;
+        const int r = row0 + 16 * i + 4 * quarter + t;
         if (r >= p.m) continue;
-        float sum = total[i][j][t] + met[(16 * i + 4 * quarter + t) * 64 + 16 * j + side];
+        float sum = total[i][j][t] + met[(16 * i + 4 * quarter + t) * 32 + 16 * j + side];
+        if (spoilt(sum))
+          sum = summed_again((const float*)p.x + (size_t)r * p.k, (const float*)p.w + (size_t)row_of_w(p, at) * p.k, p.k);
         if (p.bias != nullptr) sum += bias;
         if (p.inter != 0) {
           const float up = __shfl_xor(sum, 8);
@@ -354,20 +523,34 @@ __global__ void __launch_bounds__(kSlices* kWave) gemm_f32_wide_kernel(GemmF32Pa
     }
 }
 
-static int launch_gemm_f32_wide(GemmF32Params p, hipStream_t stream) {
-  p.row_tiles = (p.m + kWideRows - 1) / kWideRows;
-  const long tiles = (long)p.row_tiles * ((p.n + kWideCols - 1) / kWideCols);
-  if (tiles > 0x3fffffL) return ATOM_TOO_LARGE;
-  p.tiles = (int)tiles;
-  constexpr int bytes = 4 * kStageFloats * sizeof(float);
+// Rows of x that are split and multiplied at a time: what the pieces of as many take is all the scratch memory there is.
+constexpr int kSplitRows = 2048;
+
+static int launch_gemm_f32_wide(GemmF32Params p, void* scratch, hipStream_t stream) {
+  constexpr int bytes = 4 * kStageBytes;
+  static_assert(bytes <= 160 * 1024 && bytes >= 4 * 64 * 32 * 4, "the stages fit in LDS, and the second half of the sums there");
   static bool allowed = false;
   if (!allowed) {
     if (hipFuncSetAttribute((const void*)gemm_f32_wide_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess)
       return ATOM_LAUNCH_FAILED;
     allowed = true;
   }
-  hipLaunchKernelGGL(gemm_f32_wide_kernel, dim3((unsigned)(tiles + kXcds - 1) / kXcds * kXcds), dim3(kSlices * kWave), bytes,
-                     stream, p);
+  const int m = p.m, out = p.inter ? p.inter : p.n;
+  p.pieces = (const bf16_t*)scratch;
+  for (int first = 0; first < m; first += kSplitRows) {
+    p.m = min(kSplitRows, m - first);
+    p.row_tiles = (p.m + kWideRows - 1) / kWideRows;
+    const long tiles = (long)p.row_tiles * ((p.n + kWideCols - 1) / kWideCols);
+    const size_t eights = (size_t)p.m * p.k / kLane;
+    if (tiles > 0x3fffffL || eights / 256 > 0x3fffffL) return ATOM_TOO_LARGE;
+    p.tiles = (int)tiles;
+    hipLaunchKernelGGL(split_f32_kernel, dim3((unsigned)((eights + 255) / 256)), dim3(256), 0, stream, (const float*)p.x,
+                       (bf16_t*)scratch, eights, p.k / kStep);
+    hipLaunchKernelGGL(gemm_f32_wide_kernel, dim3((unsigned)(tiles + kXcds - 1) / kXcds * kXcds), dim3(kSlices * kWave), bytes,
+                       stream, p);
+    p.x = (const float*)p.x + (size_t)p.m * p.k;
+    p.y = (char*)p.y + (size_t)p.m * out * (p.y_bf16 ? 2 : 4);
+  }
   return launch_status();
 }
 
@@ -378,73 +561,86 @@ static int launch_gemm_f32(GemmF32Params p, hipStream_t stream) {
   if (tiles > 0x3fffffL) return ATOM_TOO_LARGE;   // 2^31 threads
   p.tiles = (int)tiles;
   const dim3 grid((unsigned)(tiles + kXcds - 1) / kXcds * kXcds), block(kSlices * kWave);
-  const bool whole = p.k % kStep == 0 && (uintptr_t)p.x % (4 * sizeof(TX)) == 0 && (uintptr_t)p.w % (4 * sizeof(TW)) == 0;
+  const bool whole = p.k % kStep == 0 && ((uintptr_t)p.x | (uintptr_t)p.w) % 16 == 0;
   if (whole)
     hipLaunchKernelGGL((gemm_f32_kernel<TX, TW, MT, NT, DEPTH, kWhole>), grid, block, 0, stream, p);
-  else if (MT * NT < 16 || p.k >= 4)
+  else if (p.k >= 4)
     hipLaunchKernelGGL((gemm_f32_kernel<TX, TW, MT, NT, DEPTH, kAny>), grid, block, 0, stream, p);
-  else if constexpr (MT * NT == 16)
+  else if constexpr (MT * NT == 1)
     hipLaunchKernelGGL((gemm_f32_kernel<TX, TW, MT, NT, DEPTH, kTerms>), grid, block, 0, stream, p);
   return launch_status();
 }
 
+// The width of the tiles of 64 rows that a product of more than 32 rows takes, the one whose rounds over the CUs take least: 16,
+// 32 or 64 columns, or, through LDS, 128.  A round takes 38, 46, 71 and 106 us at
+// K 4,096 (465 rows by 24,576: 48, 24, 12 and 6 rounds of 1,800, 1,100, 843 and 645 us in all).
+static int f32_columns(int m, int n, bool wide) {
+  const long cus = device_cus(), rows = (m + 63) / 64;
+  const auto cost = [&](int cols, int round) { return (rows * ((n + cols - 1) / cols) + cus - 1) / cus * round; };
+  const long c1 = cost(16, 38), c2 = cost(32, 46), c4 = cost(64, 71), c8 = cost(128, 106);
+  if (wide && c8 <= c4 && c8 <= c2 && c8 <= c1) return 128;
+  return c1 <= c2 && c1 <= c4 ? 16 : c2 <= c4 ? 32 : 64;
+}
+
+static bool f32_wide(const void* x, int x_dtype, const void* w, int w_dtype, int m, int n, int k) {
+  return x_dtype == ATOM_F32 && w_dtype == ATOM_F32 && m > 64 && k % kStep == 0 && ((uintptr_t)x | (uintptr_t)w) % 16 == 0 &&
+         f32_columns(m, n, true) == 128;
+}
+
 template <typename TX, typename TW>
 static int choose_gemm_f32(const GemmF32Params& p, hipStream_t stream) {
-  // Tiles two wide read x half as often, which pays from where there is one for most CUs on.  24,576 x 4,096, narrow and
-  // wide: 16 rows 111 and 93 us, 32 rows 155 and 116; 4,096 x 12,288 (128
-  // wide tiles): 32 rows 89 and 116 us.
-  if (p.k < 4) return launch_gemm_f32<TX, TW, 4, 4, 2>(p, stream);
+  // Tiles two wide read x half as often, which pays from where there is one for most CUs on.
+  if (p.k < 4) return launch_gemm_f32<TX, TW, 1, 1, 4>(p, stream);
   const long cus = device_cus();
   const bool wide_fills = p.n / 32 >= cus * 3 / 4;
   if (p.m <= 16) {
-    if (p.m > 4 && wide_fills) return launch_gemm_f32<TX, TW, 1, 2, 6>(p, stream);
-    return launch_gemm_f32<TX, TW, 1, 1, 8>(p, stream);
+    if (p.m > 4 && wide_fills) return launch_gemm_f32<TX, TW, 1, 2, 3>(p, stream);
+    return launch_gemm_f32<TX, TW, 1, 1, 4>(p, stream);
   }
   if (p.m <= 32) {
-    if (wide_fills) return launch_gemm_f32<TX, TW, 2, 2, 3>(p, stream);
-    return launch_gemm_f32<TX, TW, 2, 1, 6>(p, stream);
+    if (wide_fills) return launch_gemm_f32<TX, TW, 2, 2, 2>(p, stream);
+    return launch_gemm_f32<TX, TW, 2, 1, 3>(p, stream);
   }
-  // 64 rows: the width whose rounds over the CUs take least, a round's time being about 13, 22, 40 and, through LDS, 64
-  // for 16, 32, 64 and 128 columns (465 rows by 6,144 x 4,096: 384 of the widest tiles are two rounds, 317 us, 768 tiles of
-  // 64 three shorter ones, 272)
-  const long rows = (p.m + 63) / 64;
-  const auto cost = [&](int cols, int round) { return (rows * ((p.n + cols - 1) / cols) + cus - 1) / cus * round; };
-  const long c1 = cost(16, 13), c2 = cost(32, 22), c4 = cost(64, 40), c8 = cost(128, 64);
-  if constexpr (sizeof(TX) == 4 && sizeof(TW) == 4) {
-    const bool whole = p.k % kStep == 0 && ((uintptr_t)p.x | (uintptr_t)p.w) % 16 == 0;
-    if (p.m > 64 && whole && c8 <= c4 && c8 <= c2 && c8 <= c1) return launch_gemm_f32_wide(p, stream);
-  }
-  if (c1 <= c2 && c1 <= c4) return launch_gemm_f32<TX, TW, 4, 1, 4>(p, stream);
-  if (c2 <= c4) return launch_gemm_f32<TX, TW, 4, 2, 3>(p, stream);
-  return launch_gemm_f32<TX, TW, 4, 4, 2>(p, stream);
+  const int columns = f32_columns(p.m, p.n, false);
+  if (columns == 16) return launch_gemm_f32<TX, TW, 4, 1, 2>(p, stream);
+  if (columns == 32) return launch_gemm_f32<TX, TW, 4, 2, 2>(p, stream);
+  return launch_gemm_f32<TX, TW, 4, 4, 1>(p, stream);
 }
 
-ATOM_EXPORT int atom_gemm_f32(const void* x, int x_dtype, const void* w, int w_dtype, const float* bias, void* y,
-                              int y_dtype, int m, int n, int k, hipStream_t stream) {
-  if (m < 0 || n <= 0 || k <= 0) return ATOM_BAD_SHAPE;
-  if ((unsigned)x_dtype > 1u || (unsigned)w_dtype > 1u || (unsigned)y_dtype > 1u) return ATOM_BAD_DTYPE;
-  if (m == 0) return ATOM_OK;
-  const GemmF32Params p{x, w, bias, y, m, n, k, 0, 0, y_dtype == ATOM_BF16, 0};
+// Bytes of scratch memory that a product takes (its x as pieces); 0: none.
+ATOM_EXPORT long atom_gemm_f32_scratch(const void* x, int x_dtype, const void* w, int w_dtype, int m, int n, int k) {
+  if (m <= 0 || n <= 0 || k <= 0 || !f32_wide(x, x_dtype, w, w_dtype, m, n, k)) return 0;
+  return 6L * min(m, kSplitRows) * k;
+}
+
+static int gemm_f32(GemmF32Params p, int x_dtype, int w_dtype, void* scratch, hipStream_t stream) {
+  if (scratch != nullptr && f32_wide(p.x, x_dtype, p.w, w_dtype, p.m, p.n, p.k)) {
+    if ((uintptr_t)scratch % 16) return ATOM_BAD_SHAPE;
+    return launch_gemm_f32_wide(p, scratch, stream);
+  }
   switch (x_dtype * 2 + w_dtype) {
     case 0: return choose_gemm_f32<float, float>(p, stream);
     case 1: return choose_gemm_f32<float, bf16_t>(p, stream);
     case 2: return choose_gemm_f32<bf16_t, float>(p, stream);
     default: return choose_gemm_f32<bf16_t, bf16_t>(p, stream);
   }
+}
+
+// scratch: null, or atom_gemm_f32_scratch's bytes, aligned to 16 (without them the product takes the narrower tiles).
+ATOM_EXPORT int atom_gemm_f32(const void* x, int x_dtype, const void* w, int w_dtype, const float* bias, void* y,
+                              int y_dtype, int m, int n, int k, void* scratch, hipStream_t stream) {
+  if (m < 0 || n <= 0 || k <= 0) return ATOM_BAD_SHAPE;
+  if ((unsigned)x_dtype > 1u || (unsigned)w_dtype > 1u || (unsigned)y_dtype > 1u) return ATOM_BAD_DTYPE;
+  if (m == 0) return ATOM_OK;
+  return gemm_f32(GemmF32Params{x, w, bias, y, m, n, k, 0, 0, y_dtype == ATOM_BF16, nullptr, 0}, x_dtype, w_dtype, scratch, stream);
 }
 
 // y[M, inter] = silu(x wg^T + bg) * (x wu^T + bu), float32, for w of `inter` gate rows and then as many up rows: the sums of
 // the plain product, gated where they are written instead of in a launch of their own that reads them back.
 ATOM_EXPORT int atom_gemm_f32_gate(const void* x, int x_dtype, const void* w, int w_dtype, const float* bias, float* y, int m,
-                                   int inter, int k, hipStream_t stream) {
+                                   int inter, int k, void* scratch, hipStream_t stream) {
   if (m < 0 || inter <= 0 || inter > 0x3fffffff || k <= 0) return ATOM_BAD_SHAPE;
   if ((unsigned)x_dtype > 1u || (unsigned)w_dtype > 1u) return ATOM_BAD_DTYPE;
   if (m == 0) return ATOM_OK;
-  const GemmF32Params p{x, w, bias, y, m, 2 * inter, k, 0, 0, 0, inter};
-  switch (x_dtype * 2 + w_dtype) {
-    case 0: return choose_gemm_f32<float, float>(p, stream);
-    case 1: return choose_gemm_f32<float, bf16_t>(p, stream);
-    case 2: return choose_gemm_f32<bf16_t, float>(p, stream);
-    default: return choose_gemm_f32<bf16_t, bf16_t>(p, stream);
-  }
+  return gemm_f32(GemmF32Params{x, w, bias, y, m, 2 * inter, k, 0, 0, 0, nullptr, inter}, x_dtype, w_dtype, scratch, stream);
 }

@@ -225,6 +225,7 @@ class HipKernels:
                    "atom_delta_chunks", "atom_delta_chunks_supports", "atom_delta_step", "atom_delta_step_supports"):
             getattr(self.lib, fn).restype = ctypes.c_int
         self.lib.atom_delta_chunks_floats.restype = ctypes.c_long
+        self.lib.atom_gemm_f32_scratch.restype = ctypes.c_long
         self.allow_library_gemm = True
         # bfloat16 products of few rows run this library's own weight-streaming kernels: up to 64 rows, and
         # up to 128 for the narrow products that atom_gemm_skinny_supports names; the BLAS library takes the rest.
@@ -908,8 +909,15 @@ class HipKernels:
         y = torch.empty((m, n), dtype=out_dtype, device=x.device)
         self._done("gemm_f32", self.lib.atom_gemm_f32(
             _ptr(x), _DTYPE_CODE[x.dtype], _ptr(weight), _DTYPE_CODE[weight.dtype], _ptr(bias), _ptr(y), self._code(y), m, n, k,
-            self._stream()))
+            _ptr(self._f32_scratch(x, weight, m, n, k)), self._stream()))
         return y
+
+    def _f32_scratch(self, x, weight, m: int, n: int, k: int) -> torch.Tensor | None:
+        """Scratch memory of a float32 product with ``n`` rows of weights: the pieces of ``x`` where its tiles read those."""
+        if m <= 64 or x.dtype != torch.float32 or weight.dtype != torch.float32:
+            return None
+        size = self.lib.atom_gemm_f32_scratch(_ptr(x), F32, _ptr(weight), F32, m, n, k)
+        return torch.empty(size, dtype=torch.uint8, device=x.device) if size else None
 
     _ROWS_GATE_ACT = {"silu": 0, "relu": 2, "gelu_tanh": 3}
     _ROWS_ACT = {"silu": 1, "relu": 2, "gelu_tanh": 3, "relu_squared": 4, "tanh": 5}
@@ -984,7 +992,8 @@ class HipKernels:
                 self._check("linear bias", bias, torch.float32, (two,))
             act = torch.empty((m, inter), dtype=x.dtype, device=x.device)
             self._done("gemm_f32_gate", self.lib.atom_gemm_f32_gate(
-                _ptr(x), F32, _ptr(weight), self._code(weight), _ptr(bias), _ptr(act), m, inter, k, self._stream()))
+                _ptr(x), F32, _ptr(weight), self._code(weight), _ptr(bias), _ptr(act), m, inter, k,
+                _ptr(self._f32_scratch(x, weight, m, two, k)), self._stream()))
             return act
         gate_up = self.linear(x, weight, bias)
         act = torch.empty((m, inter), dtype=x.dtype, device=x.device)

@@ -1,0 +1,66 @@
+"""Float32 products as sums of bfloat16 pieces: the products through LDS and without agree to the bit, their error is that of
+float32 sums, and operands whose pieces say nothing (infinities, NaN, numbers near the ends of the range) are summed again."""
+
+import pytest
+import torch
+
+from helpers import gpu_ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def rnd(shape, seed, scale=1.0):
+    return (torch.randn(shape, generator=torch.Generator().manual_seed(seed)) * scale).to(DEV)
+
+
+def through_lds(ops, x, w):
+    return ops._f32_scratch(x, w, x.shape[0], w.shape[0], x.shape[1]) is not None
+
+
+# K of one step, of a last slice that is short, of slices that are empty; rows and columns at the edges of tiles; two portions
+@pytest.mark.parametrize("m,n,k", [(449, 4099, 32), (449, 4096, 288), (512, 4100, 1056), (2112, 4096, 64), (465, 8192, 4096)])
+def test_wide_products_round_like_narrow_ones(m, n, k):
+    ops = gpu_ops()
+    x, w, b = rnd((m, k), 1), rnd((n, k), 2), rnd((n,), 3)
+    assert through_lds(ops, x, w)
+    y = ops.linear(x, w, b)
+    want = x.double() @ w.double().T + b.double()
+    assert float((y.double() - want).norm() / want.norm()) <= 2.0 ** -24 * (4 + (k / 128) ** 0.5)
+    if k >= 1024:   # what is off is off independently row by row: the rows' mean is off by less (three deviations of it)
+        off = y.double() - want
+        assert float(off.mean(0).norm()) <= 3 * float(off.norm()) / m
+    for rows in (slice(0, 1), slice(m - 1, m), slice(m // 2, m // 2 + 20)):
+        assert torch.equal(ops.linear(x[rows].contiguous(), w, b), y[rows])
+    gate = ops.linear_silu(x, w[:n // 2 * 2].contiguous())
+    assert torch.equal(ops.linear_silu(x[:3].contiguous(), w[:n // 2 * 2].contiguous()), gate[:3])
+
+
+@pytest.mark.parametrize("m,n,k", [(3, 70, 96), (449, 4096, 96)])
+def test_values_that_pieces_cannot_hold(m, n, k):
+    ops = gpu_ops()
+    x, w = rnd((m, k), 1), rnd((n, k), 2)
+    inf, nan = float("inf"), float("nan")
+    x[0, 5], x[1, 7], x[2, 9] = inf, nan, 3.4e38          # hi of the last is infinite
+    w[:, 9] *= 1e-6
+    w[3, 5], w[4, 5], w[5, 11], w[6, 13] = 0.0, -1.0, -inf, nan
+    y = ops.linear(x, w).cpu()
+    terms = x.cpu().double()[:, None] * w.cpu().double()[None, :40]
+    want = terms.sum(-1)
+    assert torch.equal(y[:, :40].isnan(), want.isnan()) and torch.equal(y[:, :40].isinf(), want.isinf())
+    held = want.isfinite()
+    off = (y[:, :40].double() - want).abs()
+    assert bool((off <= (32 + k / 32) * 2.0 ** -24 * terms.abs().sum(-1))[held].all())
+    if m <= 40:
+        assert int(held.sum()) > 10
+
+
+@pytest.mark.parametrize("m,n,k", [(3, 70, 96), (449, 4096, 96)])
+def test_numbers_below_the_range_of_pieces(m, n, k):
+    ops = gpu_ops()
+    x, w = rnd((m, k), 1, 2.0 ** -118), rnd((n, k), 2)
+    x[1] = 0.0
+    y = ops.linear(x, w).cpu()
+    terms = x.cpu().double()[:, None] * w.cpu().double()[None, :40]
+    assert float(y[1].abs().max()) == 0
+    assert bool(((y[:, :40].double() - terms.sum(-1)).abs() <= (32 + k / 32) * 2.0 ** -24 * terms.abs().sum(-1) + 2.0 ** -149).all())
