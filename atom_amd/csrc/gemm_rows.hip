@@ -49,6 +49,10 @@ struct RowsParams {
   int act;               // plain: an activation on the product (0 none, 1 SiLU, 2 ReLU, 3 tanh-GELU, 4 ReLU squared, 5 tanh);
                          // gate: that of the gate (0 SiLU, 2, 3)
   float eps;
+  const bf16_t* times;   // plain: [times_rows, times_ld] at its first column; the product times row times_ids[m] of it (0 for
+  const int* times_ids;  // an id that is no row), or null
+  long times_ld;
+  int times_rows;
 };
 
 __device__ __forceinline__ float tanh_gelu(float v) {
@@ -256,6 +260,10 @@ __global__ void __launch_bounds__(512, (MR > 4 ? 3 : 4)) gemm_rows_kernel(RowsPa
     else if (p.act == 3) v = tanh_gelu(v);
     else if (p.act == 4) v = fmaxf(v, 0.f) * fmaxf(v, 0.f);
     else if (p.act == 5) v = tanhf(v);
+    if (p.times) {
+      const int id = p.times_ids[m];
+      v *= (unsigned)id < (unsigned)p.times_rows ? to_f32(p.times[(size_t)id * p.times_ld + col]) : 0.f;
+    }
     if (p.out_f32) reinterpret_cast<float*>(p.y)[(size_t)m * p.n + col] = v;
     else reinterpret_cast<bf16_t*>(p.y)[(size_t)m * p.n + col] = from_f32<bf16_t>(v);
   }
@@ -287,7 +295,8 @@ ATOM_EXPORT int atom_gemm_rows_supports(int m, int n, int k) {
 
 // mode 0 (plain): y [m, n], bfloat16 or float32 (out_f32), act(product + bias) with act 1 SiLU, 2 ReLU, 3 tanh-GELU,
 // 4 the square of ReLU, 5 tanh (0: none); `batch` > 1: that many products of the same sizes side by side, product b
-// reading x + b batch_x and w + b batch_w and writing y + b batch_y (elements; no bias, row choice or pending norm).   mode 1 (gate): w is [2 n, k], y [m, n] bfloat16,
+// reading x + b batch_x and w + b batch_w and writing y + b batch_y (elements; no bias, row choice or pending norm); `times`:
+// row times_ids[i] of a bfloat16 table multiplies row i after the activation.   mode 1 (gate): w is [2 n, k], y [m, n] bfloat16,
 // act the gate's activation (0 SiLU, 2 ReLU, 3 tanh-GELU).
 // mode 2 (residual): res [m, n] float32 += product, ss_out [m, atom_gemm_rows_parts(n, cols)], and, with g_next [n],
 // xg_out [m, n] = bf16(res * g_next).
@@ -300,7 +309,7 @@ ATOM_EXPORT int atom_gemm_rows(const void* x, const int* rows, const float* ss, 
                                const float* bias, void* y, float* res, float* ss_out, void* xg_out,
                                const float* g_next, int m, int n, int k, int mode, int out_f32, int cols,
                                int waves_override, int act, int batch, long batch_x, long batch_w, long batch_y,
-                               hipStream_t stream) {
+                               const void* times, const int* times_ids, long times_ld, int times_rows, hipStream_t stream) {
   if (m < 0 || n <= 0 || k <= 0 || mode < 0 || mode > 2) return ATOM_BAD_SHAPE;
   if (act < 0 || act > 5 || (mode == ROWS_GATE && act != 0 && act != 2 && act != 3)) return ATOM_UNSUPPORTED;
   if (act != 0 && mode == ROWS_RESIDUAL) return ATOM_UNSUPPORTED;
@@ -308,6 +317,7 @@ ATOM_EXPORT int atom_gemm_rows(const void* x, const int* rows, const float* ss, 
   if (batch > 1 && (mode != ROWS_PLAIN || rows || ss || bias || (batch_x % 8) || (batch_w % 8))) return ATOM_UNSUPPORTED;
   if (!rows_cols_ok(cols) || (mode == ROWS_GATE && cols != 16)) return ATOM_UNSUPPORTED;
   if (!atom_gemm_rows_supports(max(m, 1), n, k)) return ATOM_UNSUPPORTED;
+  if (times && (mode != ROWS_PLAIN || batch > 1 || !times_ids || times_ld < n || times_rows < 1)) return ATOM_BAD_SHAPE;
   if (m == 0) return ATOM_OK;
   if (!x || !w || (ss && ss_parts < 1)) return ATOM_BAD_SHAPE;
   if (mode == ROWS_RESIDUAL ? (!res || !ss_out || (xg_out && !g_next)) : !y) return ATOM_BAD_SHAPE;
@@ -322,6 +332,7 @@ ATOM_EXPORT int atom_gemm_rows(const void* x, const int* rows, const float* ss, 
   p.tiles = rows_tiles(n, mode, cols);
   p.cols = cols;
   p.act = act;
+  p.times = (const bf16_t*)times; p.times_ids = times_ids; p.times_ld = times_ld; p.times_rows = times_rows;
   p.batch_x = batch_x; p.batch_w = batch_w; p.batch_y = batch_y;
   int waves = rows_waves(m, p.tiles, k);
   if (waves_override == 4 || waves_override == 8) waves = waves_override;

@@ -174,3 +174,152 @@ ATOM_EXPORT int atom_rglru_scan(const float* u, const float* gr, const float* gi
                                                      slot_of_seq, (T*)out, channels, scale));
   return launch_status();
 }
+
+// ------------------------------------------------------------------ a decode step: one token a request
+//
+// From the projection's columns to the gated output in two launches instead of four (convolution, the gates' two products,
+// the scan; each some 4 us of a decode step whatever it does).  The first forms both gates' products; every one of its
+// blocks convolves the inputs of its channels anew (four values a channel) and nothing is moved up, so the second, which has
+// a channel a thread, finds the carried inputs as they were, convolves its own channel, and alone moves them up.
+// Width 2,048 in 8 blocks of 256, one request: 16.3 us with the gaps between launches, 8.6 so.
+
+constexpr int kStepTaps = 4;
+constexpr int kStepSeqs = 8;       // the most requests of a step
+constexpr int kStepCols = 8;       // channels of a block whose gates it forms
+
+struct RglruStep {
+  const float* proj;               // [tokens, ld]: the input branch, then the other at y_off
+  long ld;
+  const void* taps;                // [channels, 4]
+  const float* conv_bias;
+  float* state;                    // a slot's row: [3, channels] carried inputs, S at state_off
+  long slot_stride, state_off;
+  const int* cu_seqlens;
+  const int* slot_of_seq;
+  const void* ra;                  // [blocks, part, part]
+  const void* ri;
+  const float* br;
+  const float* bi;
+  const float* lam;
+  float* gates;                    // [2, tokens, channels]
+  void* out;
+  int num_seqs, tokens, channels, part, y_off;
+  float scale;
+};
+
+// The convolved input of channel c, and (win) what the request carries of it.
+template <typename T>
+__device__ __forceinline__ float convolved(const RglruStep& p, int t, int slot, int c, float (&win)[kStepTaps]) {
+  const float* tail = p.state + (size_t)slot * p.slot_stride;
+  win[kStepTaps - 1] = p.proj[(size_t)t * p.ld + c];
+#pragma unroll
+  for (int j = 0; j < kStepTaps - 1; ++j) win[j] = tail[(size_t)j * p.channels + c];
+  const Four<T> w = reinterpret_cast<const Four<T>*>(p.taps)[c];
+  float s = 0.f;
+#pragma unroll
+  for (int j = 0; j < kStepTaps; ++j) s = fmaf(to_f32(w.at[j]), win[j], s);
+  return s + p.conv_bias[c];
+}
+
+// grid (part / 8, blocks); PL: weights of a row that a lane holds, part / 64.  A wave forms four of the block's sixteen
+// products (8 channels, 2 gates), each of a row of weights with every request's channels.
+template <typename T, int PL>
+__global__ void __launch_bounds__(256) rglru_step_gates_kernel(RglruStep p) {
+  constexpr int PART = PL * kWave, OUTS = 2 * kStepCols / 4;
+  __shared__ float us[kStepSeqs][PART];
+  struct alignas(PL * sizeof(T)) Lane { T at[PL]; };
+  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+  const int c0 = blockIdx.y * PART;
+  Lane w[OUTS];
+#pragma unroll
+  for (int o = 0; o < OUTS; ++o) {
+    const int which = wave * OUTS + o, col = blockIdx.x * kStepCols + which % kStepCols;
+    w[o] = *reinterpret_cast<const Lane*>((const T*)(which < kStepCols ? p.ra : p.ri) + ((size_t)c0 + col) * PART + lane * PL);
+  }
+  for (int s = 0; s < p.num_seqs; ++s) {
+    const int t = p.cu_seqlens[s], slot = p.slot_of_seq[s];
+    if (slot < 0 || p.cu_seqlens[s + 1] == t) continue;
+    for (int c = tid; c < PART; c += 256) {
+      float win[kStepTaps];
+      us[s][c] = convolved<T>(p, t, slot, c0 + c, win);
+    }
+  }
+  __syncthreads();
+  for (int s = 0; s < p.num_seqs; ++s) {
+    const int t = p.cu_seqlens[s];
+    if (p.slot_of_seq[s] < 0 || p.cu_seqlens[s + 1] == t) continue;
+    float u[PL];
+#pragma unroll
+    for (int e = 0; e < PL; ++e) u[e] = us[s][lane * PL + e];
+#pragma unroll
+    for (int o = 0; o < OUTS; ++o) {
+      const int which = wave * OUTS + o, col = blockIdx.x * kStepCols + which % kStepCols;
+      float sum = 0.f;
+#pragma unroll
+      for (int e = 0; e < PL; ++e) sum = fmaf(u[e], to_f32(w[o].at[e]), sum);
+      sum = wave_sum(sum);
+      if (lane == 0) p.gates[((size_t)(which < kStepCols ? 0 : p.tokens) + t) * p.channels + c0 + col] = sum;
+    }
+  }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(64) rglru_step_kernel(RglruStep p) {
+  const int c = blockIdx.x * 64 + threadIdx.x, s = blockIdx.y;
+  const int t = p.cu_seqlens[s], slot = p.slot_of_seq[s];
+  if (c >= p.channels || p.cu_seqlens[s + 1] == t) return;
+  T* out = (T*)p.out + (size_t)t * p.channels + c;
+  if (slot < 0) {
+    *out = from_f32<T>(0.f);
+    return;
+  }
+  float* row = p.state + (size_t)slot * p.slot_stride;
+  const float l = p.lam[c], S0 = row[p.state_off + c], y = p.proj[(size_t)t * p.ld + p.y_off + c];
+  const float gr = p.gates[(size_t)t * p.channels + c], gi = p.gates[((size_t)p.tokens + t) * p.channels + c];
+  float win[kStepTaps];
+  const float u = convolved<T>(p, t, slot, c, win);
+  const float rate = -p.scale * (l > 20.f ? l : log1pf(expf(l)));
+  const Step step = token_step(gr, gi, u, p.br[c], p.bi[c], rate);
+  const float S = fmaf(step.a, S0, step.b);
+  *out = from_f32<T>(S * gelu_tanh_y(y));
+  row[p.state_off + c] = S;
+#pragma unroll
+  for (int j = 0; j < kStepTaps - 1; ++j) row[(size_t)j * p.channels + c] = win[j + 1];
+}
+
+// 1 if the kernels take these sizes.
+ATOM_EXPORT int atom_rglru_step_supports(int num_seqs, int channels, int part, int taps) {
+  return num_seqs >= 1 && num_seqs <= kStepSeqs && taps == kStepTaps && (part == 64 || part == 128 || part == 256 || part == 512) &&
+         channels > 0 && channels % part == 0 && channels / part <= 65535;
+}
+
+// Requests bring one token each, or none; taps, ra, ri and out of the type `dtype`, whose tensors begin at multiples of 16 bytes.
+ATOM_EXPORT int atom_rglru_step(const float* proj, long ld, int y_off, const void* taps, const float* conv_bias, int dtype,
+                                float* state, long slot_stride, long state_off, const int* cu_seqlens, const int* slot_of_seq,
+                                int num_seqs, int tokens, const void* ra, const void* ri, const float* br, const float* bi,
+                                const float* lam, float* gates, void* out, int channels, int part, float scale,
+                                hipStream_t stream) {
+  if (!atom_rglru_step_supports(num_seqs, channels, part, kStepTaps)) return ATOM_UNSUPPORTED;
+  if ((unsigned)dtype > 1u) return ATOM_BAD_DTYPE;
+  if (ld < channels || y_off < 0 || y_off + channels > ld || tokens < 0 || tokens > num_seqs) return ATOM_BAD_SHAPE;
+  if (state_off < (long)(kStepTaps - 1) * channels || slot_stride < state_off + channels) return ATOM_BAD_SHAPE;
+  if (!proj || !taps || !conv_bias || !state || !cu_seqlens || !slot_of_seq || !ra || !ri || !br || !bi || !lam || !gates || !out)
+    return ATOM_BAD_SHAPE;
+  if (((uintptr_t)taps | (uintptr_t)ra | (uintptr_t)ri) & 15) return ATOM_BAD_SHAPE;
+  if (tokens == 0) return ATOM_OK;
+  const RglruStep p{proj, ld, taps, conv_bias, state, slot_stride, state_off, cu_seqlens, slot_of_seq, ra, ri, br, bi, lam,
+                    gates, out, num_seqs, tokens, channels, part, y_off, scale};
+  const dim3 grid(part / kStepCols, channels / part);
+#define GO(PL) hipLaunchKernelGGL((rglru_step_gates_kernel<T, PL>), grid, dim3(256), 0, stream, p)
+  ATOM_DISPATCH_DTYPE(dtype, {
+    switch (part) {
+      case 64: GO(1); break;
+      case 128: GO(2); break;
+      case 256: GO(4); break;
+      default: GO(8); break;
+    }
+    hipLaunchKernelGGL((rglru_step_kernel<T>), dim3((channels + 63) / 64, num_seqs), dim3(64), 0, stream, p);
+  });
+#undef GO
+  return launch_status();
+}

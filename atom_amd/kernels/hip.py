@@ -176,6 +176,7 @@ class PendingProduct:
 
 _void_p = ctypes.c_void_p
 _NO_SLICES = (None, 0, ctypes.c_long(0), None)
+_NO_FACTOR = (None, None, ctypes.c_long(0), 0)
 
 
 def _ptr(t: torch.Tensor | None):
@@ -222,7 +223,8 @@ class HipKernels:
                    "atom_attention_together", "atom_attention_together_tiles", "atom_attention_together_tiles_supports",
                    "atom_together_sum_parts", "atom_streams_step", "atom_embedding_sinusoid", "atom_softcap_rows",
                    "atom_selective_scan", "atom_step_sizes", "atom_experts_few", "atom_experts_few_supports", "atom_keys_as_values_heads_write",
-                   "atom_delta_chunks", "atom_delta_chunks_supports", "atom_delta_step", "atom_delta_step_supports"):
+                   "atom_delta_chunks", "atom_delta_chunks_supports", "atom_delta_step", "atom_delta_step_supports",
+                   "atom_rglru_step", "atom_rglru_step_supports"):
             getattr(self.lib, fn).restype = ctypes.c_int
         self.lib.atom_delta_chunks_floats.restype = ctypes.c_long
         self.lib.atom_gemm_f32_scratch.restype = ctypes.c_long
@@ -250,6 +252,7 @@ class HipKernels:
         self.use_fused_decode = True    # decode-only steps of few rows: norm, rotation and cache write inside attention
         self.use_delta_chunks = True   # the delta rule of prompts in chunks of 64 tokens
         self.use_delta_step = True     # ... and of single tokens in one launch with what is before and behind it
+        self.use_rglru_step = True     # the real-gated recurrence of single tokens in two launches
         self.use_together_tiles = True  # attention with the heads together on the matrix cores, for prompt portions
         self.use_mfma_latent = True     # attention over latent pages on the matrix cores (bfloat16, sizes it is built for)
         self.use_latent_tiles = True    # ... its form for a latent of 128, 256 or 512 entries and 64 rotated ones
@@ -468,7 +471,7 @@ class HipKernels:
         return folded <= split
 
     def _rows_launch(self, x, weight, bias, mode: int, y=None, res=None, ss_out=None, xg_out=None, g_next=None,
-                     out_f32: bool = False, act: int = 0):
+                     out_f32: bool = False, act: int = 0, times=None):
         m, k = x.shape
         n = weight.shape[0] // 2 if mode == 1 else weight.shape[0]
         self._check("linear weight", weight, torch.bfloat16, (weight.shape[0], k))
@@ -483,10 +486,18 @@ class HipKernels:
         else:
             self._check("linear input", x, torch.bfloat16, (m, k))
             head = (_ptr(x), None, None, 0, ctypes.c_float(0.0))
+        factor = _NO_FACTOR
+        if times is not None:
+            table, col_off, ids = times
+            self._check("table of factors", table, torch.bfloat16, (None, None))
+            self._check("rows of factors", ids, torch.int32, (m,))
+            if col_off < 0 or col_off + n > table.shape[1]:
+                raise KernelError("linear: the columns asked for are not in the table of factors")
+            factor = self._at(table, col_off), _ptr(ids), ctypes.c_long(table.shape[1]), table.shape[0]
         self._done("gemm_rows", self.lib.atom_gemm_rows(
             *head, _ptr(weight), _ptr(bias), _ptr(y), _ptr(res), _ptr(ss_out), _ptr(xg_out), _ptr(g_next), m, n, k,
             mode, int(out_f32), 16 if mode == 1 else self.rows_cols(n), int(self.rows_waves), act, 1, ctypes.c_long(0),
-            ctypes.c_long(0), ctypes.c_long(0), self._stream()))
+            ctypes.c_long(0), ctypes.c_long(0), *factor, self._stream()))
 
     def _rows_product(self, x, weight, bias, out_dtype):
         y = torch.empty((x.shape[0], weight.shape[0]), dtype=out_dtype, device=weight.device)
@@ -953,7 +964,7 @@ class HipKernels:
             self._done("gemm_rows", self.lib.atom_gemm_rows(
                 _ptr(xs), None, None, 0, ctypes.c_float(0.0), _ptr(weights), None, _ptr(ys), None, None, None, None, m, n, k,
                 0, int(out_dtype == torch.float32), self.rows_cols(n), int(self.rows_waves), 0, B, ctypes.c_long(m * k),
-                ctypes.c_long(n * k), ctypes.c_long(m * n), self._stream()))
+                ctypes.c_long(n * k), ctypes.c_long(m * n), *_NO_FACTOR, self._stream()))
             return [ys[b] for b in range(B)]
         return [self.linear(xs[b], weights[b], None, out_dtype=out_dtype) for b in range(B)]
 
@@ -1726,6 +1737,16 @@ class HipKernels:
                                                         self._stream()))
         return out
 
+    def linear_token_gate(self, x, weight, table, col_off: int, ids):
+        """``gelu_tanh(x @ weight.T)`` times the tokens' rows of ``table`` from column ``col_off`` on, in ``x``'s type, as one
+        launch where the few-rows product takes it, else None (the product and ``token_gate``).  A step of one row, 256
+        columns of 2,048: 4.0 us with the product's epilogue, 7.9 in two launches."""
+        if not x.shape[0] or table.dtype != torch.bfloat16 or not self._rows_takes(x, weight):
+            return None
+        y = torch.empty((x.shape[0], weight.shape[0]), dtype=x.dtype, device=weight.device)
+        self._rows_launch(x, weight, None, 0, y=y, act=self._ROWS_ACT["gelu_tanh"], times=(table, col_off, ids))
+        return y
+
     def token_gate(self, raw, table, col_off: int, ids, out):
         """``out[t, j] = gelu_tanh(raw[t, j]) * table[ids[t], col_off + j]``."""
         tokens, dim = raw.shape
@@ -1765,6 +1786,38 @@ class HipKernels:
 
     #: tokens of a run of the gated recurrence's scan (the kernel's own constant)
     RGLRU_RUN = 64
+
+    def rglru_step(self, proj, y_off: int, taps_weight, conv_bias, state, state_off: int, cu_seqlens_q, slot_of_seq, ra, ri,
+                   ra_bias, ri_bias, lam, out, decay_scale: float):
+        """For steps whose requests bring one token each: ``conv_silu_state`` (no activation), both gates' per-block products
+        ``ra`` / ``ri`` [blocks, part, part] and ``rglru_scan`` in two launches, from ``proj`` (float32 [tokens, *], the input
+        branch first, the other from column ``y_off``).  Returns ``out``, or None where the kernels do not take these sizes: up
+        to 8 requests, four taps, blocks of 64, 128, 256 or 512 channels."""
+        tokens, channels = out.shape
+        seqs, blocks, part = slot_of_seq.numel(), ra.shape[0], ra.shape[1]
+        dt = out.dtype
+        if (not self.use_rglru_step or taps_weight.dtype != dt or ra.dtype != dt or tokens > seqs
+                or not self.lib.atom_rglru_step_supports(seqs, channels, part, taps_weight.shape[1])):
+            return None
+        self._check("branches", proj, torch.float32, (tokens, None))
+        self._check("taps", taps_weight, dt, (channels, 4))
+        self._check("state", state, torch.float32, (None, None))
+        self._check("cu_seqlens_q", cu_seqlens_q, torch.int32, (seqs + 1,))
+        self._check("slot_of_seq", slot_of_seq, torch.int32, (seqs,))
+        for w in (ra, ri):
+            self._check("recurrence gate", w, dt, (blocks, part, part))
+        for b in (conv_bias, ra_bias, ri_bias, lam):
+            self._check("channel parameter", b, torch.float32)
+            if b.numel() != channels:
+                raise KernelError("rglru_step: biases and decays need one entry per channel")
+        self._check("recurrence out", out, (torch.float32, torch.bfloat16))
+        gates = torch.empty((2, tokens, channels), dtype=torch.float32, device=out.device)
+        self._done("rglru_step", self.lib.atom_rglru_step(
+            _ptr(proj), ctypes.c_long(proj.shape[1]), y_off, _ptr(taps_weight), _ptr(conv_bias), self._code(out), _ptr(state),
+            ctypes.c_long(state.shape[1]), ctypes.c_long(state_off), _ptr(cu_seqlens_q), _ptr(slot_of_seq), seqs, tokens,
+            _ptr(ra), _ptr(ri), _ptr(ra_bias), _ptr(ri_bias), _ptr(lam), _ptr(gates), _ptr(out), channels, part,
+            ctypes.c_float(decay_scale), self._stream()))
+        return out
 
     def rglru_scan(self, u, gates, ra_bias, ri_bias, lam, proj, y_off: int, state, state_off: int, cu_seqlens_q,
                    slot_of_seq, out, decay_scale: float, max_q_len: int | None = None):

@@ -64,6 +64,13 @@ class RealGatedRecurrence(Mixer):
         T, c = x.shape[0], self.width
         part = c // self.blocks
         proj = ops.linear(x, self.params["in.weight"], self.params["in.bias"], out_dtype=torch.float32)   # x | y
+        step = getattr(ops, "rglru_step", None) if ctx.max_q_len == 1 else None
+        if step is not None:
+            out = torch.empty((T, c), dtype=x.dtype, device=x.device)
+            if step(proj, c, self.params["conv.weight"], self.params["conv.bias"], cache.state, self.conv_floats,
+                    ctx.cu_seqlens_q, ctx.slot_of_seq, self.params["ra.weight"], self.params["ri.weight"], self.params["ra.bias"],
+                    self.params["ri.bias"], self.params["lam"], out, self.decay_scale) is not None:
+                return ops.linear(out, self.params["o.weight"], None, defer=True)
         u = torch.empty((T, c), dtype=torch.float32, device=x.device)
         ops.conv_silu_state(proj, c, self.params["conv.weight"], cache.state, ctx.cu_seqlens_q, ctx.slot_of_seq, u,
                             max_q_len=ctx.max_q_len, bias=self.params["conv.bias"], activation="none")

@@ -44,9 +44,12 @@ class TokenSide(FeedForward):
         if table.shape[1] != self.num_layers * self.dim:
             raise ValueError(f"the token table has {table.shape[1]} columns, {self.num_layers} layers of {self.dim} "
                              "need others")
-        raw = ops.linear(reads, self.params["gate.weight"], None, out_dtype=torch.float32)
-        gated = torch.empty((raw.shape[0], self.dim), dtype=ctx.dtype, device=raw.device)
-        ops.token_gate(raw, table, self.layer * self.dim, ctx.token_ids, gated)
+        few = getattr(ops, "linear_token_gate", None)
+        gated = few(reads, self.params["gate.weight"], table, self.layer * self.dim, ctx.token_ids) if few is not None else None
+        if gated is None:
+            raw = ops.linear(reads, self.params["gate.weight"], None, out_dtype=torch.float32)
+            gated = torch.empty((raw.shape[0], self.dim), dtype=ctx.dtype, device=raw.device)
+            ops.token_gate(raw, table, self.layer * self.dim, ctx.token_ids, gated)
         y = ops.linear(gated, self.params["proj.weight"], None, out_dtype=torch.float32)
         out = None
         if ctx.dtype != torch.float32:

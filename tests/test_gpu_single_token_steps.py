@@ -67,3 +67,47 @@ def test_delta_step_leaves_other_sizes_alone():
     for sizes in ((4, 2, 32, 32, 4, 0, 0), (4, 2, 64, 128, 4, 0, 0), (6, 2, 64, 64, 4, 0, 0), (4, 2, 64, 64, 3, 0, 0),
                   (4, 2, 64, 64, 4, 24, 0), (4, 2, 64, 64, 4, 0, 80)):
         assert not ops.lib.atom_delta_step_supports(*sizes)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("blocks,part,lens,slots", [(3, 64, [1], [2]), (2, 128, [1, 0, 1, 1], [1, 2, -1, 0]),
+                                                    (1, 256, [1] * 8, [7, 6, 5, 4, 3, 2, 1, 0]), (2, 512, [1, 1, 1], [0, -1, 3])])
+def test_rglru_step(blocks, part, lens, slots, dtype):
+    ops = gpu_ops()
+    C, T = blocks * part, sum(lens)
+    proj = rnd((T, 2 * C + 5), 1)
+    taps, conv_bias = rnd((C, 4), 2, 0.5).to(dtype), rnd((C,), 3, 0.3)
+    ra, ri = (rnd((blocks, part, part), s, part ** -0.5).to(dtype) for s in (4, 5))
+    br, bi, lam = rnd((blocks, part), 6), rnd((blocks, part), 7), rnd((C,), 8) - 2
+    off = 3 * C + 1
+    state = rnd((8, off + C), 9, 0.5)
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    some, places = i32(sorted(set(cu))), i32([s for n, s in zip(lens, slots) if n])
+
+    want_state = state.double()
+    u = torch.empty((T, C), dtype=torch.float64)
+    PLAIN.conv_silu_state(proj, C, taps, want_state, some, places, u, bias=conv_bias, activation="none")
+    parts = u.view(T, blocks, part).transpose(0, 1)
+    gates = torch.stack([torch.matmul(parts, w.double().transpose(1, 2)).transpose(0, 1).reshape(T, C) for w in (ra, ri)])
+    want = torch.empty((T, C), dtype=torch.float64)
+    PLAIN.rglru_scan(u, gates, br, bi, lam, proj, C + 5, want_state, off, some, places, want, 8.0)
+
+    dev = lambda t: t.to(DEV)  # noqa: E731
+    got, out = dev(state), torch.full((T, C), 7.0, dtype=dtype, device=DEV)
+    assert ops.rglru_step(dev(proj), C + 5, dev(taps), dev(conv_bias), got, off, dev(i32(cu)), dev(i32(slots)), dev(ra), dev(ri),
+                          dev(br), dev(bi), dev(lam), out, 8.0) is out
+    assert float((got.cpu().double() - want_state).norm() / want_state.norm()) <= 2e-6
+    assert float((out.cpu().double() - want).norm() / want.norm()) <= (4e-3 if dtype == torch.bfloat16 else 4e-6)
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 256, 2048), (3, 37, 136), (8, 64, 512)])
+def test_product_times_rows_of_a_table(m, n, k):
+    ops = gpu_ops()
+    x, w, table = rnd((m, k), 1).bfloat16(), rnd((n, k), 2, k ** -0.5).bfloat16(), rnd((50, 3 * n), 3).bfloat16()
+    ids = i32([49, 0, -1, 7, 50, 3, 3, 1][:m])
+    got = ops.linear_token_gate(x.to(DEV), w.to(DEV), table.to(DEV), n, ids.to(DEV))
+    factor = torch.where(((ids >= 0) & (ids < 50))[:, None], table[ids.clamp(0, 49).long(), n:2 * n].double(), 0.0)
+    want = torch.nn.functional.gelu(x.double() @ w.double().T, approximate="tanh") * factor
+    assert float((got.cpu().double() - want).norm() / want.norm()) <= 4e-3
