@@ -224,7 +224,8 @@ class HipKernels:
                    "atom_together_sum_parts", "atom_streams_step", "atom_embedding_sinusoid", "atom_softcap_rows",
                    "atom_selective_scan", "atom_step_sizes", "atom_experts_few", "atom_experts_few_supports", "atom_keys_as_values_heads_write",
                    "atom_delta_chunks", "atom_delta_chunks_supports", "atom_delta_step", "atom_delta_step_supports",
-                   "atom_rglru_step", "atom_rglru_step_supports"):
+                   "atom_rglru_step", "atom_rglru_step_supports", "atom_space_step",
+                   "atom_space_step_supports", "atom_mix_step", "atom_mix_step_supports"):
             getattr(self.lib, fn).restype = ctypes.c_int
         self.lib.atom_delta_chunks_floats.restype = ctypes.c_long
         self.lib.atom_gemm_f32_scratch.restype = ctypes.c_long
@@ -252,6 +253,7 @@ class HipKernels:
         self.use_fused_decode = True    # decode-only steps of few rows: norm, rotation and cache write inside attention
         self.use_delta_chunks = True   # the delta rule of prompts in chunks of 64 tokens
         self.use_delta_step = True     # ... and of single tokens in one launch with what is before and behind it
+        self.use_scan_step = True      # state-space and time-mixing recurrences of single tokens with what stands around them
         self.use_rglru_step = True     # the real-gated recurrence of single tokens in two launches
         self.use_together_tiles = True  # attention with the heads together on the matrix cores, for prompt portions
         self.use_mfma_latent = True     # attention over latent pages on the matrix cores (bfloat16, sizes it is built for)
@@ -1519,6 +1521,63 @@ class HipKernels:
             int(min_q_len), self._stream()))
         return out
 
+    def space_step(self, proj, x_off: int, taps_weight, conv_bias, state, state_off: int, cu_seqlens_q, slot_of_seq, step_bias,
+                   a_log, skip, weight, eps: float, out, heads: int, groups: int, dim: int, vdim: int, norm_groups: int):
+        """For steps whose requests bring one token each: ``conv_silu_state``, ``linear_scan`` (one decay per head from raw step
+        sizes, a skip) and ``group_norm_gate`` (gated first) in two launches, from ``proj`` (float32 [tokens, *]: z | x | B | C |
+        step sizes, x at ``x_off``) to ``out``.  Returns ``out``, or None where the kernels do not take these sizes: heads of 64
+        or 128 rows by 64 columns, four taps, one group of the norm."""
+        if (not self.use_scan_step or taps_weight.dtype != out.dtype or state.shape[1] % 4 or state_off % 4 or proj.shape[1] % 4
+                or not self.lib.atom_space_step_supports(heads, groups, dim, vdim, taps_weight.shape[1], norm_groups)):
+            return None
+        tokens, seqs, inner = proj.shape[0], slot_of_seq.numel(), heads * vdim
+        channels = inner + 2 * groups * dim
+        self._check("state-space projection", proj, torch.float32)
+        self._check("taps", taps_weight, out.dtype, (channels, 4))
+        self._check("convolution bias", conv_bias, torch.float32, (channels,))
+        self._check("state", state, torch.float32, (None, None))
+        self._check("cu_seqlens_q", cu_seqlens_q, torch.int32, (seqs + 1,))
+        self._check("slot_of_seq", slot_of_seq, torch.int32, (seqs,))
+        for t in (step_bias, a_log, skip):
+            self._check("head parameter", t, torch.float32, (heads,))
+        self._check("norm weight", weight, torch.float32, (inner,))
+        self._check("gated read-out", out, (torch.float32, torch.bfloat16), (tokens, inner))
+        y = torch.empty((tokens, inner), dtype=torch.float32, device=out.device)
+        self._done("space_step", self.lib.atom_space_step(
+            _ptr(proj), ctypes.c_long(proj.shape[1]), x_off, _ptr(taps_weight), _ptr(conv_bias), self._code(out), _ptr(state),
+            ctypes.c_long(state.shape[1]), ctypes.c_long(state_off), _ptr(cu_seqlens_q), _ptr(slot_of_seq), seqs, _ptr(step_bias),
+            _ptr(a_log), _ptr(skip), _ptr(weight), ctypes.c_float(eps), _ptr(y), _ptr(out), heads, groups, dim, vdim,
+            self._stream()))
+        return out
+
+    def mix_step(self, r, k, v, g, squashed, decay2, decay_bias, bonus, weight, state, state_off: int, cu_seqlens_q,
+                 slot_of_seq, out, heads: int, dim: int, eps: float):
+        """For steps whose requests bring one token each: the decays' product ``squashed @ decay2.T``, ``linear_scan`` with a
+        bonus and decays ``exp(-exp(. + decay_bias))`` per channel, and ``group_norm_gate`` (a group a head, gated last by ``g``)
+        in one launch.  Returns ``out``, or None where the kernel does not take these sizes: heads of 64 by 64, ranks of 32 to
+        128 in steps of 32."""
+        rank = squashed.shape[1]
+        if (not self.use_scan_step or decay2.dtype != out.dtype or state.shape[1] % 4 or state_off % 4
+                or not self.lib.atom_mix_step_supports(heads, dim, rank)):
+            return None
+        tokens, seqs, c = out.shape[0], slot_of_seq.numel(), heads * dim
+        for t in (r, k, v, g):
+            self._check("time-mixing input", t, torch.float32, (tokens, c))
+        self._check("squashed decays", squashed, torch.float32, (tokens, rank))
+        self._check("decay weight", decay2, out.dtype, (c, rank))
+        self._check("decay bias", decay_bias, torch.float32, (c,))
+        self._check("bonus", bonus, torch.float32, (heads, dim))
+        self._check("norm weight", weight, torch.float32, (c,))
+        self._check("state", state, torch.float32, (None, None))
+        self._check("cu_seqlens_q", cu_seqlens_q, torch.int32, (seqs + 1,))
+        self._check("slot_of_seq", slot_of_seq, torch.int32, (seqs,))
+        self._check("gated read-out", out, (torch.float32, torch.bfloat16), (tokens, c))
+        self._done("mix_step", self.lib.atom_mix_step(
+            _ptr(r), _ptr(k), _ptr(v), _ptr(g), _ptr(squashed), _ptr(decay2), self._code(out), _ptr(decay_bias), _ptr(bonus),
+            _ptr(weight), _ptr(state), ctypes.c_long(state.shape[1]), ctypes.c_long(state_off), _ptr(cu_seqlens_q),
+            _ptr(slot_of_seq), seqs, _ptr(out), heads, dim, rank, ctypes.c_float(eps), self._stream()))
+        return out
+
     def token_shift(self, x, mu, mixes, state, state_off: int, cu_seqlens_q, slot_of_seq, token_seq):
         """``mixes[s, t] = x[t] + (x[t - 1] - x[t]) * mu[s]``; the row before a request's first token of the step is
         what its state slot holds at ``state_off`` (float32, zeros for a fresh request), and the request's last row
@@ -1739,8 +1798,7 @@ class HipKernels:
 
     def linear_token_gate(self, x, weight, table, col_off: int, ids):
         """``gelu_tanh(x @ weight.T)`` times the tokens' rows of ``table`` from column ``col_off`` on, in ``x``'s type, as one
-        launch where the few-rows product takes it, else None (the product and ``token_gate``).  A step of one row, 256
-        columns of 2,048: 4.0 us with the product's epilogue, 7.9 in two launches."""
+        launch where the few-rows product takes it, else None (the product and ``token_gate``)."""
         if not x.shape[0] or table.dtype != torch.bfloat16 or not self._rows_takes(x, weight):
             return None
         y = torch.empty((x.shape[0], weight.shape[0]), dtype=x.dtype, device=weight.device)

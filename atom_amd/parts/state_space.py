@@ -73,6 +73,13 @@ class StateSpaceMixer(Mixer):
         T = x.shape[0]
         H, V, N, G, inner, C = self.num_heads, self.value_dim, self.state_size, self.groups, self.inner, self.channels
         proj = ops.linear(x, self.params["in.weight"], None, out_dtype=torch.float32)     # z | x | B | C | dt
+        step = getattr(ops, "space_step", None) if ctx.max_q_len == 1 else None
+        if step is not None:
+            out = torch.empty((T, inner), dtype=x.dtype, device=x.device)
+            if step(proj, inner, self.params["conv.weight"], self.params["conv.bias"], cache.state, self.conv_floats,
+                    ctx.cu_seqlens_q, ctx.slot_of_seq, self.params["dt_bias"], self.params["A_log"], self.params["D"],
+                    self.params["norm.weight"], self.norm_eps, out, H, G, N, V, self.norm_groups) is not None:
+                return ops.linear(out, self.params["o.weight"], None, defer=True)
         xbc = torch.empty((T, C), dtype=torch.float32, device=x.device)
         ops.conv_silu_state(proj, C, self.params["conv.weight"], cache.state, ctx.cu_seqlens_q, ctx.slot_of_seq, xbc,
                             max_q_len=ctx.max_q_len, bias=self.params["conv.bias"], activation="silu", x_offset=inner)

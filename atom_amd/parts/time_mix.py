@@ -76,6 +76,13 @@ class TimeMixRecurrence(Mixer):
         # each of r, k, v and the gate reads a mix of its own
         r, k, v, g = ops.linear_side_by_side(mixes[:4], self.params["rkvg.weight"].view(4, c, W), out_dtype=torch.float32)
         squashed = ops.linear_act(mixes[4], self.params["decay1.weight"], None, "tanh", out_dtype=torch.float32)
+        step = getattr(ops, "mix_step", None) if ctx.max_q_len == 1 else None
+        if step is not None:
+            out = torch.empty((T, c), dtype=x.dtype, device=x.device)
+            if step(r, k, v, g, squashed, self.params["decay2.weight"], self.params["decay.bias"], self.params["bonus"],
+                    self.params["norm.weight"], cache.state, W, ctx.cu_seqlens_q, ctx.slot_of_seq, out, H, K,
+                    self.norm_eps) is not None:
+                return ops.linear(out, self.params["o.weight"], None, defer=True)
         raw = torch.empty((T, c), dtype=torch.float32, device=x.device)
         ops.heads_gemm(squashed, 0, rank, 0, self.params["decay2.weight"].view(1, c, rank), raw, 0, c, 0, 1, T, c, rank,
                        exact=True)

@@ -111,3 +111,71 @@ def test_product_times_rows_of_a_table(m, n, k):
     factor = torch.where(((ids >= 0) & (ids < 50))[:, None], table[ids.clamp(0, 49).long(), n:2 * n].double(), 0.0)
     want = torch.nn.functional.gelu(x.double() @ w.double().T, approximate="tanh") * factor
     assert float((got.cpu().double() - want).norm() / want.norm()) <= 4e-3
+
+
+STEPS = [([1], [2]), ([1, 0, 1, 1], [1, 2, -1, 0])]
+
+
+def places_of(lens, slots):
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    return cu, i32(sorted(set(cu))), i32([s for n, s in zip(lens, slots) if n])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("lens,slots", STEPS)
+@pytest.mark.parametrize("heads,groups,dim", [(4, 1, 64), (6, 2, 128), (70, 1, 128)])
+def test_space_step(heads, groups, dim, lens, slots, dtype):
+    ops = gpu_ops()
+    V, T = 64, sum(lens)
+    inner = heads * V
+    C = inner + 2 * groups * dim
+    proj = rnd((T, inner + C + (heads + 3) // 4 * 4), 1)
+    taps, conv_bias = rnd((C, 4), 2, 0.5).to(dtype), rnd((C,), 3, 0.3)
+    step_bias, a_log, skip, norm = rnd((heads,), 4) - 1, rnd((heads,), 5, 0.5), rnd((heads,), 6), 1 + rnd((inner,), 7, 0.2)
+    off = 3 * C + 4
+    state = rnd((4, off + inner * dim), 8, 0.3)
+    cu, some, places = places_of(lens, slots)
+
+    want_state = state.double()
+    xbc, y, want = (torch.empty((T, n), dtype=torch.float64) for n in (C, inner, inner))
+    PLAIN.conv_silu_state(proj, C, taps, want_state, some, places, xbc, bias=conv_bias, x_offset=inner)
+    PLAIN.linear_scan(xbc, inner + groups * dim, groups, xbc, inner, groups, xbc, 0, proj, inner + C, want_state, off, some,
+                      places, y, heads, dim, V, per_channel=False, skip=skip, step_bias=step_bias, a_log=a_log)
+    PLAIN.group_norm_gate(y, 1, norm, 1e-5, want, gate=proj, gate_off=0, gate_first=True)
+
+    dev = lambda t: t.to(DEV)  # noqa: E731
+    got, out = dev(state), torch.full((T, inner), 7.0, dtype=dtype, device=DEV)
+    assert ops.space_step(dev(proj), inner, dev(taps), dev(conv_bias), got, off, dev(i32(cu)), dev(i32(slots)), dev(step_bias),
+                          dev(a_log), dev(skip), dev(norm), 1e-5, out, heads, groups, dim, V, 1) is out
+    assert float((got.cpu().double() - want_state).norm() / want_state.norm()) <= 2e-6
+    assert float((out.cpu().double() - want).norm() / want.norm()) <= (4e-3 if dtype == torch.bfloat16 else 4e-6)
+    assert torch.equal(got[3].cpu(), state[3])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("lens,slots", STEPS)
+@pytest.mark.parametrize("heads,rank", [(1, 32), (5, 64), (3, 96), (32, 128)])
+def test_mix_step(heads, rank, lens, slots, dtype):
+    ops = gpu_ops()
+    T, c = sum(lens), heads * 64
+    r, k, v, g = (rnd((T, c), s) for s in (1, 2, 3, 4))
+    squashed, decay2 = torch.tanh(rnd((T, rank), 5)), rnd((c, rank), 6, 0.2).to(dtype)
+    bias, bonus, norm = rnd((c,), 7) - 2, rnd((heads, 64), 8, 0.3), 1 + rnd((c,), 9, 0.2)
+    state = rnd((4, 8 + c * 64), 10, 0.3)
+    cu, some, places = places_of(lens, slots)
+
+    want_state = state.double()
+    y, want = (torch.empty((T, c), dtype=torch.float64) for _ in range(2))
+    PLAIN.linear_scan(r, 0, heads, k, 0, heads, v, 0, squashed.double() @ decay2.double().T, 0, want_state, 8, some, places, y,
+                      heads, 64, 64, w_bias=bias, bonus=bonus)
+    PLAIN.group_norm_gate(y, heads, norm, 1e-5, want, gate=g)
+
+    dev = lambda t: t.to(DEV)  # noqa: E731
+    got, out = dev(state), torch.full((T, c), 7.0, dtype=dtype, device=DEV)
+    assert ops.mix_step(dev(r), dev(k), dev(v), dev(g), dev(squashed), dev(decay2), dev(bias), dev(bonus), dev(norm), got, 8,
+                        dev(i32(cu)), dev(i32(slots)), out, heads, 64, 1e-5) is out
+    assert float((got.cpu().double() - want_state).norm() / want_state.norm()) <= 2e-6
+    assert float((out.cpu().double() - want).norm() / want.norm()) <= (4e-3 if dtype == torch.bfloat16 else 4e-6)
+    assert torch.equal(got[3].cpu(), state[3])
