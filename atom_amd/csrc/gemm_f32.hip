@@ -326,19 +326,30 @@ gemm_f32_kernel(GemmF32Params p) {
   }
 }
 
-// Many rows, float32 operands, K a multiple of 32: tiles of 64 rows and 128 columns whose operands go through LDS, in whole
-// cache lines straight from memory.  x comes as planes of pieces, made once by a kernel of its own; pieces of w are formed by
-// the one wave that multiplies them.  A block is two groups of four waves, each with four of the slices, a wave with 64 x 32
-// of the tile, so that a step's splitting (two of w's 16-row parts) takes a third of the cycles of its 48 matrix
-// instructions; in 32 x 64 it would take more than they do.  A stage is 32 terms of the tile's 192 rows, double buffered; the
-// 16-byte pieces of a row change places by its row number, so that the rows a wave reads at once lie in different banks.
-// While a stage is multiplied, the next one's operands are read from LDS and the stage behind that comes from memory: 56 KB a
-// stage and CU, at the 35 to 40 KB a microsecond that a CU draws, are what bounds it.  465 rows by 24,576 x 4,096 take 645 us,
-// 145 TFLOP/s (945 with the float32 instructions, whose rate is 157 at most), by 4,096 x 4,096 109 (161), by 4,096 x 12,288
-// 305 (475).  Five stages in LDS with all eight waves on each (32 x 32 of the tile a wave) took 705, 120 and 340.
-constexpr int kWideRows = 64, kWideCols = 128;
-constexpr int kPlaneBytes = kWideRows * kStep * 2;                     // a stage of one plane of x
-constexpr int kStageBytes = 3 * kPlaneBytes + kWideCols * kStep * 4;
+// Many rows, float32 operands, K a multiple of 32: tiles of 64 or 128 rows and 128 columns whose operands go through LDS, in
+// whole cache lines straight from memory.  x comes as planes of pieces, made once by a kernel of its own; pieces of w are formed
+// where it is multiplied.  A block is two groups of four waves, a wave with 64 x 32 of the tile, so that a step's splitting
+// (two of w's 16-row parts) takes a third of the cycles of its 48 matrix instructions; in 32 x 64 it would take more than they
+// do.  A stage is 32 terms of the tile's rows, double buffered; the 16-byte pieces of a row change places by its row number, so
+// that the rows a wave reads at once lie in different banks.  While a stage is multiplied, the next one's operands are read from
+// LDS and the stage behind that comes from memory: 56 KB for two groups of four slices each, 40 KB in tiles of 128 rows, at the
+// 35 to 40 KB a microsecond that a CU draws, are what bounds it.  465 rows by 24,576 x 4,096 take 595 us in tiles of 128 rows and
+// 645 in tiles of 64 (945 with the float32 instructions), by 4,096 x 4,096, where only the lower ones are a tile for every CU, 109
+// (161), by 4,096 x 12,288 309 (475); 1,024 rows by 24,576 1,145, 180 TFLOP/s (1,885; the float32 instructions' rate is 157).
+// Five stages in LDS with all eight waves on each (32 x 32 of 64 x 128 a wave) took 705, 120 and 340 at 465 rows.
+constexpr int kWideCols = 128;
+
+// ROWS 64: the block's halves take half of K each.  ROWS 128: they take 64 rows each and all of K, and the first four slices'
+// sums wait in LDS.
+template <int ROWS>
+struct Wide {
+  static constexpr int groups = 128 / ROWS;                            // of waves that share K
+  static constexpr int plane = ROWS * kStep * 2;                       // bytes of a stage of one plane of x,
+  static constexpr int stage = 3 * plane + kWideCols * kStep * 4;      // and of a stage
+  static constexpr int sums = ROWS * kWideCols * 4;                    // the sums of half of K
+  static constexpr int bytes = groups == 2 ? 4 * stage : 2 * stage + sums;
+  static_assert(bytes <= 160 * 1024 && bytes >= sums, "it all fits in LDS");
+};
 
 __global__ void __launch_bounds__(256) split_f32_kernel(const float* __restrict__ x, bf16_t* __restrict__ pieces, size_t eights,
                                                                   int steps) {
@@ -352,32 +363,36 @@ __global__ void __launch_bounds__(256) split_f32_kernel(const float* __restrict_
   for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(pieces + (i * eights + at) * kLane) = p[i];
 }
 
+template <int ROWS>
 __global__ void __launch_bounds__(kSlices* kWave) gemm_f32_wide_kernel(GemmF32Params p) {
+  constexpr int GROUPS = Wide<ROWS>::groups, kPlaneBytes = Wide<ROWS>::plane, kStageBytes = Wide<ROWS>::stage;
   extern __shared__ __align__(16) char wide[];   // [group][buffer][kStageBytes]: x's planes, then w
   const int tile = blockIdx.x % kXcds * (gridDim.x / kXcds) + blockIdx.x / kXcds;
   if (tile >= p.tiles) return;
-  const int row0 = tile % p.row_tiles * kWideRows;
+  const int row0 = tile % p.row_tiles * ROWS;
   const int col0 = tile / p.row_tiles * kWideCols;
   const int tid = threadIdx.x, lane = tid % kWave, side = lane % kSide, quarter = lane / kSide;
-  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), group = wave / 4, w4 = wave % 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), w4 = wave % 4;
+  const int group = GROUPS == 2 ? wave / 4 : 0, r0 = GROUPS == 2 ? 0 : wave / 4 * 64;   // the wave's share of K, or of the rows
 
   const int steps = p.k / kStep;
   const int share = (steps + kSlices - 1) / kSlices;
-  const int low = min(steps, 4 * share);
+  const int low = GROUPS == 2 ? min(steps, 4 * share) : steps;
   const int count = group ? steps - low : low;      // this group's steps
   const int k0 = group ? low * kStep : 0;
 
   // Loads of a stage: 16 rows of a plane of x each (piece `lane % 4` of a row in LDS is the row's piece of that number turned
   // by the row), then 8 rows of w each (piece `lane % 8`).
-  constexpr int X_LOADS = 3 * kWideRows / 16, LOADS = (X_LOADS + kWideCols / 8) / 4;
+  constexpr int X_LOADS = 3 * ROWS / 16, LOADS = (X_LOADS + kWideCols / 8) * GROUPS / kSlices;
+  const int loader = GROUPS == 2 ? w4 : wave;
   const char* from[LOADS];
   int size[LOADS];                                  // bytes of a term
 #pragma unroll
   for (int j = 0; j < LOADS; ++j) {
-    const int load = LOADS * w4 + j;
+    const int load = LOADS * loader + j;
     if (load < X_LOADS) {
-      const int r = load % 4 * 16 + lane / 4;
-      from[j] = (const char*)(p.pieces + ((size_t)(load / 4) * p.m + min(row0 + r, p.m - 1)) * p.k + k0 +
+      const int r = load % (ROWS / 16) * 16 + lane / 4;
+      from[j] = (const char*)(p.pieces + ((size_t)(load / (ROWS / 16)) * p.m + min(row0 + r, p.m - 1)) * p.k + k0 +
                               (lane % 4 ^ (r >> 2 & 3)) * 8);
       size[j] = 2;
     } else {
@@ -391,7 +406,7 @@ __global__ void __launch_bounds__(kSlices* kWave) gemm_f32_wide_kernel(GemmF32Pa
     const int term = min(stage, max(count - 1, 0)) * kStep;
 #pragma unroll
     for (int j = 0; j < LOADS; ++j)
-      load_to_lds(from[j] + term * size[j], lds_address(mine + buffer * kStageBytes + (LOADS * w4 + j) * 1024));
+      load_to_lds(from[j] + term * size[j], lds_address(mine + buffer * kStageBytes + (LOADS * loader + j) * 1024));
   };
   f32x4 acc[4][2], total[4][2];
 #pragma unroll
@@ -416,13 +431,17 @@ __global__ void __launch_bounds__(kSlices* kWave) gemm_f32_wide_kernel(GemmF32Pa
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int r = 16 * i + side;
+      const int r = r0 + 16 * i + side;
 #pragma unroll
       for (int t = 0; t < 3; ++t)
         o.a[i][t] = *reinterpret_cast<const bf16x8*>(xs + t * kPlaneBytes + r * kStep * 2 + (quarter ^ (r >> 2 & 3)) * 16);
     }
   };
-  int until = share;                                // steps until the slice ends
+  int until = share, slice = 0;                     // steps until the slice ends
+  // the first four slices' sums: those of the other half of the block, or the wave's own
+  float* met = (float*)(wide + (GROUPS == 2 ? 0 : 2 * kStageBytes)) + (GROUPS == 2 ? w4 : wave) * 64 * 32;
+  const auto place = [&](int i, int j, int t) { return (16 * i + 4 * quarter + t) * 32 + 16 * j + side; };
+  const bool second = GROUPS == 1 && steps > 4 * share;   // there are more slices than four
   const auto multiply = [&](const Operands& o, float sign, bool last) {
     bf16x8 bp[2][3];
     f32x4 part[2][4];
@@ -458,6 +477,16 @@ __global__ void __launch_bounds__(kSlices* kWave) gemm_f32_wide_kernel(GemmF32Pa
           for (int t = 0; t < 4; ++t) total[i][j][t] += acc[i][j][t];
           acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
+      if (second && ++slice == kSlices / 2) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) met[place(i, j, t)] = total[i][j][t];
+            total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+          }
+      }
     }
   };
   // A stage's operands are read from LDS while the stage before is multiplied; its buffer then takes the stage after next.
@@ -481,20 +510,19 @@ __global__ void __launch_bounds__(kSlices* kWave) gemm_f32_wide_kernel(GemmF32Pa
     if (stage + 1 < low) pass(odd, even, stage + 1);
   }
 
-  // the second group's half of the sum joins the first's
-  __syncthreads();
-  float* met = (float*)wide + w4 * 64 * 32;         // the wave's 64 x 32
+  if constexpr (GROUPS == 2) {                      // the second group's half of the sum joins the first's
+    __syncthreads();
+    if (group) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        float* there = met + (16 * i + 4 * quarter + t) * 32 + 16 * j + side;
-        if (group) *there = total[i][j][t];
-      }
-  __syncthreads();
-  if (group) return;
+          for (int t = 0; t < 4; ++t) met[place(i, j, t)] = total[i][j][t];
+    }
+    __syncthreads();
+    if (group) return;
+  }
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -505,9 +533,10 @@ __global__ void __launch_bounds__(kSlices* kWave) gemm_f32_wide_kernel(GemmF32Pa
       const float bias = p.bias != nullptr ? p.bias[c + (p.inter != 0 && side >= 8 ? p.inter : 0)] : 0.f;
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        const int r = row0 + 16 * i + 4 * quarter + t;
+        const int r = row0 + r0 + 16 * i + 4 * quarter + t;
         if (r >= p.m) continue;
-        float sum = total[i][j][t] + met[(16 * i + 4 * quarter + t) * 32 + 16 * j + side];
+        float sum = total[i][j][t];
+        if (GROUPS == 2 || second) sum = GROUPS == 2 ? sum + met[place(i, j, t)] : met[place(i, j, t)] + sum;
         if (spoilt(sum))
           sum = summed_again((const float*)p.x + (size_t)r * p.k, (const float*)p.w + (size_t)row_of_w(p, at) * p.k, p.k);
         if (p.bias != nullptr) sum += bias;
@@ -526,12 +555,13 @@ __global__ void __launch_bounds__(kSlices* kWave) gemm_f32_wide_kernel(GemmF32Pa
 // Rows of x that are split and multiplied at a time: what the pieces of as many take is all the scratch memory there is.
 constexpr int kSplitRows = 2048;
 
+template <int ROWS>
 static int launch_gemm_f32_wide(GemmF32Params p, void* scratch, hipStream_t stream) {
-  constexpr int bytes = 4 * kStageBytes;
-  static_assert(bytes <= 160 * 1024 && bytes >= 4 * 64 * 32 * 4, "the stages fit in LDS, and the second half of the sums there");
+  constexpr int bytes = Wide<ROWS>::bytes;
   static bool allowed = false;
   if (!allowed) {
-    if (hipFuncSetAttribute((const void*)gemm_f32_wide_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess)
+    if (hipFuncSetAttribute((const void*)gemm_f32_wide_kernel<ROWS>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) !=
+        hipSuccess)
       return ATOM_LAUNCH_FAILED;
     allowed = true;
   }
@@ -539,15 +569,15 @@ static int launch_gemm_f32_wide(GemmF32Params p, void* scratch, hipStream_t stre
   p.pieces = (const bf16_t*)scratch;
   for (int first = 0; first < m; first += kSplitRows) {
     p.m = min(kSplitRows, m - first);
-    p.row_tiles = (p.m + kWideRows - 1) / kWideRows;
+    p.row_tiles = (p.m + ROWS - 1) / ROWS;
     const long tiles = (long)p.row_tiles * ((p.n + kWideCols - 1) / kWideCols);
     const size_t eights = (size_t)p.m * p.k / kLane;
     if (tiles > 0x3fffffL || eights / 256 > 0x3fffffL) return ATOM_TOO_LARGE;
     p.tiles = (int)tiles;
     hipLaunchKernelGGL(split_f32_kernel, dim3((unsigned)((eights + 255) / 256)), dim3(256), 0, stream, (const float*)p.x,
                        (bf16_t*)scratch, eights, p.k / kStep);
-    hipLaunchKernelGGL(gemm_f32_wide_kernel, dim3((unsigned)(tiles + kXcds - 1) / kXcds * kXcds), dim3(kSlices * kWave), bytes,
-                       stream, p);
+    hipLaunchKernelGGL((gemm_f32_wide_kernel<ROWS>), dim3((unsigned)(tiles + kXcds - 1) / kXcds * kXcds), dim3(kSlices * kWave),
+                       bytes, stream, p);
     p.x = (const float*)p.x + (size_t)p.m * p.k;
     p.y = (char*)p.y + (size_t)p.m * out * (p.y_bf16 ? 2 : 4);
   }
@@ -571,20 +601,24 @@ static int launch_gemm_f32(GemmF32Params p, hipStream_t stream) {
   return launch_status();
 }
 
-// The width of the tiles of 64 rows that a product of more than 32 rows takes, the one whose rounds over the CUs take least: 16,
-// 32 or 64 columns, or, through LDS, 128.  A round takes 38, 46, 71 and 106 us at
-// K 4,096 (465 rows by 24,576: 48, 24, 12 and 6 rounds of 1,800, 1,100, 843 and 645 us in all).
+// The tiles that a product of more than 32 rows takes, those whose rounds over the CUs take least: 64 rows by 16, 32 or 64
+// columns, or, through LDS, by 128, or 128 rows by 128 (kTall).  A round takes 38, 46, 71, 106 and 185 us at K 4,096 (465
+// rows by 24,576: 48, 24, 12, 6 and 3 rounds of 1,800, 1,100, 843, 645 and 595 us in all; 180 rows: 5 rounds of 64 columns 378,
+// three of 128 332, two of 128 rows 345).
+constexpr int kTall = 256;
 static int f32_columns(int m, int n, bool wide) {
-  const long cus = device_cus(), rows = (m + 63) / 64;
-  const auto cost = [&](int cols, int round) { return (rows * ((n + cols - 1) / cols) + cus - 1) / cus * round; };
-  const long c1 = cost(16, 38), c2 = cost(32, 46), c4 = cost(64, 71), c8 = cost(128, 106);
-  if (wide && c8 <= c4 && c8 <= c2 && c8 <= c1) return 128;
+  const long cus = device_cus();
+  const auto cost = [&](int rows, int cols, int round) {
+    return ((long)((m + rows - 1) / rows) * ((n + cols - 1) / cols) + cus - 1) / cus * round;
+  };
+  const long c1 = cost(64, 16, 38), c2 = cost(64, 32, 46), c4 = cost(64, 64, 71), c8 = cost(64, 128, 106), c16 = cost(128, 128, 185);
+  if (wide && min(c8, c16) <= min(c1, min(c2, c4))) return c16 < c8 ? kTall : 128;
   return c1 <= c2 && c1 <= c4 ? 16 : c2 <= c4 ? 32 : 64;
 }
 
 static bool f32_wide(const void* x, int x_dtype, const void* w, int w_dtype, int m, int n, int k) {
   return x_dtype == ATOM_F32 && w_dtype == ATOM_F32 && m > 64 && k % kStep == 0 && ((uintptr_t)x | (uintptr_t)w) % 16 == 0 &&
-         f32_columns(m, n, true) == 128;
+         f32_columns(m, n, true) >= 128;
 }
 
 template <typename TX, typename TW>
@@ -616,7 +650,8 @@ ATOM_EXPORT long atom_gemm_f32_scratch(const void* x, int x_dtype, const void* w
 static int gemm_f32(GemmF32Params p, int x_dtype, int w_dtype, void* scratch, hipStream_t stream) {
   if (scratch != nullptr && f32_wide(p.x, x_dtype, p.w, w_dtype, p.m, p.n, p.k)) {
     if ((uintptr_t)scratch % 16) return ATOM_BAD_SHAPE;
-    return launch_gemm_f32_wide(p, scratch, stream);
+    return f32_columns(p.m, p.n, true) == kTall ? launch_gemm_f32_wide<128>(p, scratch, stream)
+                                                : launch_gemm_f32_wide<64>(p, scratch, stream);
   }
   switch (x_dtype * 2 + w_dtype) {
     case 0: return choose_gemm_f32<float, float>(p, stream);

@@ -18,8 +18,9 @@ def through_lds(ops, x, w):
     return ops._f32_scratch(x, w, x.shape[0], w.shape[0], x.shape[1]) is not None
 
 
-# K of one step, of a last slice that is short, of slices that are empty; rows and columns at the edges of tiles; two portions
-@pytest.mark.parametrize("m,n,k", [(449, 4099, 32), (449, 4096, 288), (512, 4100, 1056), (2112, 4096, 64), (465, 8192, 4096)])
+# K of one step, of a last slice that is short, of slices that are empty; rows and columns at the edges of both tiles; two portions
+@pytest.mark.parametrize("m,n,k", [(449, 4099, 32), (449, 4096, 288), (512, 4100, 1056), (2112, 4096, 64), (465, 8192, 4096),
+                                   (100, 30000, 32), (1000, 4160, 96), (129, 24580, 192), (1025, 8192, 4096)])
 def test_wide_products_round_like_narrow_ones(m, n, k):
     ops = gpu_ops()
     x, w, b = rnd((m, k), 1), rnd((n, k), 2), rnd((n,), 3)
