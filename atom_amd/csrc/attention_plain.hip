@@ -216,11 +216,11 @@ ATOM_EXPORT int atom_mean_of_norms(const void* const* xs, const float* const* ws
 
 template <typename T>
 __global__ void __launch_bounds__(256)
-embedding_positions_kernel(const T* __restrict__ table, const T* __restrict__ rows, const int* __restrict__ ids,
+embedding_positions_kernel(const T* __restrict__ table, const T* __restrict__ rows, int* ids, FedTokens fed,
                            const int* __restrict__ positions, float* __restrict__ out, int width, int vocab,
                            int max_positions) {
   const size_t t = blockIdx.x;
-  int id = ids[t], p = positions[t];
+  int id = fed_id(ids, (int)t, fed, blockIdx.y == 0 && threadIdx.x == 0), p = positions[t];
   id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);
   p = p < 0 ? 0 : (p >= max_positions ? max_positions - 1 : p);
   const T* a = table + (size_t)id * width;
@@ -230,14 +230,17 @@ embedding_positions_kernel(const T* __restrict__ table, const T* __restrict__ ro
   for (int i = blockIdx.y * blockDim.x + threadIdx.x; i < width; i += step) out[t * width + i] = to_f32(a[i]) + to_f32(b[i]);
 }
 
-ATOM_EXPORT int atom_embedding_positions(const void* table, const void* rows, int dtype, const int* ids,
+ATOM_EXPORT int atom_embedding_positions(const void* table, const void* rows, int dtype, int* ids,
                                          const int* positions, float* out, int tokens, int width, int vocab,
-                                         int max_positions, hipStream_t stream) {
+                                         int max_positions, const int* source, const int* sampled, int num_sampled,
+                                         hipStream_t stream) {
+  if (source != nullptr && (sampled == nullptr || num_sampled < 0)) return ATOM_BAD_SHAPE;
+  const FedTokens fed{source, sampled, num_sampled};
   if (tokens < 0 || width <= 0 || vocab <= 0 || max_positions <= 0) return ATOM_BAD_SHAPE;
   if (table == nullptr || rows == nullptr || ids == nullptr || positions == nullptr || out == nullptr) return ATOM_BAD_SHAPE;
   if (tokens == 0) return ATOM_OK;
   ATOM_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((embedding_positions_kernel<T>), dim3(tokens, blocks_of_row(width)), dim3(256), 0, stream,
-                                                 (const T*)table, (const T*)rows, ids, positions, out, width, vocab,
+                                                 (const T*)table, (const T*)rows, ids, fed, positions, out, width, vocab,
                                                  max_positions));
   return launch_status();
 }

@@ -42,6 +42,23 @@ static inline unsigned blocks_of_row(int entries) {
   return blocks < 1024 ? blocks : 1024;
 }
 
+// Token ids that are still on the device: token t's id is sampled[source[t]] where that names one of the `count` sampled rows (what
+// the last step's sampler left there), else ids[t].  A kernel that looks tokens up takes them so and leaves them in ids for the
+// kernels behind it (a launch of its own before an embedding of few tokens is 4 us of a decode step).
+struct FedTokens {
+  const int* source;   // null: ids as they are
+  const int* sampled;
+  int count;
+};
+
+__device__ __forceinline__ int fed_id(int* ids, int t, const FedTokens& fed, bool leaves) {
+  const int src = fed.source != nullptr ? fed.source[t] : -1;
+  if (src < 0 || src >= fed.count) return ids[t];
+  const int id = fed.sampled[src];
+  if (leaves) ids[t] = id;   // (nobody reads the old one: whoever looks this token up goes by its source)
+  return id;
+}
+
 // Four neighbouring elements of either type as float32.
 template <typename T>
 struct alignas(4 * sizeof(T)) Four {

@@ -122,10 +122,10 @@ struct SplitSum {
 // ------------------------------------------------------------------ embedding
 
 template <typename TT, typename TO>
-__global__ void embedding_kernel(const TT* __restrict__ table, const int* __restrict__ ids,
+__global__ void embedding_kernel(const TT* __restrict__ table, int* ids, FedTokens fed,
                                  TO* __restrict__ out, int hidden, int vocab) {
   const int t = blockIdx.x;
-  const int id = ids[t];
+  const int id = fed_id(ids, t, fed, blockIdx.y == 0 && threadIdx.x == 0);
   const bool ok = id >= 0 && id < vocab;
   const TT* row = table + (size_t)(ok ? id : 0) * hidden;
   TO* dst = out + (size_t)t * hidden;
@@ -137,13 +137,17 @@ __global__ void embedding_kernel(const TT* __restrict__ table, const int* __rest
   }
 }
 
-ATOM_EXPORT int atom_embedding(const void* table, int table_dtype, const int* ids, void* out,
-                               int out_dtype, int tokens, int hidden, int vocab, hipStream_t stream) {
+// source, sampled: see FedTokens (source null: ids as they are, and not written).
+ATOM_EXPORT int atom_embedding(const void* table, int table_dtype, int* ids, void* out,
+                               int out_dtype, int tokens, int hidden, int vocab, const int* source, const int* sampled,
+                               int num_sampled, hipStream_t stream) {
+  if (source != nullptr && (sampled == nullptr || num_sampled < 0)) return ATOM_BAD_SHAPE;
+  const FedTokens fed{source, sampled, num_sampled};
   if (tokens < 0 || hidden <= 0 || vocab <= 0) return ATOM_BAD_SHAPE;
   if (tokens == 0) return ATOM_OK;
   dim3 grid(tokens, blocks_of_row(hidden)), block(256);
 #define LAUNCH(TT, TO) \
-  hipLaunchKernelGGL((embedding_kernel<TT, TO>), grid, block, 0, stream, (const TT*)table, ids, (TO*)out, hidden, vocab)
+  hipLaunchKernelGGL((embedding_kernel<TT, TO>), grid, block, 0, stream, (const TT*)table, ids, fed, (TO*)out, hidden, vocab)
   if (table_dtype == ATOM_F32 && out_dtype == ATOM_F32) LAUNCH(float, float);
   else if (table_dtype == ATOM_BF16 && out_dtype == ATOM_BF16) LAUNCH(bf16_t, bf16_t);
   else if (table_dtype == ATOM_BF16 && out_dtype == ATOM_F32) LAUNCH(bf16_t, float);

@@ -227,10 +227,10 @@ ATOM_EXPORT int atom_layernorm(const void* x, int x_dtype, float* residual, cons
 // ------------------------------------------------------------------ embedding rows times a constant, float32 out
 
 template <typename TT>
-__global__ void embedding_scaled_kernel(const TT* __restrict__ table, const int* __restrict__ ids,
+__global__ void embedding_scaled_kernel(const TT* __restrict__ table, int* ids, FedTokens fed,
                                         float* __restrict__ out, int hidden, int vocab, float scale) {
   const int t = blockIdx.x;
-  int id = ids[t];
+  int id = fed_id(ids, t, fed, blockIdx.y == 0 && threadIdx.x == 0);
   id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);
   const TT* src = table + (size_t)id * hidden;
   float* dst = out + (size_t)t * hidden;
@@ -239,13 +239,16 @@ __global__ void embedding_scaled_kernel(const TT* __restrict__ table, const int*
   for (int i = blockIdx.y * blockDim.x + threadIdx.x; i < hidden; i += step) dst[i] = to_f32(src[i]) * scale;
 }
 
-ATOM_EXPORT int atom_embedding_scaled(const void* table, int table_dtype, const int* ids, float* out, int tokens,
-                                      int hidden, int vocab, float scale, hipStream_t stream) {
+ATOM_EXPORT int atom_embedding_scaled(const void* table, int table_dtype, int* ids, float* out, int tokens,
+                                      int hidden, int vocab, float scale, const int* source, const int* sampled,
+                                      int num_sampled, hipStream_t stream) {
+  if (source != nullptr && (sampled == nullptr || num_sampled < 0)) return ATOM_BAD_SHAPE;
+  const FedTokens fed{source, sampled, num_sampled};
   if (tokens < 0 || hidden <= 0 || vocab <= 0) return ATOM_BAD_SHAPE;
   if (tokens == 0) return ATOM_OK;
   const dim3 grid(tokens, blocks_of_row(hidden));
   ATOM_DISPATCH_DTYPE(table_dtype, hipLaunchKernelGGL((embedding_scaled_kernel<T>), grid, dim3(256), 0, stream,
-                                                       (const T*)table, ids, out, hidden, vocab, scale));
+                                                       (const T*)table, ids, fed, out, hidden, vocab, scale));
   return launch_status();
 }
 

@@ -84,6 +84,9 @@ class StepContext:
     # the step's token ids (int32 [T], on the device) and the model's shared token tables by checkpoint prefix,
     # for parts other than the embedding that look a token up; set by the model before its first layer
     token_ids: torch.Tensor | None = None
+    # (source, sampled): ids that the last step's sampler left on the device (``ops.feed_tokens``) and that have not joined
+    # the token ids yet; the embedding takes them where it can, else the model feeds them before it
+    feed: tuple | None = None
     tables: dict = field(default_factory=dict)
     # host-side copies, for mixers that walk requests themselves; None in a replayed step
     seq_starts: list[int] | None = None   # first row of each request in the token axis

@@ -252,14 +252,12 @@ class EngineCore:
 
         (d_tokens, d_positions, d_token_seq, d_starts, d_ctx, d_cached, d_slots, d_want, d_feed) = (
             at(k) for k in range(fixed))
-        if feeds:
-            self.ops.feed_tokens(d_tokens, d_feed, self.sampled)
         ctx = StepContext(ops=self.ops, dtype=self.dtype, device=self.device, num_tokens=total, num_seqs=num_seqs,
                           positions=d_positions, token_seq=d_token_seq, cu_seqlens_q=d_starts, context_lens=d_ctx,
                           cached_lens=d_cached, slot_of_seq=d_slots, num_prefill=view.num_prefill,
                           max_q_len=max(q_lens), max_context_len=int(context_lens.max()),
                           seq_starts=[int(s) for s in starts[:-1]], seq_lens=q_lens, seq_cached=cached,
-                          state_slots=state_slots)
+                          state_slots=state_slots, feed=(d_feed, self.sampled) if feeds else None)
         for gi, g in enumerate(mgr.groups):
             ctx.block_tables[gi] = at(fixed + 2 * gi).view(num_seqs, widths[gi])
             ctx.slot_mappings[gi] = at(fixed + 1 + 2 * gi)

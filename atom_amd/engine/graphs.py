@@ -276,7 +276,8 @@ class DecodeGraphs:
         stream = torch.cuda.Stream(device=core.device)
         stream.wait_stream(torch.cuda.current_stream(core.device))
         with torch.cuda.stream(stream):
-            core.ops.feed_tokens(tokens, feed, core.sampled)
+            # rows whose token the last step's sampler left on the device take it from there
+            ctx.feed = (feed, core.sampled)
             # first-use allocations happen here
             core.model.forward(ctx, tokens, core.storage.bindings, want, core.storage.embedding_binding)
         stream.synchronize()
@@ -293,8 +294,7 @@ class DecodeGraphs:
         try:
             ctx, tokens, want, feed = self._context(cap)    # a fresh context: nothing remembered from the warm-up
             with torch.cuda.graph(cap.graph, pool=self.pool, stream=stream):
-                # rows whose token the last step's sampler left on the device take it from there
-                core.ops.feed_tokens(tokens, feed, core.sampled)
+                ctx.feed = (feed, core.sampled)
                 cap.logits = core.model.forward(ctx, tokens, core.storage.bindings, want,
                                                 core.storage.embedding_binding)
         finally:

@@ -529,7 +529,18 @@ class HipKernels:
 
     # ------------------------------------------------------------------ kernels
 
-    def embedding(self, table: torch.Tensor, ids: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
+    #: the embeddings below take ``feed`` = (source, sampled): ``feed_tokens`` of their ids, in their own launch
+    embeddings_take_feed = True
+
+    def _fed(self, ids, feed):
+        if feed is None:
+            return None, None, 0
+        source, sampled = feed
+        self._check("token sources", source, torch.int32, (ids.numel(),))
+        self._check("sampled ids", sampled, torch.int32, (None,))
+        return _ptr(source), _ptr(sampled), sampled.numel()
+
+    def embedding(self, table: torch.Tensor, ids: torch.Tensor, out: torch.Tensor, feed=None) -> torch.Tensor:
         vocab, hidden = table.shape
         tokens = ids.numel()
         self._check("embedding table", table, (torch.float32, torch.bfloat16))
@@ -537,7 +548,7 @@ class HipKernels:
         self._check("embedding out", out, (torch.float32, torch.bfloat16), (tokens, hidden))
         self._done("embedding", self.lib.atom_embedding(
             _ptr(table), self._code(table), _ptr(ids), _ptr(out), self._code(out), tokens, hidden, vocab,
-            self._stream()))
+            *self._fed(ids, feed), self._stream()))
         return out
 
     def feed_tokens(self, ids: torch.Tensor, source: torch.Tensor, sampled: torch.Tensor) -> torch.Tensor:
@@ -1051,7 +1062,7 @@ class HipKernels:
             self._stream()))
         return out
 
-    def embedding_scaled(self, table, ids, out, scale: float):
+    def embedding_scaled(self, table, ids, out, scale: float, feed=None):
         """``out = table[ids] * scale`` in float32."""
         vocab, hidden = table.shape
         tokens = ids.numel()
@@ -1060,7 +1071,7 @@ class HipKernels:
         self._check("embedding out", out, torch.float32, (tokens, hidden))
         self._done("embedding_scaled", self.lib.atom_embedding_scaled(
             _ptr(table), self._code(table), _ptr(ids), _ptr(out), tokens, hidden, vocab, ctypes.c_float(scale),
-            self._stream()))
+            *self._fed(ids, feed), self._stream()))
         return out
 
     def sum_concat(self, hidden, residual, first, out):
@@ -1700,7 +1711,7 @@ class HipKernels:
                                                                 ctypes.c_float(eps), self._stream()))
         return out
 
-    def embedding_positions(self, table, rows, ids, positions, out):
+    def embedding_positions(self, table, rows, ids, positions, out, feed=None):
         """``out = table[ids] + rows[positions]`` in float32."""
         vocab, hidden = table.shape
         tokens = ids.numel()
@@ -1711,7 +1722,7 @@ class HipKernels:
         self._check("embedding out", out, torch.float32, (tokens, hidden))
         self._done("embedding_positions", self.lib.atom_embedding_positions(
             _ptr(table), _ptr(rows), self._code(table), _ptr(ids), _ptr(positions), _ptr(out), tokens, hidden, vocab,
-            rows.shape[0], self._stream()))
+            rows.shape[0], *self._fed(ids, feed), self._stream()))
         return out
 
     def scale_rows(self, x, scale: float):

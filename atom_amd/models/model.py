@@ -143,6 +143,9 @@ class CausalLM(Part):
         at ``want_rows`` (None: nothing is wanted, the cache is only filled).  ``embedding_cache`` is the binding
         of an embedding that keeps something per request."""
         ctx.token_ids, ctx.tables = token_ids, self.tables
+        if ctx.feed is not None and not (self.embedding.takes_feed and getattr(ctx.ops, "embeddings_take_feed", False)):
+            ctx.ops.feed_tokens(token_ids, *ctx.feed)
+            ctx.feed = None
         if self.embedding.cache_need() is not None:
             hidden = first = self.embedding.forward(ctx, token_ids, embedding_cache)
         else:

@@ -216,6 +216,9 @@ class Embedding(Part):
     """Token ids to the model's first hidden rows.  Built with ``vocab_size``, ``hidden_size`` and whatever
     else its choice names (a multiplier, say)."""
 
+    #: True where ``forward`` hands ``ctx.feed`` on to an operation that takes it; elsewhere the model feeds the ids first
+    takes_feed = False
+
     def cache_need(self):
         """What the embedding keeps per request between steps (a ``StateNeed``), or None.  An embedding with a
         need is called as ``forward(ctx, ids, cache)`` with the binding the engine made for it."""

@@ -15,13 +15,19 @@ class TokenEmbedding(Embedding):
         self.vocab_size = vocab_size
         self.hidden_size = hidden_size
         self.weight_name = weight_name   # the table's checkpoint name under the prefix (empty: the prefix itself)
+        self.takes_feed = type(self) in (TokenEmbedding, ScaledEmbedding, PositionedEmbedding)   # whose forward this file knows
 
     def param_specs(self):
         return {"weight": ParamSpec.single(self.weight_name, (self.vocab_size, self.hidden_size))}
 
+    @staticmethod
+    def _feed(ctx):
+        """The keyword for an operation that takes the tokens still on the device, where there are any."""
+        return {} if ctx.feed is None else {"feed": ctx.feed}
+
     def forward(self, ctx, ids: torch.Tensor) -> torch.Tensor:
         out = torch.empty((ids.numel(), self.hidden_size), dtype=ctx.dtype, device=ids.device)
-        return ctx.ops.embedding(self.params["weight"], ids, out)
+        return ctx.ops.embedding(self.params["weight"], ids, out, **self._feed(ctx))
 
 
 class ScaledEmbedding(TokenEmbedding):
@@ -35,7 +41,7 @@ class ScaledEmbedding(TokenEmbedding):
 
     def forward(self, ctx, ids: torch.Tensor) -> torch.Tensor:
         out = torch.empty((ids.numel(), self.hidden_size), dtype=torch.float32, device=ids.device)
-        return ctx.ops.embedding_scaled(self.params["weight"], ids, out, self.scale)
+        return ctx.ops.embedding_scaled(self.params["weight"], ids, out, self.scale, **self._feed(ctx))
 
 
 class PositionedEmbedding(TokenEmbedding):
@@ -56,7 +62,8 @@ class PositionedEmbedding(TokenEmbedding):
 
     def forward(self, ctx, ids: torch.Tensor) -> torch.Tensor:
         out = torch.empty((ids.numel(), self.hidden_size), dtype=torch.float32, device=ids.device)
-        return ctx.ops.embedding_positions(self.params["weight"], self.params["positions"], ids, ctx.positions, out)
+        return ctx.ops.embedding_positions(self.params["weight"], self.params["positions"], ids, ctx.positions, out,
+                                           **self._feed(ctx))
 
 
 class SinusoidalEmbedding(TokenEmbedding):

@@ -179,3 +179,23 @@ def test_mix_step(heads, rank, lens, slots, dtype):
     assert float((got.cpu().double() - want_state).norm() / want_state.norm()) <= 2e-6
     assert float((out.cpu().double() - want).norm() / want.norm()) <= (4e-3 if dtype == torch.bfloat16 else 4e-6)
     assert torch.equal(got[3].cpu(), state[3])
+
+
+@pytest.mark.parametrize("which", ["embedding", "embedding_scaled", "embedding_positions"])
+def test_embeddings_of_tokens_still_on_the_device(which):
+    """As after ``feed_tokens``, which it takes the place of: the rows, and the ids left for the kernels behind it.  Several
+    blocks a row; sources that name no sampled row leave the id."""
+    ops = gpu_ops()
+    table, rows = rnd((40, 2500), 1).bfloat16().to(DEV), rnd((9, 2500), 2).bfloat16().to(DEV)
+    ids, source, sampled = (i32(v).to(DEV) for v in ([7, 0, 39, 3, 1], [2, -1, 0, 3, 1], [11, 12, 13]))
+    rest = {"embedding": (), "embedding_scaled": (2.5,), "embedding_positions": ()}[which]
+
+    def run(ids, **kw):
+        out = torch.empty((5, 2500), dtype=torch.float32, device=DEV)
+        if which == "embedding_positions":
+            return ops.embedding_positions(table, rows, ids, i32([0, 8, 3, 1, 2]).to(DEV), out, **kw)
+        return getattr(ops, which)(table, ids, out, *rest, **kw)
+
+    fed = ops.feed_tokens(ids.clone(), source, sampled)
+    assert fed.tolist() == [13, 0, 11, 3, 12]
+    assert torch.equal(run(ids, feed=(source, sampled)), run(fed)) and torch.equal(ids, fed)
