@@ -57,13 +57,29 @@ sum_norm_kernel(float* __restrict__ stream, float alpha, SumTerms terms, const f
 typedef __attribute__((ext_vector_type(4))) float sn_f32x4;
 typedef __attribute__((ext_vector_type(4))) __bf16 sn_bf16x4;
 
-template <typename T, int V>
+// SHIFT: every request brings one token, and `out` receives the new rows as shift_rows blends them, out = x + (x' - x) * mu
+// with x' what the request's slot holds, where the new row is left.  (Two rows of 2,048: 3.6 us behind a sum_norm of 4.0 in a
+// launch of its own.)
+struct ShiftOne {
+  const float* mu;
+  float* state;
+  long slot_stride, state_off;
+  const int* slot_of_seq;
+  const int* token_seq;
+};
+
+template <typename T, int V, bool SHIFT>
 __global__ void __launch_bounds__(256)
 sum_norm_vec_kernel(float* __restrict__ stream, float alpha, SumTerms terms, const float* __restrict__ weight, float eps,
-                    T* __restrict__ out, int width) {
+                    T* __restrict__ out, int width, ShiftOne shift) {
   __shared__ float scratch[16];
   const size_t base = (size_t)blockIdx.x * width;
   sn_f32x4 v[V], w[V];
+  float* kept = nullptr;
+  if constexpr (SHIFT) {
+    const int seq = shift.token_seq[blockIdx.x], slot = seq >= 0 ? shift.slot_of_seq[seq] : -1;
+    if (slot >= 0) kept = shift.state + (size_t)slot * shift.slot_stride + shift.state_off;
+  }
 #pragma unroll
   for (int j = 0; j < V; ++j) {
     const int i = (threadIdx.x + 256 * j) * 4;
@@ -96,6 +112,18 @@ sum_norm_vec_kernel(float* __restrict__ stream, float alpha, SumTerms terms, con
 #pragma unroll
     for (int j = 0; j < V; ++j) v[j] += terms.scale[k] * y[j];
   }
+  sn_f32x4 prev[SHIFT ? V : 1], mu[SHIFT ? V : 1];
+  if constexpr (SHIFT) {
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      const int i = (threadIdx.x + 256 * j) * 4;
+      prev[j] = mu[j] = sn_f32x4{0.f, 0.f, 0.f, 0.f};
+      if (i < width) {
+        if (kept != nullptr) prev[j] = *reinterpret_cast<const sn_f32x4*>(kept + i);
+        mu[j] = *reinterpret_cast<const sn_f32x4*>(shift.mu + i);
+      }
+    }
+  }
   float inv = 1.f;
   if (weight != nullptr) {
     float ss = 0.f;
@@ -111,6 +139,10 @@ sum_norm_vec_kernel(float* __restrict__ stream, float alpha, SumTerms terms, con
     if (i >= width) break;
     sn_f32x4 o = weight != nullptr ? v[j] * inv * w[j] : v[j];
     *reinterpret_cast<sn_f32x4*>(stream + base + i) = o;
+    if constexpr (SHIFT) {
+      if (kept != nullptr) *reinterpret_cast<sn_f32x4*>(kept + i) = o;
+      o = o + (prev[j] - o) * mu[j];
+    }
     if (out != nullptr) {
       if constexpr (sizeof(T) == 2) {
         sn_bf16x4 b;
@@ -142,8 +174,8 @@ ATOM_EXPORT int atom_sum_norm(float* stream, float alpha, const void* y0, int d0
   for (int i = 0; i < n; ++i) vec = vec && (size_t)terms.y[i] % 16 == 0;
   if (vec) {
 #define ATOM_SUM_NORM_VEC(V)                                                                                        \
-  ATOM_DISPATCH_DTYPE(out_dtype, hipLaunchKernelGGL((sum_norm_vec_kernel<T, V>), dim3(rows), dim3(256), 0, stream_id, stream, \
-                                                     alpha, terms, weight, eps, (T*)out, width))
+  ATOM_DISPATCH_DTYPE(out_dtype, hipLaunchKernelGGL((sum_norm_vec_kernel<T, V, false>), dim3(rows), dim3(256), 0, stream_id, \
+                                                     stream, alpha, terms, weight, eps, (T*)out, width, ShiftOne{}))
     if (width <= 1024) ATOM_SUM_NORM_VEC(1);
     else if (width <= 2048) ATOM_SUM_NORM_VEC(2);
     else if (width <= 4096) ATOM_SUM_NORM_VEC(4);
@@ -153,6 +185,36 @@ ATOM_EXPORT int atom_sum_norm(float* stream, float alpha, const void* y0, int d0
   }
   ATOM_DISPATCH_DTYPE(out_dtype, hipLaunchKernelGGL((sum_norm_kernel<T>), dim3(rows), dim3(256), smem, stream_id, stream,
                                                      alpha, terms, weight, eps, (T*)out, width));
+  return launch_status();
+}
+
+// The same with the rows blended with their predecessors on the way out; every request brings one token.  ATOM_UNSUPPORTED where
+// the rows cannot be read four entries at a time.
+ATOM_EXPORT int atom_sum_norm_shift(float* stream, float alpha, const void* y0, int d0, float s0, const void* y1, int d1,
+                                    float s1, const void* y2, int d2, float s2, const void* y3, int d3, float s3, int n,
+                                    const float* weight, float eps, void* out, int out_dtype, int rows, int width,
+                                    const float* mu, float* state, long slot_stride, long state_off, const int* slot_of_seq,
+                                    const int* token_seq, hipStream_t stream_id) {
+  if (rows < 0 || width <= 0 || n < 0 || n > 4 || !stream || !out || !weight) return ATOM_BAD_SHAPE;
+  if (!mu || !state || !slot_of_seq || !token_seq || state_off < 0 || slot_stride < state_off + width) return ATOM_BAD_SHAPE;
+  SumTerms terms{{y0, y1, y2, y3}, {d0, d1, d2, d3}, {s0, s1, s2, s3}, n};
+  uintptr_t ends = (uintptr_t)stream | (uintptr_t)weight | (uintptr_t)out | (uintptr_t)mu | (uintptr_t)state;
+  for (int i = 0; i < n; ++i) {
+    if (terms.y[i] == nullptr) return ATOM_BAD_SHAPE;
+    if (terms.dtype[i] != ATOM_F32 && terms.dtype[i] != ATOM_BF16) return ATOM_BAD_DTYPE;
+    ends |= (uintptr_t)terms.y[i];
+  }
+  if (width % 4 || width > 8192 || ends % 16 || slot_stride % 4 || state_off % 4) return ATOM_UNSUPPORTED;
+  if (rows == 0) return ATOM_OK;
+  const ShiftOne shift{mu, state, slot_stride, state_off, slot_of_seq, token_seq};
+#define ATOM_SUM_NORM_SHIFT(V)                                                                                              \
+  ATOM_DISPATCH_DTYPE(out_dtype, hipLaunchKernelGGL((sum_norm_vec_kernel<T, V, true>), dim3(rows), dim3(256), 0, stream_id, \
+                                                     stream, alpha, terms, weight, eps, (T*)out, width, shift))
+  if (width <= 1024) ATOM_SUM_NORM_SHIFT(1);
+  else if (width <= 2048) ATOM_SUM_NORM_SHIFT(2);
+  else if (width <= 4096) ATOM_SUM_NORM_SHIFT(4);
+  else ATOM_SUM_NORM_SHIFT(8);
+#undef ATOM_SUM_NORM_SHIFT
   return launch_status();
 }
 

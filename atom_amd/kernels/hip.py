@@ -225,7 +225,7 @@ class HipKernels:
                    "atom_selective_scan", "atom_step_sizes", "atom_experts_few", "atom_experts_few_supports", "atom_keys_as_values_heads_write",
                    "atom_delta_chunks", "atom_delta_chunks_supports", "atom_delta_step", "atom_delta_step_supports",
                    "atom_rglru_step", "atom_rglru_step_supports", "atom_space_step",
-                   "atom_space_step_supports", "atom_mix_step", "atom_mix_step_supports"):
+                   "atom_space_step_supports", "atom_mix_step", "atom_mix_step_supports", "atom_sum_norm_shift"):
             getattr(self.lib, fn).restype = ctypes.c_int
         self.lib.atom_delta_chunks_floats.restype = ctypes.c_long
         self.lib.atom_gemm_f32_scratch.restype = ctypes.c_long
@@ -254,6 +254,7 @@ class HipKernels:
         self.use_delta_chunks = True   # the delta rule of prompts in chunks of 64 tokens
         self.use_delta_step = True     # ... and of single tokens in one launch with what is before and behind it
         self.use_scan_step = True      # state-space and time-mixing recurrences of single tokens with what stands around them
+        self.use_sum_norm_shift = True # single tokens: a norm's sum with the token shift behind it
         self.use_rglru_step = True     # the real-gated recurrence of single tokens in two launches
         self.use_together_tiles = True  # attention with the heads together on the matrix cores, for prompt portions
         self.use_mfma_latent = True     # attention over latent pages on the matrix cores (bfloat16, sizes it is built for)
@@ -391,6 +392,11 @@ class HipKernels:
             if not ok:
                 raise KernelError(f"{name}: shape {tuple(have)} does not match {tuple(shape)}")
         return t
+
+    @staticmethod
+    def _unaligned(*tensors) -> bool:
+        """Whether any of the tensors (None: there is none) begins where 16-byte accesses cannot."""
+        return any(t is not None and t.data_ptr() % 16 for t in tensors)
 
     def _done(self, what: str, status: int):
         if status != 0:
@@ -1433,6 +1439,7 @@ class HipKernels:
         in steps of 16."""
         ranks = tuple(0 if w is None else w.shape[1] for w in (decay2, gate2))
         if (not self.use_delta_step or taps_weight.dtype != out.dtype or state.shape[1] % 4 or state_off % 4
+                or self._unaligned(state, taps_weight, decay2, gate2)
                 or not self.lib.atom_delta_step_supports(heads, kv_heads, dim, vdim, taps_weight.shape[1], *ranks)):
             return None
         tokens, seqs = proj.shape[0], slot_of_seq.numel()
@@ -1539,6 +1546,7 @@ class HipKernels:
         step sizes, x at ``x_off``) to ``out``.  Returns ``out``, or None where the kernels do not take these sizes: heads of 64
         or 128 rows by 64 columns, four taps, one group of the norm."""
         if (not self.use_scan_step or taps_weight.dtype != out.dtype or state.shape[1] % 4 or state_off % 4 or proj.shape[1] % 4
+                or self._unaligned(proj, state, taps_weight, weight, out)
                 or not self.lib.atom_space_step_supports(heads, groups, dim, vdim, taps_weight.shape[1], norm_groups)):
             return None
         tokens, seqs, inner = proj.shape[0], slot_of_seq.numel(), heads * vdim
@@ -1569,6 +1577,7 @@ class HipKernels:
         128 in steps of 32."""
         rank = squashed.shape[1]
         if (not self.use_scan_step or decay2.dtype != out.dtype or state.shape[1] % 4 or state_off % 4
+                or self._unaligned(state, decay2)
                 or not self.lib.atom_mix_step_supports(heads, dim, rank)):
             return None
         tokens, seqs, c = out.shape[0], slot_of_seq.numel(), heads * dim
@@ -1866,6 +1875,7 @@ class HipKernels:
         seqs, blocks, part = slot_of_seq.numel(), ra.shape[0], ra.shape[1]
         dt = out.dtype
         if (not self.use_rglru_step or taps_weight.dtype != dt or ra.dtype != dt or tokens > seqs
+                or self._unaligned(taps_weight, ra, ri)
                 or not self.lib.atom_rglru_step_supports(seqs, channels, part, taps_weight.shape[1])):
             return None
         self._check("branches", proj, torch.float32, (tokens, None))
@@ -2025,6 +2035,38 @@ class HipKernels:
             _ptr(stream), ctypes.c_float(alpha), *terms, len(summands), _ptr(weight), ctypes.c_float(eps), _ptr(out),
             self._code(out) if out is not None else 0, rows, width, self._stream()))
         return stream
+
+    def sum_norm_shift(self, stream, alpha: float, summands, scales, weight, eps: float, mu, out, state, state_off: int,
+                       slot_of_seq, token_seq):
+        """For steps whose requests bring one token each: ``sum_norm`` of ``stream`` and ``shift_rows`` of its new rows into
+        ``out`` in one launch.  Returns ``out``, or None where the kernel does not take these rows (widths that are a multiple
+        of four up to 8,192)."""
+        rows, width = stream.shape
+        if (not self.use_sum_norm_shift or width % 4 or width > 8192 or state.shape[1] % 4 or state_off % 4
+                or self._unaligned(stream, mu, out, weight, state, *summands)):
+            return None
+        self._check("stream", stream, torch.float32)
+        if len(summands) > 4 or len(summands) != len(scales):
+            raise KernelError("sum_norm_shift: up to four summands, a scale each")
+        for y in summands:
+            self._check("summand", y, (torch.float32, torch.bfloat16), (rows, width))
+        self._check("norm weight", weight, torch.float32, (width,))
+        self._check("shift weight", mu, torch.float32, (width,))
+        self._check("shifted rows", out, (torch.float32, torch.bfloat16), (rows, width))
+        self._check("state", state, torch.float32, (None, None))
+        self._check("slot_of_seq", slot_of_seq, torch.int32, (None,))
+        self._check("token_seq", token_seq, torch.int32, (rows,))
+        terms = []
+        for i in range(4):
+            if i < len(summands):
+                terms += [_ptr(summands[i]), self._code(summands[i]), ctypes.c_float(scales[i])]
+            else:
+                terms += [None, 0, ctypes.c_float(0.0)]
+        self._done("sum_norm_shift", self.lib.atom_sum_norm_shift(
+            _ptr(stream), ctypes.c_float(alpha), *terms, len(summands), _ptr(weight), ctypes.c_float(eps), _ptr(out),
+            self._code(out), rows, width, _ptr(mu), _ptr(state), ctypes.c_long(state.shape[1]), ctypes.c_long(state_off),
+            _ptr(slot_of_seq), _ptr(token_seq), self._stream()))
+        return out
 
     def shift_rows(self, x, mu, out, state, state_off: int, cu_seqlens_q, slot_of_seq, token_seq):
         """``out[t] = x[t] + (x[t - 1] - x[t]) * mu``; the row before a request's first token of the step is what its

@@ -11,7 +11,7 @@ from dataclasses import dataclass, field
 import torch
 
 from ..cache.kinds import kind_of
-from ..parts.base import BLOCKS, EMBEDDINGS, HEADS, JOINS, NORMS, Part, PartChoice, PendingPost
+from ..parts.base import BLOCKS, EMBEDDINGS, HEADS, JOINS, NORMS, Part, PartChoice, Pending
 
 
 @dataclass(frozen=True)
@@ -153,14 +153,14 @@ class CausalLM(Part):
         residual = None
         for run, cache in zip(self.order, caches):
             block = self.blocks[run.layer]
-            if isinstance(hidden, PendingPost) and (run.enters or not block.accepts_pending_post):
+            if isinstance(hidden, Pending) and (run.enters or not isinstance(hidden, block.accepts_pending)):
                 hidden = hidden.resolve(ctx)
             if run.enters:
                 hidden, residual = self.join.forward(ctx, hidden, residual, first)
             hidden, residual = block.forward(ctx, hidden, residual, cache)
         if want_rows is None or want_rows.numel() == 0:
             return None
-        if isinstance(hidden, PendingPost):
+        if isinstance(hidden, Pending):
             hidden = hidden.resolve(ctx)
         if not self.final_norm.accepts_deferred:
             hidden = ctx.ops.materialize(hidden)

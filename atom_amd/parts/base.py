@@ -167,9 +167,14 @@ class ScaledSum:
     dtype = torch.float32
 
 
-class PendingPost:
+class Pending:
+    """What a block hands on instead of its stream or its last summand, for the next block's first kernel to take along.  A block
+    names the kinds it takes (``accepts_pending``); anything else is handed ``resolve(ctx)``."""
+
+
+class PendingPost(Pending):
     """A sublayer's result whose own norm has not been applied yet: ``norm(x)`` is to join the residual stream.  A block
-    that ``accepts_pending_post`` forms it, adds it and norms the stream for its first sublayer in one kernel; anything
+    that takes it forms it, adds it and norms the stream for its first sublayer in one kernel; anything
     else is handed ``resolve(ctx)``, the summand itself in float32."""
 
     def __init__(self, x, norm):
@@ -177,6 +182,20 @@ class PendingPost:
 
     def resolve(self, ctx):
         return self.norm.forward(ctx, self.x, out_dtype=torch.float32)
+
+
+class PendingSum(Pending):
+    """A stream that is still to become ``norm(alpha * stream + sum_i scales[i] * terms[i])``; ``copy``: with its rows in the
+    step's type beside it."""
+
+    def __init__(self, stream, alpha: float, terms, scales, norm, copy: bool):
+        self.stream, self.alpha, self.terms, self.scales, self.norm, self.copy = stream, alpha, terms, scales, norm, copy
+
+    def resolve(self, ctx):
+        reads = self.norm.forward_sum(ctx, self.terms, self.scales, self.stream, self.alpha, copy=self.copy)
+        if reads is not self.stream:
+            ctx.memo[("stream copy", self.stream.data_ptr())] = reads
+        return self.stream
 
 
 class StreamUpdate:
@@ -296,8 +315,8 @@ class FeedForward(Part):
 
 
 class Block(Part):
-    #: True when ``forward`` takes a ``PendingPost`` for ``hidden``
-    accepts_pending_post = False
+    #: the kinds of ``Pending`` that ``forward`` takes for ``hidden``
+    accepts_pending: tuple = ()
 
     def forward(self, ctx, hidden: torch.Tensor, residual: torch.Tensor | None, cache):
         """Returns (hidden, residual) for the next block."""

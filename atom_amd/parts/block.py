@@ -6,7 +6,7 @@ from __future__ import annotations
 
 import torch
 
-from .base import BLOCKS, FEED_FORWARDS, MIXERS, NORMS, Block, ParamSpec, PartChoice, PendingPost, ScaledSum, StreamUpdate
+from .base import BLOCKS, FEED_FORWARDS, MIXERS, NORMS, Block, ParamSpec, PartChoice, PendingPost, PendingSum, ScaledSum, StreamUpdate
 
 
 class PreNormBlock(Block):
@@ -55,7 +55,7 @@ class SandwichBlock(Block):
     one block to the next through a ``PendingPost`` (two kernels of 5.0 and 4.0 us in a step of 4 rows of 2,048, one of
     4.1 so)."""
 
-    accepts_pending_post = True
+    accepts_pending = (PendingPost,)
 
     def __init__(self, mixer: PartChoice, feed_forward: PartChoice | None, norm: PartChoice, prefix: str = "",
                  names: dict[str, str] | None = None):
@@ -170,7 +170,11 @@ class NormedSumBlock(Block):
     stream, which is float32 and kept whole (nothing pending); its rows in the step's type, for the products that
     read them, come out of the kernel that norms it.  A mixer with ``reads_stream`` is handed the float32 rows.
     ``names["mixer"]`` may be empty: the mixer then takes the layer's own prefix.  A checkpoint that holds the second
-    norm's weight for a layer without feed-forward gets the second step with nothing added: ``x <- norm2(alpha x)``."""
+    norm's weight for a layer without feed-forward gets the second step with nothing added: ``x <- norm2(alpha x)``.
+    In steps of single tokens the last norm may be left to the next block (a ``PendingSum``), whose mixer can take the sum
+    and the norm into its own first kernel (``forward_pending``)."""
+
+    accepts_pending = (PendingSum,)
 
     def __init__(self, mixer: PartChoice, feed_forward: PartChoice | None, norm: PartChoice, alpha: float = 1.0,
                  prefix: str = "", names: dict[str, str] | None = None):
@@ -210,20 +214,31 @@ class NormedSumBlock(Block):
         ops = ctx.ops
         if residual is not None:
             raise ValueError("this block takes the whole stream, with nothing pending beside it")
-        stream = ops.materialize(hidden)
+        mixed = None
+        if isinstance(hidden, PendingSum):
+            stream, ahead = hidden.stream, getattr(self._mixer, "forward_pending", None)
+            mixed = ahead(ctx, hidden, cache) if ahead is not None else None
+            if mixed is None:
+                hidden.resolve(ctx)
+        else:
+            stream = ops.materialize(hidden)
         if stream.dtype != torch.float32:
             raise ValueError("this block keeps a float32 stream: the embedding before it must write float32")
-        reads = ctx.memo.pop(("stream copy", stream.data_ptr()), None)
-        if self._mixer.reads_stream:
-            reads = stream
-        elif reads is None:
-            reads = stream if ctx.dtype == torch.float32 else ops.cast_rows(stream, ctx.dtype)
-        terms, scales = self._summands(ops, self._mixer.forward(ctx, reads, cache))
+        if mixed is None:
+            reads = ctx.memo.pop(("stream copy", stream.data_ptr()), None)
+            if self._mixer.reads_stream:
+                reads = stream
+            elif reads is None:
+                reads = stream if ctx.dtype == torch.float32 else ops.cast_rows(stream, ctx.dtype)
+            mixed = self._mixer.forward(ctx, reads, cache)
+        terms, scales = self._summands(ops, mixed)
         # the copy is for the feed-forward, or for the next block's mixer where that reads one
         reads = self.mixer_norm.forward_sum(ctx, terms, scales, stream, self.alpha,
                                             copy=self.ffn is not None or not self._mixer.reads_stream)
         if self.ffn is not None:
             terms, scales = self._summands(ops, self.ffn.forward(ctx, reads))
+            if ctx.max_q_len == 1 and hasattr(self._mixer, "forward_pending") and hasattr(ops, "sum_norm_shift"):
+                return PendingSum(stream, self.alpha, terms, scales, self.ffn_norm, not self._mixer.reads_stream), None
             reads = self.ffn_norm.forward_sum(ctx, terms, scales, stream, self.alpha, copy=not self._mixer.reads_stream)
         elif self.ffn_norm is not None:
             reads = self.ffn_norm.forward_sum(ctx, [], [], stream, self.alpha, copy=not self._mixer.reads_stream)

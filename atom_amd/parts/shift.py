@@ -11,6 +11,7 @@ from __future__ import annotations
 import torch
 
 from .base import MIXERS, Mixer, ParamSpec, PartChoice, StateNeed
+from .norm import RMSNorm
 from .parallel import JointNeed
 
 
@@ -46,6 +47,20 @@ class ShiftedMixer(Mixer):
         blended = torch.empty(tuple(x.shape), dtype=ctx.dtype, device=x.device)
         ctx.ops.shift_rows(x, self.params["mu"], blended, cache.parts[0].state, 0, ctx.cu_seqlens_q, ctx.slot_of_seq,
                            ctx.token_seq)
+        return self.inner.forward(ctx, blended, cache.parts[1])
+
+
+    def forward_pending(self, ctx, pending, cache):
+        """In a step of single tokens: the sum and the norm that the stream waits for and the blend of its new rows in one
+        kernel; None where there is none for these rows (nothing has been done then)."""
+        if not isinstance(pending.norm, RMSNorm):
+            return None
+        stream = pending.stream
+        blended = torch.empty(tuple(stream.shape), dtype=ctx.dtype, device=stream.device)
+        if ctx.ops.sum_norm_shift(stream, pending.alpha, pending.terms, pending.scales, pending.norm.params["weight"],
+                                  pending.norm.eps, self.params["mu"], blended, cache.parts[0].state, 0, ctx.slot_of_seq,
+                                  ctx.token_seq) is None:
+            return None
         return self.inner.forward(ctx, blended, cache.parts[1])
 
 

@@ -199,3 +199,26 @@ def test_embeddings_of_tokens_still_on_the_device(which):
     fed = ops.feed_tokens(ids.clone(), source, sampled)
     assert fed.tolist() == [13, 0, 11, 3, 12]
     assert torch.equal(run(ids, feed=(source, sampled)), run(fed)) and torch.equal(ids, fed)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("width,terms", [(4, 1), (1020, 2), (2048, 2), (4100, 1), (8192, 4)])
+def test_sum_norm_shift(width, terms, dtype):
+    """The bits of ``sum_norm`` and ``shift_rows`` in turn: rows with a slot, padding rows, a request that sits out."""
+    ops = gpu_ops()
+    dev = lambda t: t.to(DEV)  # noqa: E731
+    stream, weight, mu = dev(rnd((4, width), 1)), dev(1 + rnd((width,), 2, 0.2)), dev(rnd((width,), 3, 0.5))
+    ys = [dev(rnd((4, width), 4 + i).to(torch.bfloat16 if i % 2 else torch.float32)) for i in range(terms)]
+    scales, state = [0.5 + i for i in range(terms)], dev(rnd((5, 8 + width), 9))
+    cu, slots, seqs = dev(i32([0, 1, 2, 2, 3, 4])), dev(i32([3, 0, 1, -1, 4])), dev(i32([0, 1, -1, 4]))
+
+    want_stream, want_state, want = stream.clone(), state.clone(), torch.empty((4, width), dtype=dtype, device=DEV)
+    ops.sum_norm(want_stream, 1.5, ys, scales, weight, 1e-5)
+    ops.shift_rows(want_stream, mu, want, want_state, 4, cu, slots, seqs)
+    out = torch.empty((4, width), dtype=dtype, device=DEV)
+    assert ops.sum_norm_shift(stream, 1.5, ys, scales, weight, 1e-5, mu, out, state, 4, slots, seqs) is out
+    assert torch.equal(stream, want_stream) and torch.equal(state, want_state)
+    # (a product and a sum may be one rounding in one kernel and two in the other)
+    assert float((out.double() - want.double()).abs().max()) <= (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -22) * float(want.abs().max())
+    assert ops.sum_norm_shift(stream[:, :3].contiguous(), 1.5, [], [], weight[:3].clone(), 1e-5, mu[:3].clone(), out[:, :3].contiguous(),
+                              state, 4, slots, seqs) is None
