@@ -53,31 +53,35 @@ ATOM_EXPORT int atom_rotation_table(const int* positions, const double* freq, fl
 }
 
 // proj [tokens, ld] float32 holds, where asked for, the latent of the queries at cq_off (cq_rank entries) and the
-// down-projection of the keys at kv_off (rank entries, then rot).  A block a token.
+// down-projection of the keys at kv_off (rank entries, then rot).
 template <typename T>
-__global__ void __launch_bounds__(256)
-latent_prepare_kernel(const float* __restrict__ proj, int ld, int cq_off, int cq_rank, const float* __restrict__ cq_w,
-                      T* __restrict__ cq, int kv_off, int rank, int rot, int rot_dims, const float* __restrict__ norm_w,
-                      float eps, const float2* __restrict__ turns, const int* __restrict__ slots, T* __restrict__ pages) {
-  __shared__ float scratch[2][4];
-  const int t = blockIdx.x;
+struct LatentRows {
+  const float* proj; int ld;
+  int cq_off, cq_rank; const float* cq_w; T* cq;
+  int kv_off, rank, rot, rot_dims; const float* norm_w; float eps;
+  const float2* turns; const int* slots; T* pages;
+};
+
+// Token t, by a block of 256 threads.
+template <typename T>
+__device__ __forceinline__ void prepare_latent(const LatentRows<T>& p, int t, float (*scratch)[4]) {
   const int tid = threadIdx.x;
-  const float* row = proj + (size_t)t * ld;
-  const int slot = slots ? slots[t] : -1;   // the same for the whole block
+  const float* row = p.proj + (size_t)t * p.ld;
+  const int slot = p.slots ? p.slots[t] : -1;   // the same for the whole block
   // both norms' sums of squares in one pass and one meeting of the waves
   float ss_q = 0.f, ss_k = 0.f;
 #pragma unroll 4
-  for (int i = tid; i < cq_rank; i += 256) ss_q += row[cq_off + i] * row[cq_off + i];
+  for (int i = tid; i < p.cq_rank; i += 256) ss_q += row[p.cq_off + i] * row[p.cq_off + i];
   if (slot >= 0) {
 #pragma unroll 4
-    for (int i = tid; i < rank; i += 256) ss_k += row[kv_off + i] * row[kv_off + i];
+    for (int i = tid; i < p.rank; i += 256) ss_k += row[p.kv_off + i] * row[p.kv_off + i];
     // the shared rotated key part: by the last wave first, while the others are still adding
-    T* dst = pages + (size_t)slot * (rank + rot) + rank;
-    for (int i = 255 - tid; i < rot; i += 256) {
-      float v = row[kv_off + rank + i];
-      if (i < rot_dims) {
-        const float2 cs = turns[(size_t)t * (rot_dims / 2) + (i >> 1)];
-        const float other = row[kv_off + rank + (i ^ 1)];
+    T* dst = p.pages + (size_t)slot * (p.rank + p.rot) + p.rank;
+    for (int i = 255 - tid; i < p.rot; i += 256) {
+      float v = row[p.kv_off + p.rank + i];
+      if (i < p.rot_dims) {
+        const float2 cs = p.turns[(size_t)t * (p.rot_dims / 2) + (i >> 1)];
+        const float other = row[p.kv_off + p.rank + (i ^ 1)];
         v = (i & 1) ? v * cs.x + other * cs.y : v * cs.x - other * cs.y;
       }
       dst[i] = from_f32<T>(v);
@@ -91,17 +95,24 @@ latent_prepare_kernel(const float* __restrict__ proj, int ld, int cq_off, int cq
   }
   __syncthreads();
   // x / sqrt(mean(x^2) + eps) * w
-  if (cq_rank > 0) {
-    const float rstd = 1.f / sqrtf((scratch[0][0] + scratch[0][1] + scratch[0][2] + scratch[0][3]) / (float)cq_rank + eps);
+  if (p.cq_rank > 0) {
+    const float rstd = 1.f / sqrtf((scratch[0][0] + scratch[0][1] + scratch[0][2] + scratch[0][3]) / (float)p.cq_rank + p.eps);
 #pragma unroll 4
-    for (int i = tid; i < cq_rank; i += 256) cq[(size_t)t * cq_rank + i] = from_f32<T>(row[cq_off + i] * rstd * cq_w[i]);
+    for (int i = tid; i < p.cq_rank; i += 256) p.cq[(size_t)t * p.cq_rank + i] = from_f32<T>(row[p.cq_off + i] * rstd * p.cq_w[i]);
   }
   if (slot >= 0) {
-    const float rstd = 1.f / sqrtf((scratch[1][0] + scratch[1][1] + scratch[1][2] + scratch[1][3]) / (float)rank + eps);
-    T* dst = pages + (size_t)slot * (rank + rot);
+    const float rstd = 1.f / sqrtf((scratch[1][0] + scratch[1][1] + scratch[1][2] + scratch[1][3]) / (float)p.rank + p.eps);
+    T* dst = p.pages + (size_t)slot * (p.rank + p.rot);
 #pragma unroll 4
-    for (int i = tid; i < rank; i += 256) dst[i] = from_f32<T>(row[kv_off + i] * rstd * norm_w[i]);
+    for (int i = tid; i < p.rank; i += 256) dst[i] = from_f32<T>(row[p.kv_off + i] * rstd * p.norm_w[i]);
   }
+}
+
+// A block a token.
+template <typename T>
+__global__ void __launch_bounds__(256) latent_prepare_kernel(LatentRows<T> p) {
+  __shared__ float scratch[2][4];
+  prepare_latent(p, blockIdx.x, scratch);
 }
 
 ATOM_EXPORT int atom_latent_prepare(const float* proj, int ld, int cq_off, int cq_rank, const float* cq_w, void* cq,
@@ -117,9 +128,9 @@ ATOM_EXPORT int atom_latent_prepare(const float* proj, int ld, int cq_off, int c
     if (rot_dims > 0 && turns == nullptr) return ATOM_BAD_SHAPE;
   }
   if (tokens == 0 || (cq_rank == 0 && slots == nullptr)) return ATOM_OK;
-  ATOM_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((latent_prepare_kernel<T>), dim3(tokens), dim3(256), 0, stream, proj, ld,
-                                                 cq_off, cq_rank, cq_w, (T*)cq, kv_off, rank, rot, rot_dims, norm_w, eps,
-                                                 (const float2*)turns, slots, (T*)pages));
+  ATOM_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((latent_prepare_kernel<T>), dim3(tokens), dim3(256), 0, stream,
+                                                 LatentRows<T>{proj, ld, cq_off, cq_rank, cq_w, (T*)cq, kv_off, rank, rot, rot_dims,
+                                                               norm_w, eps, (const float2*)turns, slots, (T*)pages}));
   return launch_status();
 }
 
@@ -693,11 +704,22 @@ constexpr int kHWideRows = 96;   // from here on the wide tiles
 
 // For fewer rows: a block owns 16 columns of one head and 16 tokens; its four waves share out K (wave v the steps v, v + 4,
 // ..., four of them in flight) and meet once to add their sums, in the order of the waves.
+// With `rows`, the last column of blocks prepares the tokens' latents, which the product does not read: one launch of a decode
+// step less.
 template <typename TX, typename TY>
 __global__ void __launch_bounds__(256)
 heads_gemm_few_kernel(const TX* __restrict__ x, long ldx, long hsx, const bf16_t* __restrict__ w, TY* __restrict__ y,
-                      long ldy, long hsy, ProductGate gate, QueryTurn turn, int m, int n, int k, float alpha) {
+                      long ldy, long hsy, ProductGate gate, QueryTurn turn, int m, int n, int k, float alpha,
+                      LatentRows<bf16_t> rows) {
   __shared__ float part[4][16][17];
+  if (rows.proj != nullptr && blockIdx.x == gridDim.x - 1) {
+    const int end = min(m, ((int)blockIdx.y + 1) * 16);
+    for (int t = blockIdx.y * 16 + blockIdx.z; t < end; t += gridDim.z) {
+      prepare_latent(rows, t, reinterpret_cast<float(*)[4]>(&part[0][0][0]));
+      __syncthreads();                       // (the same trips for the whole block)
+    }
+    return;
+  }
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, r = lane % 16, g = lane / 16;
   const int h = blockIdx.z, row0 = blockIdx.y * 16, col0 = blockIdx.x * 16;
   if (col0 >= n) {   // the column of blocks behind the product's
@@ -776,7 +798,7 @@ ATOM_EXPORT int atom_heads_gemm_mfma(const void* x, int x_dtype, long ldx, long 
     grid = dim3((n + 15) / 16 + (rot > 0 ? 1 : 0), (m + 15) / 16, heads);
 #define FEW(TX, TY)                                                                                                 \
   hipLaunchKernelGGL((heads_gemm_few_kernel<TX, TY>), grid, block, 0, stream, (const TX*)x, ldx, hsx, (const bf16_t*)w, \
-                     (TY*)y, ldy, hsy, g, q, m, n, k, alpha)
+                     (TY*)y, ldy, hsy, g, q, m, n, k, alpha, LatentRows<bf16_t>{})
     switch (x_dtype * 2 + y_dtype) {
       case 0: FEW(float, float); break;
       case 1: FEW(float, bf16_t); break;
@@ -792,5 +814,31 @@ ATOM_EXPORT int atom_heads_gemm_mfma(const void* x, int x_dtype, long ldx, long 
   else
     hipLaunchKernelGGL((heads_gemm_split_kernel<bf16_t>), grid, block, 0, stream, (const float*)x, ldx, hsx,
                        (const bf16_t*)w, (bf16_t*)y, ldy, hsy, g, q, m, n, k, alpha);
+  return launch_status();
+}
+
+// The queries' absorption and the tokens' latents in one launch, for up to 95 tokens: head h's queries at h (dim + rot) of a row of
+// proj, `dim` entries that w [heads, rank, dim] brings into the latent space and `rot` rotated ones, times scale, go to
+// q_abs [tokens, heads, rank + rot]; the latents at kv_off go to row slots[t] of the pages (see atom_latent_prepare).
+ATOM_EXPORT int atom_latent_absorb(const float* proj, int ld, int kv_off, int rank, int rot, int rot_dims, const float* norm_w,
+                                   float eps, const void* turns, const int* slots, void* pages, const void* w, void* q_abs,
+                                   int heads, int tokens, int dim, float scale, hipStream_t stream) {
+  if (tokens < 0 || heads <= 0 || heads > 65535 || rank <= 0 || rot <= 0 || rot_dims < 0 || rot_dims > rot || (rot_dims & 1) ||
+      dim <= 0)
+    return ATOM_BAD_SHAPE;
+  if (!proj || !norm_w || !slots || !pages || !w || !q_abs || (rot_dims > 0 && !turns)) return ATOM_BAD_SHAPE;
+  if (kv_off < 0 || kv_off + rank + rot > ld || (long)heads * (dim + rot) > ld) return ATOM_BAD_SHAPE;
+  if (tokens >= kHWideRows || !atom_heads_gemm_mfma_supports(ATOM_F32, ATOM_BF16, 0, ld, dim + rot, dim)) return ATOM_UNSUPPORTED;
+  if (((uintptr_t)proj | (uintptr_t)w) & 15) return ATOM_BAD_SHAPE;
+  if (tokens == 0) return ATOM_OK;
+  const int width = rank + rot;
+  const QueryTurn q{proj + dim, (bf16_t*)q_abs + rank, ld, dim + rot, (long)heads * width, width, (const float2*)turns, rot, rot_dims,
+                    scale};
+  const LatentRows<bf16_t> rows{proj, ld, 0, 0, nullptr, nullptr, kv_off, rank, rot, rot_dims, norm_w, eps, (const float2*)turns,
+                                slots, (bf16_t*)pages};
+  const dim3 grid((rank + 15) / 16 + 2, (tokens + 15) / 16, heads);
+  hipLaunchKernelGGL((heads_gemm_few_kernel<float, bf16_t>), grid, dim3(256), 0, stream, proj, (long)ld, (long)(dim + rot),
+                     (const bf16_t*)w, (bf16_t*)q_abs, (long)heads * width, (long)width, ProductGate{}, q, tokens, rank, dim, scale,
+                     rows);
   return launch_status();
 }

@@ -225,7 +225,7 @@ class HipKernels:
                    "atom_selective_scan", "atom_step_sizes", "atom_experts_few", "atom_experts_few_supports", "atom_keys_as_values_heads_write",
                    "atom_delta_chunks", "atom_delta_chunks_supports", "atom_delta_step", "atom_delta_step_supports",
                    "atom_rglru_step", "atom_rglru_step_supports", "atom_space_step",
-                   "atom_space_step_supports", "atom_mix_step", "atom_mix_step_supports", "atom_sum_norm_shift"):
+                   "atom_space_step_supports", "atom_mix_step", "atom_mix_step_supports", "atom_sum_norm_shift", "atom_latent_absorb"):
             getattr(self.lib, fn).restype = ctypes.c_int
         self.lib.atom_delta_chunks_floats.restype = ctypes.c_long
         self.lib.atom_gemm_f32_scratch.restype = ctypes.c_long
@@ -1176,6 +1176,30 @@ class HipKernels:
             _ptr(norm_weight) if slots is not None else None, ctypes.c_float(eps), _ptr(turns) if pairs else None,
             _ptr(slots), _ptr(pages) if slots is not None else None, self._code(cq if cq is not None else pages), tokens,
             self._stream()))
+
+    def latent_absorb(self, proj, pages, slots, kv_off: int, rank: int, rot: int, norm_weight, eps: float, turns, weight, out,
+                      heads: int, dim: int, scale: float):
+        """``latent_prepare`` (no query latent) and the queries' absorbing product with their turn (``heads_gemm``) in one launch,
+        for bfloat16 steps of fewer than 96 tokens: ``proj`` float32 [tokens, *] with head h's queries, ``dim`` entries and then
+        ``rot`` rotated ones, at ``h (dim + rot)``; ``weight`` [heads, rank, dim]; ``out`` [tokens, heads, rank + rot].  Returns
+        ``out``, or None where the launch does not take this step."""
+        tokens, ld = proj.shape
+        if (out.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or not 1 <= tokens < 96 or not rot
+                or tokens < self.heads_mfma_from or self._unaligned(proj, weight)
+                or not self.lib.atom_heads_gemm_mfma_supports(F32, BF16, ctypes.c_long(0), ctypes.c_long(ld),
+                                                              ctypes.c_long(dim + rot), dim)):
+            return None
+        self._check("projections", proj, torch.float32)
+        self._check("latent norm weight", norm_weight, torch.float32, (rank,))
+        self._check("slot mapping", slots, torch.int32, (tokens,))
+        self._check("latent pages", pages, torch.bfloat16, (None, None, rank + rot))
+        self._check("key up-projection", weight, torch.bfloat16, (heads, rank, dim))
+        self._check("absorbed queries", out, torch.bfloat16, (tokens, heads, rank + rot))
+        pairs = self._pairs(turns, tokens, rot)
+        self._done("latent_absorb", self.lib.atom_latent_absorb(
+            _ptr(proj), ld, kv_off, rank, rot, 2 * pairs, _ptr(norm_weight), ctypes.c_float(eps), _ptr(turns) if pairs else None,
+            _ptr(slots), _ptr(pages), _ptr(weight), _ptr(out), heads, tokens, dim, ctypes.c_float(scale), self._stream()))
+        return out
 
     def _pairs(self, turns, tokens: int, rot: int) -> int:
         """How many pairs of a rotated part of ``rot`` entries a rotation table turns."""

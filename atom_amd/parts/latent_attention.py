@@ -139,14 +139,19 @@ class LatentAttention(Mixer):
             latent_q = new(T, self.query_rank)
             query = (0, self.params["q_down_norm.weight"], latent_q)
         writes = self.own_keys and cache.writes
-        if writes or query is not None:
+        q_abs = new(T, H, width)
+        absorb = getattr(ops, "latent_absorb", None) if writes and query is None else None
+        done = absorb is not None and absorb(proj, cache.pages, ctx.slot_mappings[cache.group], self.down_offset, rank, r,
+                                             self.p("down_norm.weight"), self.norm_eps, turns, self.up_k, q_abs, H, d,
+                                             self.scale) is not None
+        if not done and (writes or query is not None):
             ops.latent_prepare(proj, cache.pages, ctx.slot_mappings[cache.group] if writes else None, self.down_offset,
                                rank, r, self.p("down_norm.weight"), self.norm_eps, turns, query)
         if query is not None:
             q = ops.linear(latent_q, self.params["q_up.weight"], None, out_dtype=torch.float32)
-        q_abs = new(T, H, width)
-        ops.heads_gemm(q, 0, q.shape[1], d + r, self.up_k, q_abs, 0, H * width, width, H, T, rank, d, alpha=self.scale,
-                       turn=QueryTurn(d, rank, r, turns, self.scale))
+        if not done:
+            ops.heads_gemm(q, 0, q.shape[1], d + r, self.up_k, q_abs, 0, H * width, width, H, T, rank, d, alpha=self.scale,
+                           turn=QueryTurn(d, rank, r, turns, self.scale))
         latent = new(T, H, rank)
         ops.latent_attention(q_abs, cache.pages, latent, self._meta(ctx, cache.group), rank, self.p("sink"), self.window)
         out = new(T, H * dv)

@@ -222,3 +222,29 @@ def test_sum_norm_shift(width, terms, dtype):
     assert float((out.double() - want.double()).abs().max()) <= (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -22) * float(want.abs().max())
     assert ops.sum_norm_shift(stream[:, :3].contiguous(), 1.5, [], [], weight[:3].clone(), 1e-5, mu[:3].clone(), out[:, :3].contiguous(),
                               state, 4, slots, seqs) is None
+
+
+@pytest.mark.parametrize("tokens,heads,dim,rank,rot,dims", [(1, 16, 128, 512, 64, 64), (20, 3, 64, 40, 16, 8), (95, 2, 8, 128, 64, 0),
+                                                            (33, 17, 24, 64, 32, 32)])
+def test_latent_absorb(tokens, heads, dim, rank, rot, dims):
+    """The bits of ``latent_prepare`` and ``heads_gemm`` in turn, tokens without a slot among them."""
+    from atom_amd.kernels.hip import QueryTurn
+
+    ops = gpu_ops()
+    kv_off = heads * (dim + rot)
+    ld = (kv_off + rank + rot + 7) // 4 * 4
+    proj, norm = rnd((tokens, ld), 1).to(DEV), (1 + rnd((rank,), 2, 0.2)).to(DEV)
+    weight = rnd((heads, rank, dim), 3, dim ** -0.5).bfloat16().to(DEV)
+    turns = ops.rotation_table(torch.arange(tokens, dtype=torch.int32, device=DEV),
+                               (0.7 ** torch.arange(dims // 2, dtype=torch.float64)).to(DEV), 1.1) if dims else None
+    slots = torch.randperm(tokens + 5, generator=torch.Generator().manual_seed(4))[:tokens].int()
+    slots[tokens // 2 + 1:tokens // 2 + 2] = -1
+    slots = slots.to(DEV)
+    pages = rnd((2, (tokens + 6) // 2, rank + rot), 5).bfloat16().to(DEV)
+    want_pages, width = pages.clone(), rank + rot
+    want, out = (torch.empty((tokens, heads, width), dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    ops.latent_prepare(proj, want_pages, slots, kv_off, rank, rot, norm, 1e-5, turns)
+    ops.heads_gemm(proj, 0, ld, dim + rot, weight, want, 0, heads * width, width, heads, tokens, rank, dim, alpha=0.3,
+                   turn=QueryTurn(dim, rank, rot, turns, 0.3))
+    assert ops.latent_absorb(proj, pages, slots, kv_off, rank, rot, norm, 1e-5, turns, weight, out, heads, dim, 0.3) is out
+    assert torch.equal(out, want) and torch.equal(pages, want_pages)
