@@ -864,7 +864,7 @@ class HipKernels:
         library's own weight-streaming kernels, 65 to 256 rows of products up to 8,192 columns wide its kernel of
         tiles and K slices cut to the chip; the rest goes to the BLAS library, as the reference's engine
         does for its matrix products; anything with a float32 operand runs this library's float32
-        kernel (the matrix cores' float32 instructions, no reduced-precision mode).  With ``defer`` the result may come back as a
+        kernel (each operand as three bfloat16 pieces, no reduced-precision mode).  With ``defer`` the result may come back as a
         ``DeferredSum`` for a kernel that adds the slices while it reads them; without ``slices`` a product of the BLAS
         library is left in one piece (a ``DeferredSum`` is then one slice and its bias), for readers that take one."""
         if isinstance(x, (DeferredSum, PendingProduct)):

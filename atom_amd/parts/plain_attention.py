@@ -30,7 +30,7 @@ def padded_head(size: int) -> int:
 
 class PlainAttention(GroupedQueryAttention):
     graph_safe = True
-    accepts_deferred = False
+    accepts_deferred = True   # the input goes to the QKV product as it is
 
     def __init__(self, hidden_size: int, num_heads: int, num_kv_heads: int, head_dim: int, value_dim: int,
                  scale: float, unit_norm: bool = False, temperature: tuple | None = None, window: int | None = None,

@@ -22,6 +22,7 @@ from .base import MIXERS, Mixer, ParamSpec, StateNeed
 
 class StateSpaceMixer(Mixer):
     graph_safe = True
+    accepts_deferred = True   # the input goes to the first product as it is
 
     def __init__(self, hidden_size: int, num_heads: int, value_dim: int, state_size: int, groups: int,
                  conv_taps: int, norm_groups: int, norm_eps: float, prefix: str = "",
