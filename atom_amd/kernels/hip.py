@@ -864,7 +864,7 @@ class HipKernels:
         library's own weight-streaming kernels, 65 to 256 rows of products up to 8,192 columns wide its kernel of
         tiles and K slices cut to the chip; the rest goes to the BLAS library, as the reference's engine
         does for its matrix products; anything with a float32 operand runs this library's float32
-        kernel (each operand as three bfloat16 pieces, no reduced-precision mode).  With ``defer`` the result may come back as a
+        kernels (a float32 operand as three bfloat16 pieces that hold its 24 bits).  With ``defer`` the result may come back as a
         ``DeferredSum`` for a kernel that adds the slices while it reads them; without ``slices`` a product of the BLAS
         library is left in one piece (a ``DeferredSum`` is then one slice and its bias), for readers that take one."""
         if isinstance(x, (DeferredSum, PendingProduct)):
@@ -1118,7 +1118,7 @@ class HipKernels:
     def linear_f32(self, x, weight, bias=None):
         """``x @ weight.T (+ bias)`` summed in float32 whatever the operands' types, float32 out: for the few
         products that have to be 32-bit sums (a router's logits).  bfloat16 operands take the engine's ordinary
-        products with float32 output; anything with a float32 operand runs the matrix cores' float32 instructions."""
+        products with float32 output; anything with a float32 operand runs the kernels of ``gemm_f32.hip``."""
         x = self.materialize(x)
         m, k = x.shape
         n = weight.shape[0]
