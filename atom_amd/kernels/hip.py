@@ -937,9 +937,10 @@ class HipKernels:
         if bias is not None:
             self._check("linear bias", bias, torch.float32, (n,))
         y = torch.empty((m, n), dtype=out_dtype, device=x.device)
+        scratch = self._f32_scratch(x, weight, m, n, k)   # held until the launch is made
         self._done("gemm_f32", self.lib.atom_gemm_f32(
             _ptr(x), _DTYPE_CODE[x.dtype], _ptr(weight), _DTYPE_CODE[weight.dtype], _ptr(bias), _ptr(y), self._code(y), m, n, k,
-            _ptr(self._f32_scratch(x, weight, m, n, k)), self._stream()))
+            _ptr(scratch), self._stream()))
         return y
 
     def _f32_scratch(self, x, weight, m: int, n: int, k: int) -> torch.Tensor | None:
@@ -1021,9 +1022,10 @@ class HipKernels:
             if bias is not None:
                 self._check("linear bias", bias, torch.float32, (two,))
             act = torch.empty((m, inter), dtype=x.dtype, device=x.device)
+            scratch = self._f32_scratch(x, weight, m, two, k)   # held until the launch is made
             self._done("gemm_f32_gate", self.lib.atom_gemm_f32_gate(
                 _ptr(x), F32, _ptr(weight), self._code(weight), _ptr(bias), _ptr(act), m, inter, k,
-                _ptr(self._f32_scratch(x, weight, m, two, k)), self._stream()))
+                _ptr(scratch), self._stream()))
             return act
         gate_up = self.linear(x, weight, bias)
         act = torch.empty((m, inter), dtype=x.dtype, device=x.device)
