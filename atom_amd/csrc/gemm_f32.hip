@@ -5,8 +5,11 @@
 // leave: 3 x 8 bits hold its 24.  A product of two values is the six products of pieces that reach its last bits (hi lo, lo
 // hi, mid mid, hi mid, mid hi, hi hi; the three left out are below 2^-24 of it, a rounding of float32, at most, and a
 // sixth of the sums' own roundings on average), each exact in float32 and added there.  An operand that is bfloat16 is one
-// piece.  Two kinds of results are summed again, term by term in float32: those that are not finite (a piece behind an
-// infinity is a NaN), and those below 1e-18 and not 0, whose operands may have pieces below bfloat16's range.
+// piece.  A float32 operand is split times 2^24, and the sums are taken back as they join: float32 values are multiples of
+// 2^-149, so all pieces of any of them are then normal bfloat16 values (without that the pieces of operands below 2^-110 lose
+// bits, which the results show where the other operand is large).  What this takes from the other end, operands from 2^104 and
+// sums of 32 terms from 2^80 on, comes out as an infinity or a NaN, as infinities do themselves (a piece behind one is a NaN);
+// results that are not finite are summed again, term by term in float32.
 //
 // K is walked 32 terms at a time.  The 32 are summed apart, smallest pieces first, and join the sum of their slice; K is cut
 // into 8 slices, whose sums are added four and four in order, then the two.  That order is the same whatever M is and
@@ -59,6 +62,10 @@ __device__ __forceinline__ float silu_times(float gate, float up) { return gate 
 template <typename T>
 constexpr int kPieces = sizeof(T) == 4 ? 3 : 1;
 
+constexpr float kUp = 0x1p24f;   // what a float32 operand is split times
+template <typename T>
+constexpr float kDown = sizeof(T) == 4 ? 0x1p-24f : 1.f;
+
 // (Two values at a time: the instruction that rounds takes two, and their widened pieces are its result's halves.)
 __device__ __forceinline__ void pieces_of(const float (&v)[kLane], bf16x8 (&p)[3]) {
   typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -103,13 +110,13 @@ struct Products<1, 1> {
 // Every other step of K is therefore formed from x's negatives and subtracted (without that 1.21e-7 and 1.87e-7 in the figures
 // above, but 9.1e-7 for 4.6e-7 in attention's averages over 300 rows).
 __device__ __forceinline__ unsigned flip_of(int step) { return step & 1 ? 0x80000000u : 0u; }
-__device__ __forceinline__ float sign_of(int step) { return step & 1 ? -1.f : 1.f; }
+template <typename TX, typename TW>
+__device__ __forceinline__ float factor_of(int step) {
+  return step & 1 ? -kDown<TX> * kDown<TW> : kDown<TX> * kDown<TW>;
+}
 
 // Whether a result is one of those that pieces may have spoilt, and the result summed in float32, in the kernels' order.
-__device__ __forceinline__ bool spoilt(float v) {
-  const float a = fabsf(v);
-  return !(a < INFINITY) || (a < 1e-18f && a > 0.f);
-}
+__device__ __forceinline__ bool spoilt(float v) { return !(fabsf(v) < INFINITY); }
 
 template <typename TX, typename TW>
 __device__ __noinline__ float summed_again(const TX* x, const TW* w, int k) {
@@ -173,12 +180,12 @@ struct Terms {
       if (late > 3) q[h] = Quad{zero, zero, zero, zero};
     }
   }
-  // `flip`: the sign bit, or 0; with it the pieces are those of the terms' negatives.
+  // `flip`: the sign bit, or 0; with it the pieces are those of the terms' negatives.  (float32: of the terms times kUp.)
   __device__ __forceinline__ void pieces(bf16x8 (&p)[kPieces<T>], unsigned flip = 0) const {
     if constexpr (sizeof(T) == 4) {
       float v[kLane];
 #pragma unroll
-      for (int e = 0; e < kLane; ++e) v[e] = __uint_as_float(__float_as_uint(q[e / 4][e % 4]) ^ flip);
+      for (int e = 0; e < kLane; ++e) v[e] = q[e / 4][e % 4] * __uint_as_float(__float_as_uint(kUp) ^ flip);
       pieces_of(v, p);
     } else {
       typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
@@ -251,7 +258,7 @@ gemm_f32_kernel(GemmF32Params p) {
             for (int j = 0; j < NT; ++j) b[d][j].last_terms(at, quarter, p.k);
           }
         }
-        const float sign = sign_of(begin + base + d);
+        const float factor = factor_of<TX, TW>(begin + base + d);
         bf16x8 ap[MT][kPieces<TX>];
 #pragma unroll
         for (int i = 0; i < MT; ++i) a[d][i].pieces(ap[i], flip_of(begin + base + d));
@@ -269,7 +276,7 @@ gemm_f32_kernel(GemmF32Params p) {
 #pragma unroll
           for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int t = 0; t < 4; ++t) acc[i][j][t] = fmaf(part[i][t], sign, acc[i][j][t]);
+            for (int t = 0; t < 4; ++t) acc[i][j][t] = fmaf(part[i][t], factor, acc[i][j][t]);
         }
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -333,9 +340,10 @@ gemm_f32_kernel(GemmF32Params p) {
 // do.  A stage is 32 terms of the tile's rows, double buffered; the 16-byte pieces of a row change places by its row number, so
 // that the rows a wave reads at once lie in different banks.  While a stage is multiplied, the next one's operands are read from
 // LDS and the stage behind that comes from memory: 56 KB for two groups of four slices each, 40 KB in tiles of 128 rows, at the
-// 35 to 40 KB a microsecond that a CU draws, are what bounds it.  465 rows by 24,576 x 4,096 take 595 us in tiles of 128 rows and
-// 645 in tiles of 64 (945 with the float32 instructions), by 4,096 x 4,096, where only the lower ones are a tile for every CU, 109
-// (161), by 4,096 x 12,288 309 (475); 1,024 rows by 24,576 1,145, 180 TFLOP/s (1,885; the float32 instructions' rate is 157).
+// 35 to 40 KB a microsecond that a CU draws, are what bounds it.  465 rows by 24,576 x 4,096 take 569 us in tiles of 128 rows (938
+// with the float32 instructions; 645 in tiles of 64, timed when those were 595), by 4,096 x 4,096, where only the lower ones are a
+// tile for every CU, 110 (164), by 4,096 x 12,288 307 (475); 1,024 rows by 24,576 1,125, 183 TFLOP/s (1,873; the float32
+// instructions' rate is 157).  Of these, w times 2^24 as it is split takes 1 to 7 %: without it 562, 106 and 287 at 465 rows.
 // Five stages in LDS with all eight waves on each (32 x 32 of 64 x 128 a wave) took 705, 120 and 340 at 465 rows.
 constexpr int kWideCols = 128;
 
@@ -442,7 +450,7 @@ __global__ void __launch_bounds__(kSlices* kWave) gemm_f32_wide_kernel(GemmF32Pa
   float* met = (float*)(wide + (GROUPS == 2 ? 0 : 2 * kStageBytes)) + (GROUPS == 2 ? w4 : wave) * 64 * 32;
   const auto place = [&](int i, int j, int t) { return (16 * i + 4 * quarter + t) * 32 + 16 * j + side; };
   const bool second = GROUPS == 1 && steps > 4 * share;   // there are more slices than four
-  const auto multiply = [&](const Operands& o, float sign, bool last) {
+  const auto multiply = [&](const Operands& o, float factor, bool last) {
     bf16x8 bp[2][3];
     f32x4 part[2][4];
     o.b[0].pieces(bp[0]);
@@ -459,7 +467,7 @@ __global__ void __launch_bounds__(kSlices* kWave) gemm_f32_wide_kernel(GemmF32Pa
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) acc[i][j][t] = fmaf(part[j][i][t], sign, acc[i][j][t]);
+        for (int t = 0; t < 4; ++t) acc[i][j][t] = fmaf(part[j][i][t], factor, acc[i][j][t]);
     }
     // matrix instructions with the second half's splitting, then the first half's adding up, between them
 #pragma unroll
@@ -503,7 +511,7 @@ __global__ void __launch_bounds__(kSlices* kWave) gemm_f32_wide_kernel(GemmF32Pa
     if (stage + 2 < count) fetch(stage & 1, stage + 2);
     if (stage + 1 < count) read(next, stage + 1);
     __builtin_amdgcn_sched_barrier(0);
-    if (stage < count) multiply(now, sign_of(k0 / kStep + stage), stage + 1 == count);
+    if (stage < count) multiply(now, factor_of<float, float>(k0 / kStep + stage), stage + 1 == count);
   };
   for (int stage = 0; stage < low; stage += 2) {
     pass(even, odd, stage);

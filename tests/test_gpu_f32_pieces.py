@@ -65,3 +65,28 @@ def test_numbers_below_the_range_of_pieces(m, n, k):
     terms = x.cpu().double()[:, None] * w.cpu().double()[None, :40]
     assert float(y[1].abs().max()) == 0
     assert bool(((y[:, :40].double() - terms.sum(-1)).abs() <= (32 + k / 32) * 2.0 ** -24 * terms.abs().sum(-1) + 2.0 ** -149).all())
+
+
+# results of ordinary size, one operand near an end of the range: x's entries about 2^x_exp, w's about 2^w_exp
+@pytest.mark.parametrize("m,n,k", [(3, 70, 96), (449, 4096, 96), (20, 33, 1027)])
+@pytest.mark.parametrize("x_exp,w_exp", [(-118, 63), (-122, 70), (-135, 50), (-140, 100), (63, -118), (90, -130), (112, -100), (-90, 118)])
+def test_operands_near_the_ends_of_the_range(m, n, k, x_exp, w_exp):
+    ops = gpu_ops()
+    x, w = (torch.ldexp(rnd(s, seed).cpu().double(), torch.tensor(e)).float().to(DEV)
+            for s, seed, e in (((m, k), 1, x_exp), ((n, k), 2, w_exp)))
+    x[1] = 0.0
+    y = ops.linear(x, w).cpu()
+    terms = x.cpu().double()[:, None] * w.cpu().double()[None, :40]
+    assert float(y[1].abs().max()) == 0
+    assert bool(((y[:, :40].double() - terms.sum(-1)).abs() <= (32 + k / 32) * 2.0 ** -24 * terms.abs().sum(-1) + 2.0 ** -149).all())
+
+
+@pytest.mark.parametrize("x_type,w_type", [(torch.float32, torch.bfloat16), (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("x_exp,w_exp", [(-122, 70), (70, -122), (110, -100), (-100, 110)])
+def test_operands_of_two_types_near_the_ends_of_the_range(x_type, w_type, x_exp, w_exp):
+    ops = gpu_ops()
+    x, w = (torch.ldexp(rnd(s, seed).cpu().double(), torch.tensor(e)).to(t).to(DEV)
+            for s, seed, e, t in (((5, 160), 1, x_exp, x_type), ((70, 160), 2, w_exp, w_type)))
+    y = ops.linear(x, w, out_dtype=torch.float32).cpu()
+    terms = x.cpu().double()[:, None] * w.cpu().double()[None]
+    assert bool(((y.double() - terms.sum(-1)).abs() <= (32 + 160 / 32) * 2.0 ** -24 * terms.abs().sum(-1)).all())
