@@ -66,22 +66,19 @@ constexpr float kUp = 0x1p24f;   // what a float32 operand is split times
 template <typename T>
 constexpr float kDown = sizeof(T) == 4 ? 0x1p-24f : 1.f;
 
-// (Two values at a time: the instruction that rounds takes two, and their widened pieces are its result's halves.)
-__device__ __forceinline__ void pieces_of(const float (&v)[kLane], bf16x8 (&p)[3]) {
+// (Two values at a time, e and e + 1 of a lane's: the instruction that rounds takes two, and their widened pieces are its
+// result's halves.)
+__device__ __forceinline__ void pieces_of_two(float a, float b, bf16x8 (&p)[3], int e) {
   typedef float f32x2 __attribute__((ext_vector_type(2)));
   typedef bf16_t bf16x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
-  for (int e = 0; e < kLane; e += 2) {
-    float a = v[e], b = v[e + 1];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      const bf16x2 both = __builtin_convertvector(f32x2{a, b}, bf16x2);
-      p[i][e] = both[0];
-      p[i][e + 1] = both[1];
-      const unsigned bits = __builtin_bit_cast(unsigned, both);
-      a -= __uint_as_float(bits << 16);
-      b -= __uint_as_float(bits & 0xffff0000u);
-    }
+  for (int i = 0; i < 3; ++i) {
+    const bf16x2 both = __builtin_convertvector(f32x2{a, b}, bf16x2);
+    p[i][e] = both[0];
+    p[i][e + 1] = both[1];
+    const unsigned bits = __builtin_bit_cast(unsigned, both);
+    a -= __uint_as_float(bits << 16);
+    b -= __uint_as_float(bits & 0xffff0000u);
   }
 }
 
@@ -183,10 +180,9 @@ struct Terms {
   // `flip`: the sign bit, or 0; with it the pieces are those of the terms' negatives.  (float32: of the terms times kUp.)
   __device__ __forceinline__ void pieces(bf16x8 (&p)[kPieces<T>], unsigned flip = 0) const {
     if constexpr (sizeof(T) == 4) {
-      float v[kLane];
+      const float up = __uint_as_float(__float_as_uint(kUp) ^ flip);
 #pragma unroll
-      for (int e = 0; e < kLane; ++e) v[e] = q[e / 4][e % 4] * __uint_as_float(__float_as_uint(kUp) ^ flip);
-      pieces_of(v, p);
+      for (int e = 0; e < kLane; e += 2) pieces_of_two(q[e / 4][e % 4] * up, q[e / 4][e % 4 + 1] * up, p, e);
     } else {
       typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
       const bf16x8 all = __builtin_shufflevector(q[0], q[1], 0, 1, 2, 3, 4, 5, 6, 7);
@@ -340,10 +336,10 @@ gemm_f32_kernel(GemmF32Params p) {
 // do.  A stage is 32 terms of the tile's rows, double buffered; the 16-byte pieces of a row change places by its row number, so
 // that the rows a wave reads at once lie in different banks.  While a stage is multiplied, the next one's operands are read from
 // LDS and the stage behind that comes from memory: 56 KB for two groups of four slices each, 40 KB in tiles of 128 rows, at the
-// 35 to 40 KB a microsecond that a CU draws, are what bounds it.  465 rows by 24,576 x 4,096 take 569 us in tiles of 128 rows (938
+// 35 to 40 KB a microsecond that a CU draws, are what bounds it.  465 rows by 24,576 x 4,096 take 583 us in tiles of 128 rows (938
 // with the float32 instructions; 645 in tiles of 64, timed when those were 595), by 4,096 x 4,096, where only the lower ones are a
-// tile for every CU, 110 (164), by 4,096 x 12,288 307 (475); 1,024 rows by 24,576 1,125, 183 TFLOP/s (1,873; the float32
-// instructions' rate is 157).  Of these, w times 2^24 as it is split takes 1 to 7 %: without it 562, 106 and 287 at 465 rows.
+// tile for every CU, 108 (164), by 4,096 x 12,288 302 (475); 1,024 rows by 24,576 1,125, 183 TFLOP/s (1,873; the float32
+// instructions' rate is 157).  (w times 2^24 as it is split is 1 to 2 % of these.)
 // Five stages in LDS with all eight waves on each (32 x 32 of 64 x 128 a wave) took 705, 120 and 340 at 465 rows.
 constexpr int kWideCols = 128;
 
@@ -455,26 +451,37 @@ __global__ void __launch_bounds__(kSlices* kWave) gemm_f32_wide_kernel(GemmF32Pa
     f32x4 part[2][4];
     o.b[0].pieces(bp[0]);
     __builtin_amdgcn_sched_barrier(0);
-    o.b[1].pieces(bp[1]);
+    // the first half's matrix instructions with the second half's splitting, the second half's with the first half's adding up
+    // (in the order of the source, because the compiler splits in one go where registers are short)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int t = 0; t < Order::count; ++t)
+      for (int t = 0; t < Order::count; ++t) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           part[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.a[i][Order::x[t]], bp[j][Order::w[t]],
                                                                t ? part[j][i] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        if (t < 4) {
+          if (j == 0) {
+            const f32x4 q = o.b[1].q[t / 2];
+            pieces_of_two(q[t % 2 * 2] * kUp, q[t % 2 * 2 + 1] * kUp, bp[1], 2 * t);
+          } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+            for (int r = 0; r < 4; ++r) acc[t][0][r] = fmaf(part[0][t][r], factor, acc[t][0][r]);
+          }
+        }
 #pragma unroll
-        for (int t = 0; t < 4; ++t) acc[i][j][t] = fmaf(part[j][i][t], factor, acc[i][j][t]);
-    }
-    // matrix instructions with the second half's splitting, then the first half's adding up, between them
+        for (int i = 0; i < 4; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          if (j == 0) __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+          else __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
+        }
+        if (t == Order::count - 1) __builtin_amdgcn_sched_barrier(0);
+      }
 #pragma unroll
-    for (int t = 0; t < 48; ++t) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
-    }
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[i][1][r] = fmaf(part[1][i][r], factor, acc[i][1][r]);
     if (--until == 0 || last) {
       until = share;
 #pragma unroll
