@@ -9,7 +9,7 @@
 // 2^-149, so all pieces of any of them are then normal bfloat16 values (without that the pieces of operands below 2^-110 lose
 // bits, which the results show where the other operand is large).  What this takes from the other end, operands from 2^104 and
 // sums of 32 terms from 2^80 on, comes out as an infinity or a NaN, as infinities do themselves (a piece behind one is a NaN);
-// results that are not finite are summed again, term by term in float32.
+// results that are not finite are summed again by the float32 instructions.
 //
 // K is walked 32 terms at a time.  The 32 are summed apart, smallest pieces first, and join the sum of their slice; K is cut
 // into 8 slices, whose sums are added four and four in order, then the two.  That order is the same whatever M is and
@@ -51,10 +51,11 @@ struct GemmF32Params {
 
 // The row of w that stands at column `at` of the output tiles: with a gate every 16 columns are 8 gate rows and the up rows
 // of the same 8 columns of y, so that both meet in one place.
-__device__ __forceinline__ int row_of_w(const GemmF32Params& p, int at) {
-  if (p.inter == 0) return min(at, p.n - 1);
-  return min(at / kSide * 8 + at % 8, p.inter - 1) + (at % kSide < 8 ? 0 : p.inter);
+__device__ __forceinline__ int row_of_w(int n, int inter, int at) {
+  if (inter == 0) return min(at, n - 1);
+  return min(at / kSide * 8 + at % 8, inter - 1) + (at % kSide < 8 ? 0 : inter);
 }
+__device__ __forceinline__ int row_of_w(const GemmF32Params& p, int at) { return row_of_w(p.n, p.inter, at); }
 
 __device__ __forceinline__ float silu_times(float gate, float up) { return gate / (1.f + expf(-gate)) * up; }
 
@@ -110,26 +111,6 @@ __device__ __forceinline__ unsigned flip_of(int step) { return step & 1 ? 0x8000
 template <typename TX, typename TW>
 __device__ __forceinline__ float factor_of(int step) {
   return step & 1 ? -kDown<TX> * kDown<TW> : kDown<TX> * kDown<TW>;
-}
-
-// Whether a result is one of those that pieces may have spoilt, and the result summed in float32, in the kernels' order.
-__device__ __forceinline__ bool spoilt(float v) { return !(fabsf(v) < INFINITY); }
-
-template <typename TX, typename TW>
-__device__ __noinline__ float summed_again(const TX* x, const TW* w, int k) {
-  const int steps = (k + kStep - 1) / kStep, share = (steps + kSlices - 1) / kSlices;
-  float total = 0.f, half = 0.f;
-  for (int slice = 0; slice < kSlices; ++slice) {
-    float sum = 0.f;
-    for (int step = slice * share; step < min((slice + 1) * share, steps); ++step) {
-      float part = 0.f;
-      for (int i = step * kStep; i < min((step + 1) * kStep, k); ++i) part = fmaf(to_f32(x[i]), to_f32(w[i]), part);
-      sum += part;
-    }
-    half = slice % (kSlices / 2) ? half + sum : sum;
-    if (slice % (kSlices / 2) == kSlices / 2 - 1) total = slice < kSlices / 2 ? half : total + half;
-  }
-  return total;
 }
 
 // How a row's terms are read, four at a time.  kWhole: K is a multiple of 32 and rows begin at multiples of 16 bytes in
@@ -190,6 +171,68 @@ struct Terms {
     }
   }
 };
+
+// Whether a result is one of those that pieces may have spoilt.
+__device__ __forceinline__ bool spoilt(float v) { return !(fabsf(v) < INFINITY); }
+
+// 16 rows and columns summed by the float32 instructions, in the kernels' steps and slices: lane (side, quarter) brings row `side` of
+// both operands and receives column `side` of rows 4 quarter .. + 3.  (One lane a result, term by term: 465 rows by 24,576 x 4,096
+// 2,600 us with one row of NaN and 91 ms with nothing else.)
+template <int LOADS, typename TX, typename TW>
+__device__ __noinline__ f32x4 summed_again(const TX* x, const TW* w, int quarter, int k) {
+  constexpr int DEPTH = 2;
+  const int steps = (k + kStep - 1) / kStep, share = (steps + kSlices - 1) / kSlices;
+  Terms<TX> a[DEPTH];
+  Terms<TW> b[DEPTH];
+  const auto fetch = [&](int d, int step) {
+    if (step >= steps) return;
+    a[d].template read<LOADS>(x, step * kStep, quarter, k);
+    b[d].template read<LOADS>(w, step * kStep, quarter, k);
+  };
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d) fetch(d, d);
+  f32x4 total = {0.f, 0.f, 0.f, 0.f}, half = total, sum = total;
+  int until = share, slice = 0;
+#pragma unroll 1
+  for (int base = 0; base < steps; base += DEPTH) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+      const int step = base + d;
+      if (step >= steps) break;
+      if (LOADS == kAny && step == k / kStep) {
+        a[d].last_terms(step * kStep, quarter, k);
+        b[d].last_terms(step * kStep, quarter, k);
+      }
+      f32x4 part = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int e = 0; e < kLane; ++e)
+        part = __builtin_amdgcn_mfma_f32_16x16x4f32(to_f32(a[d].q[e / 4][e % 4]), to_f32(b[d].q[e / 4][e % 4]), part, 0, 0, 0);
+      fetch(d, step + DEPTH);
+      sum += part;
+      if (--until == 0 || step + 1 == steps) {
+        until = share;
+        half += sum;
+        sum = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (++slice == kSlices / 2 || step + 1 == steps) {
+          total += half;
+          half = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+      }
+    }
+  }
+  return total;
+}
+
+// Row r, column c of what summed_again left in the wave's lanes.
+__device__ __forceinline__ float picked(f32x4 sums, int r, int c) {
+  float v = 0.f;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const float other = __shfl(sums[t], r / 4 * kSide + c);
+    if (r % 4 == t) v = other;
+  }
+  return v;
+}
 
 template <typename TX, typename TW, int MT, int NT, int DEPTH, int LOADS>
 __global__ void __launch_bounds__(kSlices* kWave)
@@ -290,7 +333,7 @@ gemm_f32_kernel(GemmF32Params p) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) met[wave][(i * kSide + quarter * 4 + t) * kSide + side] = acc[i][j][t];
     __syncthreads();
-    const auto sum_of = [&](int e) {   // entry e % 16 of row e / 16, of rows and columns that are there
+    const auto sum_of = [&](int e) {   // entry e % 16 of row e / 16
       float sum = 0.f;
 #pragma unroll
       for (int half = 0; half < kSlices; half += kSlices / 2) {
@@ -299,18 +342,26 @@ gemm_f32_kernel(GemmF32Params p) {
         for (int s = 1; s < kSlices / 2; ++s) part += met[half + s][e];
         sum = half ? sum + part : part;
       }
-      if constexpr (kPieces<TX> * kPieces<TW> > 1) {
-        if (spoilt(sum))
-          sum = summed_again((const TX*)p.x + (size_t)(row0 + e / kSide) * p.k,
-                             (const TW*)p.w + (size_t)row_of_w(p, col0 + j * kSide + e % kSide) * p.k, p.k);
-      }
       return sum;
+    };
+    // of the 16 rows that hold row r, which a whole wave asks for together
+    const auto again = [&](int r) {
+      return summed_again<LOADS>((const TX*)p.x + (size_t)min(row0 + r / kSide * kSide + side, p.m - 1) * p.k,
+                          (const TW*)p.w + (size_t)row_of_w(p, col0 + j * kSide + side) * p.k, quarter, p.k);
     };
     if (p.inter != 0) {
       for (int e = tid; e < MT * kSide * 8; e += kSlices * kWave) {
         const int r = row0 + e / 8, c = (col0 + j * kSide) / 2 + e % 8;
-        if (r >= p.m || c >= p.inter) continue;
         float gate = sum_of(e / 8 * kSide + e % 8), up = sum_of(e / 8 * kSide + 8 + e % 8);
+        if constexpr (kPieces<TX> * kPieces<TW> > 1) {
+          if (__any(spoilt(gate) || spoilt(up))) {
+            const f32x4 sums = again(e / 8);
+            const float g = picked(sums, e / 8 % kSide, e % 8), u = picked(sums, e / 8 % kSide, 8 + e % 8);
+            if (spoilt(gate)) gate = g;
+            if (spoilt(up)) up = u;
+          }
+        }
+        if (r >= p.m || c >= p.inter) continue;
         if (p.bias != nullptr) gate += p.bias[c], up += p.bias[p.inter + c];
         ((float*)p.y)[(size_t)r * p.inter + c] = silu_times(gate, up);
       }
@@ -318,8 +369,14 @@ gemm_f32_kernel(GemmF32Params p) {
     }
     for (int e = tid; e < MT * kSide * kSide; e += kSlices * kWave) {
       const int r = row0 + e / kSide, c = col0 + j * kSide + e % kSide;
-      if (r >= p.m || c >= p.n) continue;
       float sum = sum_of(e);
+      if constexpr (kPieces<TX> * kPieces<TW> > 1) {
+        if (__any(spoilt(sum))) {
+          const float other = picked(again(e / kSide), e / kSide % kSide, e % kSide);
+          if (spoilt(sum)) sum = other;
+        }
+      }
+      if (r >= p.m || c >= p.n) continue;
       if (p.bias != nullptr) sum += p.bias[c];
       if (p.y_bf16)
         ((bf16_t*)p.y)[(size_t)r * p.n + c] = from_f32<bf16_t>(sum);
@@ -365,6 +422,32 @@ __global__ void __launch_bounds__(256) split_f32_kernel(const float* __restrict_
   v.pieces(p, flip_of(at / 4 % steps));
 #pragma unroll
   for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(pieces + (i * eights + at) * kLane) = p[i];
+}
+
+// The place of row 16 i + 4 quarter + t, column 16 j + side among a wave's 64 x 32 sums in LDS.
+__device__ __forceinline__ int place_of(int i, int j, int t, int quarter, int side) {
+  return (16 * i + 4 * quarter + t) * 32 + 16 * j + side;
+}
+
+// The wide kernel's: of a wave's 64 x 32 sums in LDS, from row `row0` and column `col0` on, those that pieces may have spoilt.
+// (Through LDS, so that the kernel has no registers to keep for it.)
+__device__ __noinline__ void sum_again_wide(const float* x, const float* w, int m, int n, int k, int inter, float* sums, int row0, int col0) {
+  const int lane = threadIdx.x % kWave, side = lane % kSide, quarter = lane / kSide;
+#pragma unroll 1
+  for (int i = 0; i < 4; ++i)
+#pragma unroll 1
+    for (int j = 0; j < 2; ++j) {
+      float* own[4];
+      bool any = false;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) own[t] = sums + place_of(i, j, t, quarter, side), any = any || spoilt(*own[t]);
+      if (!__any(any)) continue;
+      const f32x4 again = summed_again<kWhole>(x + (size_t)min(row0 + 16 * i + side, m - 1) * k,
+                                               w + (size_t)row_of_w(n, inter, col0 + 16 * j + side) * k, quarter, k);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        if (spoilt(*own[t])) *own[t] = again[t];
+    }
 }
 
 template <int ROWS>
@@ -444,7 +527,7 @@ __global__ void __launch_bounds__(kSlices* kWave) gemm_f32_wide_kernel(GemmF32Pa
   int until = share, slice = 0;                     // steps until the slice ends
   // the first four slices' sums: those of the other half of the block, or the wave's own
   float* met = (float*)(wide + (GROUPS == 2 ? 0 : 2 * kStageBytes)) + (GROUPS == 2 ? w4 : wave) * 64 * 32;
-  const auto place = [&](int i, int j, int t) { return (16 * i + 4 * quarter + t) * 32 + 16 * j + side; };
+  const auto place = [&](int i, int j, int t) { return place_of(i, j, t, quarter, side); };
   const bool second = GROUPS == 1 && steps > 4 * share;   // there are more slices than four
   const auto multiply = [&](const Operands& o, float factor, bool last) {
     bf16x8 bp[2][3];
@@ -538,6 +621,32 @@ __global__ void __launch_bounds__(kSlices* kWave) gemm_f32_wide_kernel(GemmF32Pa
     __syncthreads();
     if (group) return;
   }
+  bool any = false;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        if (GROUPS == 2 || second)
+          total[i][j][t] = GROUPS == 2 ? total[i][j][t] + met[place(i, j, t)] : met[place(i, j, t)] + total[i][j][t];
+        any = any || spoilt(total[i][j][t]);
+      }
+  if (__any(any)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) met[place(i, j, t)] = total[i][j][t];
+    sum_again_wide((const float*)p.x, (const float*)p.w, p.m, p.n, p.k, p.inter, met, row0 + r0, col0 + 32 * w4);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) total[i][j][t] = met[place(i, j, t)];
+  }
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -551,9 +660,6 @@ __global__ void __launch_bounds__(kSlices* kWave) gemm_f32_wide_kernel(GemmF32Pa
         const int r = row0 + r0 + 16 * i + 4 * quarter + t;
         if (r >= p.m) continue;
         float sum = total[i][j][t];
-        if (GROUPS == 2 || second) sum = GROUPS == 2 ? sum + met[place(i, j, t)] : met[place(i, j, t)] + sum;
-        if (spoilt(sum))
-          sum = summed_again((const float*)p.x + (size_t)r * p.k, (const float*)p.w + (size_t)row_of_w(p, at) * p.k, p.k);
         if (p.bias != nullptr) sum += bias;
         if (p.inter != 0) {
           const float up = __shfl_xor(sum, 8);

@@ -90,3 +90,51 @@ def test_operands_of_two_types_near_the_ends_of_the_range(x_type, w_type, x_exp,
     y = ops.linear(x, w, out_dtype=torch.float32).cpu()
     terms = x.cpu().double()[:, None] * w.cpu().double()[None]
     assert bool(((y.double() - terms.sum(-1)).abs() <= (32 + 160 / 32) * 2.0 ** -24 * terms.abs().sum(-1)).all())
+
+
+# tiles of every kernel; K below four, ragged, of whole steps
+@pytest.mark.parametrize("m,n,k", [(1, 70, 3), (3, 70, 1027), (9, 9000, 64), (30, 9000, 96), (40, 100, 130), (70, 5000, 100), (300, 3000, 96),
+                                   (449, 4096, 64), (2100, 4100, 288)])
+def test_results_that_are_not_finite_come_from_float32_sums(m, n, k):
+    """Large operands whose results are ordinary numbers, beside infinities and NaN; a row's result is its own."""
+    ops = gpu_ops()
+    x, w = rnd((m, k), 1), rnd((n, k), 2, 2.0 ** -20)
+    x[m // 2] *= 2.0 ** 122
+    x[m - 1, k // 2], w[n // 2, k - 1] = float("inf"), float("nan")
+    w[n - 1] *= 2.0 ** -70
+    big, cols = m // 2, slice(max(0, n - 40), n)
+    y = ops.linear(x, w)
+    terms = x[big].cpu().double() * w[cols].cpu().double()
+    if m > 1:
+        off = (y[big, cols].cpu().double() - terms.sum(-1)).abs()
+        held = terms.sum(-1).isfinite()
+        assert bool((off <= (32 + k / 32) * 2.0 ** -24 * terms.abs().sum(-1))[held].all()) and int(held.sum()) >= 39
+    assert not bool(y[m - 1].isfinite().any()) and bool(y[:, n // 2].isnan().all())
+    for row in {0, big, m - 1}:
+        assert torch.equal(ops.linear(x[row:row + 1].contiguous(), w)[0].nan_to_num(7.0), y[row].nan_to_num(7.0))
+    w = w[:n // 2 * 2].contiguous()
+    gate, want = ops.linear_silu(x, w), ops.linear(x, w)
+    a, b = want[:, :n // 2], want[:, n // 2:]
+    want = a / (1 + torch.exp(-a)) * b
+    close = (gate - want).abs() <= 1e-5 * want.abs()
+    assert bool((close | (gate == want) | (gate.isnan() & want.isnan())).all())
+
+
+def test_results_that_are_not_finite_cost_little():
+    ops = gpu_ops()
+
+    def passes(x, w, n=3):
+        events = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        ops.linear(x, w)
+        events[0].record()
+        for _ in range(n):
+            ops.linear(x, w)
+        events[1].record()
+        torch.cuda.synchronize()
+        return events[0].elapsed_time(events[1])
+
+    for m in (8, 465):
+        x, w = rnd((m, 4096), 1), rnd((8192, 4096), 2)
+        plain = passes(x, w)
+        x[:, 7] = float("nan")
+        assert passes(x, w) <= 10 * plain     # summed one by one: 30 and 130 times
