@@ -129,8 +129,7 @@ class LLMEngine:
         free, total = torch.cuda.mem_get_info(dev)
         used = total - free
         graphs = 0 if self.config.enforce_eager else self._graph_estimate()
-        scratch = max((part.scratch_bytes(self.ops, self.config.max_num_batched_tokens, self.config.max_num_seqs)
-                       for block in self.model.blocks for part in block.walk()), default=0)
+        scratch = LLMEngine._scratch(self, self.config.max_num_batched_tokens, self.config.max_num_seqs)
         safety = int(total * 0.02)
         budget = max(0, min(int(total * self.config.gpu_memory_utilization) - used - graphs - scratch - safety, free))
         logger.info("Memory budget: total_gpu=%.2fGB, free=%.2fGB, utilization=%s, in_use=%.2fGB, "
@@ -178,7 +177,11 @@ class LLMEngine:
             logits_rows += len(prefill_sizes) * sum(cfg.cudagraph_prefill_slots + n for n in mixed)
             rows = max(rows, max(prefill_sizes) + max(mixed))
         live = rows * (4 * spec.hidden_size + 8 * widest) * 4
-        return logits_rows * spec.vocab_size * 4 + 2 * live + (128 << 20)
+        return logits_rows * spec.vocab_size * 4 + 2 * live + self._scratch(rows, rows) + (128 << 20)
+
+    def _scratch(self, tokens: int, seqs: int) -> int:
+        """The largest scratch memory that a part takes in a step of ``tokens`` tokens."""
+        return max((part.scratch_bytes(self.ops, tokens, seqs) for block in self.model.blocks for part in block.walk()), default=0)
 
     def _log_capacity(self) -> None:
         """How many requests the pages hold at once, by context length

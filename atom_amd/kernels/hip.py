@@ -943,6 +943,13 @@ class HipKernels:
             _ptr(scratch), self._stream()))
         return y
 
+    # rows of x that a float32 product splits at a time (the kernel's own constant)
+    F32_SPLIT_ROWS = 2048
+
+    def product_scratch(self, rows: int, k: int) -> int:
+        """Bytes of scratch memory that a float32 product of up to ``rows`` rows over ``k`` terms takes at most."""
+        return 6 * min(rows, self.F32_SPLIT_ROWS) * k if rows > 64 and k % 32 == 0 else 0
+
     def _f32_scratch(self, x, weight, m: int, n: int, k: int) -> torch.Tensor | None:
         """Scratch memory of a float32 product with ``n`` rows of weights: the pieces of ``x`` where its tiles read those."""
         if m <= 64 or x.dtype != torch.float32 or weight.dtype != torch.float32:

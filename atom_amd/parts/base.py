@@ -91,8 +91,13 @@ class Part:
             yield from child.walk()
 
     def scratch_bytes(self, ops, tokens: int, seqs: int) -> int:
-        """Device memory that a step of ``tokens`` tokens of ``seqs`` requests takes in this part beside the activations."""
-        return 0
+        """Device memory that a step of ``tokens`` tokens of ``seqs`` requests takes in this part beside the activations: here
+        what its float32 products split their input into."""
+        product = getattr(ops, "product_scratch", None)
+        if product is None:
+            return 0
+        return max((product(tokens, p.shape[1]) for p in self.params.values() if p.dim() == 2 and p.dtype == torch.float32),
+                   default=0)
 
     def full_name(self, local: str) -> str:
         """The checkpoint name of ``local`` under this part's prefix; an empty ``local`` names the prefix itself

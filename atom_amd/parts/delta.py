@@ -65,10 +65,11 @@ class GatedDeltaRule(Mixer):
         return StateNeed((self.conv_floats + self.num_heads * self.head_dim * self.value_dim,), torch.float32)
 
     def scratch_bytes(self, ops, tokens, seqs):
+        products = super().scratch_bytes(ops, tokens, seqs)
         if not hasattr(ops, "delta_scratch"):
-            return 0
+            return products
         places, floats = ops.delta_scratch(tokens, seqs, self.num_heads, self.head_dim, self.value_dim, self.decay == "channel")
-        return 4 * places * floats
+        return max(products, 4 * places * floats)
 
     @property
     def decay_width(self) -> int:

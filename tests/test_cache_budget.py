@@ -36,3 +36,38 @@ def test_the_delta_rules_chunks_are_left_their_scratch_memory(monkeypatch):
     assert _budget([rule(32, 128)], 16384, monkeypatch) == plain - (1 << 30) // place * place     # 264 places are beyond the bound
     assert _budget([rule(32, 32)], 16384, monkeypatch) == plain                                   # walked whatever their length
     assert _budget([rule(32, 128)], 127, monkeypatch) == _budget([rule(32, 128, "channel")], 255, monkeypatch) == plain
+
+
+def _f32_mlp(hidden, inter, dtype=torch.float32):
+    part = GatedMLP(hidden, inter)
+    part.params = {name: torch.empty(spec.shape, dtype=dtype, device="meta") for name, spec in part.param_specs().items()}
+    return part
+
+
+def test_float32_products_are_left_their_scratch_memory(monkeypatch):
+    ops = _ops()
+    ops.F32_SPLIT_ROWS = HipKernels.F32_SPLIT_ROWS
+    ops.product_scratch = lambda *a: HipKernels.product_scratch(ops, *a)
+    monkeypatch.setattr("test_cache_budget._ops", lambda: ops)
+    plain = _budget([_f32_mlp(1024, 4096, torch.bfloat16)], 4096, monkeypatch)
+    assert _budget([_f32_mlp(512, 1024), _f32_mlp(1024, 4096)], 4096, monkeypatch) == plain - 6 * 2048 * 4096
+    assert _budget([_f32_mlp(1024, 4096)], 300, monkeypatch) == plain - 6 * 300 * 4096
+    assert _budget([_f32_mlp(1024, 4096)], 64, monkeypatch) == _budget([_f32_mlp(1000, 4100)], 4096, monkeypatch) == plain
+    rule = GatedDeltaRule(512, 8, 4, 128, 128, 4, 1e-6)
+    rule.params = {"o.weight": torch.empty(512, 65536, device="meta")}
+    assert _budget([rule], 256, monkeypatch) == plain - 6 * 256 * 65536
+
+
+def test_decode_graphs_are_left_the_scratch_memory_of_their_products():
+    ops = SimpleNamespace(product_scratch=lambda rows, k: 6 * rows * k)
+    config = SimpleNamespace(cudagraph_capture_sizes=[1, 128], max_num_seqs=128, cudagraph_prefill_sizes=[], cudagraph_prefill_slots=2,
+                             max_num_batched_tokens=4096, max_model_len=4096)
+
+    def estimate(dtype):
+        engine = LLMEngine.__new__(LLMEngine)
+        engine.config, engine.ops = config, ops
+        block = SimpleNamespace(walk=lambda: [_f32_mlp(1024, 4096, dtype)])
+        engine.model = SimpleNamespace(blocks=[block], spec=SimpleNamespace(hidden_size=1024, vocab_size=100))
+        return engine._graph_estimate()
+
+    assert estimate(torch.float32) == estimate(torch.bfloat16) + 6 * 128 * 4096

@@ -138,3 +138,14 @@ def test_results_that_are_not_finite_cost_little():
         plain = passes(x, w)
         x[:, 7] = float("nan")
         assert passes(x, w) <= 10 * plain     # summed one by one: 30 and 130 times
+
+
+def test_scratch_memory_is_within_what_the_cache_leaves_it():
+    ops = gpu_ops()
+    taken = 0
+    for m in (65, 100, 465, 2048, 2049, 5000):
+        for n, k in ((100, 32), (4096, 4096), (24576, 4096), (4096, 12288), (30000, 48)):
+            size = ops.lib.atom_gemm_f32_scratch(None, 0, None, 0, m, n, k)
+            assert size <= ops.product_scratch(m, k)
+            taken += size == ops.product_scratch(m, k) > 0
+    assert taken
