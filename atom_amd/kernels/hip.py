@@ -1397,9 +1397,21 @@ class HipKernels:
         floats = self.lib.atom_delta_chunks_floats(heads, dim, vdim)
         return min(tokens // 64 + seqs, max(1, self.DELTA_SCRATCH_BYTES // (4 * floats))), floats
 
+    def delta_walkers(self, seq_lens: list[int], per_channel: bool) -> float:
+        """How many requests of the longest portion's length the portions that go in chunks come to."""
+        least = self.DELTA_CHUNKS_FROM[per_channel]
+        return sum(n for n in seq_lens if n >= least) / max(seq_lens)
+
+    def delta_columns(self, heads: int, vdim: int, walkers: float) -> int:
+        """Value columns of a block that walks a request's chunks: two tiles of 16 where blocks of one would be more than the
+        CUs.  A chunk takes a block 4.3 us with one tile and a CU to itself, 9.1 with one tile and two blocks a CU, 7.3 with two
+        tiles: 5,569 tokens of four requests, 16 heads of 128 x 128, 290 us with one tile and 233 with two; one prompt of
+        2,048 tokens beside two requests that bring a token each, which return at once, 146 and 233."""
+        return 32 if vdim % 32 == 0 and heads * (vdim // 16) * walkers > self.num_cus else 16
+
     def delta_rule(self, qkv, gates, a_off: int, b_off: int, a_log, dt_bias, state, state_off: int, cu_seqlens_q,
                    slot_of_seq, out, heads: int, kv_heads: int, dim: int, vdim: int, decay=None,
-                   per_channel: bool = False, max_q_len: int | None = None, min_q_len: int = 1):
+                   per_channel: bool = False, max_q_len: int | None = None, min_q_len: int = 1, walkers: float | None = None):
         """The gated delta recurrence over each request's tokens.  ``qkv`` float32 [tokens, 2 kv_heads dim + heads
         vdim] (q | k | v after convolution and SiLU); ``gates`` float32 [tokens, *] with the raw beta inputs at
         ``b_off`` and, unless ``decay`` (float32 [tokens, *]) holds them, the raw decay inputs at ``a_off``: one
@@ -1410,7 +1422,8 @@ class HipKernels:
 
         Requests that bring ``DELTA_CHUNKS_FROM`` tokens or more take chunks of 64 tokens as matrix products (heads of 64 or
         128 key channels); their inputs are left as they are.  ``max_q_len`` and ``min_q_len``: the most and the fewest tokens
-        a request brings, or bounds of them (default: all tokens, and one), which say what need not be launched."""
+        a request brings, or bounds of them (default: all tokens, and one), which say what need not be launched.  ``walkers``:
+        what ``delta_walkers`` says of the requests (default: the most there can be); it picks a block's columns, not the result."""
         tokens, channels = qkv.shape
         seqs = slot_of_seq.numel()
         decay = gates if decay is None else decay
@@ -1436,7 +1449,8 @@ class HipKernels:
                 _ptr(qkv), tokens, channels, _ptr(gates), gates.shape[1], _ptr(decay), decay.shape[1], a_off, b_off,
                 int(bool(per_channel)), _ptr(a_log), _ptr(dt_bias), _ptr(state),
                 ctypes.c_long(state.shape[1]), ctypes.c_long(state_off), _ptr(cu_seqlens_q), _ptr(slot_of_seq), seqs,
-                _ptr(out), heads, kv_heads, dim, vdim, least, _ptr(scratch), room, self._stream()))
+                _ptr(out), heads, kv_heads, dim, vdim, least, _ptr(scratch), room,
+                self.delta_columns(heads, vdim, min(seqs, tokens // least) if walkers is None else walkers), self._stream()))
             if min_q_len >= least:
                 return out
         self._done("delta_rule", self.lib.atom_delta_rule(

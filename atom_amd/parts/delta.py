@@ -152,10 +152,14 @@ class GatedDeltaRule(Mixer):
         gate, gate_off = proj, at["gate"]
         if self.gate_low_rank:
             gate, gate_off = self._second(ops, proj, at["gate"], self.params["gate2.weight"]), 0
+        known = {}
+        if ctx.max_q_len > 1 and ctx.seq_lens:
+            known["min_q_len"] = min(ctx.seq_lens)
+            if hasattr(ops, "delta_walkers"):
+                known["walkers"] = ops.delta_walkers(ctx.seq_lens, self.decay == "channel")
         ops.delta_rule(qkv, proj, decay_off, at["beta"], self.params["A_log"], self.params["dt_bias"], cache.state,
                        self.conv_floats, ctx.cu_seqlens_q, ctx.slot_of_seq, read, H, self.num_kv_heads, self.head_dim,
-                       dv, decay=decay, per_channel=self.decay == "channel", max_q_len=ctx.max_q_len,
-                       min_q_len=min(ctx.seq_lens) if ctx.max_q_len > 1 and ctx.seq_lens else 1)
+                       dv, decay=decay, per_channel=self.decay == "channel", max_q_len=ctx.max_q_len, **known)
         out = torch.empty((T, H * dv), dtype=x.dtype, device=x.device)
         ops.delta_out(read, gate, gate_off, self.params["norm.weight"], self.norm_eps, out,
                       activation=self.gate_activation)
