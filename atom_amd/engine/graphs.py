@@ -316,8 +316,8 @@ class DecodeGraphs:
 
     def run(self, entries, cached: list[int]) -> torch.Tensor | None:
         """Float32 logits at the entries' wanted places (a portion's last row, a single token), in the
-        order of the entries; None if nothing is wanted.  For a step of single tokens the tensor may be the graph's own
-        output, valid until the graph's next replay."""
+        order of the entries; None if nothing is wanted.  Where the first entries of a step of single tokens want theirs, and
+        they alone, the tensor is the graph's own output, valid until the graph's next replay; elsewhere it is a copy."""
         shape = self.shape_for(entries)
         cap = self.captured.get(shape) or self._capture(shape)
         logits_row = self._fill(cap, entries, cached)
@@ -341,4 +341,4 @@ class DecodeGraphs:
         parts = [cap.logits[lo:hi] for lo, hi in runs]
         if len(parts) > 1:
             return torch.cat(parts)
-        return parts[0].clone() if shape[0] else parts[0]
+        return parts[0].clone() if shape[0] or runs[0][0] else parts[0]
