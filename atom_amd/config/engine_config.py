@@ -32,10 +32,11 @@ class Config:
     cudagraph_capture_sizes: list[int] = field(default_factory=lambda: [1, 2, 4, 8, 16, 32, 48, 64, 128, 256])
     # Steps that hold prompt portions beside decode tokens are replayed as graphs too when the portions
     # together have at most one of these many tokens (one graph per listed size and decode size of 8 and more).
-    # Empty: on an MI355X such steps keep the GPU busy when launched one by one, as long as they are launched ahead
-    # (deferred_output), and a graph pads every step to its bucket; only where the token budget and the layers are so
-    # small that launching takes longer than the work does are two sizes chosen (LLMEngine._prefill_graph_sizes).
-    cudagraph_prefill_sizes: list[int] = field(default_factory=list)
+    # Empty: none are.  None: the engine chooses.  On an MI355X such steps keep the GPU busy when launched one by one, as
+    # long as they are launched ahead (deferred_output), and a graph pads every step to its bucket; only where the token budget
+    # and the layers are so small that launching takes longer than the work does are two sizes chosen
+    # (LLMEngine._prefill_graph_sizes).
+    cudagraph_prefill_sizes: list[int] | None = None
     cudagraph_prefill_slots: int = 2      # prompt portions such a graph holds at most
     hf_overrides: dict | None = None
     dtype: str = "bf16"

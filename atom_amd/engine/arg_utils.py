@@ -81,7 +81,8 @@ class EngineArgs:
                             help="Decode batch sizes captured as HIP graphs.")
         parser.add_argument("--cudagraph-prefill-sizes", type=str, default="[]",
                             help="Ours: prompt-token capacities of graphs for steps with prompt portions beside decode "
-                                 "tokens, e.g. [512]; empty (the default): such steps are launched one by one, ahead of time.")
+                                 "tokens, e.g. [512]; empty (the default): such steps are launched one by one, ahead of time; "
+                                 "auto: graphs where the token budget and the layers are small.")
         parser.add_argument("--cudagraph-prefill-slots", type=int, default=2,
                             help="Ours: prompt portions one such graph holds at most.")
         parser.add_argument("--load-dummy", type=str, nargs="?", const="random", default=None,
@@ -114,7 +115,8 @@ class EngineArgs:
         kwargs = {f.name: getattr(self, f.name) for f in fields(self) if f.name != "model"}
         kwargs["kv_cache_block_size"] = kwargs.pop("block_size")
         kwargs["cudagraph_capture_sizes"] = parse_size_list(kwargs["cudagraph_capture_sizes"])
-        kwargs["cudagraph_prefill_sizes"] = parse_size_list(kwargs["cudagraph_prefill_sizes"])
+        sizes = kwargs["cudagraph_prefill_sizes"]
+        kwargs["cudagraph_prefill_sizes"] = None if sizes == "auto" else parse_size_list(sizes)
         kwargs.pop("level")
         if kwargs.pop("cudagraph_mode") == "NONE":
             kwargs["enforce_eager"] = True

@@ -138,7 +138,7 @@ class LLMEngine:
                     budget / 2**30)
         return budget
 
-    # Where no sizes are configured, steps with prompt portions are replayed if the token budget is at most this ...
+    # Where the sizes are left to the engine, steps with prompt portions are replayed if the token budget is at most this ...
     SMALL_BUDGET_TOKENS = 128
     # ... and a layer's weights are below this.  Launching a layer takes the host some 110 us (nine launches of 12 us, the
     # step's arrays apart), working it some 36 us beside its bytes at 5 TB/s, and rows up to 128 are padded for next to
@@ -149,7 +149,7 @@ class LLMEngine:
     def _prefill_graph_sizes(self) -> list[int]:
         """Portion sizes (tokens of a step's prompt portions together) that graphs are captured for."""
         cfg = self.config
-        if cfg.cudagraph_prefill_sizes:
+        if cfg.cudagraph_prefill_sizes is not None:
             return list(cfg.cudagraph_prefill_sizes)
         budget = min(cfg.max_num_batched_tokens, cfg.max_model_len or cfg.max_num_batched_tokens)
         heaviest = max((sum(p.numel() * p.element_size() for part in block.walk() for p in part.params.values())
