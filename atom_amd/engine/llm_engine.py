@@ -140,11 +140,15 @@ class LLMEngine:
 
     # Where the sizes are left to the engine, steps with prompt portions are replayed if the token budget is at most this ...
     SMALL_BUDGET_TOKENS = 128
-    # ... and a layer's weights are below this.  Launching a layer takes the host some 110 us (nine launches of 12 us, the
-    # step's arrays apart), working it some 36 us beside its bytes at 5 TB/s, and rows up to 128 are padded for next to
-    # nothing because the weights' bytes bound the products.  Three layers of 96 in float32, 16 tokens a step beside up to
-    # three decoding requests: 390 us launched, 95 replayed.
-    SMALL_LAYER_BYTES = 256 << 20
+    # ... and a layer's weights are at most this.  Launching a step of four layers takes the host 480 to 1,000 us; a graph pads
+    # it to its bucket, which is next to nothing in bfloat16, where the weights' bytes bound products of up to 128 rows, but not in
+    # float32 (24,576 x 4,096: one row 69 us, 32 rows 107).  Steps with portions of 16 to 120 tokens beside up to 30 decoding
+    # requests, launched over replayed: in bfloat16 1.2 to 2.6 with layers of 5 to 127 MB (Qwen3 layers of width 512 to 2,048, and
+    # four designs of width 1,024 and 2,048), 0.99 to 1.29 with 192 MB, 0.84 to 0.99 with 416 MB; in float32 1.3 to 1.6 with
+    # 11 MB and less, 1.1 to 1.3 with 43 MB of Qwen3 but down to 0.97 with 50 MB of the designs, 0.72 to 1.04 with 172 MB and
+    # more.  (A replayed step's attention is launched for the longest context the engine allows: 40,960 tokens instead of 1,300
+    # make these 0.01 to 0.16 less.)
+    SMALL_LAYER_BYTES = {torch.bfloat16: 200 << 20, torch.float32: 32 << 20}
 
     def _prefill_graph_sizes(self) -> list[int]:
         """Portion sizes (tokens of a step's prompt portions together) that graphs are captured for."""
@@ -154,7 +158,7 @@ class LLMEngine:
         budget = min(cfg.max_num_batched_tokens, cfg.max_model_len or cfg.max_num_batched_tokens)
         heaviest = max((sum(p.numel() * p.element_size() for part in block.walk() for p in part.params.values())
                         for block in self.model.blocks), default=0)
-        if budget > self.SMALL_BUDGET_TOKENS or heaviest > self.SMALL_LAYER_BYTES:
+        if budget > self.SMALL_BUDGET_TOKENS or heaviest > self.SMALL_LAYER_BYTES[self.dtype]:
             return []
         return sorted({n for n in (budget // 4, budget) if n >= 2})
 

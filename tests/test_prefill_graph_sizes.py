@@ -11,6 +11,7 @@ from atom_amd.engine.llm_engine import LLMEngine
 
 def sizes(configured, batched=64, max_len=4096, layer_bytes=1 << 20, dtype=torch.bfloat16):
     engine = LLMEngine.__new__(LLMEngine)
+    engine.dtype = dtype
     part = SimpleNamespace(params={"weight": torch.empty(layer_bytes // dtype.itemsize, dtype=dtype, device="meta")})
     engine.config = SimpleNamespace(cudagraph_prefill_sizes=configured, max_num_batched_tokens=batched, max_model_len=max_len)
     engine.model = SimpleNamespace(blocks=[SimpleNamespace(walk=lambda: [part])])
@@ -24,6 +25,11 @@ def test_what_the_caller_says_holds():
 def test_the_engine_chooses_where_nothing_is_said():
     assert Config.__dataclass_fields__["cudagraph_prefill_sizes"].default is None
     assert sizes(None) == [16, 64] and sizes(None, batched=16384) == [] and sizes(None, layer_bytes=1 << 30) == []
+
+
+def test_float32_layers_are_padded_dearly():
+    for layer, half, single in ((1 << 20, [16, 64], [16, 64]), (100 << 20, [16, 64], []), (250 << 20, [], [])):
+        assert sizes(None, layer_bytes=layer) == half and sizes(None, layer_bytes=layer, dtype=torch.float32) == single
 
 
 def test_the_command_line_says_none_some_or_leaves_it_to_the_engine():
