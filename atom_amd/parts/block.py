@@ -82,7 +82,8 @@ class SandwichBlock(Block):
 
     def forward(self, ctx, hidden, residual, cache):
         ops = ctx.ops
-        if isinstance(hidden, PendingPost) and residual is not None and hidden.norm.eps == self.mixer_pre.eps:
+        if (isinstance(hidden, PendingPost) and residual is not None and type(self.mixer_pre) is type(hidden.norm)
+                and hidden.norm.eps == self.mixer_pre.eps):
             hidden = hidden.norm.forward_post(ctx, hidden.x, residual, self.mixer_pre)
         else:
             if isinstance(hidden, PendingPost):
