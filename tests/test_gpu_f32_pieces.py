@@ -149,3 +149,19 @@ def test_scratch_memory_is_within_what_the_cache_leaves_it():
             assert size <= ops.product_scratch(m, k)
             taken += size == ops.product_scratch(m, k) > 0
     assert taken
+
+
+# through linear (a float32 operand), and bfloat16 by bfloat16 where a caller asks for the float32 kernels
+@pytest.mark.parametrize("x_type,w_type", [(torch.float32, torch.bfloat16), (torch.bfloat16, torch.float32), (torch.bfloat16, torch.bfloat16)])
+@pytest.mark.parametrize("m,n,k", [(1, 70, 1027), (9, 9000, 4096), (40, 300, 96), (300, 3000, 1040), (465, 4096, 4096)])
+def test_products_of_other_types(m, n, k, x_type, w_type):
+    """The error of float32 sums of a step's 32 terms, as float32 operands have it; a row does not depend on its batch."""
+    ops = gpu_ops()
+    x, w = rnd((m, k), 1).to(x_type), rnd((n, k), 2).to(w_type)
+    y = ops._linear_f32(x, w, None, torch.float32, m, n, k)
+    want = x.double() @ w.double().T
+    off = float((y.double() - want).norm() / want.norm())
+    print(f"{x_type} by {w_type}, {m} x {n} x {k}: {off:.3g}")
+    assert off <= 2.0 ** -24 * (4 + (k / 128) ** 0.5)
+    for row in {0, m // 2, m - 1}:
+        assert torch.equal(ops._linear_f32(x[row:row + 1].contiguous(), w, None, torch.float32, 1, n, k)[0], y[row])
