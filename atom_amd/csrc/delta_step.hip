@@ -12,9 +12,11 @@
 // S^T k and S^T q, come from one pass over it, o = S_new^T q = (g S)^T q + u (k . q), so that rows meet (lanes, then
 // waves through LDS) once a token.
 //
-// What bounds it is that chain: two dependent rounds of loads, four barriers.  Heads of 128 x 128, two a q/k head, a layer and
-// step: with decays per channel and both low-rank products, one request of 8 q/k heads, six launches before, 9.6 us less; two
-// requests of 4, 10.1 us less (runs of 16 steps: 6,888 -> 6,735 us with one such layer, 7,944 -> 7,620 with two).
+// What bounds it is that chain: two dependent rounds of loads, four barriers.  Against the launches one by one, heads of 128 x
+// 128, two a q/k head, a layer and step of 1 / 4 / 8 / 16 / 32 / 64 requests, us less: 8 q/k heads with a decay a head (four
+// launches) 4.2 / 8.0 / 14 / 24 / 39 / 66; with decays per channel and both low-rank products (six) 6.1 / 16 / 25 / 31 / 49 / 78;
+// 4 q/k heads so 8.5 / 11 / 15 / 21 / 33 / 52 (runs of 16 steps: 6,888 -> 6,735 us with one such layer, 7,944 -> 7,620 with two).
+// So steps of any number of requests take it.
 #include "common.h"
 
 constexpr int kStepThreads = 1024;

@@ -14,14 +14,14 @@
 // K is walked 32 terms at a time.  The 32 are summed apart, smallest pieces first, and join the sum of their slice; K is cut
 // into 8 slices, whose sums are added four and four in order, then the two.  That order is the same whatever M is and
 // whichever tile and kernel a launch uses, so a row's result does not depend on its batch.  Against float64 (random normal
-// operands, 2-norm of the difference over that of the result): 9.9e-8 at K 4,096
-// and 1.43e-7 at 12,288, where the float32 instructions' sums of 16 terms are 1.38e-7 and 2.00e-7 off.
+// operands, 2-norm of the difference over that of the result): 9.9e-8 at K 4,096 (with one operand in bfloat16 the same, with
+// both 9.6e-8) and 1.43e-7 at 12,288, where the float32 instructions' sums of 16 terms are 1.38e-7 and 2.00e-7 off.
 //
 // A block is 8 waves, one a slice, all on the same output tile of 16 MT rows and 16 NT columns; a wave reads its
 // operands straight from memory into the registers that the matrix instructions take, DEPTH steps ahead of their use
-// (no LDS before the slices meet).  Few rows are bound by the weights' bytes: one row by 24,576 x 4,096 takes 69 us, 5.8 TB/s
-// (72 with the float32 instructions), 8 rows 74 (88), 32 rows 112 (120).  Many rows take the kernel
-// with LDS below where its tiles fill the chip.
+// (no LDS before the slices meet).  Few rows are bound by the weights' bytes: one row by 24,576 x 4,096 takes 70 us, 5.8 TB/s
+// (71 with the float32 instructions), 8 rows 72 (83), 32 rows 107 (117).  Many rows take the kernel with LDS below where its
+// tiles fill the chip and K is a multiple of 32; else 465 rows by 24,576 x 4,112 take 804 us (952), by 4,096 x 4,112 133 (160).
 #include "common.h"
 #include "lds_loads.h"
 

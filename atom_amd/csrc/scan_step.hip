@@ -8,8 +8,9 @@
 //
 // A lane holds four neighbouring columns of every RG-th row of S; all loads that depend on nothing but the request's slot go
 // out together, and rows meet once (lanes, then waves through LDS).  What bounds them is two dependent rounds of loads and
-// three barriers.  Four requests, two layers of state space (64 heads of 128 x 64) and one of time mixing (32 heads of 64 x
-// 64): 26.8 us less a step, four launches fewer (a prompt of 5,569 tokens and 16 steps 9,685 -> 9,257 us).
+// three barriers.  Against the launches one by one, two layers of state space (64 heads of 128 x 64) and one of time mixing (32
+// heads of 64 x 64), four launches fewer in a step of 1 / 4 / 8 / 16 / 32 / 64 requests: 24 / 27 / 31 / 44 / 68 / 98 us less, so
+// steps of any number of requests take them (a prompt of 5,569 tokens and 16 steps of four requests 9,685 -> 9,257 us).
 #include "common.h"
 
 constexpr int kStepTaps = 4;

@@ -59,7 +59,7 @@ typedef __attribute__((ext_vector_type(4))) __bf16 sn_bf16x4;
 
 // SHIFT: every request brings one token, and `out` receives the new rows as shift_rows blends them, out = x + (x' - x) * mu
 // with x' what the request's slot holds, where the new row is left.  (Two rows of 2,048: 3.6 us behind a sum_norm of 4.0 in a
-// launch of its own.)
+// launch of its own; three of them in a step of 1 / 4 / 8 / 64 requests, width 2,048: 4.5 / 5.4 / 7.8 / 7.8 us less.)
 struct ShiftOne {
   const float* mu;
   float* state;
