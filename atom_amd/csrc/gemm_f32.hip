@@ -20,8 +20,10 @@
 // A block is 8 waves, one a slice, all on the same output tile of 16 MT rows and 16 NT columns; a wave reads its
 // operands straight from memory into the registers that the matrix instructions take, DEPTH steps ahead of their use
 // (no LDS before the slices meet).  Few rows are bound by the weights' bytes: one row by 24,576 x 4,096 takes 70 us, 5.8 TB/s
-// (71 with the float32 instructions), 8 rows 72 (83), 32 rows 107 (117).  Many rows take the kernel with LDS below where its
+// (71 with the float32 instructions), 8 rows 72 (83), 32 rows 98 (117).  Many rows take the kernel with LDS below where its
 // tiles fill the chip and K is a multiple of 32; else 465 rows by 24,576 x 4,112 take 804 us (952), by 4,096 x 4,112 133 (160).
+// What splitting costs shows where the bytes come from caches or are few: one row by 1,024 x 1,024 5.3 us (4.9), x 1,040 5.7
+// (4.9), by 4,096 x 4,096 read again and again 13.6 (12.8), 300 rows by 4,096 x 96 14.9 (12.2), by 4,096 x 8 1.2 times as long.
 #include "common.h"
 #include "lds_loads.h"
 
@@ -753,7 +755,9 @@ static int choose_gemm_f32(const GemmF32Params& p, hipStream_t stream) {
     return launch_gemm_f32<TX, TW, 1, 1, 4>(p, stream);
   }
   if (p.m <= 32) {
-    if (wide_fills) return launch_gemm_f32<TX, TW, 2, 2, 2>(p, stream);
+    // One step ahead, in 116 registers: two blocks a CU, where two steps ahead, in 148, leave room for one.  20 rows by 9,728 x
+    // 96 4.4 and 5.9 us (4.5 with the float32 instructions), x 1,024 16.7 and 19.2 (17.3), by 24,576 x 4,096 86 and 92.
+    if (wide_fills) return launch_gemm_f32<TX, TW, 2, 2, 1>(p, stream);
     return launch_gemm_f32<TX, TW, 2, 1, 3>(p, stream);
   }
   const int columns = f32_columns(p.m, p.n, false);
