@@ -137,7 +137,7 @@ def test_results_that_are_not_finite_cost_little():
         x, w = rnd((m, 4096), 1), rnd((8192, 4096), 2)
         plain = passes(x, w)
         x[:, 7] = float("nan")
-        assert passes(x, w) <= 10 * plain     # summed one by one: 30 and 130 times
+        assert passes(x, w) <= 15 * plain     # 5 to 6 times; summed one by one 30 and 130 times
 
 
 def test_scratch_memory_is_within_what_the_cache_leaves_it():
