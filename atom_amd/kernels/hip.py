@@ -207,6 +207,7 @@ class HipKernels:
                    "atom_attention_prefill_tile_rows", "atom_attention_decode_fused",
                    "atom_attention_decode_fused_supports", "atom_gemm_rows", "atom_gemm_rows_parts",
                    "atom_gemm_rows_supports", "atom_gemm_tile", "atom_gemm_tile_splits", "atom_gemm_tile_supports",
+                   "atom_gemm_many", "atom_gemm_many_plan", "atom_gemm_many_supports",
                    "atom_layernorm", "atom_embedding_scaled", "atom_sum_concat", "atom_gated_act", "atom_latent_prepare", "atom_rotation_table",
                    "atom_heads_gemm", "atom_latent_attention", "atom_conv_silu_state", "atom_delta_rule",
                    "atom_delta_out", "atom_router_choose", "atom_experts_gate_up", "atom_experts_down",
@@ -229,6 +230,7 @@ class HipKernels:
             getattr(self.lib, fn).restype = ctypes.c_int
         self.lib.atom_delta_chunks_floats.restype = ctypes.c_long
         self.lib.atom_gemm_f32_scratch.restype = ctypes.c_long
+        self.lib.atom_gemm_many_scratch.restype = ctypes.c_long
         self.allow_library_gemm = True
         # bfloat16 products of few rows run this library's own weight-streaming kernels: up to 64 rows, and
         # up to 128 for the narrow products that atom_gemm_skinny_supports names; the BLAS library takes the rest.
@@ -242,6 +244,10 @@ class HipKernels:
         self.use_tile_gemm = True
         self.tile_rows = (65, 256)
         self.tile_max_width = 8192
+        # bfloat16 products of more rows: the kernel of large tiles; the BLAS library takes what that one does not
+        self.use_many_gemm = True
+        self.many_rows = 257
+        self._many_plans: dict[tuple, tuple] = {}
         self.narrow_row_tiles = True   # tiles of 12 or 8 columns in the few-rows product where they spread better
         self.rows_waves = 0     # 4 or 8 forces the waves a block of that kernel (0: its own choice)
         self.use_mfma_attention = True
@@ -853,6 +859,52 @@ class HipKernels:
                     and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
                     and self.lib.atom_gemm_tile_supports(m, n, k))
 
+    # scratch memory that a product's cut tiles take at most (the kernel's own constant)
+    MANY_SCRATCH = 128 << 20
+
+    def _many(self, x, weight, gate: bool = False) -> bool:
+        """Whether the kernel of large tiles takes ``x @ weight.T`` (``gate``: weight = gate rows, then up rows)."""
+        m, k = x.shape
+        n = weight.shape[0] // 2 if gate else weight.shape[0]
+        return bool(self.use_many_gemm and m >= self.many_rows and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
+                    and (x.data_ptr() | weight.data_ptr()) % 16 == 0
+                    and self.lib.atom_gemm_many_supports(m, n, k, int(gate)))
+
+    @staticmethod
+    def _many_pays(n: int, k: int, bias) -> bool:
+        """Whether the kernel of large tiles is the faster one for a product that ends in nothing but its bias.  Against the BLAS
+        library, 257 to 5,569 rows: with K from 8,192 on 0.91 to 2.0 times as fast (1.2 in the mean: 32B down at 4,111 rows 1,348
+        -> 796 us, at 536 256 -> 139; 8B down at 536 94 -> 65), 10,240 columns of K 5,120 0.92 to 1.3 (4,111 rows 451 -> 342);
+        shorter K 0.6 to 1.4 (0.95 from 1,500 rows on, 0.63 at 257 rows by 2,048 x 2,048), which the library keeps.  A bias is
+        one pass of the library's float32 sums more and, for bfloat16, another that rounds."""
+        return bias is not None or k >= 8192 or (k >= 5120 and n >= 4096)
+
+    def _many_launch(self, x, weight, bias, out_dtype, gate: bool = False, act: int = 0, slices: bool = False):
+        """``act(x @ weight.T + bias)``, or with ``gate`` ``act(x @ gate.T + ..) * (x @ up.T + ..)``, by the kernel of large
+        tiles.  ``slices``: the product may come back as a ``DeferredSum`` (no activation then)."""
+        m, k = x.shape
+        n = weight.shape[0] // 2 if gate else weight.shape[0]
+        key = (m, n, k, gate, slices)
+        plan = self._many_plans.get(key)
+        if plan is None:
+            found = (ctypes.c_int * 4)()
+            self._done("gemm_many_plan", self.lib.atom_gemm_many_plan(m, n, k, int(gate), int(slices), self.num_cus, found))
+            plan = (*found, self.lib.atom_gemm_many_scratch(m, n, int(gate), found[0], found[1], found[2]))
+            if len(self._many_plans) >= 4096:
+                self._many_plans.clear()
+            self._many_plans[key] = plan
+        tile, whole, cut, apart, scratch = plan
+        if apart:
+            parts = torch.empty((cut, m, n), dtype=torch.float32, device=x.device)
+            y = None
+        else:
+            parts = torch.empty(scratch, dtype=torch.uint8, device=x.device) if scratch else None
+            y = torch.empty((m, n), dtype=out_dtype, device=x.device)
+        self._done("gemm_many", self.lib.atom_gemm_many(
+            _ptr(x), _ptr(weight), None if apart else _ptr(bias), _ptr(y), _ptr(parts), m, n, k, int(gate), act,
+            int(out_dtype == torch.float32), tile, whole, cut, apart, self._stream()))
+        return DeferredSum(parts, bias, out_dtype) if apart else y
+
     def _skinny(self, x, weight) -> bool:
         m, k = x.shape
         return bool(self.use_skinny_gemm and m <= self.skinny_max_rows and x.dtype == torch.bfloat16
@@ -910,6 +962,8 @@ class HipKernels:
                 _ptr(x), _ptr(weight), None, None, _ptr(partial), m, n, k, 0, 0, self._stream()))
             result = DeferredSum(partial, bias, out_dtype)
             return result if defer else self.materialize(result)
+        if m and self._many_pays(n, k, bias) and self._many(x, weight):
+            return self._many_launch(x, weight, bias, out_dtype, slices=defer and slices and n <= k)
         if x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and self.allow_library_gemm:
             pieces = self._library_slices(m, n, k) if defer and slices else 1
             if pieces > 1:
@@ -958,6 +1012,7 @@ class HipKernels:
         return torch.empty(size, dtype=torch.uint8, device=x.device) if size else None
 
     _ROWS_GATE_ACT = {"silu": 0, "relu": 2, "gelu_tanh": 3}
+    _MANY_GATE_ACT = {"silu": 1, "relu": 2, "gelu_tanh": 3}
     _ROWS_ACT = {"silu": 1, "relu": 2, "gelu_tanh": 3, "relu_squared": 4, "tanh": 5}
 
     def linear_act(self, x, weight, bias, activation: str, out_dtype=None):
@@ -972,6 +1027,13 @@ class HipKernels:
             y = torch.empty((m, weight.shape[0]), dtype=out_dtype or x.dtype, device=weight.device)
             self._rows_launch(x, weight, bias, 0, y=y, act=self._ROWS_ACT[activation], out_f32=y.dtype == torch.float32)
             return y
+        x = self.materialize(x)
+        if m and activation in ("relu", "relu_squared") and self._many_alone(x, weight):
+            self._check("linear input", x, torch.bfloat16)
+            self._check("linear weight", weight, torch.bfloat16, (weight.shape[0], x.shape[1]))
+            if bias is not None:
+                self._check("linear bias", bias, torch.float32, (weight.shape[0],))
+            return self._many_launch(x, weight, bias, out_dtype or x.dtype, act=self._ROWS_ACT[activation])
         up = self.linear(x, weight, bias, out_dtype=out_dtype)
         out = torch.empty(tuple(up.shape), dtype=up.dtype, device=up.device)
         return self.unary_act(up, out, activation)
@@ -1034,9 +1096,40 @@ class HipKernels:
                 _ptr(x), F32, _ptr(weight), self._code(weight), _ptr(bias), _ptr(act), m, inter, k,
                 _ptr(scratch), self._stream()))
             return act
+        if m and self._many_alone(x, weight, gate=True):
+            return self._many_gated(x, weight, bias, "silu")
         gate_up = self.linear(x, weight, bias)
         act = torch.empty((m, inter), dtype=x.dtype, device=x.device)
         return self.silu_mul(gate_up, act)
+
+    def linear_gated(self, x, weight, bias, activation: str):
+        """``act(x @ Wg.T + bg) * (x @ Wu.T + bu)`` for ``weight`` = gate rows then up rows: the epilogue of the product for
+        a handful of rows and for many, else the product and the gate entry by entry."""
+        if activation not in self._ACTIVATIONS:
+            raise KernelError(f"linear_gated: unknown activation {activation!r}; known: {sorted(self._ACTIVATIONS)}")
+        if weight.shape[0] % 2:
+            raise KernelError("linear_gated: the weight must hold as many gate rows as up rows")
+        if isinstance(x, (DeferredSum, PendingProduct)):
+            x = self.materialize(x)
+        if x.shape[0] and not self._rows_takes(x, weight):
+            x = self.materialize(x)
+            if self._many_alone(x, weight, gate=True):
+                return self._many_gated(x, weight, bias, activation)
+        # a product of few rows waits for the gate, which becomes its epilogue
+        both = self.linear(x, weight, bias, defer=True, slices=False)
+        act = torch.empty((both.shape[0], weight.shape[0] // 2), dtype=both.dtype, device=both.device)
+        return self.gated_act(both, act, activation)
+
+    def _many_alone(self, x, weight, gate: bool = False) -> bool:
+        """Whether the kernel of large tiles takes this product and no kernel of fewer rows does."""
+        return not self._tile(x, weight) and not self._skinny(x, weight) and self._many(x, weight, gate)
+
+    def _many_gated(self, x, weight, bias, activation: str):
+        self._check("linear input", x, torch.bfloat16)
+        self._check("linear weight", weight, torch.bfloat16, (weight.shape[0], x.shape[1]))
+        if bias is not None:
+            self._check("linear bias", bias, torch.float32, (weight.shape[0],))
+        return self._many_launch(x, weight, bias, x.dtype, gate=True, act=self._MANY_GATE_ACT[activation])
 
     # ------------------------------------------------------------------ layer norm and the float32 stream
 

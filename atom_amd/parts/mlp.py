@@ -1,7 +1,6 @@
 """Gated dense feed-forward: ``down(act(gate(x)) * up(x))`` with gate and up in one packed
 product, gate rows first (atom/models/qwen3.py:166-198,321-322; atom/model_ops/activation.py:78-82).
-SiLU runs the fused gate products; ReLU and tanh-GELU are the epilogue of a product of few rows and an elementwise
-kernel behind one of many."""
+The gate is the epilogue of the product where its kernel offers one, else an elementwise kernel behind it."""
 
 from __future__ import annotations
 
@@ -41,11 +40,13 @@ class GatedMLP(FeedForward):
 
     def forward(self, ctx, x):
         ops = ctx.ops
+        weight, bias = self.params["gate_up.weight"], self.p("gate_up.bias")
         if self.activation == "silu":
-            act = ops.linear_silu(x, self.params["gate_up.weight"], self.p("gate_up.bias"))
+            act = ops.linear_silu(x, weight, bias)
+        elif hasattr(ops, "linear_gated"):
+            act = ops.linear_gated(x, weight, bias, self.activation)
         else:
-            # a product of few rows waits for the gate, which becomes its epilogue; for many the gate is an elementwise kernel
-            both = ops.linear(x, self.params["gate_up.weight"], self.p("gate_up.bias"), defer=True, slices=False)
+            both = ops.linear(x, weight, bias, defer=True, slices=False)
             act = torch.empty((both.shape[0], self.intermediate_size), dtype=both.dtype, device=both.device)
             ops.gated_act(both, act, self.activation)
         # the down product may come back as slices that the next norm adds while it reads them
