@@ -280,6 +280,18 @@ class CacheManager:
             out.append(max(0, last + 1 - max(len(table), self._first_page_needed(gi, cached))))
         return out
 
+    def holds(self, req_id, upto: int, reserve: int | None = None) -> bool:
+        """Whether the request is open and has a page for every position before ``upto`` (and ``reserve``) in groups that keep
+        theirs: then ``cover`` has nothing to do.  (False where a group gives pages back, whose check is ``cover``'s.)"""
+        req = self._requests.get(req_id)
+        if req is None:
+            return False
+        end = upto if reserve is None or reserve < upto else reserve
+        for g, table in zip(self.groups, req.tables):
+            if not g.keeps_all or len(table) * g.page_size < end:
+                return False
+        return True
+
     def can_cover(self, req_id, cached: int, upto: int, reserve: int | None = None) -> bool:
         return all(need <= pool.num_free
                    for need, pool in zip(self.pages_missing(req_id, cached, upto, reserve), self.pools))

@@ -132,6 +132,7 @@ class EngineCore:
         if len(set(ids)) != len(ids):
             raise ValueError("a request appears twice in one step")
         vocab = self.model.vocab_size
+        lacking, cached_now = [], []
         for e in entries:
             if not e.tokens:
                 raise ValueError(f"request {e.req_id!r}: a step entry needs at least one token")
@@ -140,28 +141,34 @@ class EngineCore:
             if e.feed is not None and (len(e.tokens) != 1 or not 0 <= e.feed < self.sampled.numel()):
                 raise ValueError(f"request {e.req_id!r}: a token read on the device must be the entry's only one "
                                  f"and name one of the {self.sampled.numel()} sampled rows")
-            if any(w < 0 or w >= len(e.tokens) for w in e.want):
+            if e.want and (min(e.want) < 0 or max(e.want) >= len(e.tokens)):
                 raise ValueError(f"request {e.req_id!r}: a wanted place is outside its {len(e.tokens)} tokens")
-            end = self.num_cached(e.req_id) + len(e.tokens)
+            cached = self.num_cached(e.req_id)
+            end = cached + len(e.tokens)
             if self.max_positions and end > self.max_positions:
                 raise ValueError(f"request {e.req_id!r}: {end} tokens exceed the model's {self.max_positions} positions")
-        if not self.can_step(entries):
+            cached_now.append(cached)
+            if not self.manager.holds(e.req_id, end, e.reserve):
+                lacking.append(e)
+        # (a request that holds all its step needs takes nothing from the pools)
+        if lacking and not self.can_step(lacking):
             from ..cache.manager import OutOfPages
             raise OutOfPages("the cache cannot hold this step's tokens")
 
-        # prompt portions first, single tokens after them (stable)
-        order = sorted(range(len(entries)), key=lambda i: len(entries[i].tokens) == 1)
-        for e in entries:
+        for e in lacking:
             self.open(e.req_id)
             cached = self.lengths[e.req_id]
             self.manager.cover(e.req_id, cached, cached + len(e.tokens), e.reserve)
-        self.storage.reset_state(self._fresh_slots)
-        self._fresh_slots = []
+        if self._fresh_slots:
+            self.storage.reset_state(self._fresh_slots)
+            self._fresh_slots = []
 
-        cached_now = [self.lengths[e.req_id] for e in entries]
-        if self.graphs is not None and self.graphs.accepts(entries, cached_now):
-            logits = self.graphs.run(entries, cached_now)
+        shape = None if self.graphs is None else self.graphs.place(entries, cached_now)
+        if shape is not None:
+            logits = self.graphs.run(entries, cached_now, shape)
         else:
+            # prompt portions first, single tokens after them (stable)
+            order = sorted(range(len(entries)), key=lambda i: len(entries[i].tokens) == 1)
             ctx, token_ids, want_rows = self._build(entries, order)
             logits = self.model.forward(ctx, token_ids, self.storage.bindings, want_rows,
                                         self.storage.embedding_binding)

@@ -37,6 +37,8 @@ import torch
 from .context import StepContext
 
 
+_COUNT = np.arange(4096, dtype=np.int32)
+
 PREFILL_SLOTS = 2    # prompt portions a replayed step holds at most, unless the engine's configuration says otherwise
 
 
@@ -58,6 +60,11 @@ class _Captured:
         # what the pinned buffer holds per request row and group: (the request's serial, pages written), so
         # that a request that keeps its row only has its new pages written
         self.row_state: list[list[tuple | None]] = []
+        # the buffer's arrays by name, its part that every step writes anew with what padding reads there, its block tables
+        self.views: dict = {}
+        self.head: np.ndarray | None = None
+        self.blank: np.ndarray | None = None
+        self.tables: list[np.ndarray] = []
 
 
 class DecodeGraphs:
@@ -104,11 +111,13 @@ class DecodeGraphs:
         return (next(p for p in self.prefill_sizes if p >= total), self.prefill_slots, n)
 
     def accepts(self, entries, cached: list[int]) -> bool:
-        if not self.usable or not entries:
-            return False
-        if self.shape_for(entries) is None:
-            return False
-        return max(c + len(e.tokens) for c, e in zip(cached, entries)) <= self.max_model_len
+        return self.place(entries, cached) is not None
+
+    def place(self, entries, cached: list[int]) -> tuple[int, int, int] | None:
+        """The bucket whose graph runs these entries, or None if the step is to be launched."""
+        if not self.usable or not entries or max(c + len(e.tokens) for c, e in zip(cached, entries)) > self.max_model_len:
+            return None
+        return self.shape_for(entries)
 
     # ------------------------------------------------------------------ layout
 
@@ -121,17 +130,25 @@ class DecodeGraphs:
         t, s = cap.num_tokens, cap.num_seqs
         pieces = [("tokens", t), ("feed", t), ("positions", t), ("token_seq", t), ("starts", s + 1),
                   ("context_lens", s), ("cached_lens", s), ("slot_of_seq", s), ("want", cap.num_logits)]
-        for gi, width in enumerate(self.widths):
-            pieces += [(f"bt{gi}", s * width), (f"slots{gi}", t)]
+        pieces += [(f"slots{gi}", t) for gi in range(len(self.widths))]
+        blanked = len(pieces)            # what every step writes anew; rows of block tables keep what they had
+        pieces += [(f"bt{gi}", s * width) for gi, width in enumerate(self.widths)]
         # what the mixers ask for: in a replayed step the shapes depend on the bucket only
         view = self._view_of(cap, self._padded_q_lens(cap, []), [0] * s)
         for key, mixer in self.core.preparers.items():
             for name, array in mixer.prepare_step(view).items():
                 pieces.append((("prepared", key, name, tuple(np.shape(array))), int(np.size(array))))
         cursor = 0
-        for name, n in pieces:
+        for i, (name, n) in enumerate(pieces):
             cap.offsets[name] = (cursor, n)
             cursor += (n + 3) // 4 * 4
+            if i + 1 == blanked:
+                cap.blank = np.zeros(cursor, dtype=np.int32)
+        for name in ["feed", "token_seq", "slot_of_seq"] + [f"slots{gi}" for gi in range(len(self.widths))]:
+            off, n = cap.offsets[name]
+            cap.blank[off:off + n] = -1
+        off, n = cap.offsets["starts"]
+        np.cumsum(self._padded_q_lens(cap, []), out=cap.blank[off + 1:off + n])
         return cursor
 
     @staticmethod
@@ -150,82 +167,89 @@ class DecodeGraphs:
         if cap.copy_pending:
             cap.copied.synchronize()   # the last copy out of this buffer has finished
             cap.copy_pending = False
-        host = cap.host.numpy()
         p, r, n = cap.shape
         mgr = self.core.manager
-
-        def view(name):
-            off, count = cap.offsets[name]
-            return host[off:off + count]
-
-        tokens, positions, token_seq, feed = view("tokens"), view("positions"), view("token_seq"), view("feed")
-        tokens[:] = 0
-        feed[:] = -1
-        positions[:] = 0
-        token_seq[:] = -1
-        ctx_lens, cached_lens, slot_of_seq = view("context_lens"), view("cached_lens"), view("slot_of_seq")
-        ctx_lens[:] = 0
-        cached_lens[:] = 0
-        slot_of_seq[:] = -1
-        starts, want = view("starts"), view("want")
-        want[:] = 0
-        if not cap.row_state:
+        if not cap.views:
+            host = cap.host.numpy()
+            cap.views = {name: host[off:off + count] for name, (off, count) in cap.offsets.items()}
+            cap.head = host[:cap.blank.size]
+            cap.tables = [cap.views[f"bt{gi}"].reshape(cap.num_seqs, width) for gi, width in enumerate(self.widths)]
             cap.row_state = [[None] * cap.num_seqs for _ in self.widths]
-        slot_arrays = [view(f"slots{gi}") for gi in range(len(self.widths))]
-        for slots in slot_arrays:
-            slots[:] = -1
-        tables = [view(f"bt{gi}").reshape(cap.num_seqs, width) for gi, width in enumerate(self.widths)]
+        view = cap.views
+        cap.head[:] = cap.blank
+        sizes = [g.page_size for g in mgr.groups]
 
-        # which request row and token rows every entry gets
-        logits_row, placed = [], []          # placed: (entry, its cached tokens, request row, first token row)
-        at, portions, singles = 0, 0, 0
-        for e, c in zip(entries, cached):
-            if len(e.tokens) > 1:
-                placed.append((e, c, portions, at))
-                logits_row.append(portions)
-                at += len(e.tokens)
-                portions += 1
-            else:
-                placed.append((e, c, cap.first_single + singles, p + singles))
-                logits_row.append(r + singles)
-                singles += 1
-        q_lens = self._padded_q_lens(cap, [len(e.tokens) for e in entries if len(e.tokens) > 1])
-        starts[0] = 0
-        np.cumsum(q_lens, out=starts[1:])
+        # which request row and token rows every entry gets; the single tokens' values are gathered and written together
+        logits_row, portion_lens = [], []
         full_cached = [0] * cap.num_seqs
-        for i, (e, c, row, first) in enumerate(placed):
+        single_tokens, single_cached, single_slots, feeds = [], [], [], []
+        single_places = [[] for _ in sizes]
+        at = 0
+        for e, c in zip(entries, cached):
             k = len(e.tokens)
-            tokens[first:first + k] = e.tokens
-            if e.feed is not None:
-                feed[first] = e.feed
-            positions[first:first + k] = np.arange(c, c + k, dtype=np.int32)
-            token_seq[first:first + k] = row
-            ctx_lens[row] = c + k
-            cached_lens[row] = c
+            if k > 1:
+                row, first = len(portion_lens), at
+                logits_row.append(row)
+                portion_lens.append(k)
+                at += k
+                view["tokens"][first:first + k] = e.tokens
+                view["positions"][first:first + k] = np.arange(c, c + k, dtype=np.int32)
+                view["token_seq"][first:first + k] = row
+                view["context_lens"][row] = c + k
+                view["cached_lens"][row] = c
+                view["slot_of_seq"][row] = mgr.state_slot(e.req_id)
+                view["want"][row] = first + k - 1
+            else:
+                row = cap.first_single + len(single_tokens)
+                logits_row.append(r + len(single_tokens))
+                single_tokens.append(e.tokens[0])
+                single_cached.append(c)
+                single_slots.append(mgr.state_slot(e.req_id))
+                feeds.append(-1 if e.feed is None else e.feed)
             full_cached[row] = c
-            slot_of_seq[row] = mgr.state_slot(e.req_id)
-            want[logits_row[i]] = first + k - 1
-            for gi, width in enumerate(self.widths):
+            serial = mgr.serial(e.req_id)
+            for gi, page_size in enumerate(sizes):
                 table = mgr.block_table(e.req_id, gi)
-                page_size = mgr.groups[gi].page_size
-                slot_arrays[gi][first:first + k] = mgr.slot_mapping(e.req_id, gi, c, k)
-                bt, state = tables[gi], cap.row_state[gi]
-                held, serial = state[row], mgr.serial(e.req_id)
-                if table[(c + k - 1) // page_size] < 0:
+                last = table[(c + k - 1) // page_size]
+                if last < 0:
                     raise AssertionError(f"request {e.req_id!r}: position {c + k - 1} has no page")
-                if held is not None and held[0] == serial and held[1] <= len(table):
+                if k > 1:
+                    view[f"slots{gi}"][first:first + k] = mgr.slot_mapping(e.req_id, gi, c, k)
+                else:
+                    single_places[gi].append(last * page_size + c % page_size)
+                state, length = cap.row_state[gi], len(table)
+                held = state[row]
+                if held is not None and held[0] == serial and held[1] <= length:
                     # pages appended since the row was last written; places whose pages a window has passed meanwhile
                     # keep their old numbers, which no query's keys name any more
-                    if held[1] < len(table):
-                        bt[row, held[1]:len(table)] = [max(page, 0) for page in table[held[1]:]]
+                    if held[1] == length:
+                        continue
+                    cap.tables[gi][row, held[1]:length] = [max(page, 0) for page in table[held[1]:]]
                 else:
-                    line = np.asarray(table, dtype=np.int32)
-                    bt[row, :len(table)] = np.where(line < 0, 0, line)
-                    bt[row, len(table):] = 0
-                state[row] = (serial, len(table))
+                    bt, line = cap.tables[gi], np.asarray(table, dtype=np.int32)
+                    bt[row, :length] = np.where(line < 0, 0, line)
+                    bt[row, length:] = 0
+                state[row] = (serial, length)
+        count = len(single_tokens)
+        if count:
+            tokens, positions, slots = np.array((single_tokens, single_cached, single_slots), dtype=np.int32)
+            seqs, rows = slice(cap.first_single, cap.first_single + count), slice(p, p + count)
+            view["tokens"][rows], view["positions"][rows] = tokens, positions
+            view["token_seq"][rows] = _COUNT[seqs] if seqs.stop <= _COUNT.size else np.arange(seqs.start, seqs.stop)
+            view["context_lens"][seqs] = positions + 1
+            view["cached_lens"][seqs], view["slot_of_seq"][seqs] = positions, slots
+            view["want"][r:r + count] = _COUNT[rows] if rows.stop <= _COUNT.size else np.arange(rows.start, rows.stop)
+            for gi, places in enumerate(single_places):
+                view[f"slots{gi}"][rows] = places
+            if max(feeds) >= 0:
+                view["feed"][rows] = feeds
+        q_lens = None
+        if portion_lens:
+            q_lens = self._padded_q_lens(cap, portion_lens)
+            np.cumsum(q_lens, out=view["starts"][1:])
             # request rows without an entry keep what they had: their context length is 0, nothing reads them
         if self.core.preparers:
-            batch = self._view_of(cap, q_lens, full_cached)
+            batch = self._view_of(cap, q_lens or self._padded_q_lens(cap, []), full_cached)
             for key, mixer in self.core.preparers.items():
                 for name, array in mixer.prepare_step(batch).items():
                     array = np.ascontiguousarray(array, dtype=np.int32)
@@ -233,7 +257,7 @@ class DecodeGraphs:
                     if piece not in cap.offsets:
                         raise AssertionError(f"{type(mixer).__name__}.prepare_step: '{name}' has shape {array.shape} "
                                              f"in this step, not the shape the graph {cap.shape} was captured with")
-                    view(piece)[:] = array.reshape(-1)
+                    view[piece][:] = array.reshape(-1)
         return logits_row
 
     def _context(self, cap: _Captured):
@@ -314,11 +338,12 @@ class DecodeGraphs:
             self._capture(shape, collect=i == 0)   # one collection (some 20 ms) before all of them
         return len(self.captured)
 
-    def run(self, entries, cached: list[int]) -> torch.Tensor | None:
+    def run(self, entries, cached: list[int], shape: tuple[int, int, int] | None = None) -> torch.Tensor | None:
         """Float32 logits at the entries' wanted places (a portion's last row, a single token), in the
         order of the entries; None if nothing is wanted.  Where the first entries of a step of single tokens want theirs, and
-        they alone, the tensor is the graph's own output, valid until the graph's next replay; elsewhere it is a copy."""
-        shape = self.shape_for(entries)
+        they alone, the tensor is the graph's own output, valid until the graph's next replay; elsewhere it is a copy.
+        ``shape``: what ``place`` said."""
+        shape = shape or self.shape_for(entries)
         cap = self.captured.get(shape) or self._capture(shape)
         logits_row = self._fill(cap, entries, cached)
         cap.dev.copy_(cap.host, non_blocking=True)
