@@ -47,7 +47,7 @@ struct GemmF32Params {
   int m, n, k;
   int row_tiles, tiles;
   int y_bf16;
-  const bf16_t* pieces;   // the wide kernel: x as three planes [m, k] of pieces
+  const bf16_t* pieces;   // the wide kernel: x's pieces [m, k / 32, 3, 32]
   int inter;   // SiLU-gate: w holds `inter` gate rows, then as many up rows (n = 2 inter); 0: a plain product
 };
 
@@ -423,7 +423,7 @@ __global__ void __launch_bounds__(256) split_f32_kernel(const float* __restrict_
   bf16x8 p[3];
   v.pieces(p, flip_of(at / 4 % steps));
 #pragma unroll
-  for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(pieces + (i * eights + at) * kLane) = p[i];
+  for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(pieces + (at / 4 * 12 + 4 * i + at % 4) * kLane) = p[i];
 }
 
 // The place of row 16 i + 4 quarter + t, column 16 j + side among a wave's 64 x 32 sums in LDS.
@@ -470,8 +470,8 @@ __global__ void __launch_bounds__(kSlices* kWave) gemm_f32_wide_kernel(GemmF32Pa
   const int count = group ? steps - low : low;      // this group's steps
   const int k0 = group ? low * kStep : 0;
 
-  // Loads of a stage: 16 rows of a plane of x each (piece `lane % 4` of a row in LDS is the row's piece of that number turned
-  // by the row), then 8 rows of w each (piece `lane % 8`).
+  // Loads of a stage: x, whose rows have twelve 16-byte pieces a step side by side (their place in LDS turned, in fours, by the
+  // row), then 8 rows of w each (piece `lane % 8`).
   constexpr int X_LOADS = 3 * ROWS / 16, LOADS = (X_LOADS + kWideCols / 8) * GROUPS / kSlices;
   const int loader = GROUPS == 2 ? w4 : wave;
   const char* from[LOADS];
@@ -480,10 +480,9 @@ __global__ void __launch_bounds__(kSlices* kWave) gemm_f32_wide_kernel(GemmF32Pa
   for (int j = 0; j < LOADS; ++j) {
     const int load = LOADS * loader + j;
     if (load < X_LOADS) {
-      const int r = load % (ROWS / 16) * 16 + lane / 4;
-      from[j] = (const char*)(p.pieces + ((size_t)(load / (ROWS / 16)) * p.m + min(row0 + r, p.m - 1)) * p.k + k0 +
-                              (lane % 4 ^ (r >> 2 & 3)) * 8);
-      size[j] = 2;
+      const int at = load * kWave + lane, r = at / 12, piece = at % 12;
+      from[j] = (const char*)p.pieces + ((size_t)min(row0 + r, p.m - 1) * p.k + k0) * 6 + (piece ^ (r >> 1 & 3)) * 16;
+      size[j] = 6;
     } else {
       const int r = (load - X_LOADS) * 8 + lane / 8;
       from[j] = (const char*)((const float*)p.w + (size_t)row_of_w(p, col0 + r) * p.k + k0 + (lane % 8 ^ (r >> 1 & 7)) * 4);
@@ -523,7 +522,7 @@ __global__ void __launch_bounds__(kSlices* kWave) gemm_f32_wide_kernel(GemmF32Pa
       const int r = r0 + 16 * i + side;
 #pragma unroll
       for (int t = 0; t < 3; ++t)
-        o.a[i][t] = *reinterpret_cast<const bf16x8*>(xs + t * kPlaneBytes + r * kStep * 2 + (quarter ^ (r >> 2 & 3)) * 16);
+        o.a[i][t] = *reinterpret_cast<const bf16x8*>(xs + r * kStep * 6 + (4 * t + (quarter ^ (r >> 1 & 3))) * 16);
     }
   };
   int until = share, slice = 0;                     // steps until the slice ends
