@@ -1,7 +1,7 @@
 // Paged attention, general form: any head size, any page size, float32 or bfloat16,
 // every query token of a mixed batch (prompt portions and single decoded tokens alike).
 //
-// One block per (query token, query head).  The token's request and absolute position
+// One block per (query token, query head), or, for many tokens, per token and two or four heads that share keys.  The token's request and absolute position
 // are given per token; the keys it sees are positions max(0, p - window + 1) .. p of that
 // request, found through the request's block table; with `chunk` only those from the start of the run of `chunk`
 // positions (counted from position 0) that p lies in.  With `softcap` a score s becomes softcap * tanh(s / softcap); with
@@ -19,22 +19,46 @@ constexpr int kAttnFew = 1024;    // blocks up to which the chip holds them all 
 constexpr int kAttnChunk = 512;  // keys per pass
 constexpr int kAttnStretch = 16; // keys a thread adds in one go
 
-// The sum of a block's kAttnItems values, for all its threads: over each 64 of them, then group by group; the same order
-// whether a block's waves hold one group each or several.
-template <int PER>
-__device__ __forceinline__ float groups_sum(const float (&v)[PER], float* scratch) {
-  const int wave = threadIdx.x / kWave, waves = kAttnItems / kWave / PER;
+// Over a block, for all its threads and each of HEADS heads: the maximum of a value a thread, or the sum of kAttnItems values, PER
+// a thread: over each 64 of them, then group by group; the same order whether a block's waves hold one group each or several.
+template <int HEADS, int PER>
+__device__ __forceinline__ void block_maxima(float (&v)[HEADS], float* scratch) {
+  const int wave = threadIdx.x / kWave;
+  constexpr int WAVES = kAttnItems / kWave / PER;
   __syncthreads();   // what was there before has been read
 #pragma unroll
-  for (int r = 0; r < PER; ++r) {
-    const float s = wave_sum(v[r]);
-    if (threadIdx.x % kWave == 0) scratch[r * waves + wave] = s;
+  for (int h = 0; h < HEADS; ++h) {
+    const float m = wave_max(v[h]);
+    if (threadIdx.x % kWave == 0) scratch[h * WAVES + wave] = m;
   }
   __syncthreads();
-  float sum = 0.f;
 #pragma unroll
-  for (int g = 0; g < kAttnItems / kWave; ++g) sum += scratch[g];
-  return sum;
+  for (int h = 0; h < HEADS; ++h) {
+    v[h] = scratch[h * WAVES];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) v[h] = fmaxf(v[h], scratch[h * WAVES + w]);
+  }
+}
+
+template <int HEADS, int PER>
+__device__ __forceinline__ void groups_sums(const float (&v)[HEADS][PER], float (&sums)[HEADS], float* scratch) {
+  constexpr int WAVES = kAttnItems / kWave / PER, GROUPS = kAttnItems / kWave;
+  const int wave = threadIdx.x / kWave;
+  __syncthreads();   // what was there before has been read
+#pragma unroll
+  for (int h = 0; h < HEADS; ++h)
+#pragma unroll
+    for (int r = 0; r < PER; ++r) {
+      const float s = wave_sum(v[h][r]);
+      if (threadIdx.x % kWave == 0) scratch[h * GROUPS + r * WAVES + wave] = s;
+    }
+  __syncthreads();
+#pragma unroll
+  for (int h = 0; h < HEADS; ++h) {
+    sums[h] = 0.f;
+#pragma unroll
+    for (int g = 0; g < GROUPS; ++g) sums[h] += scratch[h * GROUPS + g];
+  }
 }
 
 // A block's items are (output entry, every `runs`-th stretch of kAttnStretch keys counted from position 0): as many runs side
@@ -42,7 +66,9 @@ __device__ __forceinline__ float groups_sum(const float (&v)[PER], float* scratc
 // thread an item (PER 1); where there are blocks enough to fill the chip, 128 threads with four items each (PER 4) leave fewer
 // of them idle at a short row's end.  Float32, 32 heads of 128: one or two tokens behind some 300 keys 26 us with one run, 15.7
 // with PER 1; a prompt of 461 tokens 250 us with PER 1, 198 with PER 4.  The items and the order of every sum are the same in both.
-template <typename T, int PER>
+// What then bounds a prompt is what its blocks read of the keys and values, 32 times over for 32 heads: HEADS query heads of a
+// block, which have one head of keys, use what is read for all of them (that prompt, four heads a head of keys: 214 -> 85 us).
+template <typename T, int PER, int HEADS>
 __global__ void __launch_bounds__(kAttnItems / PER)
 paged_attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ k_cache,
                                const T* __restrict__ v_cache, T* __restrict__ out,
@@ -52,40 +78,44 @@ paged_attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ k_
                                const float* __restrict__ sink, const float* __restrict__ slopes,
                                const float* __restrict__ gate, long gate_ld, int od, int key_fours, int value_fours) {
   extern __shared__ __align__(16) float smem[];
-  float* qs = smem;                  // d
-  float* probs = qs + (d + 3) / 4 * 4;   // kAttnChunk
-  float* scratch = probs + kAttnChunk;  // 16
-  float* shares = scratch + 16;         // kAttnItems
+  const int dq = (d + 3) / 4 * 4;
+  float* qs = smem;                                // HEADS x dq
+  float* probs = qs + HEADS * dq;                  // HEADS x kAttnChunk
+  float* scratch = probs + HEADS * kAttnChunk;     // HEADS x 16
+  float* shares = scratch + HEADS * 16;            // HEADS x kAttnItems
   constexpr int kAttnThreads = kAttnItems / PER;
   const int t = blockIdx.x;
-  const int h = blockIdx.y;
-  const int kvh = h / (hq / hkv);
+  const int h0 = blockIdx.y * HEADS;
+  const int kvh = h0 / (hq / hkv);
   const int tid = threadIdx.x;
   const int seq = token_seq[t];
   const int pos = positions[t];
-  T* dst = out + ((size_t)t * hq + h) * od;
+  T* dst = out + ((size_t)t * hq + h0) * od;
   if (seq < 0) {  // padding row
-    for (int i = tid; i < od; i += kAttnThreads) dst[i] = from_f32<T>(0.f);
+    for (int i = tid; i < HEADS * od; i += kAttnThreads) dst[i] = from_f32<T>(0.f);
     return;
   }
   const int* table = block_tables + (size_t)seq * max_blocks;
-  const T* qr = q + ((size_t)t * hq + h) * d;
-  for (int i = tid; i < d; i += kAttnThreads) qs[i] = to_f32(qr[i]) * scale;
+  const T* qr = q + ((size_t)t * hq + h0) * d;
+  for (int i = tid; i < d; i += kAttnThreads)
+#pragma unroll
+    for (int h = 0; h < HEADS; ++h) qs[h * dq + i] = to_f32(qr[h * d + i]) * scale;
   __syncthreads();
 
   int first = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
   if (chunk > 0 && pos / chunk * chunk > first) first = pos / chunk * chunk;
   const int last = pos;  // inclusive
   const int wide = min(kAttnItems, (d + kWave - 1) / kWave * kWave), runs = kAttnItems / wide;
-  float acc[PER];
+  float acc[HEADS][PER], run_max[HEADS], run_sum[HEADS], slope[HEADS];
 #pragma unroll
-  for (int r = 0; r < PER; ++r) acc[r] = 0.f;
-  float run_max = -INFINITY, run_sum = 0.f;
-  if (sink != nullptr) {   // as if a key with that score and a value of zeros had been seen already
-    run_max = sink[h];
-    run_sum = 1.f;
+  for (int h = 0; h < HEADS; ++h) {
+#pragma unroll
+    for (int r = 0; r < PER; ++r) acc[h][r] = 0.f;
+    // a sink: as if a key with that score and a value of zeros had been seen already
+    run_max[h] = sink != nullptr ? sink[h0 + h] : -INFINITY;
+    run_sum[h] = sink != nullptr ? 1.f : 0.f;
+    slope[h] = slopes != nullptr ? slopes[h0 + h] : 0.f;
   }
-  const float slope = slopes != nullptr ? slopes[h] : 0.f;
 
   // chunks are aligned to multiples of kAttnChunk from position 0, so the grouping of
   // keys does not move with the window start
@@ -93,50 +123,70 @@ paged_attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ k_
     const int lo = base > first ? base : first;
     const int hi = (base + kAttnChunk - 1 < last) ? base + kAttnChunk - 1 : last;
     const int n = hi - lo + 1;
-    float local_max = -INFINITY;
+    float new_max[HEADS];
+#pragma unroll
+    for (int h = 0; h < HEADS; ++h) new_max[h] = -INFINITY;
     for (int j = tid; j < n; j += kAttnThreads) {
       const int key = lo + j;
       const int page = table[key / page_size];
       const int off = key % page_size;
       const T* kr = k_cache + (((size_t)page * hkv + kvh) * page_size + off) * (size_t)d;
-      float s = 0.f;
+      float s[HEADS];
+#pragma unroll
+      for (int h = 0; h < HEADS; ++h) s[h] = 0.f;
       if (key_fours) {   // rows of four-element pieces: a piece a load
 #pragma unroll 8
         for (int i = 0; i < d; i += 4) {
           const Four<T> four = *reinterpret_cast<const Four<T>*>(kr + i);
-          const float4 qi = *reinterpret_cast<const float4*>(qs + i);
-          s += qi.x * to_f32(four.at[0]);
-          s += qi.y * to_f32(four.at[1]);
-          s += qi.z * to_f32(four.at[2]);
-          s += qi.w * to_f32(four.at[3]);
+#pragma unroll
+          for (int h = 0; h < HEADS; ++h) {
+            const float4 qi = *reinterpret_cast<const float4*>(qs + h * dq + i);
+            s[h] += qi.x * to_f32(four.at[0]);
+            s[h] += qi.y * to_f32(four.at[1]);
+            s[h] += qi.z * to_f32(four.at[2]);
+            s[h] += qi.w * to_f32(four.at[3]);
+          }
         }
       } else {
-        for (int i = 0; i < d; ++i) s += qs[i] * to_f32(kr[i]);
-      }
-      if (softcap > 0.f) s = softcap * tanhf(s / softcap);
-      s = fmaf(slope, (float)(key - pos), s);
-      probs[j] = s;
-      local_max = fmaxf(local_max, s);
-    }
-    const float chunk_max = block_max(local_max, scratch);
-    const float new_max = fmaxf(run_max, chunk_max);
-    const float rescale = (run_max == -INFINITY) ? 0.f : expf(run_max - new_max);
-    static_assert(kAttnChunk == kAttnItems, "a key of a chunk an item");
-    float p[PER];
+        for (int i = 0; i < d; ++i)
 #pragma unroll
-    for (int r = 0; r < PER; ++r) {
-      const int j = tid + r * kAttnThreads;
-      p[r] = j < n ? expf(probs[j] - new_max) : 0.f;
-      if (j < n) probs[j] = p[r];
+          for (int h = 0; h < HEADS; ++h) s[h] += qs[h * dq + i] * to_f32(kr[i]);
+      }
+#pragma unroll
+      for (int h = 0; h < HEADS; ++h) {
+        if (softcap > 0.f) s[h] = softcap * tanhf(s[h] / softcap);
+        s[h] = fmaf(slope[h], (float)(key - pos), s[h]);
+        probs[h * kAttnChunk + j] = s[h];
+        new_max[h] = fmaxf(new_max[h], s[h]);
+      }
     }
-    const float chunk_sum = groups_sum<PER>(p, scratch);  // also orders the probs[] writes
-    run_sum = run_sum * rescale + chunk_sum;
-    run_max = new_max;
+    block_maxima<HEADS, PER>(new_max, scratch);
+    float rescale[HEADS], p[HEADS][PER], chunk_sum[HEADS];
+    static_assert(kAttnChunk == kAttnItems, "a key of a chunk an item");
+#pragma unroll
+    for (int h = 0; h < HEADS; ++h) {
+      new_max[h] = fmaxf(run_max[h], new_max[h]);
+      rescale[h] = (run_max[h] == -INFINITY) ? 0.f : expf(run_max[h] - new_max[h]);
+#pragma unroll
+      for (int r = 0; r < PER; ++r) {
+        const int j = tid + r * kAttnThreads;
+        p[h][r] = j < n ? expf(probs[h * kAttnChunk + j] - new_max[h]) : 0.f;
+        if (j < n) probs[h * kAttnChunk + j] = p[h][r];
+      }
+    }
+    groups_sums<HEADS, PER>(p, chunk_sum, scratch);  // also orders the probs[] writes
+#pragma unroll
+    for (int h = 0; h < HEADS; ++h) {
+      run_sum[h] = run_sum[h] * rescale[h] + chunk_sum[h];
+      run_max[h] = new_max[h];
+    }
 #pragma unroll
     for (int r = 0; r < PER; ++r) {
       const int item = tid + r * kAttnThreads, entry = item % wide, run = item / wide;
       if (entry >= d || run >= runs) continue;
-      float a = acc[r] * rescale;
+      float a[HEADS];
+#pragma unroll
+      for (int h = 0; h < HEADS; ++h) a[h] = acc[h][r] * rescale[h];
       for (int from = base + run * kAttnStretch; from <= hi; from += runs * kAttnStretch) {
         const int stop = min(from + kAttnStretch, hi + 1);
         // page by page: a page's values of one entry lie side by side
@@ -150,27 +200,37 @@ paged_attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ k_
             for (; j + 4 <= here; j += 4) {
               const Four<T> four = *reinterpret_cast<const Four<T>*>(vr + j);
 #pragma unroll
-              for (int e = 0; e < 4; ++e) a += pr[j + e] * to_f32(four.at[e]);
+              for (int h = 0; h < HEADS; ++h)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) a[h] += pr[h * kAttnChunk + j + e] * to_f32(four.at[e]);
             }
           }
-          for (; j < here; ++j) a += pr[j] * to_f32(vr[j]);
+          for (; j < here; ++j)
+#pragma unroll
+            for (int h = 0; h < HEADS; ++h) a[h] += pr[h * kAttnChunk + j] * to_f32(vr[j]);
           key += here;
         }
       }
-      acc[r] = a;
+#pragma unroll
+      for (int h = 0; h < HEADS; ++h) acc[h][r] = a[h];
     }
     __syncthreads();  // probs[] is rewritten by the next chunk
   }
-  float inv = 1.f / run_sum;
-  if (gate != nullptr) inv /= 1.f + expf(-gate[(size_t)t * gate_ld + h]);
 #pragma unroll
-  for (int r = 0; r < PER; ++r) shares[tid + r * kAttnThreads] = acc[r];
-  __syncthreads();
-  for (int entry = tid; entry < od; entry += kAttnThreads) {   // the runs' shares
-    float sum = 0.f;
-    for (int r = 0; r < runs; ++r) sum += shares[r * wide + entry];
-    dst[entry] = from_f32<T>(sum * inv);
+  for (int h = 0; h < HEADS; ++h) {
+    run_sum[h] = 1.f / run_sum[h];
+    if (gate != nullptr) run_sum[h] /= 1.f + expf(-gate[(size_t)t * gate_ld + h0 + h]);
+#pragma unroll
+    for (int r = 0; r < PER; ++r) shares[h * kAttnItems + tid + r * kAttnThreads] = acc[h][r];
   }
+  __syncthreads();
+#pragma unroll
+  for (int h = 0; h < HEADS; ++h)
+    for (int entry = tid; entry < od; entry += kAttnThreads) {   // the runs' shares
+      float sum = 0.f;
+      for (int r = 0; r < runs; ++r) sum += shares[h * kAttnItems + r * wide + entry];
+      dst[h * od + entry] = from_f32<T>(sum * run_sum[h]);
+    }
 }
 
 ATOM_EXPORT int atom_paged_attention_generic(const void* q, const void* k_cache, const void* v_cache, void* out,
@@ -185,20 +245,23 @@ ATOM_EXPORT int atom_paged_attention_generic(const void* q, const void* k_cache,
   if (d > kAttnItems) return ATOM_TOO_LARGE;
   if (hq > 65535) return ATOM_TOO_LARGE;
   if (tokens == 0) return ATOM_OK;
-  const size_t smem = (size_t)((d + 3) / 4 * 4 + kAttnChunk + 16 + kAttnItems) * sizeof(float);
-  const dim3 grid(tokens, hq);
   // four keys' entries, or an entry of four keys, a load where they begin at multiples of their size in memory
   const size_t four = dtype == ATOM_F32 ? 16 : 8;
   const int key_fours = d % 4 == 0 && (uintptr_t)k_cache % four == 0;
   const int value_fours = page_size % 4 == 0 && (uintptr_t)v_cache % four == 0;
-#define LAUNCH(PER)                                                                                                  \
-  ATOM_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((paged_attention_generic_kernel<T, PER>), grid, dim3(kAttnItems / PER), smem, \
+#define LAUNCH(PER, HEADS)                                                                                           \
+  ATOM_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((paged_attention_generic_kernel<T, PER, HEADS>), dim3(tokens, hq / (HEADS)), \
+                                                 dim3(kAttnItems / PER),                                             \
+                                                 (HEADS) * ((d + 3) / 4 * 4 + kAttnChunk + 16 + kAttnItems) * sizeof(float), \
                                                  stream, (const T*)q, (const T*)k_cache, (const T*)v_cache, (T*)out,  \
                                                  token_seq, positions, block_tables, max_blocks, hq, hkv, d, page_size, \
                                                  scale, window, chunk, softcap, sink, slopes, gate, gate_ld, od, key_fours, \
                                                  value_fours))
-  if ((long)tokens * hq <= kAttnFew) LAUNCH(1);
-  else LAUNCH(4);
+  const int group = hq / hkv;
+  if ((long)tokens * hq <= kAttnFew) LAUNCH(1, 1);
+  else if (group % 4 == 0) LAUNCH(4, 4);
+  else if (group % 2 == 0) LAUNCH(4, 2);
+  else LAUNCH(4, 1);
 #undef LAUNCH
   return launch_status();
 }
