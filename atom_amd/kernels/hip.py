@@ -871,13 +871,16 @@ class HipKernels:
                     and self.lib.atom_gemm_many_supports(m, n, k, int(gate)))
 
     @staticmethod
-    def _many_pays(n: int, k: int, bias) -> bool:
+    def _many_pays(m: int, n: int, k: int, bias) -> bool:
         """Whether the kernel of large tiles is the faster one for a product that ends in nothing but its bias.  Against the BLAS
         library, 257 to 5,569 rows: with K from 8,192 on 0.91 to 2.0 times as fast (1.2 in the mean: 32B down at 4,111 rows 1,348
         -> 796 us, at 536 256 -> 139; 8B down at 536 94 -> 65), 10,240 columns of K 5,120 0.92 to 1.3 (4,111 rows 451 -> 342);
-        shorter K 0.6 to 1.4 (0.95 from 1,500 rows on, 0.63 at 257 rows by 2,048 x 2,048), which the library keeps.  A bias is
-        one pass of the library's float32 sums more and, for bfloat16, another that rounds."""
-        return bias is not None or k >= 8192 or (k >= 5120 and n >= 4096)
+        numbers of columns that are no multiple of 256, from two million results on, 0.9 to 1.7 (1.07 in the mean of 15 such
+        widths: 5,569 rows by 8,512 x 2,048 228 -> 166, by 6,176 in float32 144 -> 140, 300 by 8,512 26 -> 21).  Other widths
+        with shorter K 0.6 to 1.4 (0.95 from 1,500 rows on, 0.63 at 257 rows by 2,048 x 2,048), which the library keeps, and so
+        it does few results (300 rows by 2,912 12 us, here 17).  A bias is one pass of the library's float32 sums more and, for
+        bfloat16, another that rounds."""
+        return bias is not None or k >= 8192 or (k >= 5120 and n >= 4096) or (n % 256 != 0 and m * n >= 2_000_000)
 
     def _many_launch(self, x, weight, bias, out_dtype, gate: bool = False, act: int = 0, slices: bool = False):
         """``act(x @ weight.T + bias)``, or with ``gate`` ``act(x @ gate.T + ..) * (x @ up.T + ..)``, by the kernel of large
@@ -962,7 +965,7 @@ class HipKernels:
                 _ptr(x), _ptr(weight), None, None, _ptr(partial), m, n, k, 0, 0, self._stream()))
             result = DeferredSum(partial, bias, out_dtype)
             return result if defer else self.materialize(result)
-        if m and self._many_pays(n, k, bias) and self._many(x, weight):
+        if m and self._many_pays(m, n, k, bias) and self._many(x, weight):
             return self._many_launch(x, weight, bias, out_dtype, slices=defer and slices and n <= k)
         if x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and self.allow_library_gemm:
             pieces = self._library_slices(m, n, k) if defer and slices else 1

@@ -69,14 +69,14 @@ def test_tiles(tile, m, n, k):
             assert off(parts.sum(0), plain) < SUMS
 
 
-@pytest.mark.parametrize("m,n,k", [(257, 8192, 8192), (300, 2560, 9728), (1000, 4096, 5120), (2305, 1024, 8256), (536, 1544, 8192)])
+@pytest.mark.parametrize("m,n,k", [(257, 8192, 8192), (300, 2560, 9728), (1000, 4096, 5120), (2305, 1024, 8256), (536, 1544, 8192), (700, 3664, 2048)])
 def test_products_of_the_engine(m, n, k):
     """As the parts call it: whole, as a sum of slices, with a bias, a gate and an activation, and replayed from a graph."""
     from atom_amd.kernels.hip import DeferredSum
 
     ops = gpu_ops()
     x, w, b = operands(m, n, k, 0, 5)
-    assert ops._many(x, w) and ops._many_pays(n, k, None)
+    assert ops._many(x, w) and ops._many_pays(m, n, k, None)
     plain = x.double() @ w.double().T
     limit = 2e-7 * k ** 0.5          # 2^-24 sqrt(k), three times that
     assert off(ops.linear(x, w, b), plain + b.double()) < ROUNDED
