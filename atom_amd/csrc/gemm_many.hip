@@ -3,15 +3,15 @@
 // act(gate) * up; a plain product may end in an activation as well.
 //
 // A block of eight waves owns a tile of 128 to 256 rows of x by 128 to 256 rows of w and walks K in stages of 64 terms, a
-// whole cache line of each row, which go straight from memory into LDS (lds_loads.h), two to four stages of them at a time.  A
+// whole cache line of each row, which go straight from memory into LDS (lds_loads.h), two to four stages of them at a time (as many as fit).  A
 // row's eight 16-byte pieces stand in LDS turned by the row's number, so that the sixteen rows a matrix operand reads lie in
 // different banks.
 //
 // What bounds it: at 2,048 rows by 24,576 x 4,096 the matrix cores are busy for 70 % of the time, at the 1.8 GHz the chip
 // holds then; the tile of 256 x 256 alone keeps them at 1.95 PFLOP/s without its loads and LDS reads, 1.6 without its loads.  So:
 //   - the operands of half a stage are read from LDS while the half before is multiplied, a few reads with every four matrix
-//     instructions; the block meets once a stage, one such group after the last read of a stage, whose buffer is
-//     then free and takes the stage S ahead, a load with every group (318 -> 309 us at the size above);
+//     instructions; the block meets once a stage, one such group after the last read of a stage, whose buffer is then free and
+//     takes the stage that many buffers ahead (SX of x, SW of w), a load with every group (318 -> 309 us at the size above);
 //   - lines come from the memory side into the die's L2 before the tile asks for them: the 32 blocks of a die form 4 x 8 tiles
 //     and share their rows, so each block touches a quarter of its lines one stage further ahead, four bytes a line (a load to a
 //     corner of LDS that nobody reads; 328 -> 298 us; every block touching all of its lines: 336);

@@ -247,6 +247,9 @@ class HipKernels:
         # bfloat16 products of more rows: the kernel of large tiles; the BLAS library takes what that one does not
         self.use_many_gemm = True
         self.many_rows = 257
+        # With a gate from 321 rows on: 0.94 to 1.54 times the pace of the library's product and the gate behind it (1.11 in the
+        # mean of six sizes, 340 to 16,384 rows), below it 0.85 to 0.95 at four of the six (300 rows by 24,576 x 4,096 77 us, here 82).
+        self.many_gate_rows = 321
         self._many_plans: dict[tuple, tuple] = {}
         self.narrow_row_tiles = True   # tiles of 12 or 8 columns in the few-rows product where they spread better
         self.rows_waves = 0     # 4 or 8 forces the waves a block of that kernel (0: its own choice)
@@ -862,11 +865,16 @@ class HipKernels:
     # scratch memory that a product's cut tiles take at most (the kernel's own constant)
     MANY_SCRATCH = 128 << 20
 
+    def many_scratch(self, rows: int) -> int:
+        """Bytes of scratch memory that a bfloat16 product of ``rows`` rows takes at most."""
+        return self.MANY_SCRATCH if rows >= self.many_rows else 0
+
     def _many(self, x, weight, gate: bool = False) -> bool:
         """Whether the kernel of large tiles takes ``x @ weight.T`` (``gate``: weight = gate rows, then up rows)."""
         m, k = x.shape
         n = weight.shape[0] // 2 if gate else weight.shape[0]
-        return bool(self.use_many_gemm and m >= self.many_rows and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
+        return bool(self.use_many_gemm and m >= (self.many_gate_rows if gate else self.many_rows)
+                    and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
                     and (x.data_ptr() | weight.data_ptr()) % 16 == 0
                     and self.lib.atom_gemm_many_supports(m, n, k, int(gate)))
 
@@ -917,8 +925,8 @@ class HipKernels:
                slices: bool = True):
         """``x @ weight.T (+ bias)``.  bfloat16 operands with at most 64 rows (narrow products: 128) run this
         library's own weight-streaming kernels, 65 to 256 rows of products up to 8,192 columns wide its kernel of
-        tiles and K slices cut to the chip; the rest goes to the BLAS library, as the reference's engine
-        does for its matrix products; anything with a float32 operand runs this library's float32
+        tiles and K slices cut to the chip; more rows its kernel of large tiles where that one is the faster
+        (``_many_pays``) and else the BLAS library; anything with a float32 operand runs this library's float32
         kernels (a float32 operand as three bfloat16 pieces that hold its 24 bits).  With ``defer`` the result may come back as a
         ``DeferredSum`` for a kernel that adds the slices while it reads them; without ``slices`` a product of the BLAS
         library is left in one piece (a ``DeferredSum`` is then one slice and its bias), for readers that take one."""

@@ -92,12 +92,13 @@ class Part:
 
     def scratch_bytes(self, ops, tokens: int, seqs: int) -> int:
         """Device memory that a step of ``tokens`` tokens of ``seqs`` requests takes in this part beside the activations: here
-        what its float32 products split their input into."""
+        what its float32 products split their input into and the parts that its bfloat16 products of many rows leave."""
         product = getattr(ops, "product_scratch", None)
         if product is None:
             return 0
-        return max((product(tokens, p.shape[1]) for p in self.params.values() if p.dim() == 2 and p.dtype == torch.float32),
-                   default=0)
+        many = getattr(ops, "many_scratch", lambda rows: 0)
+        return max((product(tokens, p.shape[1]) if p.dtype == torch.float32 else many(tokens)
+                    for p in self.params.values() if p.dim() == 2 and p.dtype in (torch.float32, torch.bfloat16)), default=0)
 
     def full_name(self, local: str) -> str:
         """The checkpoint name of ``local`` under this part's prefix; an empty ``local`` names the prefix itself
