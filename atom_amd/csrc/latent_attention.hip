@@ -553,10 +553,17 @@ heads_gemm_split_kernel(const float* __restrict__ x, long ldx, long hsx, const b
   }
 }
 
-// For many rows: a block of 2 x 2 waves owns 64 tokens x 128 columns, a wave 32 x 64 of them; K is walked 64 at a time
-// (whole lines of bfloat16 rows), the next 64's pieces asked for before this step's products.  `vec`: y, its strides and the
-// gate's suit eight columns at a time (n % 8 = 0).
-constexpr int kHWideTokens = 64;
+// For many rows: a block of 2 x 2 waves owns 64 tokens x 128 columns, a wave 32 x 64 of them.  K is walked 64 at a time (whole
+// lines of bfloat16 rows): a stage's rows go from memory to registers two stages ahead and from there, rounded, to one of two
+// buffers in LDS, a row's eight pieces turned by its number, so that the sixteen rows a matrix operand reads lie in different
+// banks.  Blocks are numbered heads first: with a multiple of eight heads all blocks of a head run on one die, whose L2 then
+// holds its weights and passes a token's row from memory once.  `vec`: y, its strides and the gate's suit eight columns at a
+// time (n % 8 = 0).
+// Bound by what L2 passes to the CUs: rows that each wave read for itself, straight into a matrix operand's layout, went there
+// twice and in half lines.  5,569 tokens of 16 heads: float32 queries of 128 by 512 columns 93.6 -> 33.7 us (4.1 TB/s of memory),
+// bfloat16 latents of 512 by 128 columns 76.3 -> 23.6 (4.8); 2,048 tokens 37.2 -> 15.9 and 28.9 -> 11.8.  Over 300 sizes (1 to
+// 32 heads, 96 to 5,569 tokens, K 8 to 512) 0.91 to 4.8 times as fast, below 1 only where both take 9 us; the same bits.
+constexpr int kHWideTokens = 64, kHWideCols = 128;
 
 template <typename TX>
 struct HeadPieces;
@@ -592,85 +599,122 @@ __global__ void __launch_bounds__(256, 2)
 heads_gemm_wide_kernel(const TX* __restrict__ x, long ldx, long hsx, const bf16_t* __restrict__ w, TY* __restrict__ y,
                        long ldy, long hsy, ProductGate gate, QueryTurn turn, int m, int n, int k, float alpha, int vec) {
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, r = lane % 16, g = lane / 16;
-  const int h = blockIdx.z;
-  if ((int)blockIdx.x * 128 >= n) {   // the column of blocks behind the product's
-    const int t0 = (int)blockIdx.y * kHWideTokens;
-    turn_queries<TY>(turn, h, t0, m - t0 < kHWideTokens ? m - t0 : kHWideTokens);
+  const int h = blockIdx.x, first_row = (int)blockIdx.z * kHWideTokens, first_col = (int)blockIdx.y * kHWideCols;
+  if (first_col >= n) {   // the column of blocks behind the product's
+    turn_queries<TY>(turn, h, first_row, m - first_row < kHWideTokens ? m - first_row : kHWideTokens);
     return;
   }
-  constexpr int RT = kHWideTokens / 32, CT = 4;   // 16-row and 16-column tiles of a wave
-  const int row0 = blockIdx.y * kHWideTokens + (wave / 2) * (RT * 16);
-  const int col0 = blockIdx.x * 128 + (wave % 2) * 64;
+  constexpr int RT = kHWideTokens / 32, CT = kHWideCols / 32;            // 16-row and 16-column tiles of a wave
+  constexpr int XP = kHWideTokens * 8 / 256, WP = kHWideCols * 8 / 256;  // pieces of eight that a thread brings to a stage
+  constexpr int kTileLd = kHWideCols + 4;
+  constexpr int kStage = (kHWideTokens + kHWideCols) * 128;
+  union Shared {
+    char stage[2][kStage];                     // rows of 128 bytes, x's and then w's
+    float tile[kHWideTokens][kTileLd];
+  };
+  __shared__ __attribute__((aligned(16))) Shared lds;
   // rows and columns beyond the product's are read as its last ones and not written
-  const TX* xrow[RT];
-  const bf16_t* wrow[CT];
+  const int piece = tid % 8;
+  const TX* xrow[XP];
+  const bf16_t* wrow[WP];
 #pragma unroll
-  for (int j = 0; j < RT; ++j)
-    xrow[j] = x + (size_t)(row0 + j * 16 + r < m ? row0 + j * 16 + r : m - 1) * ldx + (size_t)h * hsx;
+  for (int j = 0; j < XP; ++j) {
+    const int row = first_row + j * 32 + tid / 8;
+    xrow[j] = x + (size_t)(row < m ? row : m - 1) * ldx + (size_t)h * hsx;
+  }
 #pragma unroll
-  for (int i = 0; i < CT; ++i)
-    wrow[i] = w + ((size_t)h * n + (col0 + i * 16 + r < n ? col0 + i * 16 + r : n - 1)) * k;
+  for (int i = 0; i < WP; ++i) {
+    const int col = first_col + i * 32 + tid / 8;
+    wrow[i] = w + ((size_t)h * n + (col < n ? col : n - 1)) * k;
+  }
   hg_f32x4 acc[CT][RT];
 #pragma unroll
   for (int i = 0; i < CT; ++i)
 #pragma unroll
     for (int j = 0; j < RT; ++j) acc[i][j] = hg_f32x4{0.f, 0.f, 0.f, 0.f};
-  HeadPieces<TX> xp[2][2][RT];
-  HeadPieces<bf16_t> wp[2][2][CT];
-  auto fetch = [&](int buffer, int k0) {
+  HeadPieces<TX> xp[2][XP];
+  HeadPieces<bf16_t> wp[2][WP];
+  auto fetch = [&](int set, int stage) {
+    const int at = stage * 64 + 8 * piece, kk = at < k ? at : k - 8;   // past the end: the last piece, counted as zeros
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int at = k0 + s * 32 + 8 * g, kk = at < k ? at : k - 8;   // past the end: the last piece, counted as zeros
+    for (int j = 0; j < XP; ++j) xp[set][j].load(xrow[j] + kk);
 #pragma unroll
-      for (int j = 0; j < RT; ++j) xp[buffer][s][j].load(xrow[j] + kk);
-#pragma unroll
-      for (int i = 0; i < CT; ++i) wp[buffer][s][i].load(wrow[i] + kk);
-    }
+    for (int i = 0; i < WP; ++i) wp[set][i].load(wrow[i] + kk);
+    __builtin_amdgcn_sched_barrier(0);
   };
-  auto multiply = [&](int buffer, int k0) {
+  const int put_at = (tid / 8) * 128 + ((piece ^ (tid / 8 % 8)) * 16);   // (rows 32 apart are turned alike)
+  auto put = [&](int set, int stage) {
+    const bool ok = stage * 64 + 8 * piece < k;
+#pragma unroll
+    for (int j = 0; j < XP; ++j) *reinterpret_cast<hg_bf16x8*>(&lds.stage[set][j * 32 * 128 + put_at]) = xp[set][j].get(ok);
+#pragma unroll
+    for (int i = 0; i < WP; ++i)
+      *reinterpret_cast<hg_bf16x8*>(&lds.stage[set][(kHWideTokens + i * 32) * 128 + put_at]) = wp[set][i].get(true);
+  };
+  auto multiply = [&](int set) {
+    const char* const xs = &lds.stage[set][((wave / 2) * (RT * 16) + r) * 128];
+    const char* const ws = &lds.stage[set][(kHWideTokens + (wave % 2) * (CT * 16) + r) * 128];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      const bool ok = k0 + s * 32 + 8 * g < k;
-      hg_bf16x8 xb[RT];
+      const int at = ((s * 4 + g) ^ (r % 8)) * 16;
+      hg_bf16x8 xb[RT], wa[CT];
 #pragma unroll
-      for (int j = 0; j < RT; ++j) xb[j] = xp[buffer][s][j].get(ok);
+      for (int j = 0; j < RT; ++j) xb[j] = *reinterpret_cast<const hg_bf16x8*>(xs + j * 16 * 128 + at);
+#pragma unroll
+      for (int i = 0; i < CT; ++i) wa[i] = *reinterpret_cast<const hg_bf16x8*>(ws + i * 16 * 128 + at);
 #pragma unroll
       for (int i = 0; i < CT; ++i)
 #pragma unroll
-        for (int j = 0; j < RT; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wp[buffer][s][i].get(true), xb[j], acc[i][j], 0, 0, 0);
+        for (int j = 0; j < RT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[i], xb[j], acc[i][j], 0, 0, 0);
     }
   };
+  // Register set and buffer 0 serve the even stages, 1 the odd ones.  A buffer is written after the barrier behind its last
+  // reads and read after the next.
+  const int stages = (k + 63) / 64;
   fetch(0, 0);
-  if (k <= 128) {   // nothing behind the second fetch: no third one that would only be thrown away
-    fetch(1, 64);
-    multiply(0, 0);
-    multiply(1, 64);
-  } else {
-    for (int k0 = 0; k0 < k; k0 += 128) {
-      fetch(1, k0 + 64);
-      __builtin_amdgcn_sched_barrier(0);
-      multiply(0, k0);
-      fetch(0, k0 + 128);
-      __builtin_amdgcn_sched_barrier(0);
-      multiply(1, k0 + 64);
-    }
+  fetch(1, 1);
+  put(0, 0);
+  __syncthreads();
+  int s = 0;
+  for (; s + 3 < stages; s += 2) {   // stage s is in buffer 0, s + 1 on its way
+    fetch(0, s + 2);
+    multiply(0);
+    put(1, s + 1);
+    __syncthreads();
+    fetch(1, s + 3);
+    multiply(1);
+    put(0, s + 2);
+    __syncthreads();
   }
-  // lane (r, g) holds columns col0 + 16 i + 4g .. + 3 of row row0 + 16 j + r; through LDS, so that whole lines are written
-  __shared__ __attribute__((aligned(16))) float tile[kHWideTokens][128 + 4];
+  const int left = stages - s;   // 1 to 3
+  if (left == 3) fetch(0, s + 2);
+  multiply(0);
+  if (left > 1) {
+    put(1, s + 1);
+    __syncthreads();
+    multiply(1);
+  }
+  if (left == 3) {
+    put(0, s + 2);
+    __syncthreads();
+    multiply(0);
+  }
+  __syncthreads();
+  // lane (r, g) holds columns 16 i + 4g .. + 3 of row 16 j + r of its wave's part; through LDS, so that whole lines are written
 #pragma unroll
   for (int j = 0; j < RT; ++j)
 #pragma unroll
     for (int i = 0; i < CT; ++i)
-      *reinterpret_cast<hg_f32x4*>(&tile[(wave / 2) * (RT * 16) + j * 16 + r][(wave % 2) * 64 + i * 16 + 4 * g]) = acc[i][j] * alpha;
+      *reinterpret_cast<hg_f32x4*>(&lds.tile[(wave / 2) * (RT * 16) + j * 16 + r][(wave % 2) * (CT * 16) + i * 16 + 4 * g]) =
+          acc[i][j] * alpha;
   __syncthreads();
-  const int c = (tid % 16) * 8, col = blockIdx.x * 128 + c;
+  const int c = (tid % 16) * 8, col = first_col + c;
   for (int t = tid / 16; t < kHWideTokens; t += 16) {
-    const int row = (int)blockIdx.y * kHWideTokens + t;
+    const int row = first_row + t;
     if (row >= m || col >= n) break;
     float v[8];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) v[q] = tile[t][c + q];
+    for (int q = 0; q < 8; ++q) v[q] = lds.tile[t][c + q];
     TY* dst = y + (size_t)row * ldy + (size_t)h * hsy + col;
     if (vec) {
       if (gate.g && gate.csg) {
@@ -777,11 +821,11 @@ ATOM_EXPORT int atom_heads_gemm_mfma(const void* x, int x_dtype, long ldx, long 
   if (m == 0) return ATOM_OK;
   dim3 grid((n + 63) / 64 + (rot > 0 ? 1 : 0), (m + 63) / 64, heads), block(256);
   if (grid.y > 65535) return ATOM_TOO_LARGE;
-  if (!split && m >= kHWideRows) {
+  if (!split && m >= kHWideRows && (n + kHWideCols - 1) / kHWideCols < 65535) {
     const long unit = 8;   // entries that are read or written together
     const int vec = n % unit == 0 && ldy % unit == 0 && hsy % unit == 0 && (size_t)y % 16 == 0 &&
                     (g.g == nullptr || g.csg == 0 || ((size_t)g.g % 16 == 0 && g.ldg % 4 == 0 && g.hsg % 4 == 0));
-    grid = dim3((n + 127) / 128 + (rot > 0 ? 1 : 0), (m + kHWideTokens - 1) / kHWideTokens, heads);
+    grid = dim3(heads, (n + kHWideCols - 1) / kHWideCols + (rot > 0 ? 1 : 0), (m + kHWideTokens - 1) / kHWideTokens);
 #define WIDE(TX, TY)                                                                                                \
   hipLaunchKernelGGL((heads_gemm_wide_kernel<TX, TY>), grid, block, 0, stream, (const TX*)x, ldx, hsx, (const bf16_t*)w, \
                      (TY*)y, ldy, hsy, g, q, m, n, k, alpha, vec)
