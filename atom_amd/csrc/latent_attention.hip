@@ -450,112 +450,34 @@ ATOM_EXPORT int atom_latent_attention(const void* q_abs, const void* pages, void
 // ------------------------------------------------------------------ the per-head products on the matrix cores
 //
 // The same product as heads_gemm with bfloat16 weights: the head's weight rows are the A operand and the tokens the B
-// operand, both read straight from memory (a float32 input is rounded to bfloat16 on the way, or, where the product is
-// to be the float32 one, split into three bfloat16 pieces that are multiplied one by one), so a lane ends up with four
-// consecutive columns of one token.  Three kernels: the exact one (a block of 2 x 2 waves owns 64 tokens x 64 columns),
-// one for many rows and one for few.  All need k % 8 == 0 and offsets and strides of x that keep its 8-element pieces
-// aligned.
+// operand (a float32 input is rounded to bfloat16 on the way, or, where the product is to be the float32 one, split into three
+// bfloat16 pieces that are multiplied one by one), so a lane ends up with four consecutive columns of one token.  Two
+// kernels: one for many rows and for the float32 product, one for few.  Both need k % 8 == 0 and offsets and strides of x
+// that keep its 8-element pieces aligned.
 
 typedef __attribute__((ext_vector_type(4))) float hg_f32x4;
 typedef __attribute__((ext_vector_type(8))) __bf16 hg_bf16x8;
 
-__device__ __forceinline__ hg_bf16x8 hg_load8(const bf16_t* p, bool ok) {
-  const hg_bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-  return ok ? *reinterpret_cast<const hg_bf16x8*>(p) : zero;
-}
-
 // A float32 input in three bfloat16 pieces, x = hi + mid + lo exactly (3 x 8 bits of mantissa): the products of each
 // piece with a bfloat16 weight are exact in float32 and the matrix cores add them in float32, so the three products
 // together are the float32 product, at three matrix instructions instead of 32 multiply-adds a lane.
-__device__ __forceinline__ void hg_load8_split(const float* p, bool ok, hg_bf16x8* hi, hg_bf16x8* mid, hg_bf16x8* lo) {
-  const hg_bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-  *hi = *mid = *lo = zero;
-  if (ok) {
-    const hg_f32x4 a = *reinterpret_cast<const hg_f32x4*>(p), b = *reinterpret_cast<const hg_f32x4*>(p + 4);
+__device__ __forceinline__ void hg_split8(hg_f32x4 a, hg_f32x4 b, bool ok, hg_bf16x8* hi, hg_bf16x8* mid, hg_bf16x8* lo) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float v = i < 4 ? a[i] : b[i - 4];
-      const __bf16 h = static_cast<__bf16>(v);
-      const float r1 = v - static_cast<float>(h);
-      const __bf16 m = static_cast<__bf16>(r1);
-      const float r2 = r1 - static_cast<float>(m);
-      (*hi)[i] = h;
-      (*mid)[i] = m;
-      (*lo)[i] = static_cast<__bf16>(r2);
-    }
-  }
-}
-
-template <typename TY>
-__global__ void __launch_bounds__(256)
-heads_gemm_split_kernel(const float* __restrict__ x, long ldx, long hsx, const bf16_t* __restrict__ w, TY* __restrict__ y,
-                       long ldy, long hsy, ProductGate gate, QueryTurn turn, int m, int n, int k, float alpha) {
-  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, r = lane % 16, g = lane / 16;
-  const int h = blockIdx.z;
-  if (blockIdx.x * 64 >= n) {   // the column of blocks behind the product's
-    turn_queries<TY>(turn, h, blockIdx.y * 64, m - (int)blockIdx.y * 64 < 64 ? m - (int)blockIdx.y * 64 : 64);
-    return;
-  }
-  const int row0 = blockIdx.y * 64 + (wave / 2) * 32;
-  const int col0 = blockIdx.x * 64 + (wave % 2) * 32;
-  const float* xrow[2];
-  bool rok[2];
-#pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
-    const int row = row0 + rt * 16 + r;
-    rok[rt] = row < m;
-    xrow[rt] = x + (size_t)(rok[rt] ? row : 0) * ldx + (size_t)h * hsx;
-  }
-  const bf16_t* wrow[2];
-  bool cok[2];
-#pragma unroll
-  for (int ct = 0; ct < 2; ++ct) {
-    const int col = col0 + ct * 16 + r;
-    cok[ct] = col < n;
-    wrow[ct] = w + ((size_t)h * n + (cok[ct] ? col : 0)) * k;
-  }
-  hg_f32x4 acc[2][2];
-#pragma unroll
-  for (int ct = 0; ct < 2; ++ct)
-#pragma unroll
-    for (int rt = 0; rt < 2; ++rt) acc[ct][rt] = hg_f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < k; k0 += 32) {
-    const int kk = k0 + 8 * g;
-    const bool kok = kk < k;
-    hg_bf16x8 xb[2], xm[2], xl[2], wa[2];
-#pragma unroll
-    for (int rt = 0; rt < 2; ++rt) hg_load8_split(xrow[rt] + kk, kok && rok[rt], &xb[rt], &xm[rt], &xl[rt]);
-#pragma unroll
-    for (int ct = 0; ct < 2; ++ct) wa[ct] = hg_load8(wrow[ct] + kk, kok && cok[ct]);
-#pragma unroll
-    for (int ct = 0; ct < 2; ++ct)
-#pragma unroll
-      for (int rt = 0; rt < 2; ++rt) {
-        // the small pieces first
-        acc[ct][rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[ct], xl[rt], acc[ct][rt], 0, 0, 0);
-        acc[ct][rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[ct], xm[rt], acc[ct][rt], 0, 0, 0);
-        acc[ct][rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[ct], xb[rt], acc[ct][rt], 0, 0, 0);
-      }
-  }
-#pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
-    const int row = row0 + rt * 16 + r;
-    if (row >= m) continue;
-#pragma unroll
-    for (int ct = 0; ct < 2; ++ct) {
-      const int col = col0 + ct * 16 + 4 * g;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (col + i < n)
-          y[(size_t)row * ldy + (size_t)h * hsy + col + i] =
-              from_f32<TY>(acc[ct][rt][i] * alpha * (gate.g ? gate_value(gate, row, h, col + i) : 1.f));
-    }
+  for (int i = 0; i < 8; ++i) {
+    const float v = !ok ? 0.f : i < 4 ? a[i] : b[i - 4];
+    const __bf16 h = static_cast<__bf16>(v);
+    const float r1 = v - static_cast<float>(h);
+    const __bf16 m = static_cast<__bf16>(r1);
+    const float r2 = r1 - static_cast<float>(m);
+    (*hi)[i] = h;
+    (*mid)[i] = m;
+    (*lo)[i] = static_cast<__bf16>(r2);
   }
 }
 
 // For many rows: a block of 2 x 2 waves owns 64 tokens x 128 columns, a wave 32 x 64 of them.  K is walked 64 at a time (whole
-// lines of bfloat16 rows): a stage's rows go from memory to registers two stages ahead and from there, rounded, to one of two
-// buffers in LDS, a row's eight pieces turned by its number, so that the sixteen rows a matrix operand reads lie in different
+// lines of bfloat16 rows): a stage's rows go from memory to registers two stages ahead and from there, rounded or in three
+// pieces (`SPLIT`), to one of two buffers in LDS, a row's eight pieces turned by its number, so that the sixteen rows a matrix operand reads lie in different
 // banks.  Blocks are numbered heads first: with a multiple of eight heads all blocks of a head run on one die, whose L2 then
 // holds its weights and passes a token's row from memory once.  `vec`: y, its strides and the gate's suit eight columns at a
 // time (n % 8 = 0).
@@ -563,6 +485,9 @@ heads_gemm_split_kernel(const float* __restrict__ x, long ldx, long hsx, const b
 // twice and in half lines.  5,569 tokens of 16 heads: float32 queries of 128 by 512 columns 93.6 -> 33.7 us (4.1 TB/s of memory),
 // bfloat16 latents of 512 by 128 columns 76.3 -> 23.6 (4.8); 2,048 tokens 37.2 -> 15.9 and 28.9 -> 11.8.  Over 300 sizes (1 to
 // 32 heads, 96 to 5,569 tokens, K 8 to 512) 0.91 to 4.8 times as fast, below 1 only where both take 9 us; the same bits.
+// The float32 product, which had tiles of 64 x 64 read straight from memory: 2,048 tokens of 8 heads by 256 x 256 36.6 -> 15.0 us,
+// of one head by 2,048 x 64 17.9 -> 10.7; 9 to 5,569 tokens 0.92 to 3.4 times as fast, below 1 only near 9 us (up to 16 tokens, or n
+// that is no multiple of 8 with a gate an entry: up to 1 us more).
 constexpr int kHWideTokens = 64, kHWideCols = 128;
 
 template <typename TX>
@@ -594,12 +519,12 @@ struct HeadPieces<float> {
   }
 };
 
-template <typename TX, typename TY>
+template <typename TX, typename TY, bool SPLIT>
 __global__ void __launch_bounds__(256, 2)
 heads_gemm_wide_kernel(const TX* __restrict__ x, long ldx, long hsx, const bf16_t* __restrict__ w, TY* __restrict__ y,
-                       long ldy, long hsy, ProductGate gate, QueryTurn turn, int m, int n, int k, float alpha, int vec) {
+                       long ldy, long hsy, ProductGate gate, QueryTurn turn, int heads, int m, int n, int k, float alpha, int vec) {
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, r = lane % 16, g = lane / 16;
-  const int h = blockIdx.x, first_row = (int)blockIdx.z * kHWideTokens, first_col = (int)blockIdx.y * kHWideCols;
+  const int h = blockIdx.x % heads, first_row = (int)blockIdx.y * kHWideTokens, first_col = (int)(blockIdx.x / heads) * kHWideCols;
   if (first_col >= n) {   // the column of blocks behind the product's
     turn_queries<TY>(turn, h, first_row, m - first_row < kHWideTokens ? m - first_row : kHWideTokens);
     return;
@@ -607,9 +532,9 @@ heads_gemm_wide_kernel(const TX* __restrict__ x, long ldx, long hsx, const bf16_
   constexpr int RT = kHWideTokens / 32, CT = kHWideCols / 32;            // 16-row and 16-column tiles of a wave
   constexpr int XP = kHWideTokens * 8 / 256, WP = kHWideCols * 8 / 256;  // pieces of eight that a thread brings to a stage
   constexpr int kTileLd = kHWideCols + 4;
-  constexpr int kStage = (kHWideTokens + kHWideCols) * 128;
+  constexpr int kPieces = SPLIT ? 3 : 1, kPlane = kHWideTokens * 128, kW = kPieces * kPlane, kStage = kW + kHWideCols * 128;
   union Shared {
-    char stage[2][kStage];                     // rows of 128 bytes, x's and then w's
+    char stage[2][kStage];                     // rows of 128 bytes, those of x's pieces and then w's
     float tile[kHWideTokens][kTileLd];
   };
   __shared__ __attribute__((aligned(16))) Shared lds;
@@ -646,26 +571,41 @@ heads_gemm_wide_kernel(const TX* __restrict__ x, long ldx, long hsx, const bf16_
   auto put = [&](int set, int stage) {
     const bool ok = stage * 64 + 8 * piece < k;
 #pragma unroll
-    for (int j = 0; j < XP; ++j) *reinterpret_cast<hg_bf16x8*>(&lds.stage[set][j * 32 * 128 + put_at]) = xp[set][j].get(ok);
+    for (int j = 0; j < XP; ++j) {
+      char* const to = &lds.stage[set][j * 32 * 128 + put_at];
+      if constexpr (SPLIT) {
+        hg_bf16x8 big, mid, low;
+        hg_split8(xp[set][j].a, xp[set][j].b, ok, &big, &mid, &low);
+        *reinterpret_cast<hg_bf16x8*>(to) = big;
+        *reinterpret_cast<hg_bf16x8*>(to + kPlane) = mid;
+        *reinterpret_cast<hg_bf16x8*>(to + 2 * kPlane) = low;
+      } else {
+        *reinterpret_cast<hg_bf16x8*>(to) = xp[set][j].get(ok);
+      }
+    }
 #pragma unroll
-    for (int i = 0; i < WP; ++i)
-      *reinterpret_cast<hg_bf16x8*>(&lds.stage[set][(kHWideTokens + i * 32) * 128 + put_at]) = wp[set][i].get(true);
+    for (int i = 0; i < WP; ++i) *reinterpret_cast<hg_bf16x8*>(&lds.stage[set][kW + i * 32 * 128 + put_at]) = wp[set][i].get(ok);
   };
   auto multiply = [&](int set) {
     const char* const xs = &lds.stage[set][((wave / 2) * (RT * 16) + r) * 128];
-    const char* const ws = &lds.stage[set][(kHWideTokens + (wave % 2) * (CT * 16) + r) * 128];
+    const char* const ws = &lds.stage[set][kW + ((wave % 2) * (CT * 16) + r) * 128];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       const int at = ((s * 4 + g) ^ (r % 8)) * 16;
-      hg_bf16x8 xb[RT], wa[CT];
+      hg_bf16x8 xb[kPieces][RT], wa[CT];
 #pragma unroll
-      for (int j = 0; j < RT; ++j) xb[j] = *reinterpret_cast<const hg_bf16x8*>(xs + j * 16 * 128 + at);
+      for (int q = 0; q < kPieces; ++q)
+#pragma unroll
+        for (int j = 0; j < RT; ++j) xb[q][j] = *reinterpret_cast<const hg_bf16x8*>(xs + q * kPlane + j * 16 * 128 + at);
 #pragma unroll
       for (int i = 0; i < CT; ++i) wa[i] = *reinterpret_cast<const hg_bf16x8*>(ws + i * 16 * 128 + at);
 #pragma unroll
-      for (int i = 0; i < CT; ++i)
+      for (int q = kPieces - 1; q >= 0; --q)   // the small pieces first
 #pragma unroll
-        for (int j = 0; j < RT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[i], xb[j], acc[i][j], 0, 0, 0);
+        for (int i = 0; i < CT; ++i)
+#pragma unroll
+          for (int j = 0; j < RT; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[i], xb[q][j], acc[i][j], 0, 0, 0);
     }
   };
   // Register set and buffer 0 serve the even stages, 1 the odd ones.  A buffer is written after the barrier behind its last
@@ -708,6 +648,28 @@ heads_gemm_wide_kernel(const TX* __restrict__ x, long ldx, long hsx, const bf16_
       *reinterpret_cast<hg_f32x4*>(&lds.tile[(wave / 2) * (RT * 16) + j * 16 + r][(wave % 2) * (CT * 16) + i * 16 + 4 * g]) =
           acc[i][j] * alpha;
   __syncthreads();
+  if (!vec) {   // column by column, all gates asked for before the first is used
+    constexpr int kStep = 256 / kHWideCols, kCount = kHWideTokens / kStep;
+    const int c = tid % kHWideCols, col = first_col + c, rows = m - first_row;
+    float f[kCount];
+    if (gate.g) {
+#pragma unroll
+      for (int q = 0; q < kCount; ++q) {
+        const int t = tid / kHWideCols + q * kStep;
+        f[q] = gate.g[(size_t)(first_row + (t < rows ? t : rows - 1)) * gate.ldg + (size_t)h * gate.hsg +
+                      (size_t)(col < n ? col : n - 1) * gate.csg];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < kCount; ++q) {
+      const int t = tid / kHWideCols + q * kStep;
+      if (t >= rows || col >= n) break;
+      float v = lds.tile[t][c];
+      if (gate.g) v *= 1.f / (1.f + expf(-f[q]));
+      y[(size_t)(first_row + t) * ldy + (size_t)h * hsy + col] = from_f32<TY>(v);
+    }
+    return;
+  }
   const int c = (tid % 16) * 8, col = first_col + c;
   for (int t = tid / 16; t < kHWideTokens; t += 16) {
     const int row = first_row + t;
@@ -716,35 +678,29 @@ heads_gemm_wide_kernel(const TX* __restrict__ x, long ldx, long hsx, const bf16_
 #pragma unroll
     for (int q = 0; q < 8; ++q) v[q] = lds.tile[t][c + q];
     TY* dst = y + (size_t)row * ldy + (size_t)h * hsy + col;
-    if (vec) {
-      if (gate.g && gate.csg) {
-        const float* gp = gate.g + row * gate.ldg + (size_t)h * gate.hsg + col;
-        const hg_f32x4 ga = *reinterpret_cast<const hg_f32x4*>(gp), gb = *reinterpret_cast<const hg_f32x4*>(gp + 4);
+    if (gate.g && gate.csg) {
+      const float* gp = gate.g + row * gate.ldg + (size_t)h * gate.hsg + col;
+      const hg_f32x4 ga = *reinterpret_cast<const hg_f32x4*>(gp), gb = *reinterpret_cast<const hg_f32x4*>(gp + 4);
 #pragma unroll
-        for (int q = 0; q < 8; ++q) v[q] *= 1.f / (1.f + expf(-(q < 4 ? ga[q] : gb[q - 4])));
-      } else if (gate.g) {
-        const float f = gate_value(gate, row, h, 0);
+      for (int q = 0; q < 8; ++q) v[q] *= 1.f / (1.f + expf(-(q < 4 ? ga[q] : gb[q - 4])));
+    } else if (gate.g) {
+      const float f = gate_value(gate, row, h, 0);
 #pragma unroll
-        for (int q = 0; q < 8; ++q) v[q] *= f;
-      }
-      if constexpr (sizeof(TY) == 2) {
-        hg_bf16x8 o;
+      for (int q = 0; q < 8; ++q) v[q] *= f;
+    }
+    if constexpr (sizeof(TY) == 2) {
+      hg_bf16x8 o;
 #pragma unroll
-        for (int q = 0; q < 8; ++q) o[q] = static_cast<__bf16>(v[q]);
-        *reinterpret_cast<hg_bf16x8*>(dst) = o;
-      } else {
-        *reinterpret_cast<hg_f32x4*>(dst) = hg_f32x4{v[0], v[1], v[2], v[3]};
-        *reinterpret_cast<hg_f32x4*>(dst + 4) = hg_f32x4{v[4], v[5], v[6], v[7]};
-      }
+      for (int q = 0; q < 8; ++q) o[q] = static_cast<__bf16>(v[q]);
+      *reinterpret_cast<hg_bf16x8*>(dst) = o;
     } else {
-#pragma unroll
-      for (int q = 0; q < 8; ++q)
-        if (col + q < n) dst[q] = from_f32<TY>(v[q] * (gate.g ? gate_value(gate, row, h, col + q) : 1.f));
+      *reinterpret_cast<hg_f32x4*>(dst) = hg_f32x4{v[0], v[1], v[2], v[3]};
+      *reinterpret_cast<hg_f32x4*>(dst + 4) = hg_f32x4{v[4], v[5], v[6], v[7]};
     }
   }
 }
 
-constexpr int kHWideRows = 96;   // from here on the wide tiles
+constexpr int kHWideRows = 96;   // from here on the wide tiles; the float32 product takes them always
 
 // For fewer rows: a block owns 16 columns of one head and 16 tokens; its four waves share out K (wave v the steps v, v + 4,
 // ..., four of them in flight) and meet once to add their sums, in the order of the waves.
@@ -819,45 +775,41 @@ ATOM_EXPORT int atom_heads_gemm_mfma(const void* x, int x_dtype, long ldx, long 
   if (!product_options(gate, ldg, hsg, csg, qx, ldqx, hsqx, qout, ldqo, hsqo, rot, rot_dims, turns, scale, &g, &q))
     return ATOM_BAD_SHAPE;
   if (m == 0) return ATOM_OK;
-  dim3 grid((n + 63) / 64 + (rot > 0 ? 1 : 0), (m + 63) / 64, heads), block(256);
-  if (grid.y > 65535) return ATOM_TOO_LARGE;
-  if (!split && m >= kHWideRows && (n + kHWideCols - 1) / kHWideCols < 65535) {
+  const dim3 block(256);
+  const long row_blocks = ((long)m + kHWideTokens - 1) / kHWideTokens;
+  const long wide_blocks = (((long)n + kHWideCols - 1) / kHWideCols + (rot > 0 ? 1 : 0)) * heads;
+  if (row_blocks > 65535) return ATOM_TOO_LARGE;
+  if (split || m >= kHWideRows) {
+    if (wide_blocks >= 1l << 24) return ATOM_TOO_LARGE;   // (threads of a grid's x dimension)
     const long unit = 8;   // entries that are read or written together
     const int vec = n % unit == 0 && ldy % unit == 0 && hsy % unit == 0 && (size_t)y % 16 == 0 &&
                     (g.g == nullptr || g.csg == 0 || ((size_t)g.g % 16 == 0 && g.ldg % 4 == 0 && g.hsg % 4 == 0));
-    grid = dim3(heads, (n + kHWideCols - 1) / kHWideCols + (rot > 0 ? 1 : 0), (m + kHWideTokens - 1) / kHWideTokens);
-#define WIDE(TX, TY)                                                                                                \
-  hipLaunchKernelGGL((heads_gemm_wide_kernel<TX, TY>), grid, block, 0, stream, (const TX*)x, ldx, hsx, (const bf16_t*)w, \
-                     (TY*)y, ldy, hsy, g, q, m, n, k, alpha, vec)
-    switch (x_dtype * 2 + y_dtype) {
-      case 0: WIDE(float, float); break;
-      case 1: WIDE(float, bf16_t); break;
-      case 2: WIDE(bf16_t, float); break;
-      default: WIDE(bf16_t, bf16_t); break;
+    const dim3 grid((unsigned)wide_blocks, (unsigned)row_blocks);
+#define WIDE(TX, TY, SPLIT)                                                                                          \
+  hipLaunchKernelGGL((heads_gemm_wide_kernel<TX, TY, SPLIT>), grid, block, 0, stream, (const TX*)x, ldx, hsx, (const bf16_t*)w, \
+                     (TY*)y, ldy, hsy, g, q, heads, m, n, k, alpha, vec)
+    switch ((split ? 4 : 0) + x_dtype * 2 + y_dtype) {
+      case 0: WIDE(float, float, false); break;
+      case 1: WIDE(float, bf16_t, false); break;
+      case 2: WIDE(bf16_t, float, false); break;
+      case 3: WIDE(bf16_t, bf16_t, false); break;
+      case 4: WIDE(float, float, true); break;
+      default: WIDE(float, bf16_t, true); break;
     }
 #undef WIDE
     return launch_status();
   }
-  if (!split) {
-    grid = dim3((n + 15) / 16 + (rot > 0 ? 1 : 0), (m + 15) / 16, heads);
+  const dim3 grid((n + 15) / 16 + (rot > 0 ? 1 : 0), (m + 15) / 16, heads);
 #define FEW(TX, TY)                                                                                                 \
   hipLaunchKernelGGL((heads_gemm_few_kernel<TX, TY>), grid, block, 0, stream, (const TX*)x, ldx, hsx, (const bf16_t*)w, \
                      (TY*)y, ldy, hsy, g, q, m, n, k, alpha, LatentRows<bf16_t>{})
-    switch (x_dtype * 2 + y_dtype) {
-      case 0: FEW(float, float); break;
-      case 1: FEW(float, bf16_t); break;
-      case 2: FEW(bf16_t, float); break;
-      default: FEW(bf16_t, bf16_t); break;
-    }
-#undef FEW
-    return launch_status();
+  switch (x_dtype * 2 + y_dtype) {
+    case 0: FEW(float, float); break;
+    case 1: FEW(float, bf16_t); break;
+    case 2: FEW(bf16_t, float); break;
+    default: FEW(bf16_t, bf16_t); break;
   }
-  if (y_dtype == ATOM_F32)
-    hipLaunchKernelGGL((heads_gemm_split_kernel<float>), grid, block, 0, stream, (const float*)x, ldx, hsx, (const bf16_t*)w,
-                       (float*)y, ldy, hsy, g, q, m, n, k, alpha);
-  else
-    hipLaunchKernelGGL((heads_gemm_split_kernel<bf16_t>), grid, block, 0, stream, (const float*)x, ldx, hsx,
-                       (const bf16_t*)w, (bf16_t*)y, ldy, hsy, g, q, m, n, k, alpha);
+#undef FEW
   return launch_status();
 }
 
