@@ -483,7 +483,8 @@ __device__ __forceinline__ void hg_split8(hg_f32x4 a, hg_f32x4 b, bool ok, hg_bf
 // time (n % 8 = 0).
 // Bound by what L2 passes to the CUs: rows that each wave read for itself, straight into a matrix operand's layout, went there
 // twice and in half lines.  5,569 tokens of 16 heads: float32 queries of 128 by 512 columns 93.6 -> 33.7 us (4.1 TB/s of memory),
-// bfloat16 latents of 512 by 128 columns 76.3 -> 23.6 (4.8); 2,048 tokens 37.2 -> 15.9 and 28.9 -> 11.8.  Over 300 sizes (1 to
+// bfloat16 latents of 512 by 128 columns 76.3 -> 23.6 (4.8), within a prompt, where the inputs come from further away and the
+// queries' rows are 192 entries apart, 97 -> 56 and 81 -> 33; 2,048 tokens 37.2 -> 15.9 and 28.9 -> 11.8.  Over 300 sizes (1 to
 // 32 heads, 96 to 5,569 tokens, K 8 to 512) 0.91 to 4.8 times as fast, below 1 only where both take 9 us; the same bits.
 // The float32 product, which had tiles of 64 x 64 read straight from memory: 2,048 tokens of 8 heads by 256 x 256 36.6 -> 15.0 us,
 // of one head by 2,048 x 64 17.9 -> 10.7; 9 to 5,569 tokens 0.92 to 3.4 times as fast, below 1 only near 9 us (up to 16 tokens, or n
