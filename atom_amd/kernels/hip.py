@@ -928,8 +928,8 @@ class HipKernels:
         tiles and K slices cut to the chip; more rows its kernel of large tiles where that one is the faster
         (``_many_pays``) and else the BLAS library; anything with a float32 operand runs this library's float32
         kernels (a float32 operand as three bfloat16 pieces that hold its 24 bits).  With ``defer`` the result may come back as a
-        ``DeferredSum`` for a kernel that adds the slices while it reads them; without ``slices`` a product of the BLAS
-        library is left in one piece (a ``DeferredSum`` is then one slice and its bias), for readers that take one."""
+        ``DeferredSum`` for a kernel that adds the slices while it reads them; without ``slices`` a product of many rows
+        is left in one piece (a ``DeferredSum`` is then one slice and its bias), for readers that take one."""
         if isinstance(x, (DeferredSum, PendingProduct)):
             x = self.materialize(x)
         m, k = x.shape
@@ -973,8 +973,13 @@ class HipKernels:
                 _ptr(x), _ptr(weight), None, None, _ptr(partial), m, n, k, 0, 0, self._stream()))
             result = DeferredSum(partial, bias, out_dtype)
             return result if defer else self.materialize(result)
-        if m and self._many_pays(m, n, k, bias) and self._many(x, weight):
-            return self._many_launch(x, weight, bias, out_dtype, slices=defer and slices and n <= k)
+        reads = defer and n <= k          # whoever reads the result takes sums, and adds the bias
+        if m and self._many_pays(m, n, k, None if reads else bias) and self._many(x, weight):
+            # sums that the library's product would hand on in float32 are handed on so by this one, in slices or as one
+            if not reads or (bias is None and not (slices and self._library_slices(m, n, k) > 1)):
+                return self._many_launch(x, weight, bias, out_dtype, slices=reads and slices)
+            y = self._many_launch(x, weight, None, torch.float32, slices=slices)
+            return DeferredSum(y.partial if isinstance(y, DeferredSum) else y.unsqueeze(0), bias, out_dtype)
         if x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and self.allow_library_gemm:
             pieces = self._library_slices(m, n, k) if defer and slices else 1
             if pieces > 1:
@@ -989,8 +994,8 @@ class HipKernels:
             # float32 out, or a bias: the library writes its float32 sums as they are, so that logits have the
             # same precision whatever the number of rows, and a bias is added before anything is rounded
             y = torch.mm(x, weight.t(), out_dtype=torch.float32)
-            if bias is not None and defer and n <= k:
-                return DeferredSum(y.unsqueeze(0), bias, out_dtype)     # whoever reads it adds the bias
+            if bias is not None and reads:
+                return DeferredSum(y.unsqueeze(0), bias, out_dtype)
             if bias is not None:
                 self._done("bias_rows", self.lib.atom_bias_rows(_ptr(y), _ptr(bias), m, n, self._stream()))
             return y if out_dtype == torch.float32 else y.to(out_dtype)

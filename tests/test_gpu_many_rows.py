@@ -129,3 +129,25 @@ def test_what_it_leaves_to_others():
     keep = torch.ones_like(got, dtype=torch.bool)
     keep[7], keep[:, 9] = False, False
     assert bool(got[:, 9].isnan().all()) and not bool(got[7].isfinite().any()) and torch.equal(got[keep], y[keep])
+
+
+# Sizes whose plan hands slices on and sizes where it does not; (884, 3104, 4224) and (629, 6504, 11840) are such that the BLAS
+# library's product would be cut in two.
+@pytest.mark.parametrize("m,n,k", [(300, 2048, 2048), (536, 4096, 8192), (884, 3104, 4224), (629, 6504, 11840), (2305, 2048, 8192)])
+@pytest.mark.parametrize("biased", [True, False])
+@pytest.mark.parametrize("slices", [True, False])
+def test_sums_for_a_reader_stay_float32(m, n, k, biased, slices):
+    """A deferred product whose reader adds a bias, or slices that the library's product would leave, is handed on in float32."""
+    from atom_amd.kernels.hip import DeferredSum
+
+    ops = gpu_ops()
+    x, w, b = operands(m, n, k, 0, 11)
+    if not biased and not (slices and ops._library_slices(m, n, k) > 1):
+        pytest.skip("the product is its tensor")
+    lazy = ops.linear(x, w, b if biased else None, defer=True, slices=slices)
+    assert isinstance(lazy, DeferredSum) and lazy.partial.dtype == torch.float32 and lazy.dtype == torch.bfloat16
+    assert lazy.splits == 1 or slices
+    assert (lazy.bias is b) if biased else (lazy.bias is None)
+    want = x.double() @ w.double().T
+    assert off(lazy.partial.double().sum(0), want) < 2e-7 * k ** 0.5
+    assert off(ops.materialize(lazy), want + (b.double() if biased else 0)) < ROUNDED
