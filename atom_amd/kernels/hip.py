@@ -247,8 +247,8 @@ class HipKernels:
         # bfloat16 products of more rows: the kernel of large tiles; the BLAS library takes what that one does not
         self.use_many_gemm = True
         self.many_rows = 257
-        # With a gate from 321 rows on: 0.94 to 1.54 times the pace of the library's product and the gate behind it (1.11 in the
-        # mean of six sizes, 340 to 16,384 rows), below it 0.85 to 0.95 at four of the six (300 rows by 24,576 x 4,096 77 us, here 82).
+        # With a gate from 321 rows on: 0.84 to 2.2 times the pace of the library's product and the gate behind it (1.18 in the mean of
+        # 1,214 products), below it 0.85 to 0.95 at four of six sizes (300 rows by 24,576 x 4,096 77 us, here 82).
         self.many_gate_rows = 321
         self._many_plans: dict[tuple, tuple] = {}
         self.narrow_row_tiles = True   # tiles of 12 or 8 columns in the few-rows product where they spread better
@@ -878,17 +878,32 @@ class HipKernels:
                     and (x.data_ptr() | weight.data_ptr()) % 16 == 0
                     and self.lib.atom_gemm_many_supports(m, n, k, int(gate)))
 
-    @staticmethod
-    def _many_pays(m: int, n: int, k: int, bias) -> bool:
-        """Whether the kernel of large tiles is the faster one for a product that ends in nothing but its bias.  Against the BLAS
-        library, 257 to 5,569 rows: with K from 8,192 on 0.91 to 2.0 times as fast (1.2 in the mean: 32B down at 4,111 rows 1,348
-        -> 796 us, at 536 256 -> 139; 8B down at 536 94 -> 65), 10,240 columns of K 5,120 0.92 to 1.3 (4,111 rows 451 -> 342);
-        numbers of columns that are no multiple of 256, from two million results on, 0.9 to 1.7 (1.07 in the mean of 15 such
-        widths: 5,569 rows by 8,512 x 2,048 228 -> 166, by 6,176 in float32 144 -> 140, 300 by 8,512 26 -> 21).  Other widths
-        with shorter K 0.6 to 1.4 (0.95 from 1,500 rows on, 0.63 at 257 rows by 2,048 x 2,048), which the library keeps, and so
-        it does few results (300 rows by 2,912 12 us, here 17).  A bias is one pass of the library's float32 sums more and, for
-        bfloat16, another that rounds."""
-        return bias is not None or k >= 8192 or (k >= 5120 and n >= 4096) or (n % 256 != 0 and m * n >= 2_000_000)
+    def _many_pays(self, m: int, n: int, k: int, bias, out_dtype=torch.bfloat16, act: bool = False) -> bool:
+        """Whether the kernel of large tiles is the faster one for a product of ``n`` rows of weights that ends in ``bias`` and,
+        with ``act``, in a gate or an activation.  ``bias``: None also where whoever reads the sums adds it.  Against the BLAS library and
+        what runs behind it, 164 weights of 128 to 51,200 by 512 to 25,600 at 257 to 8,192 rows (mean of the ratios; and how many of
+        them are below 0.97), for products that end in nothing:
+        - K from 8,192 on: 1.20 (85 of 477; 5,120 x 25,600 at 4,111 rows 1.63, 8,192 x 8,192 0.89 to 1.38);
+        - K from 5,120, 4,096 columns and more: 1.06 (6 of 56) where the library's tiles of 256 x 256 are a quarter of the CUs or
+          fewer, 1.17 (4 of 21) where they need three rounds of the CUs (10,240 x 5,120 at 4,111 rows 1.28); other numbers of tiles
+          0.99 (60 of 169), which the library keeps;
+        - columns that are no multiple of 256, two to 80 million results: 1.13 (57 of 425; 8,512 x 2,048 at 4,111 rows 1.20).  Fewer
+          rows 1.08 (12 of 46) and, with K from 3,072 on, where fewer than 1,000 are few, 1.01 (28 of 73); more results 0.97 (19 of 38).
+        Anything behind the library's product is a pass over its results: of one pass (a float32 result's bias, an activation, a gate)
+        1.15 to 1.25, of two (a bias in float32 and its rounding) and more 1.4 to 1.5.  The library keeps small products, which it
+        finishes in less (384 rows by 640 x 1,536 with ReLU 10 us, here 14), and one pass at 320 rows and fewer (300 rows by 6,144 x
+        4,096 0.91 to 0.94)."""
+        if k >= 8192:
+            return True
+        passes = act + (0 if bias is None else 1 if out_dtype == torch.float32 else 2)
+        if passes:
+            return m * n * k >= 1.25e9 if passes > 1 else m >= self.many_gate_rows and m * n * k >= 2.5e9
+        if k >= 5120 and n >= 4096:
+            tile = self.chip.library_tile
+            tiles = -(-m // tile) * -(-n // tile)
+            if 4 * tiles <= self.num_cus or -(-tiles // self.num_cus) == 3:
+                return True
+        return n % 256 != 0 and 2e6 <= m * n <= 8e7 and m >= (450 if k < 3072 else 1000)
 
     def _many_launch(self, x, weight, bias, out_dtype, gate: bool = False, act: int = 0, slices: bool = False):
         """``act(x @ weight.T + bias)``, or with ``gate`` ``act(x @ gate.T + ..) * (x @ up.T + ..)``, by the kernel of large
@@ -974,7 +989,7 @@ class HipKernels:
             result = DeferredSum(partial, bias, out_dtype)
             return result if defer else self.materialize(result)
         reads = defer and n <= k          # whoever reads the result takes sums, and adds the bias
-        if m and self._many_pays(m, n, k, None if reads else bias) and self._many(x, weight):
+        if m and self._many_pays(m, n, k, None if reads else bias, out_dtype) and self._many(x, weight):
             # sums that the library's product would hand on in float32 are handed on so by this one, in slices or as one
             if not reads or (bias is None and not (slices and self._library_slices(m, n, k) > 1)):
                 return self._many_launch(x, weight, bias, out_dtype, slices=reads and slices)
@@ -1044,7 +1059,7 @@ class HipKernels:
             self._rows_launch(x, weight, bias, 0, y=y, act=self._ROWS_ACT[activation], out_f32=y.dtype == torch.float32)
             return y
         x = self.materialize(x)
-        if m and activation in ("relu", "relu_squared") and self._many_alone(x, weight):
+        if m and activation in ("relu", "relu_squared") and self._many_alone(x, weight, bias, out_dtype or x.dtype):
             self._check("linear input", x, torch.bfloat16)
             self._check("linear weight", weight, torch.bfloat16, (weight.shape[0], x.shape[1]))
             if bias is not None:
@@ -1112,7 +1127,7 @@ class HipKernels:
                 _ptr(x), F32, _ptr(weight), self._code(weight), _ptr(bias), _ptr(act), m, inter, k,
                 _ptr(scratch), self._stream()))
             return act
-        if m and self._many_alone(x, weight, gate=True):
+        if m and self._many_alone(x, weight, bias, x.dtype, gate=True):
             return self._many_gated(x, weight, bias, "silu")
         gate_up = self.linear(x, weight, bias)
         act = torch.empty((m, inter), dtype=x.dtype, device=x.device)
@@ -1129,16 +1144,18 @@ class HipKernels:
             x = self.materialize(x)
         if x.shape[0] and not self._rows_takes(x, weight):
             x = self.materialize(x)
-            if self._many_alone(x, weight, gate=True):
+            if self._many_alone(x, weight, bias, x.dtype, gate=True):
                 return self._many_gated(x, weight, bias, activation)
         # a product of few rows waits for the gate, which becomes its epilogue
         both = self.linear(x, weight, bias, defer=True, slices=False)
         act = torch.empty((both.shape[0], weight.shape[0] // 2), dtype=both.dtype, device=both.device)
         return self.gated_act(both, act, activation)
 
-    def _many_alone(self, x, weight, gate: bool = False) -> bool:
-        """Whether the kernel of large tiles takes this product and no kernel of fewer rows does."""
-        return not self._tile(x, weight) and not self._skinny(x, weight) and self._many(x, weight, gate)
+    def _many_alone(self, x, weight, bias, out_dtype, gate: bool = False) -> bool:
+        """Whether the kernel of large tiles takes this product that ends in a gate or an activation, and no kernel of fewer rows
+        does."""
+        return (self._many(x, weight, gate) and self._many_pays(x.shape[0], weight.shape[0], x.shape[1], bias, out_dtype, True)
+                and not self._tile(x, weight) and not self._skinny(x, weight))
 
     def _many_gated(self, x, weight, bias, activation: str):
         self._check("linear input", x, torch.bfloat16)

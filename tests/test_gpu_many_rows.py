@@ -151,3 +151,33 @@ def test_sums_for_a_reader_stay_float32(m, n, k, biased, slices):
     want = x.double() @ w.double().T
     assert off(lazy.partial.double().sum(0), want) < 2e-7 * k ** 0.5
     assert off(ops.materialize(lazy), want + (b.double() if biased else 0)) < ROUNDED
+
+
+# The lines of the rule that gives products to the kernel of large tiles: what the BLAS library finishes earlier stays with it.
+@pytest.mark.parametrize("call,m,n,k,takes", [
+    ("bias", 300, 640, 1536, False), ("bias", 384, 2048, 2048, True), ("bias32", 536, 1408, 1664, False), ("bias32", 300, 6144, 4096, False),
+    ("bias32", 2048, 4096, 2048, True), ("bias deferred", 300, 2048, 2048, False), ("bias deferred", 300, 2048, 8192, True),
+    ("relu", 384, 640, 1536, False), ("relu", 300, 6144, 4096, False), ("relu", 321, 6144, 4096, True), ("relu", 300, 2048, 8192, True),
+    ("silu", 384, 640, 1536, False), ("silu", 320, 6144, 4096, False), ("silu", 321, 6144, 4096, True), ("silu bias", 321, 2048, 2048, True),
+    ("gelu_tanh", 700, 640, 1536, False), ("gelu_tanh", 700, 4096, 2048, True),
+    ("", 1024, 4096, 5120, True), ("", 1025, 4096, 5120, False), ("", 4111, 10240, 5120, True), ("", 2305, 10240, 5120, False),
+    ("", 536, 16000, 3008, True), ("", 384, 16000, 3008, False), ("", 700, 4928, 4032, False), ("", 5569, 18704, 704, False)])
+def test_which_products_it_takes(call, m, n, k, takes, monkeypatch):
+    ops = gpu_ops()
+    x, w, b = operands(m, n, k, 0, 3)
+    taken, launch = [], ops._many_launch
+    monkeypatch.setattr(ops, "_many_launch", lambda *a, **kw: taken.append(1) or launch(*a, **kw))
+    plain = x.double() @ w.double().T
+    if call in ("silu", "silu bias", "gelu_tanh"):
+        b = b if "bias" in call else None
+        y = ops.linear_gated(x, w, b, call) if call == "gelu_tanh" else ops.linear_silu(x, w, b)
+        gate, up = (plain if b is None else plain + b.double()).split(n // 2, 1)
+        want = activation(call.split()[0])(gate) * up
+    elif call == "relu":
+        y, want = ops.linear_act(x, w, None, "relu"), torch.relu(plain)
+    else:
+        y = ops.linear(x, w, b if call else None, out_dtype=torch.float32 if call == "bias32" else None, defer="deferred" in call)
+        y, want = ops.materialize(y), plain + b.double() if call else plain
+    assert bool(taken) == takes
+    # the library's way rounds a gate's two halves, or the product before its activation, to bfloat16 first
+    assert off(y, want) < (ROUNDED if takes or call in ("", "bias", "bias32", "bias deferred") else 2 * ROUNDED)
