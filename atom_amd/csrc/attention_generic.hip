@@ -1,8 +1,8 @@
 // Paged attention, general form: any head size, any page size, float32 or bfloat16,
 // every query token of a mixed batch (prompt portions and single decoded tokens alike).
 //
-// One block per (query token, query head), or, for many tokens, per token and two or four heads that share keys.  The token's request and absolute position
-// are given per token; the keys it sees are positions max(0, p - window + 1) .. p of that
+// One block per (query token, query head), or, for many tokens, per token and two or four heads that share keys.  The
+// token's request and absolute position are given per token; the keys it sees are positions max(0, p - window + 1) .. p of that
 // request, found through the request's block table; with `chunk` only those from the start of the run of `chunk`
 // positions (counted from position 0) that p lies in.  With `softcap` a score s becomes softcap * tanh(s / softcap); with
 // `slopes` head h's score of key j then loses slopes[h] * (p - j); exp(sink[h]) joins head h's denominator with no key and
@@ -16,6 +16,7 @@
 
 constexpr int kAttnItems = 512;   // (entry, run of keys) pairs a block has
 constexpr int kAttnFew = 1024;    // blocks up to which the chip holds them all at once with 512 threads each
+constexpr int kAttnFours = 600;  // blocks of four heads from which on a launch has enough of them
 constexpr int kAttnChunk = 512;  // keys per pass
 constexpr int kAttnStretch = 16; // keys a thread adds in one go
 
@@ -233,6 +234,18 @@ paged_attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ k_
     }
 }
 
+// Heads that a block of 128 threads takes; 0: a block of 512 threads each.  Four where that leaves two blocks or more a CU: 484 sizes
+// (seven layouts of 6 to 64 heads, prompts of 20 to 1,000 tokens, portions behind 2,000 keys, decoded tokens behind 300 and 2,000; both
+// types) take 0.9 % longer than each's best of one, two and four; with four always 2.5 % (32 heads over 8, 33 tokens 10.7 us, with
+// two 8.5, with one 8.8; 461 tokens 121, 188 and 332).
+ATOM_EXPORT int atom_paged_attention_generic_heads(int tokens, int hq, int hkv) {
+  const long rows = (long)tokens * hq;
+  const int group = hq / hkv;
+  if (rows <= kAttnFew) return 0;
+  if (group % 4 == 0 && rows / 4 >= kAttnFours) return 4;
+  return group % 2 == 0 ? 2 : 1;
+}
+
 ATOM_EXPORT int atom_paged_attention_generic(const void* q, const void* k_cache, const void* v_cache, void* out,
                                              const int* token_seq, const int* positions,
                                              const int* block_tables, int max_blocks, int dtype, int tokens,
@@ -257,10 +270,10 @@ ATOM_EXPORT int atom_paged_attention_generic(const void* q, const void* k_cache,
                                                  token_seq, positions, block_tables, max_blocks, hq, hkv, d, page_size, \
                                                  scale, window, chunk, softcap, sink, slopes, gate, gate_ld, od, key_fours, \
                                                  value_fours))
-  const int group = hq / hkv;
-  if ((long)tokens * hq <= kAttnFew) LAUNCH(1, 1);
-  else if (group % 4 == 0) LAUNCH(4, 4);
-  else if (group % 2 == 0) LAUNCH(4, 2);
+  const int heads = atom_paged_attention_generic_heads(tokens, hq, hkv);
+  if (heads == 0) LAUNCH(1, 1);
+  else if (heads == 4) LAUNCH(4, 4);
+  else if (heads == 2) LAUNCH(4, 2);
   else LAUNCH(4, 1);
 #undef LAUNCH
   return launch_status();

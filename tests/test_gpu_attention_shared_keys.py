@@ -17,13 +17,16 @@ DEV = "cuda:0"
                                                    (12, 1, 300, 8, 40), (2, 2, 64, 16, 530)])
 @pytest.mark.parametrize("extras", [{}, {"softcap": 3.0, "window": 100, "sink": 1, "slopes": 1, "gate": 1, "od": 1}])
 def test_rows_are_those_of_single_tokens(dtype, hq, hkv, d, page, longest, extras):
+    check_rows(dtype, hq, hkv, d, page, longest, extras, 1024 // hq + 7)             # more than the launches that take a block a head
+
+
+def check_rows(dtype, hq, hkv, d, page, longest, extras, tokens):
     from atom_amd.kernels.hip import AttentionMeta
 
     ops = gpu_ops()
     ops.use_mfma_attention = False
     try:
         g = torch.Generator(device=DEV).manual_seed(3)
-        tokens = 1024 // hq + 7                           # more than the launches that take a block a head
         lens = [longest, 1, longest // 2]
         blocks = -(-longest // page)
         pages = torch.randperm(3 * blocks, generator=torch.Generator().manual_seed(1)).to(torch.int32).view(3, blocks).to(DEV)
@@ -55,3 +58,19 @@ def test_rows_are_those_of_single_tokens(dtype, hq, hkv, d, page, longest, extra
             assert torch.equal(run([t])[0], many[t])
     finally:
         ops.use_mfma_attention = True
+
+
+# 600 blocks of four heads and a few more (fewer take two heads each), groups of four and eight
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("hq,hkv,d,page,longest", [(4, 1, 32, 16, 513), (8, 1, 36, 4, 300), (12, 3, 128, 16, 512), (24, 1, 65, 6, 77)])
+@pytest.mark.parametrize("extras", [{}, {"softcap": 3.0, "window": 100, "sink": 1, "slopes": 1, "gate": 1, "od": 1}])
+def test_rows_of_four_heads_a_block(dtype, hq, hkv, d, page, longest, extras):
+    check_rows(dtype, hq, hkv, d, page, longest, extras, 2400 // hq + 7)
+
+
+def test_heads_a_block():
+    heads = gpu_ops().lib.atom_paged_attention_generic_heads
+    assert heads(32, 32, 8) == 0                                                     # a block a head, 512 threads
+    assert heads(33, 32, 8) == heads(74, 32, 8) == heads(2000, 6, 3) == 2            # few blocks of four; a group of two
+    assert heads(75, 32, 8) == heads(461, 32, 8) == heads(38, 64, 8) == 4
+    assert heads(33, 32, 32) == heads(500, 6, 2) == 1
