@@ -451,6 +451,22 @@ ATOM_EXPORT long atom_gemm_many_scratch(int m, int n, int gate, int tile, int wh
   return cut * slices * T.bm * T.bn * 4;
 }
 
+// The most memory that the parts of a product of `from` to `to` rows take by its plan, handed out as slices or not.  (A plan
+// holds for all rows between two multiples of 64, which every tile's rows are.)
+ATOM_EXPORT long atom_gemm_many_scratch_most(int from, int to, int n, int k, int gate, int num_cus) {
+  long most = 0;
+  for (long m = (from + 63L) / 64 * 64;; m += 64) {
+    const int rows = (int)(m < to ? m : to);
+    for (int as_slices = 0; rows >= from && as_slices <= (gate ? 0 : 1); ++as_slices) {
+      int plan[4];
+      if (atom_gemm_many_plan(rows, n, k, gate, as_slices, num_cus, plan) != ATOM_OK) continue;
+      const long bytes = plan[3] ? 4L * plan[2] * rows * n : atom_gemm_many_scratch(rows, n, gate, plan[0], plan[1], plan[2]);
+      if (bytes > most) most = bytes;
+    }
+    if (m >= to) return most;
+  }
+}
+
 // plan: tile, tiles that stay whole, slices, whether the parts go to [slices, m, n] in `parts` (then all tiles are cut, and
 // y, bias and act are not used).
 ATOM_EXPORT int atom_gemm_many(const void* x, const void* w, const float* bias, void* y, float* parts, int m, int n, int k,

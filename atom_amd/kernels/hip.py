@@ -231,6 +231,7 @@ class HipKernels:
         self.lib.atom_delta_chunks_floats.restype = ctypes.c_long
         self.lib.atom_gemm_f32_scratch.restype = ctypes.c_long
         self.lib.atom_gemm_many_scratch.restype = ctypes.c_long
+        self.lib.atom_gemm_many_scratch_most.restype = ctypes.c_long
         self.allow_library_gemm = True
         # bfloat16 products of few rows run this library's own weight-streaming kernels: up to 64 rows, and
         # up to 128 for the narrow products that atom_gemm_skinny_supports names; the BLAS library takes the rest.
@@ -251,6 +252,7 @@ class HipKernels:
         # 1,214 products), below it 0.85 to 0.95 at four of six sizes (300 rows by 24,576 x 4,096 77 us, here 82).
         self.many_gate_rows = 321
         self._many_plans: dict[tuple, tuple] = {}
+        self._many_most: dict[tuple, int] = {}
         self.narrow_row_tiles = True   # tiles of 12 or 8 columns in the few-rows product where they spread better
         self.rows_waves = 0     # 4 or 8 forces the waves a block of that kernel (0: its own choice)
         self.use_mfma_attention = True
@@ -865,9 +867,17 @@ class HipKernels:
     # scratch memory that a product's cut tiles take at most (the kernel's own constant)
     MANY_SCRATCH = 128 << 20
 
-    def many_scratch(self, rows: int) -> int:
-        """Bytes of scratch memory that a bfloat16 product of ``rows`` rows takes at most."""
-        return self.MANY_SCRATCH if rows >= self.many_rows else 0
+    def many_scratch(self, rows: int, n: int, k: int) -> int:
+        """Bytes of scratch memory that a bfloat16 product of up to ``rows`` rows with a weight of ``n`` x ``k``, gated or not,
+        takes at most."""
+        if not self.use_many_gemm or rows < self.many_rows:
+            return 0
+        key = (rows, n, k)
+        if key not in self._many_most:
+            most = self.lib.atom_gemm_many_scratch_most
+            self._many_most[key] = max(most(self.many_rows, rows, n, k, 0, self.num_cus),
+                                       0 if n % 2 else most(self.many_rows, rows, n // 2, k, 1, self.num_cus))
+        return self._many_most[key]
 
     def _many(self, x, weight, gate: bool = False) -> bool:
         """Whether the kernel of large tiles takes ``x @ weight.T`` (``gate``: weight = gate rows, then up rows)."""

@@ -96,8 +96,8 @@ class Part:
         product = getattr(ops, "product_scratch", None)
         if product is None:
             return 0
-        many = getattr(ops, "many_scratch", lambda rows: 0)
-        return max((product(tokens, p.shape[1]) if p.dtype == torch.float32 else many(tokens)
+        many = getattr(ops, "many_scratch", lambda rows, n, k: 0)
+        return max((product(tokens, p.shape[1]) if p.dtype == torch.float32 else many(tokens, *p.shape)
                     for p in self.params.values() if p.dim() == 2 and p.dtype in (torch.float32, torch.bfloat16)), default=0)
 
     def full_name(self, local: str) -> str:

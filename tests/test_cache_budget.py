@@ -1,5 +1,6 @@
 """What the cache's budget leaves free: memory a step takes in its parts beside the activations."""
 
+import ctypes
 from types import SimpleNamespace
 
 import torch
@@ -71,3 +72,36 @@ def test_decode_graphs_are_left_the_scratch_memory_of_their_products():
         return engine._graph_estimate()
 
     assert estimate(torch.float32) == estimate(torch.bfloat16) + 6 * 128 * 4096
+
+
+def test_bfloat16_products_of_many_rows_are_left_what_their_plans_take(monkeypatch):
+    from atom_amd.kernels.build import build
+
+    ops = _ops()
+    ops.lib = ctypes.CDLL(build())
+    ops.lib.atom_gemm_many_scratch.restype = ops.lib.atom_gemm_many_scratch_most.restype = ctypes.c_long
+    ops.use_many_gemm, ops.many_rows, ops.num_cus, ops._many_most = True, 257, 256, {}
+    ops.product_scratch = lambda rows, k: 0
+    ops.many_scratch = lambda *a: HipKernels.many_scratch(ops, *a)
+    monkeypatch.setattr("test_cache_budget._ops", lambda: ops)
+
+    def taken(rows, n, k, gate, apart):
+        plan = (ctypes.c_int * 4)()
+        if ops.lib.atom_gemm_many_plan(rows, n, k, gate, apart, 256, plan) != 0:
+            return 0
+        tile, whole, slices, as_slices = plan
+        return 4 * slices * rows * n if as_slices else ops.lib.atom_gemm_many_scratch(rows, n, gate, tile, whole, slices)
+
+    def most(part, tokens):
+        return max(taken(m, n // 2 if gate else n, k, gate, apart) for n, k in (tuple(p.shape) for p in part.params.values() if p.dim() == 2)
+                   for m in range(257, tokens + 1) for gate, apart in ((0, 0), (0, 1), (1, 0)))
+
+    plain = _budget([GatedMLP(512, 1024)], 4096, monkeypatch)
+    for hidden, inter, tokens in ((512, 1024, 4096), (1024, 2048, 700), (2560, 9728, 2000), (576, 1096, 300)):
+        part = _f32_mlp(hidden, inter, torch.bfloat16)
+        assert _budget([part], tokens, monkeypatch) == plain - most(part, tokens)
+        assert most(part, tokens) <= 128 << 20 and (most(part, tokens) > 0 or tokens == 300)
+    assert _budget([_f32_mlp(1024, 4096, torch.bfloat16)], 256, monkeypatch) == plain
+    assert _budget([_f32_mlp(100, 300, torch.bfloat16)], 4096, monkeypatch) == plain     # no size the kernel takes
+    small = _f32_mlp(1024, 2816, torch.bfloat16)
+    assert most(small, 2048) < 100 << 20                                                 # not the bound of all plans
