@@ -523,9 +523,11 @@ struct HeadPieces<float> {
 template <typename TX, typename TY, bool SPLIT>
 __global__ void __launch_bounds__(256, 2)
 heads_gemm_wide_kernel(const TX* __restrict__ x, long ldx, long hsx, const bf16_t* __restrict__ w, TY* __restrict__ y,
-                       long ldy, long hsy, ProductGate gate, QueryTurn turn, int heads, int m, int n, int k, float alpha, int vec) {
+                       long ldy, long hsy, ProductGate gate, QueryTurn turn, int beside, int m, int n, int k, float alpha, int vec) {
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, r = lane % 16, g = lane / 16;
-  const int h = blockIdx.x % heads, first_row = (int)blockIdx.y * kHWideTokens, first_col = (int)(blockIdx.x / heads) * kHWideCols;
+  // `beside` heads lie side by side in x, all of them or, with the heads in z, one
+  const int h = blockIdx.x % beside + blockIdx.z;
+  const int first_row = (int)blockIdx.y * kHWideTokens, first_col = (int)(blockIdx.x / beside) * kHWideCols;
   if (first_col >= n) {   // the column of blocks behind the product's
     turn_queries<TY>(turn, h, first_row, m - first_row < kHWideTokens ? m - first_row : kHWideTokens);
     return;
@@ -778,17 +780,19 @@ ATOM_EXPORT int atom_heads_gemm_mfma(const void* x, int x_dtype, long ldx, long 
   if (m == 0) return ATOM_OK;
   const dim3 block(256);
   const long row_blocks = ((long)m + kHWideTokens - 1) / kHWideTokens;
-  const long wide_blocks = (((long)n + kHWideCols - 1) / kHWideCols + (rot > 0 ? 1 : 0)) * heads;
   if (row_blocks > 65535) return ATOM_TOO_LARGE;
   if (split || m >= kHWideRows) {
-    if (wide_blocks >= 1l << 24) return ATOM_TOO_LARGE;   // (threads of a grid's x dimension)
+    const long col_blocks = ((long)n + kHWideCols - 1) / kHWideCols + (rot > 0 ? 1 : 0);
+    const long most = 1l << 24;   // blocks of a grid's x dimension, which has fewer than 2^32 threads
+    if (col_blocks >= most) return ATOM_TOO_LARGE;
+    const int beside = col_blocks * heads < most ? heads : 1;   // (2.1e9 columns of all heads and more: the heads in z)
     const long unit = 8;   // entries that are read or written together
     const int vec = n % unit == 0 && ldy % unit == 0 && hsy % unit == 0 && (size_t)y % 16 == 0 &&
                     (g.g == nullptr || g.csg == 0 || ((size_t)g.g % 16 == 0 && g.ldg % 4 == 0 && g.hsg % 4 == 0));
-    const dim3 grid((unsigned)wide_blocks, (unsigned)row_blocks);
+    const dim3 grid((unsigned)(col_blocks * beside), (unsigned)row_blocks, (unsigned)(heads / beside));
 #define WIDE(TX, TY, SPLIT)                                                                                          \
   hipLaunchKernelGGL((heads_gemm_wide_kernel<TX, TY, SPLIT>), grid, block, 0, stream, (const TX*)x, ldx, hsx, (const bf16_t*)w, \
-                     (TY*)y, ldy, hsy, g, q, heads, m, n, k, alpha, vec)
+                     (TY*)y, ldy, hsy, g, q, beside, m, n, k, alpha, vec)
     switch ((split ? 4 : 0) + x_dtype * 2 + y_dtype) {
       case 0: WIDE(float, float, false); break;
       case 1: WIDE(float, bf16_t, false); break;

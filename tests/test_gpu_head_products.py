@@ -45,3 +45,26 @@ def test_per_head_products_of_many_tokens(heads, m, n, gated, k, x_type, exact, 
         got = y[:, h * hsy:h * hsy + n]
         assert bool(((got - want).abs() <= bound).all()), f"head {h}: {float(((got - want).abs() / bound).max()):.2f} of the bound"
         assert bool((y[:, h * hsy + n:(h + 1) * hsy] == 7.0).all()), "columns between the heads' were written"
+
+
+def test_more_columns_than_a_grids_first_dimension_holds_blocks():
+    """2^31 columns of two heads and a few more: the heads in the grid's third dimension."""
+    from atom_amd.kernels.hip import HipKernels
+
+    if torch.cuda.mem_get_info(DEV)[0] < 48 << 30:
+        pytest.skip("34 GB of weights")
+    ops = HipKernels(DEV)
+    ops.heads_split_from = 1
+    heads, k, n = 2, 8, (1 << 30) + 64
+    x = rnd((1, heads * k), 1).to(DEV)
+    w = torch.empty((heads, n, k), dtype=torch.bfloat16, device=DEV).normal_()
+    y = torch.empty((1, heads * n), dtype=torch.bfloat16, device=DEV)
+    ops.heads_gemm(x, 0, heads * k, k, w, y, 0, heads * n, n, heads, 1, n, k, exact=True)
+    for h in range(heads):
+        for at in (0, n // 2 - 77, n - 300):
+            want = w[h, at:at + 300].double() @ x[0, h * k:(h + 1) * k].double()
+            got = y[0, h * n + at:h * n + at + 300].double()
+            terms = w[h, at:at + 300].double().abs() @ x[0, h * k:(h + 1) * k].double().abs()
+            assert bool(((got - want).abs() <= (3 * k + 8) * 2.0 ** -24 * terms + 2.0 ** -8 * want.abs()).all()), (h, at)
+    del w, y
+    torch.cuda.empty_cache()
