@@ -110,9 +110,6 @@ class DecodeGraphs:
             return None
         return (next(p for p in self.prefill_sizes if p >= total), self.prefill_slots, n)
 
-    def accepts(self, entries, cached: list[int]) -> bool:
-        return self.place(entries, cached) is not None
-
     def place(self, entries, cached: list[int]) -> tuple[int, int, int] | None:
         """The bucket whose graph runs these entries, or None if the step is to be launched."""
         if not self.usable or not entries or max(c + len(e.tokens) for c, e in zip(cached, entries)) > self.max_model_len:
@@ -274,7 +271,7 @@ class DecodeGraphs:
                           cu_seqlens_q=view("starts"), context_lens=view("context_lens"),
                           cached_lens=view("cached_lens"), slot_of_seq=view("slot_of_seq"),
                           num_prefill=cap.first_single, max_q_len=max(p, 1),
-                          # a bound, not the batch's own: no request of a replayed step is longer (accepts())
+                          # a bound, not the batch's own: no request of a replayed step is longer (place())
                           max_context_len=self.max_model_len, replayed=True)
         for gi, (g, width) in enumerate(zip(core.manager.groups, self.widths)):
             ctx.block_tables[gi] = view(f"bt{gi}").view(cap.num_seqs, width)

@@ -331,3 +331,27 @@ def test_a_page_is_named_only_when_all_its_tokens_are_known():
     mgr.open("c")
     assert mgr.match_prefix("c", [1, 2, 3, 4, 5, 6, 7, 0, 9]) == 4      # not under the placeholder
     mgr.check()
+
+
+@pytest.mark.parametrize("groups", [[GroupSpec(4, 64)], [GroupSpec(4, 64), GroupSpec(16, 64)], [GroupSpec(4, 64, window=6)],
+                                    [GroupSpec(8, 64), GroupSpec(4, 64, window=6)], [GroupSpec(4, 64, chunk=8)], []])
+@pytest.mark.parametrize("held", [0, 1, 3, 4, 5, 15, 16, 17, 33])
+def test_a_request_that_holds_its_step_lacks_nothing(groups, held):
+    """``holds`` says yes only where ``cover`` has nothing to do, and always where every group keeps its keys."""
+    m = CacheManager(groups, 2)
+    assert not m.holds("a", 1)
+    m.open("a")
+    if held:
+        m.cover("a", 0, held)
+    keeps = all(g.keeps_all for g in groups)
+    for cached in {0, max(0, held - 1), held}:
+        for upto in range(cached + 1, held + 20):
+            for reserve in (None, 0, upto - 1, upto, upto + 1, upto + 9):
+                lacks = any(m.pages_missing("a", cached, upto, reserve))
+                holds = m.holds("a", upto, reserve)
+                assert holds == (keeps and not lacks)
+                if holds:
+                    before = [list(m.block_table("a", g)) for g in range(len(groups))]
+                    m.cover("a", cached, upto, reserve)
+                    assert before == [list(m.block_table("a", g)) for g in range(len(groups))]
+    m.check()
