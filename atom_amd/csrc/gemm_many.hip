@@ -7,17 +7,18 @@
 // row's eight 16-byte pieces stand in LDS turned by the row's number, so that the sixteen rows a matrix operand reads lie in
 // different banks.
 //
-// What bounds it: at 2,048 rows by 24,576 x 4,096 the matrix cores are busy for 70 % of the time, at the 1.8 GHz the chip
-// holds then; the tile of 256 x 256 alone keeps them at 1.95 PFLOP/s without its loads and LDS reads, 1.6 without its loads.  So:
+// What bounds it: at 2,048 rows by 24,576 x 4,096 (314 to 323 us, 1.3 PFLOP/s) the matrix cores are busy for 70 % of the time, at
+// the 1.8 GHz the chip holds then; the tile of 256 x 256 alone keeps them at 1.95 PFLOP/s without its loads and LDS reads, 1.6
+// without its loads.  So:
 //   - the operands of half a stage are read from LDS while the half before is multiplied, a few reads with every four matrix
 //     instructions; the block meets once a stage, one such group after the last read of a stage, whose buffer is then free and
-//     takes the stage that many buffers ahead (SX of x, SW of w), a load with every group (318 -> 309 us at the size above);
-//   - lines come from the memory side into the die's L2 before the tile asks for them: the 32 blocks of a die form 4 x 8 tiles
-//     and share their rows, so each block touches a quarter of its lines one stage further ahead, four bytes a line (a load to a
-//     corner of LDS that nobody reads; 328 -> 298 us; every block touching all of its lines: 336);
+//     takes the stage that many buffers ahead (SX of x, SW of w), a load with every group (when the kernel was first built 318
+//     -> 309 us at the size above);
 //   - blocks go to the dies in turn; each die takes a run of tiles of its own, in bands of four row tiles.
-// Tried and not taken: stages of 32 terms, half lines, in four and five buffers (329; by tiles of 128 x 256 433, 367 with whole
-// lines), four waves with 128 x 128 each, which read a third less from LDS (343).
+// Tried then and not taken: stages of 32 terms, half lines, in four and five buffers (329; by tiles of 128 x 256 433, 367 with
+// whole lines), four waves with 128 x 128 each, which read a third less from LDS (343).  Blocks that touch a quarter of their lines
+// a stage further ahead, which the other blocks of their die read as well, take longer in every tile whose LDS has room for it
+// (90 sizes: 128 x 128 1.05 times, 256 x 128 1.05, 256 x 192 1.02, 192 x 256 1.01).
 //
 // Where the tiles' last round would leave CUs idle, its tiles are cut along K (`slices`): their parts go to `scratch` in the
 // order of the registers, and a second launch adds them, in slice order, and writes y.  A caller that adds slices itself may
@@ -95,13 +96,9 @@ __device__ __forceinline__ int in_runs(int at, int count) {
   return xcd * (count / kXcds) + min(xcd, count % kXcds) + at / kXcds;
 }
 
-// A load of `Bytes` (4 or 16) a lane from base + offset to LDS: lane l's land at `lds` + Bytes l.
-template <int Bytes>
+// A load of 16 bytes a lane from base + offset to LDS: lane l's land at `lds` + 16 l.
 __device__ __forceinline__ void load_at_to_lds(const void* base, unsigned offset, unsigned lds) {
-  if constexpr (Bytes == 16)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base) : "memory");
-  else
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(offset), "s"(base) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base) : "memory");
 }
 
 // Waits until all but this wave's last LEFT loads have arrived and its LDS reads are done, then for the block.
@@ -116,11 +113,9 @@ struct Many {
   static constexpr int MF = MF_, NF = NF_, WM = WM_, WN = WN_, SX = SX_, SW = SW_;
   static constexpr bool GATE = GATE_;
   static constexpr int bm = 16 * MF * WM, bn = 16 * NF * WN, out = GATE ? bn / 2 : bn;
-  static constexpr int xstage = bm * kRowBytes, wstage = bn * kRowBytes;       // LDS: the stages of w, those of x, a corner
+  static constexpr int xstage = bm * kRowBytes, wstage = bn * kRowBytes;       // LDS: the stages of w, those of x
   static constexpr int xloads = bm / 8 / kWaves, wloads = bn / 8 / kWaves;     // loads a wave
-  static constexpr int xfrom = SW * wstage, staged = xfrom + SX * xstage;
-  static constexpr bool touches = staged + kWaves * 256 <= kLdsBytes;
-  static constexpr int lds = staged + (touches ? kWaves * 256 : 0);
+  static constexpr int xfrom = SW * wstage, lds = xfrom + SX * xstage;
   static constexpr int NO = GATE ? NF / 2 : NF;                                // fours of columns of y a lane holds of a row
   static_assert(WM * WN == kWaves && (!GATE || NF % 2 == 0), "as many gate as up rows a wave");
   static_assert(bm % 64 == 0 && bn % 64 == 0, "whole loads");
@@ -176,23 +171,11 @@ __global__ void __launch_bounds__(64 * kWaves, 2) gemm_many_kernel(ManyParams p)
 #pragma unroll
   for (int j = 0; j < LW; ++j) wfrom[j] = (unsigned)row_of((j * kWaves + wave) * 8 + (lane >> 3)) * row_bytes + turned;
   const auto load_x = [&](int j, int stage, int buf) {
-    load_at_to_lds<16>(xs + (size_t)stage * kRowBytes, xfrom[j], lds0 + G::xfrom + buf * G::xstage + (j * kWaves + wave) * 1024);
+    load_at_to_lds(xs + (size_t)stage * kRowBytes, xfrom[j], lds0 + G::xfrom + buf * G::xstage + (j * kWaves + wave) * 1024);
   };
   const auto load_w = [&](int j, int stage, int buf) {
-    load_at_to_lds<16>(ws + (size_t)stage * kRowBytes, wfrom[j], lds0 + buf * G::wstage + (j * kWaves + wave) * 1024);
+    load_at_to_lds(ws + (size_t)stage * kRowBytes, wfrom[j], lds0 + buf * G::wstage + (j * kWaves + wave) * 1024);
   };
-  // The quarter of the lines that this block touches ahead: the first four waves 16 rows of w each, the others of x.
-  const int quarter = wave % 4 * 16 + (lane & 15);
-  const unsigned ahead = (unsigned)row_of(wave < 4 ? (mtile & 3) * (BN / 4) + quarter % (BN / 4)
-                                                   : BN + (ntile & 3) * (BM / 4) + quarter % (BM / 4)) * row_bytes;
-  const char* const touch_base = wave < 4 ? ws : xs;
-  const int touch_ahead = wave < 4 ? SW : SX;
-  const auto touch = [&](int stage) {
-    const size_t at = (size_t)(touch_base + (size_t)min(stage + touch_ahead, stages - 1) * kRowBytes);   // the same in all lanes:
-    const unsigned high = __builtin_amdgcn_readfirstlane((int)(at >> 32)), low = __builtin_amdgcn_readfirstlane((int)at);
-    if (lane < 16) load_at_to_lds<4>((const void*)((size_t)high << 32 | low), ahead, lds0 + G::staged + wave * 256);
-  };
-
   f32x4 acc[MF][NF];
 #pragma unroll
   for (int a = 0; a < MF; ++a)
@@ -240,9 +223,9 @@ __global__ void __launch_bounds__(64 * kWaves, 2) gemm_many_kernel(ManyParams p)
   using Set0 = std::integral_constant<int, 0>;
   using Set1 = std::integral_constant<int, 1>;
   using Apart = std::integral_constant<int, -1>;
-  // A stage's loads go out as x, w, touch; the next stage has arrived when no more than these of the newest are left: w and the
-  // touch where w is a stage further ahead than x, else the touch and the stages behind the next with theirs.
-  constexpr int T = G::touches, LEFT = SW > SX ? LW + T : (SX - 2) * (LX + LW + T) + T;
+  // A stage's loads go out as x, w; the next stage has arrived when no more than these of the newest are left: w where it is a
+  // stage further ahead than x, else the stages behind the next.
+  constexpr int LEFT = SW > SX ? LW : (SX - 2) * (LX + LW);
   using Meet = std::integral_constant<int, LEFT>;
   using MeetLast = std::integral_constant<int, 0>;
   const auto nothing = [](int, int) {};
@@ -254,9 +237,8 @@ __global__ void __launch_bounds__(64 * kWaves, 2) gemm_many_kernel(ManyParams p)
       for (int j = 0; j < LX; ++j) load_x(j, s, s);
 #pragma unroll
     for (int j = 0; j < LW; ++j) load_w(j, s, s);
-    if (T && SW == SX && s > 0 && s < SX - 1) touch(s);   // (so that the first stages' waits count what the others' do)
   }
-  stage_barrier<(SX - 1) * LX + (SW - 1) * LW + (SW == SX ? (SX - 2) * T : 0)>();
+  stage_barrier<(SX - 1) * LX + (SW - 1) * LW>();
 #pragma unroll
   for (int i = 0; i < NF; ++i) read_w(Set0{}, i, at0);
 #pragma unroll
@@ -267,9 +249,7 @@ __global__ void __launch_bounds__(64 * kWaves, 2) gemm_many_kernel(ManyParams p)
   int wbuf = 0, xbuf = 0;
   const auto stage = [&](auto more_x, auto more_w, auto meet, auto more, int s) {
     const int wnext = wbuf + 1 == SW ? 0 : wbuf + 1, xnext = xbuf + 1 == SX ? 0 : xbuf + 1;
-    half(Set0{}, Yes{}, Apart{}, wbuf * G::wstage + at1, xbuf * G::xstage + at1, [&](int g, int) {
-      if (decltype(more_w)::value && G::touches && g == 3) touch(s);
-    });
+    half(Set0{}, Yes{}, Apart{}, wbuf * G::wstage + at1, xbuf * G::xstage + at1, nothing);
     if constexpr (decltype(more)::value)
       half(Set1{}, Yes{}, meet, wnext * G::wstage + at0, xnext * G::xstage + at0, [&](int g, int groups) {
         constexpr int N = (decltype(more_x)::value ? LX : 0) + (decltype(more_w)::value ? LW : 0);
