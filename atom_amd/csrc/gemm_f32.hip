@@ -389,16 +389,17 @@ gemm_f32_kernel(GemmF32Params p) {
 }
 
 // Many rows, float32 operands, K a multiple of 32: tiles of 64 or 128 rows and 128 columns whose operands go through LDS, in
-// whole cache lines straight from memory.  x comes as planes of pieces, made once by a kernel of its own; pieces of w are formed
-// where it is multiplied.  A block is two groups of four waves, a wave with 64 x 32 of the tile, so that a step's splitting
+// whole cache lines straight from memory.  x comes in pieces, a row's twelve of a step side by side, made once by a kernel of its
+// own; pieces of w are formed where it is multiplied.  A block is two groups of four waves, a wave with 64 x 32 of the tile, so that a step's splitting
 // (two of w's 16-row parts) takes a third of the cycles of its 48 matrix instructions; in 32 x 64 it would take more than they
 // do.  A stage is 32 terms of the tile's rows, double buffered; the 16-byte pieces of a row change places by its row number, so
 // that the rows a wave reads at once lie in different banks.  While a stage is multiplied, the next one's operands are read from
 // LDS and the stage behind that comes from memory: 56 KB for two groups of four slices each, 40 KB in tiles of 128 rows, at the
-// 35 to 40 KB a microsecond that a CU draws, are what bounds it.  465 rows by 24,576 x 4,096 take 583 us in tiles of 128 rows (938
+// 35 to 40 KB a microsecond that a CU draws, are what bounds it.  465 rows by 24,576 x 4,096 take 573 us in tiles of 128 rows (938
 // with the float32 instructions; 645 in tiles of 64, timed when those were 595), by 4,096 x 4,096, where only the lower ones are a
-// tile for every CU, 108 (164), by 4,096 x 12,288 302 (475); 1,024 rows by 24,576 1,125, 183 TFLOP/s (1,873; the float32
-// instructions' rate is 157).  (w times 2^24 as it is split is 1 to 2 % of these.)
+// tile for every CU, 108 (164), by 4,096 x 12,288 299 (475); 1,024 rows by 24,576 1,120, 184 TFLOP/s (1,873; the float32
+// instructions' rate is 157).  (w times 2^24 as it is split is 1 to 2 % of these.  With x's pieces in three planes, a plane's rows
+// half a line a step, the four are 600, 112, 310 and 1,151.)
 // Five stages in LDS with all eight waves on each (32 x 32 of 64 x 128 a wave) took 705, 120 and 340 at 465 rows.
 constexpr int kWideCols = 128;
 
@@ -407,8 +408,8 @@ constexpr int kWideCols = 128;
 template <int ROWS>
 struct Wide {
   static constexpr int groups = 128 / ROWS;                            // of waves that share K
-  static constexpr int plane = ROWS * kStep * 2;                       // bytes of a stage of one plane of x,
-  static constexpr int stage = 3 * plane + kWideCols * kStep * 4;      // and of a stage
+  static constexpr int xs = ROWS * kStep * 6;                          // bytes of x in a stage: rows of three times kStep pieces,
+  static constexpr int stage = xs + kWideCols * kStep * 4;             // and of a stage, w behind them
   static constexpr int sums = ROWS * kWideCols * 4;                    // the sums of half of K
   static constexpr int bytes = groups == 2 ? 4 * stage : 2 * stage + sums;
   static_assert(bytes <= 160 * 1024 && bytes >= sums, "it all fits in LDS");
@@ -454,8 +455,8 @@ __device__ __noinline__ void sum_again_wide(const float* x, const float* w, int 
 
 template <int ROWS>
 __global__ void __launch_bounds__(kSlices* kWave) gemm_f32_wide_kernel(GemmF32Params p) {
-  constexpr int GROUPS = Wide<ROWS>::groups, kPlaneBytes = Wide<ROWS>::plane, kStageBytes = Wide<ROWS>::stage;
-  extern __shared__ __align__(16) char wide[];   // [group][buffer][kStageBytes]: x's planes, then w
+  constexpr int GROUPS = Wide<ROWS>::groups, kStageBytes = Wide<ROWS>::stage;
+  extern __shared__ __align__(16) char wide[];   // [group][buffer][kStageBytes]: x's pieces, then w
   const int tile = blockIdx.x % kXcds * (gridDim.x / kXcds) + blockIdx.x / kXcds;
   if (tile >= p.tiles) return;
   const int row0 = tile % p.row_tiles * ROWS;
@@ -509,7 +510,7 @@ __global__ void __launch_bounds__(kSlices* kWave) gemm_f32_wide_kernel(GemmF32Pa
   };
   const auto read = [&](Operands& o, int stage) {
     const char* xs = mine + (stage & 1) * kStageBytes;
-    const char* ws = xs + 3 * kPlaneBytes;
+    const char* ws = xs + Wide<ROWS>::xs;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int r = 32 * w4 + 16 * j + side;
