@@ -83,12 +83,22 @@ def test_products_of_the_engine(m, n, k):
     y32 = ops.linear(x, w, b, out_dtype=torch.float32)
     assert off(y32, plain + b.double()) < limit
     lazy = ops.linear(x, w, b, defer=True)
-    assert isinstance(lazy, torch.Tensor) or lazy.splits > 1
-    assert off(lazy.partial.double().sum(0) + b.double() if isinstance(lazy, DeferredSum) else lazy, plain + b.double()) < ROUNDED
+    if n <= k:                       # a product that a reader adds: slices, by each of these plans
+        assert isinstance(lazy, DeferredSum) and lazy.splits > 1 and lazy.bias is b
+        assert off(lazy.partial.double().sum(0), plain) < limit
+    else:
+        assert isinstance(lazy, torch.Tensor) and off(lazy, plain + b.double()) < ROUNDED
     assert off(ops.linear_act(x, w, b, "relu_squared"), torch.relu(plain + b.double()) ** 2) < ROUNDED
     half = (plain + b.double()).split(n // 2, 1)
+    # (gates of fewer than 321 rows, or of halves that are not eights, are the library's)
+    gated = m >= 321 and n % 16 == 0
+    assert ops._many_alone(x, w, b, torch.bfloat16, gate=True) == gated
     for name in ("silu", "relu", "gelu_tanh"):
         assert off(ops.linear_gated(x, w, b, name), activation(name)(half[0]) * half[1]) < ROUNDED
+    assert off(ops.linear_silu(x, w, b), activation("silu")(half[0]) * half[1]) < ROUNDED
+    free = plain.split(n // 2, 1)
+    assert off(ops.linear_silu(x, w), activation("silu")(free[0]) * free[1]) < ROUNDED
+    assert off(ops.linear_act(x, w, None, "relu"), torch.relu(plain)) < ROUNDED
     static, out = x.clone(), None
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
@@ -179,5 +189,4 @@ def test_which_products_it_takes(call, m, n, k, takes, monkeypatch):
         y = ops.linear(x, w, b if call else None, out_dtype=torch.float32 if call == "bias32" else None, defer="deferred" in call)
         y, want = ops.materialize(y), plain + b.double() if call else plain
     assert bool(taken) == takes
-    # the library's way rounds a gate's two halves, or the product before its activation, to bfloat16 first
-    assert off(y, want) < (ROUNDED if takes or call in ("", "bias", "bias32", "bias deferred") else 2 * ROUNDED)
+    assert off(y, want) < ROUNDED
