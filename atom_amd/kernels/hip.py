@@ -891,28 +891,38 @@ class HipKernels:
     def _many_pays(self, m: int, n: int, k: int, bias, out_dtype=torch.bfloat16, act: bool = False) -> bool:
         """Whether the kernel of large tiles is the faster one for a product of ``n`` rows of weights that ends in ``bias`` and,
         with ``act``, in a gate or an activation.  ``bias``: None also where whoever reads the sums adds it.  Against the BLAS library and
-        what runs behind it, 164 weights of 128 to 51,200 by 512 to 25,600 at 257 to 8,192 rows (mean of the ratios; and how many of
+        what runs behind it, 164 weights of 128 to 51,200 by 512 to 25,600 at 257 to 8,192 rows, those of K from
+        8,192 on and of whole rounds 122 and 34 up to 16,384 (mean of the ratios; and how many of
         them are below 0.97), for products that end in nothing:
-        - K from 8,192 on: 1.20 (85 of 477; 5,120 x 25,600 at 4,111 rows 1.63, 8,192 x 8,192 0.89 to 1.38);
-        - K from 5,120, 4,096 columns and more: 1.06 (6 of 56) where the library's tiles of 256 x 256 are a quarter of the CUs or
-          fewer, 1.17 (4 of 21) where they need three rounds of the CUs (10,240 x 5,120 at 4,111 rows 1.28); other numbers of tiles
-          0.99 (60 of 169), which the library keeps;
+        - K from 8,192 on: 1.32 (102 of 1,242; 5,120 x 25,600 at 4,111 rows 1.75, 8,192 x 8,192 1.48), deferred 1.27 (127), where the
+          library's tiles of 256 x 256 leave more than a 16th of their rounds of the CUs empty and a single round is no fuller than
+          nine 16ths.  Full rounds 0.96 (120 of 147; 4,096 x 12,288 at 8,192 and 16,384 rows 0.91 and 0.90) and single rounds of more
+          1.00 (63 of 120; 4,096 x 14,336 at 2,560 rows 0.86) the library keeps;
+        - K from 5,120, 4,096 columns and more: 1.06 (6 of 56) where those tiles are a quarter of the CUs or fewer, 1.29 (1 of 9) where they
+          need three rounds of the CUs and leave that much of them empty (10,240 x 5,120 at 4,111 rows 1.35; 8,192 x 5,120 at 6,144,
+          three whole rounds, 0.92); other numbers of tiles 0.99 (60 of 169), which the library keeps;
         - columns that are no multiple of 256, two to 80 million results: 1.13 (57 of 425; 8,512 x 2,048 at 4,111 rows 1.20).  Fewer
           rows 1.08 (12 of 46) and, with K from 3,072 on, where fewer than 1,000 are few, 1.01 (28 of 73); more results 0.97 (19 of 38).
         Anything behind the library's product is a pass over its results: of one pass (a float32 result's bias, an activation, a gate)
-        1.15 to 1.25, of two (a bias in float32 and its rounding) and more 1.4 to 1.5.  The library keeps small products, which it
-        finishes in less (384 rows by 640 x 1,536 with ReLU 10 us, here 14), and one pass at 320 rows and fewer (300 rows by 6,144 x
-        4,096 0.91 to 0.94)."""
-        if k >= 8192:
-            return True
+        1.15 to 1.25, of two (a bias in float32 and its rounding) and more 1.4 to 1.5.  Behind whole rounds of the library's tiles
+        a gate or an activation alone makes less: with K from 8,192 on 0.96 (35 of 52), which the library keeps, from 4,096 on 1.01
+        (7 of 78; 24,576 x 4,096 at 16,384 rows 0.96).  It keeps small products as well, which it finishes in less (384 rows by
+        640 x 1,536 with ReLU 10 us, here 14), and one pass at 320 rows and fewer (300 rows by 6,144 x 4,096 0.91 to 0.94)."""
         passes = act + (0 if bias is None else 1 if out_dtype == torch.float32 else 2)
+        tile = self.chip.library_tile
+        tiles = -(-m // tile) * -(-n // tile)
+        rounds = -(-tiles // self.num_cus)
+        if passes > 1:
+            return k >= 8192 or m * n * k >= 1.25e9
+        if passes and k >= 8192:
+            return not act or tiles % self.num_cus != 0
         if passes:
-            return m * n * k >= 1.25e9 if passes > 1 else m >= self.many_gate_rows and m * n * k >= 2.5e9
-        if k >= 5120 and n >= 4096:
-            tile = self.chip.library_tile
-            tiles = -(-m // tile) * -(-n // tile)
-            if 4 * tiles <= self.num_cus or -(-tiles // self.num_cus) == 3:
-                return True
+            return m >= self.many_gate_rows and m * n * k >= 2.5e9
+        room = 16 * tiles < 15 * rounds * self.num_cus       # the library's rounds are not full
+        if k >= 8192 and room and (rounds > 1 or 16 * tiles <= 9 * self.num_cus):
+            return True
+        if k >= 5120 and n >= 4096 and (4 * tiles <= self.num_cus or (rounds == 3 and room)):
+            return True
         return n % 256 != 0 and 2e6 <= m * n <= 8e7 and m >= (450 if k < 3072 else 1000)
 
     def _many_launch(self, x, weight, bias, out_dtype, gate: bool = False, act: int = 0, slices: bool = False):

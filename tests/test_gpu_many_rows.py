@@ -171,7 +171,11 @@ def test_sums_for_a_reader_stay_float32(m, n, k, biased, slices):
     ("silu", 384, 640, 1536, False), ("silu", 320, 6144, 4096, False), ("silu", 321, 6144, 4096, True), ("silu bias", 321, 2048, 2048, True),
     ("gelu_tanh", 700, 640, 1536, False), ("gelu_tanh", 700, 4096, 2048, True),
     ("", 1024, 4096, 5120, True), ("", 1025, 4096, 5120, False), ("", 4111, 10240, 5120, True), ("", 2305, 10240, 5120, False),
-    ("", 536, 16000, 3008, True), ("", 384, 16000, 3008, False), ("", 700, 4928, 4032, False), ("", 5569, 18704, 704, False)])
+    ("", 536, 16000, 3008, True), ("", 384, 16000, 3008, False), ("", 700, 4928, 4032, False), ("", 5569, 18704, 704, False),
+    # K from 8,192 on: rounds of the library's tiles that are full, and single ones of more than nine 16ths of the CUs
+    ("", 2048, 8192, 8192, False), ("", 1900, 7680, 8192, False), ("deferred", 4096, 8192, 8192, False), ("bias deferred", 2305, 4096, 8192, False),
+    ("", 2304, 4096, 8192, True), ("deferred", 2048, 4096, 9728, True), ("", 4111, 8192, 8192, True), ("bias", 2048, 8192, 8192, True),
+    ("relu", 2048, 8192, 8192, False), ("relu", 1900, 7680, 8192, True), ("", 6144, 8192, 5120, False), ("", 4111, 8192, 5120, True)])
 def test_which_products_it_takes(call, m, n, k, takes, monkeypatch):
     ops = gpu_ops()
     x, w, b = operands(m, n, k, 0, 3)
@@ -186,7 +190,7 @@ def test_which_products_it_takes(call, m, n, k, takes, monkeypatch):
     elif call == "relu":
         y, want = ops.linear_act(x, w, None, "relu"), torch.relu(plain)
     else:
-        y = ops.linear(x, w, b if call else None, out_dtype=torch.float32 if call == "bias32" else None, defer="deferred" in call)
-        y, want = ops.materialize(y), plain + b.double() if call else plain
+        y = ops.linear(x, w, b if "bias" in call else None, out_dtype=torch.float32 if call == "bias32" else None, defer="deferred" in call)
+        y, want = ops.materialize(y), plain + b.double() if "bias" in call else plain
     assert bool(taken) == takes
     assert off(y, want) < ROUNDED
