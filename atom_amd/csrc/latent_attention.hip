@@ -487,8 +487,9 @@ __device__ __forceinline__ void hg_split8(hg_f32x4 a, hg_f32x4 b, bool ok, hg_bf
 // queries' rows are 192 entries apart, 97 -> 56 and 81 -> 33; 2,048 tokens 37.2 -> 15.9 and 28.9 -> 11.8.  Over 300 sizes (1 to
 // 32 heads, 96 to 5,569 tokens, K 8 to 512) 0.91 to 4.8 times as fast, below 1 only where both take 9 us; the same bits.
 // The float32 product, which had tiles of 64 x 64 read straight from memory: 2,048 tokens of 8 heads by 256 x 256 36.6 -> 15.0 us,
-// of one head by 2,048 x 64 17.9 -> 10.7; 9 to 5,569 tokens 0.92 to 3.4 times as fast, below 1 only near 9 us (up to 16 tokens, or n
-// that is no multiple of 8 with a gate an entry: up to 1 us more).
+// of one head by 2,048 x 64 17.9 -> 10.7; 9 to 5,569 tokens 0.84 to 3.4 times as fast, below 0.97 at 27 of 352 sizes, all of 16 tokens
+// and fewer (K 64: 3.4 -> 3.8 us, 128 by 512: 4.5 -> 4.8) or with n that is no multiple of 8 and a gate an entry (8.3 -> 9.2).  With a
+// path of its own for one stage those of K 64 take 3.7 us and all others 2 % longer.
 constexpr int kHWideTokens = 64, kHWideCols = 128;
 
 template <typename TX>

@@ -891,9 +891,8 @@ class HipKernels:
     def _many_pays(self, m: int, n: int, k: int, bias, out_dtype=torch.bfloat16, act: bool = False) -> bool:
         """Whether the kernel of large tiles is the faster one for a product of ``n`` rows of weights that ends in ``bias`` and,
         with ``act``, in a gate or an activation.  ``bias``: None also where whoever reads the sums adds it.  Against the BLAS library and
-        what runs behind it, 164 weights of 128 to 51,200 by 512 to 25,600 at 257 to 8,192 rows, those of K from
-        8,192 on and of whole rounds 122 and 34 up to 16,384 (mean of the ratios; and how many of
-        them are below 0.97), for products that end in nothing:
+        what runs behind it, 164 weights of 128 to 51,200 by 512 to 25,600 at 257 to 8,192 rows (K from 8,192 on and whole rounds: 160,
+        up to 16,384 rows; the mean of the ratios, and how many of them are below 0.97), for products that end in nothing:
         - K from 8,192 on: 1.32 (102 of 1,242; 5,120 x 25,600 at 4,111 rows 1.75, 8,192 x 8,192 1.48), deferred 1.27 (127), where the
           library's tiles of 256 x 256 leave more than a 16th of their rounds of the CUs empty and a single round is no fuller than
           nine 16ths.  Full rounds 0.96 (120 of 147; 4,096 x 12,288 at 8,192 and 16,384 rows 0.91 and 0.90) and single rounds of more
