@@ -3,6 +3,7 @@
 #include "common.h"
 
 constexpr int kScanStage = 16;   // tokens staged at a time
+constexpr int kScanRunTimes = 256;   // floats of scratch memory a run and head takes for its decays, where runs are matrix products
 
 struct ScanArgs {
   const float* r; long ldr; int r_div;       // head h reads r-head h / r_div, K entries each
@@ -22,7 +23,8 @@ struct ScanArgs {
   int most;                                  // the walk leaves out requests of more tokens (0: none)
   int run_len;                               // R, a multiple of kScanStage; 0: a request is one run whatever its length
   float* run_state;                          // [places, H, K, V]: B of a run after pass 1, the state before it after pass 2
-  float* run_decay;                          // [places, H, K]: the product of a run's decays
+  float* run_decay;                          // [places, H, K]: the product of a run's decays; [places, H, kScanRunTimes] where
+                                             // runs are matrix products
 };
 
 // Which request and which of its runs the block with index b works on: the last s with cu[s] / R + s <= b.

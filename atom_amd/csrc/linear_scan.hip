@@ -315,7 +315,8 @@ __global__ void __launch_bounds__(256) linear_scan_fold_kernel(ScanArgs a) {
   }
 }
 
-// shortest: a lower bound of the tokens a request brings, which says what need not be launched.
+// shortest: a lower bound of the tokens a request brings, which says what need not be launched.  run_state [places, H, K, V];
+// run_decay [places, H, K], with w_mode 2 [places, H, max(K, kScanRunTimes)].
 ATOM_EXPORT int atom_linear_scan(const float* r, long ldr, int r_div, const float* k, long ldk, int k_div, const float* v,
                                  long ldv, const float* w, long ldw, int w_per_channel, const float* w_bias, int w_mode,
                                  const float* a_log, const float* v_scale, long ldvs, const float* bonus, const float* skip, float* out,

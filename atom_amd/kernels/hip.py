@@ -1667,6 +1667,7 @@ class HipKernels:
         return ctypes.c_void_p(t.data_ptr() + t.element_size() * offset)
 
     SCAN_RUN = 64     # tokens of a run of the linear recurrences (a multiple of 16)
+    SCAN_RUN_TIMES = 256   # floats of scratch memory a run and head takes for its decays where these are formed from raw steps
 
     def linear_scan(self, r, r_off: int, r_heads: int, k, k_off: int, k_heads: int, v, v_off: int, w, w_off: int,
                     state, state_off: int, cu_seqlens_q, slot_of_seq, out, heads: int, dim: int, vdim: int,
@@ -1721,7 +1722,8 @@ class HipKernels:
             run_len = self.SCAN_RUN
             places = -(-tokens // run_len) + seqs
             run_state = torch.empty((places, heads, dim, vdim), dtype=torch.float32, device=out.device)
-            run_decay = torch.empty((places, heads, dim), dtype=torch.float32, device=out.device)
+            times = dim if a_log is None else max(dim, self.SCAN_RUN_TIMES)
+            run_decay = torch.empty((places, heads, times), dtype=torch.float32, device=out.device)
         self._done("linear_scan", self.lib.atom_linear_scan(
             self._at(r, r_off), L(r.shape[1]), heads // r_heads, self._at(k, k_off), L(k.shape[1]), heads // k_heads,
             self._at(v, v_off), L(v.shape[1]), self._at(w, w_off), L(w.shape[1]), int(bool(per_channel)), _ptr(bias),
