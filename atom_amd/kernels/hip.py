@@ -1549,9 +1549,9 @@ class HipKernels:
 
     def delta_columns(self, heads: int, vdim: int, walkers: float) -> int:
         """Value columns of a block that walks a request's chunks: two tiles of 16 where blocks of one would be more than the
-        CUs.  A chunk takes a block 2.9 us with one tile and a CU to itself, 4.9 with one tile and two blocks a CU, 4.8 with two
-        tiles: 5,569 tokens of four requests, heads of 128 x 128, 16 heads 158 us with one tile and 173 with two, 32 heads 292 and
-        258; one prompt of 2,048 tokens, 16 heads 92 and 154."""
+        CUs.  A chunk takes a block 2.6 us with one tile and a CU to itself, 4.4 with two tiles: 5,569 tokens of four requests,
+        heads of 128 x 128, 16 heads 143 us with one tile and 149 with two, 32 heads 249 and 224; one prompt of 2,048 tokens,
+        16 heads 86 and 142."""
         return 32 if vdim % 32 == 0 and heads * (vdim // 16) * walkers > self.num_cus else 16
 
     def delta_rule(self, qkv, gates, a_off: int, b_off: int, a_log, dt_bias, state, state_off: int, cu_seqlens_q,
