@@ -222,7 +222,7 @@ class HipKernels:
                    "atom_mean_of_norms", "atom_embedding_positions", "atom_unary_act", "atom_stream_add", "atom_scale_rows",
                    "atom_stream_norm", "atom_sum_norm", "atom_shift_rows", "atom_qkv_rot_write",
                    "atom_attention_together", "atom_attention_together_tiles", "atom_attention_together_tiles_supports",
-                   "atom_together_sum_parts", "atom_streams_step", "atom_embedding_sinusoid", "atom_softcap_rows",
+                   "atom_together_sum_parts", "atom_attention_together_few", "atom_attention_together_few_supports", "atom_streams_step", "atom_embedding_sinusoid", "atom_softcap_rows",
                    "atom_selective_scan", "atom_step_sizes", "atom_experts_few", "atom_experts_few_supports", "atom_keys_as_values_heads_write",
                    "atom_delta_chunks", "atom_delta_chunks_supports", "atom_delta_step", "atom_delta_step_supports",
                    "atom_rglru_step", "atom_rglru_step_supports", "atom_space_step",
@@ -268,6 +268,7 @@ class HipKernels:
         self.use_sum_norm_shift = True # single tokens: a norm's sum with the token shift behind it
         self.use_rglru_step = True     # the real-gated recurrence of single tokens in two launches
         self.use_together_tiles = True  # attention with the heads together on the matrix cores, for prompt portions
+        self.use_together_few = True    # ... and for few tokens whose keys are cut over several blocks
         self.use_mfma_latent = True     # attention over latent pages on the matrix cores (bfloat16, sizes it is built for)
         self.use_latent_tiles = True    # ... its form for a latent of 128, 256 or 512 entries and 64 rotated ones
         # routed experts: from this many (token, choice) pairs on, the pairs are sorted by expert and run as grouped
@@ -2380,6 +2381,15 @@ class HipKernels:
             parts = max(1, min(-(-2 * self.num_cus // max(sets, 1)), -(-reach // 64))) if sets < self.num_cus else 1
         ws_ml = ws_o = ws_s = None
         stride = block_tables.shape[1] * page_size
+        if (parts > 1 and self.use_together_few and dt == torch.bfloat16 and not self._unaligned(q, k_cache, v_cache)
+                and self.lib.atom_attention_together_few_supports(H, G, D, DV, page_size, int(talk is not None), int(parts))):
+            ws_ml = self.workspace("together_ml", tokens * H * parts * 2)
+            ws_o = self.workspace("together_o", tokens * parts * H * DV * (1 if talk is None else G))
+            self._done("attention_together_few", self.lib.atom_attention_together_few(
+                _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(token_seq), _ptr(positions), _ptr(block_tables),
+                block_tables.shape[1], tokens, H, G, D, DV, page_size, ctypes.c_float(scale), _ptr(head_scale), _ptr(sink),
+                _ptr(talk), int(window or 0), int(parts), _ptr(ws_ml), _ptr(ws_o), self._stream()))
+            return out
         if parts > 1:
             ws_ml = self.workspace("together_ml", tokens * H * parts * 2)
             ws_o = self.workspace("together_o", tokens * parts * H * DV)
