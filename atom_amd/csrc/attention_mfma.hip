@@ -81,8 +81,15 @@ __device__ __forceinline__ int first_visible(const AttnParams& p, int pos) {
   return max(lo, 0);
 }
 
-__device__ __forceinline__ float capped(const AttnParams& p, float s) {
-  return p.cap_out > 0.f ? p.cap_out * tanhf(s * p.cap_in) : s;
+// Raw scores bounded, where there is a bound: one branch for all of them.  (Asked score by score it was a jump for each, around a
+// tanh that nothing took, between the products and the exponentials of every tile.)
+template <int N>
+__device__ __forceinline__ void cap_scores(const AttnParams& p, f32x4 (&s)[N]) {
+  if (p.cap_out <= 0.f) return;
+#pragma unroll
+  for (int b = 0; b < N; ++b)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[b][i] = p.cap_out * tanhf(s[b][i] * p.cap_in);
 }
 
 __device__ __forceinline__ float head_slope(const AttnParams& p, int head) {
@@ -345,12 +352,17 @@ __global__ void __launch_bounds__(kWave) attention_mfma_kernel(AttnParams p) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) s[rt][i] = penalised(p, s[rt][i], slope, rel + i);
       }
+      {
+        f32x4 one[1] = {s[rt]};
+        cap_scores(p, one);
+        s[rt] = one[0];
+      }
       float sc[4];
       float mx = -INFINITY;
       if (whole) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          sc[i] = capped(p, s[rt][i]);
+          sc[i] = s[rt][i];
           mx = fmaxf(mx, sc[i]);
         }
       } else {
@@ -360,7 +372,7 @@ __global__ void __launch_bounds__(kWave) attention_mfma_kernel(AttnParams p) {
         for (int i = 0; i < 4; ++i) {
           const int key = k0 + 4 * g + i;
           const bool vis = key <= hi && key >= lo && key >= kb;
-          sc[i] = vis ? capped(p, s[rt][i]) : -INFINITY;
+          sc[i] = vis ? s[rt][i] : -INFINITY;
           mx = fmaxf(mx, sc[i]);
         }
       }
@@ -442,7 +454,7 @@ __global__ void __launch_bounds__(TOGETHER ? 8 * kWave : kWave, (D <= 128 ? 2 : 
   constexpr int AREA = 32 * KLDS;  // LDS bytes of a wave: the key rows of a step, later its result
   extern __shared__ __attribute__((aligned(16))) char decode_lds[];
   const int lane = threadIdx.x & (kWave - 1);
-  const int wave = threadIdx.x / kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   char* klds = decode_lds + wave * AREA;
   const int r16 = lane & 15;
   const int g = lane >> 4;
@@ -667,12 +679,13 @@ __global__ void __launch_bounds__(TOGETHER ? 8 * kWave : kWave, (D <= 128 ? 2 : 
 #pragma unroll
         for (int e = 0; e < 8; ++e) s[rt][e / 4][e % 4] = penalised(p, s[rt][e / 4][e % 4], slope, rel + e);
       }
+      cap_scores(p, s[rt]);
       float sc[8];
       float mx = -INFINITY;
       if (whole) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          sc[e] = capped(p, s[rt][e / 4][e % 4]);
+          sc[e] = s[rt][e / 4][e % 4];
           mx = fmaxf(mx, sc[e]);
         }
       } else {
@@ -681,7 +694,7 @@ __global__ void __launch_bounds__(TOGETHER ? 8 * kWave : kWave, (D <= 128 ? 2 : 
         for (int e = 0; e < 8; ++e) {
           const int key = k0 + 8 * g + e;
           const bool vis = key < ke && key >= lo;
-          sc[e] = vis ? capped(p, s[rt][e / 4][e % 4]) : -INFINITY;
+          sc[e] = vis ? s[rt][e / 4][e % 4] : -INFINITY;
           mx = fmaxf(mx, sc[e]);
         }
       }
@@ -907,10 +920,13 @@ static int launch_decode(const AttnParams& p, int seqs, hipStream_t stream) {
 // Needs D % 64 == 0 and page_size % 8 == 0.
 constexpr float kLazyMax = 8.f;
 
-// EXTRAS: with a penalty on distance, a gate per head or heads written narrower than D (a variant of its own, because the
-// penalty's branch costs the plain kernel a tenth of its pace).
-template <int D, int GH, int TK, int KS, int RT, bool EXTRAS>
+// WITH: PREFILL_BOUND, scores that are bounded; PREFILL_EXTRAS, those that may be, a penalty on distance, a gate per head or heads
+// written narrower than D (variants of their own, because the penalty's branch costs the plain kernel a tenth of its pace).
+enum PrefillWith : int { PREFILL_PLAIN = 0, PREFILL_BOUND = 1, PREFILL_EXTRAS = 2 };
+
+template <int D, int GH, int TK, int KS, int RT, int WITH>
 __global__ void __launch_bounds__(256 * KS, (D <= 128 && KS == 1 ? 2 : 1)) attention_prefill_tiled_kernel(AttnParams p) {
+  constexpr bool EXTRAS = WITH == PREFILL_EXTRAS;
   constexpr int KCH = D / 32;
   constexpr int DT = D / 16;
   constexpr int ROWS = 16 * RT;          // query tokens of a wave: 32, or 16 where a launch of 32 would leave CUs idle
@@ -929,12 +945,13 @@ __global__ void __launch_bounds__(256 * KS, (D <= 128 && KS == 1 ? 2 : 1)) atten
   constexpr int NS = RT * DT * 4 + 2 * RT;           // floats a lane hands over when the halves are added
   constexpr int SMEM_TILES = KS * TILE_ELEMS * 2, SMEM_SUMS = KS > 1 ? 4 * NS * kWave * 4 : 0;
   __shared__ __attribute__((aligned(16))) char smem[SMEM_TILES > SMEM_SUMS ? SMEM_TILES : SMEM_SUMS];
-  const int part = threadIdx.x / 256;    // which half of the key tiles (always 0 with KS = 1)
+  // (the same in a wave's lanes: branches on it and on the wave's rows are scalar ones)
+  const int part = KS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / 256) : 0;   // which half of the key tiles
   const int tid = threadIdx.x % 256;
   bf16_t* const ks = reinterpret_cast<bf16_t*>(smem) + part * TILE_ELEMS;
   bf16_t* const vs = ks + TK * KSTR;
   const int lane = tid & (kWave - 1);
-  const int wave = tid / kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int r16 = lane & 15;
   const int g = lane >> 4;
   const int group = p.hq / p.hkv;
@@ -1153,6 +1170,7 @@ __global__ void __launch_bounds__(256 * KS, (D <= 128 && KS == 1 ? 2 : 1)) atten
             for (int i = 0; i < 4; ++i) s[rt][b][i] = penalised(p, s[rt][b][i], slope, rel + (16 * b + i));
         }
       }
+      if constexpr (WITH != PREFILL_PLAIN) cap_scores(p, s[rt]);
       float sc[4 * KB];
       float mx = -INFINITY;
       if (whole) {
@@ -1160,7 +1178,7 @@ __global__ void __launch_bounds__(256 * KS, (D <= 128 && KS == 1 ? 2 : 1)) atten
         for (int b = 0; b < KB; ++b)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            sc[4 * b + i] = capped(p, s[rt][b][i]);
+            sc[4 * b + i] = s[rt][b][i];
             mx = fmaxf(mx, sc[4 * b + i]);
           }
       } else {
@@ -1173,7 +1191,7 @@ __global__ void __launch_bounds__(256 * KS, (D <= 128 && KS == 1 ? 2 : 1)) atten
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const bool vis = 16 * b + i <= hi && 16 * b + i >= lo;
-            sc[4 * b + i] = vis ? capped(p, s[rt][b][i]) : -INFINITY;
+            sc[4 * b + i] = vis ? s[rt][b][i] : -INFINITY;
             mx = fmaxf(mx, sc[4 * b + i]);
           }
       }
@@ -1287,7 +1305,7 @@ ATOM_EXPORT int atom_attention_prefill_tile_rows(int d, int page_size, int group
   return 32 * (4 / gh);
 }
 
-template <int D, bool EXTRAS>
+template <int D, int WITH>
 static int launch_prefill_tiled_as(const AttnParams& p, int num_tiles, int rows_per_tile, bool halves, bool low,
                                 hipStream_t stream) {
   const int group = p.hq / p.hkv;
@@ -1300,22 +1318,22 @@ static int launch_prefill_tiled_as(const AttnParams& p, int num_tiles, int rows_
     if (halves && low) {   // ... and 16 tokens a wave: two blocks for every entry of the list
       block = dim3(512);
       grid = dim3(2 * num_tiles * (p.hq / gh), 1);
-      if (gh == 4) hipLaunchKernelGGL((attention_prefill_tiled_kernel<D, 4, TK, 2, 1, EXTRAS>), grid, block, 0, stream, p);
-      else if (gh == 2) hipLaunchKernelGGL((attention_prefill_tiled_kernel<D, 2, TK, 2, 1, EXTRAS>), grid, block, 0, stream, p);
-      else hipLaunchKernelGGL((attention_prefill_tiled_kernel<D, 1, TK, 2, 1, EXTRAS>), grid, block, 0, stream, p);
+      if (gh == 4) hipLaunchKernelGGL((attention_prefill_tiled_kernel<D, 4, TK, 2, 1, WITH>), grid, block, 0, stream, p);
+      else if (gh == 2) hipLaunchKernelGGL((attention_prefill_tiled_kernel<D, 2, TK, 2, 1, WITH>), grid, block, 0, stream, p);
+      else hipLaunchKernelGGL((attention_prefill_tiled_kernel<D, 1, TK, 2, 1, WITH>), grid, block, 0, stream, p);
       return launch_status();
     }
     if (halves) {   // eight waves a block, the key tiles taken in turn by its two halves
       block = dim3(512);
-      if (gh == 4) hipLaunchKernelGGL((attention_prefill_tiled_kernel<D, 4, TK, 2, 2, EXTRAS>), grid, block, 0, stream, p);
-      else if (gh == 2) hipLaunchKernelGGL((attention_prefill_tiled_kernel<D, 2, TK, 2, 2, EXTRAS>), grid, block, 0, stream, p);
-      else hipLaunchKernelGGL((attention_prefill_tiled_kernel<D, 1, TK, 2, 2, EXTRAS>), grid, block, 0, stream, p);
+      if (gh == 4) hipLaunchKernelGGL((attention_prefill_tiled_kernel<D, 4, TK, 2, 2, WITH>), grid, block, 0, stream, p);
+      else if (gh == 2) hipLaunchKernelGGL((attention_prefill_tiled_kernel<D, 2, TK, 2, 2, WITH>), grid, block, 0, stream, p);
+      else hipLaunchKernelGGL((attention_prefill_tiled_kernel<D, 1, TK, 2, 2, WITH>), grid, block, 0, stream, p);
       return launch_status();
     }
   }
-  if (gh == 4) hipLaunchKernelGGL((attention_prefill_tiled_kernel<D, 4, TK, 1, 2, EXTRAS>), grid, block, 0, stream, p);
-  else if (gh == 2) hipLaunchKernelGGL((attention_prefill_tiled_kernel<D, 2, TK, 1, 2, EXTRAS>), grid, block, 0, stream, p);
-  else hipLaunchKernelGGL((attention_prefill_tiled_kernel<D, 1, TK, 1, 2, EXTRAS>), grid, block, 0, stream, p);
+  if (gh == 4) hipLaunchKernelGGL((attention_prefill_tiled_kernel<D, 4, TK, 1, 2, WITH>), grid, block, 0, stream, p);
+  else if (gh == 2) hipLaunchKernelGGL((attention_prefill_tiled_kernel<D, 2, TK, 1, 2, WITH>), grid, block, 0, stream, p);
+  else hipLaunchKernelGGL((attention_prefill_tiled_kernel<D, 1, TK, 1, 2, WITH>), grid, block, 0, stream, p);
   return launch_status();
 }
 
@@ -1323,8 +1341,9 @@ template <int D>
 static int launch_prefill_tiled(const AttnParams& p, int num_tiles, int rows_per_tile, bool halves, bool low,
                                 hipStream_t stream) {
   if (p.slopes != nullptr || p.gate != nullptr || p.od != D)
-    return launch_prefill_tiled_as<D, true>(p, num_tiles, rows_per_tile, halves, low, stream);
-  return launch_prefill_tiled_as<D, false>(p, num_tiles, rows_per_tile, halves, low, stream);
+    return launch_prefill_tiled_as<D, PREFILL_EXTRAS>(p, num_tiles, rows_per_tile, halves, low, stream);
+  if (p.cap_out > 0.f) return launch_prefill_tiled_as<D, PREFILL_BOUND>(p, num_tiles, rows_per_tile, halves, low, stream);
+  return launch_prefill_tiled_as<D, PREFILL_PLAIN>(p, num_tiles, rows_per_tile, halves, low, stream);
 }
 
 template <int D>
