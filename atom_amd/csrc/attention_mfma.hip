@@ -903,9 +903,11 @@ static int launch_decode(const AttnParams& p, int seqs, hipStream_t stream) {
 // A block of four waves owns a tile of query tokens of GH query heads that share a KV head
 // (GH = 4, 2 or 1, a divisor of the group size): wave w has head (w % GH) and the 32 tokens
 // number (w / GH) of the tile, so a block covers 32 * 4 / GH tokens.  Keys are walked TK (64 or 32) at a
-// time; the block loads each K tile (TK keys x D) and V^T tile (D x TK keys) once, through
-// registers (the next tile's loads are in flight while this one is multiplied) into LDS, where all
-// four waves read them as matrix-core operands.  Products, softmax and layouts are those of the
+// time; the block loads each K tile (TK keys x D) and V^T tile (D x TK keys) once, through registers into one of two
+// LDS buffers, where all four waves read them as matrix-core operands.  While a tile's scores are formed the next one
+// goes from registers to the other buffer and the loads of the one after it go out, a piece between two products: put
+// between two barriers of their own they were a third of a tile's time (4,900 cycles, 1,060 of them address arithmetic
+// and the issue of loads, 720 the stores and barriers).  Products, softmax and layouts are those of the
 // kernel above, with both products on v_mfma_f32_16x16x32_bf16: 32 keys of a tile are the k
 // dimension of one step of the second product, in the order (4 g + i, 16 + 4 g + i) that the first product
 // leaves them in a lane.
@@ -920,8 +922,8 @@ static int launch_decode(const AttnParams& p, int seqs, hipStream_t stream) {
 // Needs D % 64 == 0 and page_size % 8 == 0.
 constexpr float kLazyMax = 8.f;
 
-// WITH: PREFILL_BOUND, scores that are bounded; PREFILL_EXTRAS, those that may be, a penalty on distance, a gate per head or heads
-// written narrower than D (variants of their own, because the penalty's branch costs the plain kernel a tenth of its pace).
+// WITH: PREFILL_BOUND, scores that are bounded; PREFILL_EXTRAS, those that may be, a penalty on distance, a gate per head, heads
+// written narrower than D or pages whose size is no power of two (variants of their own, because the penalty's branch costs the plain kernel a tenth of its pace).
 enum PrefillWith : int { PREFILL_PLAIN = 0, PREFILL_BOUND = 1, PREFILL_EXTRAS = 2 };
 
 template <int D, int GH, int TK, int KS, int RT, int WITH>
@@ -944,12 +946,11 @@ __global__ void __launch_bounds__(256 * KS, (D <= 128 && KS == 1 ? 2 : 1)) atten
   constexpr int TILE_ELEMS = TK * KSTR + D * VSTR;   // a K tile and a V^T tile
   constexpr int NS = RT * DT * 4 + 2 * RT;           // floats a lane hands over when the halves are added
   constexpr int SMEM_TILES = KS * TILE_ELEMS * 2, SMEM_SUMS = KS > 1 ? 4 * NS * kWave * 4 : 0;
-  __shared__ __attribute__((aligned(16))) char smem[SMEM_TILES > SMEM_SUMS ? SMEM_TILES : SMEM_SUMS];
+  __shared__ __attribute__((aligned(16))) char smem[2 * SMEM_TILES > SMEM_SUMS ? 2 * SMEM_TILES : SMEM_SUMS];
   // (the same in a wave's lanes: branches on it and on the wave's rows are scalar ones)
   const int part = KS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / 256) : 0;   // which half of the key tiles
   const int tid = threadIdx.x % 256;
-  bf16_t* const ks = reinterpret_cast<bf16_t*>(smem) + part * TILE_ELEMS;
-  bf16_t* const vs = ks + TK * KSTR;
+  bf16_t* const tiles_lds = reinterpret_cast<bf16_t*>(smem) + part * (2 * TILE_ELEMS);   // two buffers: K rows, then V^T rows
   const int lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int r16 = lane & 15;
@@ -1047,76 +1048,98 @@ __global__ void __launch_bounds__(256 * KS, (D <= 128 && KS == 1 ? 2 : 1)) atten
   bf16x8 kreg[PT], vreg[PT];
   const uint32_t page_elems = (uint32_t)p.hkv * ps * D;    // elements of a page, all heads
   const int k_head = kvh * ps * D, v_head = kvh * D * ps;  // this KV head's part of a key page and of a value page
-  // The pages of a tile are looked up a tile before its loads go out (`pages_of`), so that no load waits for a
-  // table entry; a thread's pieces of V^T all lie in one page (256 is a multiple of the pieces per row).
+  // The pages of a tile are looked up a tile before its loads go out, so that no load waits for a table entry; a
+  // thread's pieces of V^T all lie in one page (256 is a multiple of the pieces per row).  Tiles behind the last key are
+  // read as that key, and used by nobody: there is no branch around a load.
   static_assert(256 % (TK / 8) == 0, "a thread's V^T pieces must share their keys");
   int kpage[PT], vpage = 0;
-  auto pages_of_as = [&](int k0, auto kind) {
-    const PageMath<decltype(kind)::value> pages{ps, p.page_shift};
-#pragma unroll
-    for (int j = 0; j < PT; ++j) {
-      const int key = min(k0 + (tid + 256 * j) / (D / 8), ke - 1);
-      kpage[j] = table[pages.index(key)];
+  const auto by_pages = [&](auto&& body) {   // sizes that are no power of two take the variant with everything
+    if constexpr (EXTRAS) {
+      if (p.page_shift < 0) {
+        body(PageMath<AnyPages::value>{ps, p.page_shift});
+        return;
+      }
     }
-    const int vkey = min(k0 + (tid % (TK / 8)) * 8, (ke - 1) & ~7);
-    vpage = table[pages.index(vkey)];
+    body(PageMath<Pow2Pages::value>{ps, p.page_shift});
   };
-  auto pages_of = [&](int k0) {
-    if (p.page_shift >= 0) pages_of_as(k0, Pow2Pages{});
-    else pages_of_as(k0, AnyPages{});
-  };
-  auto load_tile_as = [&](int k0, auto kind) {
-    const PageMath<decltype(kind)::value> pages{ps, p.page_shift};
-    const int vkey = min(k0 + (tid % (TK / 8)) * 8, (ke - 1) & ~7);
-    const bf16_t* vbase = p.v_cache + (uint64_t)(uint32_t)vpage * page_elems + (v_head + pages.within(vkey));
-#pragma unroll
-    for (int j = 0; j < PT; ++j) {
-      const int q = tid + 256 * j;
-      const int key = min(k0 + q / (D / 8), ke - 1);
+  const auto k_key = [&](int k0, int j) { return min(k0 + (tid + 256 * j) / (D / 8), ke - 1); };
+  const auto v_key = [&](int k0) { return min(k0 + (tid % (TK / 8)) * 8, (ke - 1) & ~7); };
+  auto look_k = [&](int k0, int j) { by_pages([&](const auto& pages) { kpage[j] = table[pages.index(k_key(k0, j))]; }); };
+  auto look_v = [&](int k0) { by_pages([&](const auto& pages) { vpage = table[pages.index(v_key(k0))]; }); };
+  auto load_k = [&](int k0, int j) {
+    by_pages([&](const auto& pages) {
       kreg[j] = *reinterpret_cast<const bf16x8*>(p.k_cache + (uint64_t)(uint32_t)kpage[j] * page_elems +
-                                                 (k_head + pages.within(key) * D + (q % (D / 8)) * 8));
-      vreg[j] = *reinterpret_cast<const bf16x8*>(vbase + (q / (TK / 8)) * ps);
-    }
+                                                 (k_head + pages.within(k_key(k0, j)) * D + ((tid + 256 * j) % (D / 8)) * 8));
+    });
   };
-  auto load_tile = [&](int k0) {
-    if (p.page_shift >= 0) load_tile_as(k0, Pow2Pages{});
-    else load_tile_as(k0, AnyPages{});
+  auto load_v = [&](int k0, int j) {
+    by_pages([&](const auto& pages) {
+      vreg[j] = *reinterpret_cast<const bf16x8*>(p.v_cache + (uint64_t)(uint32_t)vpage * page_elems +
+                                                 (v_head + pages.within(v_key(k0)) + ((tid + 256 * j) / (TK / 8)) * ps));
+    });
   };
-  auto store_tile = [&]() {
-#pragma unroll
-    for (int j = 0; j < PT; ++j) {
-      const int q = tid + 256 * j;
-      *reinterpret_cast<bf16x8*>(ks + (q / (D / 8)) * KSTR + (q % (D / 8)) * 8) = kreg[j];
-      // Within every 32 keys of a V^T row the keys are laid in the order in which the second product
-      // takes them: lane group g holds keys 4 g .. 4 g + 3 and 16 + 4 g .. 16 + 4 g + 3 (what the first
-      // product left it), so these eight lie together at 8 g: key c goes to 8 ((c % 16) / 4) + 4 (c / 16) + c % 4.
-      const bf16x4 lo = {vreg[j][0], vreg[j][1], vreg[j][2], vreg[j][3]};
-      const bf16x4 hi = {vreg[j][4], vreg[j][5], vreg[j][6], vreg[j][7]};
-      const int c0 = (q % (TK / 8)) * 8;              // first key of the piece within the tile
-      const int in32 = c0 % 32;
-      const int at_lo = 8 * ((in32 % 16) / 4) + 4 * (in32 / 16);
-      bf16_t* dst = vs + (q / (TK / 8)) * VSTR + (c0 - in32);
-      *reinterpret_cast<bf16x4*>(dst + at_lo) = lo;
-      *reinterpret_cast<bf16x4*>(dst + at_lo + 8) = hi;   // keys c0 + 4 ..: the next lane group
-    }
+  auto store_k = [&](bf16_t* ks, int j) {
+    const int q = tid + 256 * j;
+    *reinterpret_cast<bf16x8*>(ks + (q / (D / 8)) * KSTR + (q % (D / 8)) * 8) = kreg[j];
+  };
+  auto store_v = [&](bf16_t* vs, int j) {
+    const int q = tid + 256 * j;
+    // Within every 32 keys of a V^T row the keys are laid in the order in which the second product
+    // takes them: lane group g holds keys 4 g .. 4 g + 3 and 16 + 4 g .. 16 + 4 g + 3 (what the first
+    // product left it), so these eight lie together at 8 g: key c goes to 8 ((c % 16) / 4) + 4 (c / 16) + c % 4.
+    const bf16x4 lo = {vreg[j][0], vreg[j][1], vreg[j][2], vreg[j][3]};
+    const bf16x4 hi = {vreg[j][4], vreg[j][5], vreg[j][6], vreg[j][7]};
+    const int c0 = (q % (TK / 8)) * 8;              // first key of the piece within the tile
+    const int in32 = c0 % 32;
+    const int at_lo = 8 * ((in32 % 16) / 4) + 4 * (in32 / 16);
+    bf16_t* dst = vs + (q / (TK / 8)) * VSTR + (c0 - in32);
+    *reinterpret_cast<bf16x4*>(dst + at_lo) = lo;
+    *reinterpret_cast<bf16x4*>(dst + at_lo + 8) = hi;   // keys c0 + 4 ..: the next lane group
   };
 
   constexpr int STEP = KS * TK;          // keys the block walks at a time
-  if (kb + part * TK < ke) {
-    pages_of(kb + part * TK);
-    load_tile(kb + part * TK);
-    if (kb + part * TK + STEP < ke) pages_of(kb + part * TK + STEP);
-  }
-  for (int kk = kb; kk < ke; kk += STEP) {
-    const int k0 = kk + part * TK;       // this half's tile
-    __syncthreads();   // the previous tile has been read by every wave
-    if (k0 < ke) store_tile();
-    __syncthreads();
-    if (k0 + STEP < ke) {
-      load_tile(k0 + STEP);
-      if (k0 + 2 * STEP < ke) pages_of(k0 + 2 * STEP);
+  // One piece of moving tiles on: the tile in the registers to the buffer, the loads of the tile at `load`, look-ups for `look`.
+  constexpr int PIECES = 2 * PT + 1;
+  auto move_on = [&](int i, bf16_t* buffer, int load, int look) {
+    if (i < 2 * PT && i % 2 == 0) {
+      store_k(buffer, i / 2);
+      load_k(load, i / 2);
+      look_k(look, i / 2);
+    } else if (i < 2 * PT) {
+      store_v(buffer + TK * KSTR, i / 2);
+      load_v(load, i / 2);
+    } else if (i == 2 * PT) {
+      look_v(look);
     }
-    if (nrows == 0 || k0 >= my_ke) continue;   // the whole wave: nothing of this tile is visible to it
+  };
+  {
+    const int k0 = kb + part * TK;
+#pragma unroll
+    for (int j = 0; j < PT; ++j) look_k(k0, j);
+    look_v(k0);
+#pragma unroll
+    for (int j = 0; j < PT; ++j) {
+      load_k(k0, j);
+      load_v(k0, j);
+    }
+#pragma unroll
+    for (int j = 0; j < PT; ++j) look_k(k0 + STEP, j);
+    look_v(k0 + STEP);
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) move_on(i, tiles_lds, k0 + STEP, k0 + 2 * STEP);
+  }
+  int buffer = 0;
+  for (int kk = kb; kk < ke; kk += STEP, buffer ^= TILE_ELEMS) {
+    const int k0 = kk + part * TK;       // this half's tile
+    __syncthreads();   // this tile is there, and the one before it has been read by every wave
+    const bf16_t* const ks = tiles_lds + buffer;
+    const bf16_t* const vs = ks + TK * KSTR;
+    bf16_t* const other = tiles_lds + (buffer ^ TILE_ELEMS);
+    if (nrows == 0 || k0 >= my_ke) {     // the whole wave: nothing of this tile is visible to it
+#pragma unroll
+      for (int i = 0; i < PIECES; ++i) move_on(i, other, k0 + 2 * STEP, k0 + 3 * STEP);
+      continue;
+    }
 
     // ---- S^T for the blocks of 16 keys
     f32x4 s[RT][KB];
@@ -1143,7 +1166,9 @@ __global__ void __launch_bounds__(256 * KS, (D <= 128 && KS == 1 ? 2 : 1)) atten
         for (int rt = 0; rt < RT; ++rt)
           s[rt][i % KB] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, q32[rt][i / KB], s[rt][i % KB], 0, 0, 0);
         if (i + AHEAD < NQK) kf[i % AHEAD] = k_operand(i + AHEAD);
+        move_on(i, other, k0 + 2 * STEP, k0 + 3 * STEP);
       }
+      static_assert(PIECES <= NQK);
       __builtin_amdgcn_sched_barrier(0);
     }
     constexpr int NPV = (KB / 2) * DT;
@@ -1294,6 +1319,7 @@ __global__ void __launch_bounds__(256 * KS, (D <= 128 && KS == 1 ? 2 : 1)) atten
 #pragma unroll
     for (int t = 0; t < DT; ++t) store_head(dst, 16 * t + 4 * g, acc[rt][t], inv, od);
   }
+  if (KS == 1 && !TWO) __syncthreads();   // the next tile's keys take the place of this one's last
   }   // the two tiles of the block
 }
 
@@ -1340,7 +1366,7 @@ static int launch_prefill_tiled_as(const AttnParams& p, int num_tiles, int rows_
 template <int D>
 static int launch_prefill_tiled(const AttnParams& p, int num_tiles, int rows_per_tile, bool halves, bool low,
                                 hipStream_t stream) {
-  if (p.slopes != nullptr || p.gate != nullptr || p.od != D)
+  if (p.slopes != nullptr || p.gate != nullptr || p.od != D || p.page_shift < 0)
     return launch_prefill_tiled_as<D, PREFILL_EXTRAS>(p, num_tiles, rows_per_tile, halves, low, stream);
   if (p.cap_out > 0.f) return launch_prefill_tiled_as<D, PREFILL_BOUND>(p, num_tiles, rows_per_tile, halves, low, stream);
   return launch_prefill_tiled_as<D, PREFILL_PLAIN>(p, num_tiles, rows_per_tile, halves, low, stream);
