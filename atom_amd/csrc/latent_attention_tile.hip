@@ -148,19 +148,20 @@ __global__ void __launch_bounds__(64 * NW, 2) latent_tile_kernel(LatentTileParam
   // keys that no row of the tile sees are read as the nearest that one does
   auto readable = [&](int key) { return key > last_pos ? last_pos : key < first_key ? first_key : key; };
   auto cache_row = [&](int key) { return table[readable(key) / p.page_size] * p.page_size + readable(key) % p.page_size; };
-  auto stage = [&](int buffer) {
-    int row = (wave * 64 + lane) / U, col = (wave * 64 + lane) % U;
-    const int* mine = slots + buffer * kTChunk;
-    for (int n = wave; n < U; n += NW) {
-      const int piece = col < KS * 4 ? col : 0;   // the two pieces of padding: anything that is there to read
-      load_to_lds(p.pages + (size_t)mine[row] * kWidth + piece * 8, lds0 + (unsigned)(buffer * kTChunk * kPitch + n * 1024));
-      row += 64 * NW / U;
-      col += 64 * NW % U;
-      if (col >= U) {
-        col -= U;
-        ++row;
-      }
-    }
+  // What a wave brings of a chunk: pieces wave, wave + NW, ... of 64 times 16 bytes.  Which row of the chunk and which 16 bytes of
+  // it a lane has in each does not change from chunk to chunk.
+  constexpr int NP = (U + NW - 1) / NW;
+  unsigned place[NP];                    // row | offset in bytes << 8
+#pragma unroll
+  for (int n = 0; n < NP; ++n) {
+    const int at = (wave + n * NW) * 64 + lane, col = at % U;
+    place[n] = (unsigned)min(at / U, kTChunk - 1) | (unsigned)(col < KS * 4 ? col : 0) << 12;   // (padding: anything that is there to read)
+  }
+  const auto slot_of = [&](int buffer, int n) { return slots[buffer * kTChunk + (place[n] & 255)]; };
+  const auto bring = [&](int buffer, int n, int row) {
+    if ((n + 1) * NW <= U || wave + n * NW < U)
+      load_to_lds(reinterpret_cast<const unsigned char*>(p.pages) + ((size_t)row * (kWidth * 2) + (place[n] >> 8)),
+                  lds0 + (unsigned)(buffer * kTChunk * kPitch + (wave + n * NW) * 1024));
   };
 
   if (my_lo < my_hi) {
@@ -169,7 +170,8 @@ __global__ void __launch_bounds__(64 * NW, 2) latent_tile_kernel(LatentTileParam
       slots[kTChunk + tid] = cache_row((my_lo + 1) * kTChunk + tid);
     }
     __syncthreads();
-    stage(0);
+#pragma unroll
+    for (int n = 0; n < NP; ++n) bring(0, n, slot_of(0, n));
   }
 
   for (int c = my_lo; c < my_hi; ++c) {
@@ -177,11 +179,12 @@ __global__ void __launch_bounds__(64 * NW, 2) latent_tile_kernel(LatentTileParam
     const int kbase = c * kTChunk;
     arrived();
     lds_barrier();
-    if (c + 1 < my_hi) stage(cur ^ 1);
-    // the page of one key of the chunk after the next, for `slots`: asked for here, by all lanes (no branch may end
-    // behind it), and first touched when everything has arrived
-    const int key2 = readable((c + 2) * kTChunk + lane);
-    int page2 = table[key2 / p.page_size];
+    // The next chunk is asked for a few pieces at a time between the groups of products: a lump of loads before them, each
+    // behind its row's look-up, leaves the matrix cores idle meanwhile.
+    const bool more = c + 1 < my_hi;
+    int row_of[NP];
+#pragma unroll
+    for (int n = 0; n < NP; ++n) row_of[n] = slot_of(cur ^ 1, n);
     const unsigned char* klds = lds + cur * kTChunk * kPitch;
 
     f32x4 s[KT][RS];
@@ -206,6 +209,10 @@ __global__ void __launch_bounds__(64 * NW, 2) latent_tile_kernel(LatentTileParam
       for (int group = 0; group < KS / G; ++group) {
         if (group + 1 < KS / G) read(group + 1, a[(group + 1) & 1]);
         __builtin_amdgcn_sched_barrier(0);
+        constexpr int PER = (NP + KS / G - 1) / (KS / G);
+#pragma unroll
+        for (int n = group * PER; n < (group + 1) * PER && n < NP; ++n)
+          if (more) bring(cur ^ 1, n, row_of[n]);
 #pragma unroll
         for (int j = 0; j < G; ++j)
 #pragma unroll
@@ -277,6 +284,10 @@ __global__ void __launch_bounds__(64 * NW, 2) latent_tile_kernel(LatentTileParam
       }
       l_run[i] = l_run[i] * a + sum;
     }
+    // the page of one key of the chunk after the next, for `slots`: asked for here, by all lanes (no branch may end
+    // behind it), and first touched when everything has arrived
+    const int key2 = readable((c + 2) * kTChunk + lane);
+    int page2 = table[key2 / p.page_size];
     lds_barrier();
     const unsigned char* vp = klds + (8 * g + r / 4) * kPitch + (wave * CT * 16 + 4 * (r % 4)) * 2;
     bf16x8 v[2];
