@@ -705,11 +705,11 @@ class HipKernels:
         """Whether the prefill kernel with shared key tiles runs blocks of eight waves (one a CU, the key tiles taken
         in turn by the block's halves) rather than of four (two a CU, each on its own).  Measured on an MI355X with
         32 / 8 heads of 128: two blocks of four waves keep each other's SIMDs busy as long as both run, so they win
-        when a CU has a queue of them (8,192 fresh tokens: 640 against 690 us) or when all blocks are about as long
-        (2,048 tokens behind 8,192 cached: 355 against 390 us); a block of eight waves does not depend on a
-        neighbour, and wins when there is none (a portion of 512 tokens behind 3,072 cached, 128 blocks: 74 against
-        99 us) or when the long blocks of a fresh prompt outlive their short neighbours (2,048 tokens: 64 against
-        72 us)."""
+        when a CU has a queue of them (3,072 fresh tokens: 113 against 117 us; 8,192: 665 with both) or when all blocks
+        are about as long (2,048 tokens behind 8,192 cached: 328 against 342 us); a block of eight waves does not depend
+        on a neighbour, and wins when there is none (1,024 tokens behind 2,048 cached, 256 blocks: 67 against 81 us) or
+        when the long blocks of a fresh prompt outlive their short neighbours (1,536 / 2,048 tokens: 40 / 58 against
+        46 / 59 us)."""
         if self.prefill_key_halves is not None:
             return bool(self.prefill_key_halves)
         if blocks <= self.num_cus:
@@ -719,9 +719,9 @@ class HipKernels:
     def _prefill_low_blocks(self, blocks: int, head_dim: int, meta) -> bool:
         """Whether the blocks of eight waves take 16 query tokens a wave instead of 32 (twice the blocks, each with
         half the products per key tile it stages): when the launch would otherwise leave half of the CUs without a
-        block (512 tokens behind 3,072 cached: 65 against 78 us), and for fresh prompts of up to a block a CU, whose
-        blocks are mostly short (549 / 768 / 1,024 tokens: 16 / 20 / 29 against 21 / 24 / 30 us; behind 2,048 cached
-        tokens the same launches take 82-90 against 62-68 us, so those keep 32 tokens a wave)."""
+        block (512 tokens behind 3,072 cached: 55 against 72 us), and for fresh prompts of up to a block a CU, whose
+        blocks are mostly short (549 / 768 / 1,024 tokens: 16 / 22 / 28 against 22 / 23 / 29 us; behind 2,048 cached
+        tokens the same launches take 68-80 against 56-67 us, so those keep 32 tokens a wave)."""
         if self.prefill_low_blocks is not None:
             return bool(self.prefill_low_blocks) and head_dim <= 128
         if head_dim > 128:
